@@ -52,6 +52,11 @@ def gemm_flops(batch, filters, n_layers):
     return 2.0 * 36 * 25 * batch * filters * (18 + (n_layers - 1) * filters)
 
 
+def conv_flops(batch, filters, n_layers):
+    """The same layers as direct 3x3 convolutions: 2 * 9 * 361 * batch * F * (18 + (L-1)*F)."""
+    return 2.0 * 9 * 361 * batch * filters * (18 + (n_layers - 1) * filters)
+
+
 def transform_bytes(batch, filters, n_layers, e):
     """Algorithmic HBM bytes per forward of the three transform kernel classes:
     external inputs + outputs of each launch, nothing counted twice.
@@ -209,11 +214,9 @@ def netbench_workload(args, pkg, netgen):
 
 def gemm_kernel_name(fp16, Fp, B):
     """The GEMM kernel the library launches for this precision, padded width and batch."""
-    if fp16 and Fp in (128, 192, 256):
-        return "wino_gemm_stream_k"
     if not fp16 and Fp in (128, 256):
-        return "wino_gemm_stream32_k"
-    return "wino_gemm_k / wino_gemm_big_k family"
+        return "wino_gemm_stream32_k (36-way batched Winograd GEMM)"
+    return "wino_gemm_k / wino_gemm_big_k family (36-way batched Winograd GEMM)"
 
 
 def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, lanes_arg,
@@ -350,17 +353,22 @@ def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, 
             ms2 += m
         ms2 /= profile_reps
     e = 2 if prec == pkg.FP16 else 4
-    gf = gemm_flops(B, F, nl)
+    # towers of direct convolutions have no transforms; their one kernel class is timed as "gemm"
+    direct = cnt[pkg.K_IN] == 0
+    gf = conv_flops(B, F, nl) if direct else gemm_flops(B, F, nl)
     in_b, out_b, fused_b = transform_bytes(B, F, nl, e)
     peak = PEAK_MFMA_F16 if prec == pkg.FP16 else PEAK_MFMA_F32
     gemm_rate = gf / (ms[pkg.K_GEMM] * 1e-3)
     Fp = (F + 63) // 64 * 64
     roofline = {
-        "kernel": gemm_kernel_name(prec == pkg.FP16, Fp, B) + " (36-way batched Winograd GEMM)",
+        "kernel": ("conv3x3_k (direct convolution + batch norm + skip + ReLU)" if direct
+                   else gemm_kernel_name(prec == pkg.FP16, Fp, B)),
         "bound": "mfma", "achieved": gemm_rate / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
         "frac": gemm_rate / peak,
-        "traffic": measured_gemm_traffic(blocks, F, precision, B),
-        "algorithmic_bytes_per_launch": 36.0 * e * (25 * B * F * 2 + F * F),
+        "traffic": None if direct else measured_gemm_traffic(blocks, F, precision, B),
+        # planes in and out and filters of a tower layer (V, M and U of a Winograd one)
+        "algorithmic_bytes_per_launch": (e * (361.0 * B * F * 2 + 9 * F * F) if direct
+                                         else 36.0 * e * (25 * B * F * 2 + F * F)),
         "avg_launch_us": ms[pkg.K_GEMM] * 1e3 / cnt[pkg.K_GEMM],
         "launches_per_forward": int(cnt[pkg.K_GEMM]),
         "flops_per_launch": gf / cnt[pkg.K_GEMM],

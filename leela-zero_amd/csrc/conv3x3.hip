@@ -1,0 +1,510 @@
+// Direct 3x3 convolution for fp16 towers on the matrix cores (gfx950): one kernel per layer,
+// convolution + batch norm + skip connection + ReLU, channels-last activations in and out.
+//
+// Why direct and not Winograd in fp16: F(4x4,3x3) needs 3.6 times fewer products, but as
+// separate kernels it moves V and M (2 x 36/16 of a layer's planes) through memory in both
+// directions, and at 256 filters that traffic, not the matrix pipe, is what a layer takes.
+// As an implicit GEMM a layer reads its planes once and its filters once per die, and the
+// fp16 matrix rate is high enough (v_mfma_f32_16x16x32_f16, fp32 accumulate) to do the
+// whole sum.  Measured per layer of a chain of dependent 256-filter layers, Winograd GEMM +
+// fused transform -> this kernel: 64 boards 26.5 -> 22.7 us one forward at a time, 24.2 -> 17.7
+// with two side by side; 200 boards 83 -> 54 (1.57 PFLOP/s; two side by side 1.71; torch.mm of
+// 8192 x 8192 fp16 matrices reached 1.33 on that card); 16 boards 12.8 -> 10.2; 1 board 9.2 -> 6.6.
+// It also rounds less: planes and 3x3 filters are the only values kept in half precision.
+#include <cmath>
+#include <stdexcept>
+
+#include "kernel_util.h"
+
+namespace lzhip {
+
+typedef int int2v __attribute__((ext_vector_type(2)));
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+
+// ---------------------------------------------------------------------------
+// Geometry.  Row m of the implicit GEMM is point (b, y, x) of the batch.  In LDS the planes
+// stand with a zero border: cell q(m) = 400 b + 20 (y + 1) + x, one zero column between board
+// rows (right border of one row and left border of the next) and one zero row between
+// boards.  A tap (r, s) is then the constant offset 20 (r - 1) + (s - 1), without bounds logic.
+constexpr int kCellsPerBoard = 400;
+// Cells that a tile of mt consecutive rows can reach: its own span (a cell more per board
+// row ended, 20 more per board ended) and 21 on either side.
+constexpr int conv_cells(int mt) {
+    return mt - 1 + (mt - 1 + 18) / 19 + 20 * ((mt - 1 + 360) / 361) + 43;
+}
+__device__ __forceinline__ unsigned conv_cell(unsigned m) {
+    const unsigned b = m / kPts, p = m - b * kPts, y = p / kBoard, x = p - y * kBoard;
+    return b * kCellsPerBoard + (y + 1) * 20 + x;
+}
+
+// Filters: [k-step][Kp / 16][64 lanes][8], k-step = (chunk of 64 input channels, tap, half of
+// the chunk), i.e. the matrix instruction's row operand in the order it is used; every load of
+// a wavefront is one contiguous KiB.  Lane l of block kb holds output channel
+// conv_channel(kb, l % 16), input channels 32 (half) + 8 (l / 16) + 0..7 of the chunk.
+// Register r of lane l of the result is row 4 (l / 16) + r of the row operand; with this order of
+// the channels the registers of two neighbouring blocks are 8 consecutive channels, and a
+// store instruction of a wavefront writes 64 contiguous bytes per point.
+__host__ __device__ constexpr int conv_channel(int kb, int i) {
+    return 32 * (kb >> 1) + 8 * (i >> 2) + 4 * (kb & 1) + (i & 3);
+}
+constexpr int kStepsPerChunk = 18;   // 9 taps x two k-steps of 32 channels
+constexpr int kFilterLookahead = 18; // most k-steps requested ahead
+
+__host__ __device__ static inline size_t conv3x3_index(int k, int c, int tap, int Kp) {
+    const int kb = 2 * (k >> 5) + ((k >> 2) & 1), i = 4 * ((k >> 3) & 3) + (k & 3);
+    const int step = ((c >> 6) * 9 + tap) * 2 + ((c >> 5) & 1);
+    const int lane = ((c >> 3) & 3) * 16 + i;
+    return (((size_t)step * (Kp / 16) + kb) * 64 + lane) * 8 + (c & 7);
+}
+
+size_t conv3x3_filter_count(int Cp, int Kp) {
+    // the look-ahead reads past the last k-step (values that no instruction uses)
+    return (size_t)(9 * Cp / 32 + kFilterLookahead) * Kp * 32;
+}
+
+// One work-group computes WR * RB * 16 points x WN * NB * 16 output channels; a wavefront owns
+// RB x NB accumulator tiles of 16 x 16.
+//
+// Operands.  The filters are read once per work-group row of wavefronts straight from the
+// die's L2 into registers (a ring of D k-steps, so that D - 1 steps of matrix instructions
+// cover the latency); no two wavefronts of a work-group column share them through LDS because
+// the LDS pipe is the busier one: it delivers RB KiB per k-step and wavefront for RB * NB
+// instructions of 16 cycles, 256 / NB of its 128 bytes per cycle, against 256 / RB of the 64 that
+// the L1 delivers.  RB = 6, NB = 4 (50 % of one, 67 % of the other) is the tile for full
+// batches.  The planes pass through LDS because every value is used nine times: the cells a
+// tile reaches are staged once per chunk of input channels, in rows padded to an odd number
+// of 16-byte pieces (conflict-free fragment reads), and the nine taps and two halves are
+// immediate offsets of one address per 16 points.
+//
+// CC == 0: chunks of 64 input channels in two LDS buffers; the next chunk's pieces are loaded
+// and stored in small groups between the matrix instructions (SGRP at a time: kept whole they
+// would take the registers that let two work-groups share a compute unit), one barrier per
+// chunk.  CC > 0 (64 CC channels, small tiles): everything is staged at once, one barrier in
+// all, since a chunk's arithmetic would be over long before the next chunk has come.
+//
+// The sum over taps and channels runs in the same order in every variant, with the same
+// instruction, so a position's result does not depend on the batch it is evaluated in.
+template <int RB, int NB, int WR, int WN, int D, int DA, int CC, int OCC>
+__global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
+    const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
+    half_t* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
+    float rfac, int n, int Cp, int Kp, int tiles_n, int seg, int n_items) {
+    constexpr bool DB = CC == 0;
+    constexpr int CH = DB ? 1 : CC;              // chunks of 64 channels staged together
+    constexpr int NT = 64 * WR * WN;
+    constexpr int MT = WR * RB * 16, CW = WN * NB * 16;
+    constexpr int CELLS = conv_cells(MT);
+    constexpr int STR = CH * 128 + 16;           // bytes per cell
+    constexpr int BUF = (CELLS + 1) * STR;       // one more cell takes the pieces past the end
+    constexpr int PPC = CH * 8;                  // 16-byte pieces per cell
+    constexpr int NP = (CELLS * PPC + NT - 1) / NT;
+    constexpr int KS = kStepsPerChunk;
+    constexpr int SGRP = 3;
+    constexpr int NG = (NP + SGRP - 1) / SGRP;   // groups of pieces per chunk (CC == 0)
+    constexpr int GS = KS / NG > 0 ? KS / NG : 1;
+    constexpr int PR = NB >= 2 ? NB / 2 : 1;     // stores per point: two blocks give 16 bytes
+    constexpr int E = NB >= 2 ? 8 : 4;           // channels per store
+    constexpr bool EARLY = RB * NB <= 4;         // skip connection requested before the arithmetic
+    static_assert(KS % D == 0 && KS % DA == 0, "rings turn a whole number of times per chunk");
+    static_assert(D <= kFilterLookahead, "filter padding");
+    static_assert(!DB || NG <= KS, "one group of pieces per k-step at most");
+    static_assert(NB == 1 || NB % 2 == 0, "blocks are stored in pairs");
+    __shared__ __attribute__((aligned(16))) unsigned char lds[DB ? 2 * BUF : BUF + 128 * DA];
+    __shared__ __attribute__((aligned(16))) float bn[2][CW];
+
+    // Work-group w runs on die w % 8; the items (row tile, channel tile; channel tile fastest)
+    // are cut into 8 contiguous segments, one per die: the channel tiles of a row tile, and row
+    // tiles next to each other, read the same planes.
+    const int item = (int)(blockIdx.x & 7) * seg + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= seg || item >= n_items) return;
+    const int tn = item % tiles_n, tm = item / tiles_n;
+    const int rows = n * kPts, m0 = tm * MT;
+    const unsigned tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const int wr = wave / WN, wn = wave % WN;
+
+    // Global offsets of this thread's pieces of the patch; cells off the board (and past the
+    // batch) get an offset outside the buffer and read as zero.
+    const unsigned q0 = conv_cell(m0) + kCellsPerBoard - 21;   // one board on: stays positive
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
+    const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wf, ((size_t)9 * Cp + 32 * kFilterLookahead) * Kp * 2);
+    unsigned poff[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const unsigned piece = tid + i * NT, cell = piece / PPC, part = piece % PPC;
+        const unsigned q = q0 + cell;
+        const unsigned b1 = q / kCellsPerBoard, r = q - b1 * kCellsPerBoard, y1 = r / 20,
+                       x = r - y1 * 20;
+        const bool ok = (cell < (unsigned)CELLS) & (b1 >= 1) & (b1 <= (unsigned)n) & (y1 >= 1) &
+                        (x < (unsigned)kBoard);
+        poff[i] = ok ? (((b1 - 1) * kPts + (y1 - 1) * kBoard + x) * (unsigned)Cp + part * 8u) * 2u
+                     : 0xfffffff0u;
+    }
+    // LDS address of piece i: a constant distance from piece 0 (but for the last, which may
+    // lie past the end, and where a row of threads is no whole number of cells)
+    const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 16u;
+    auto laddr = [&](int i) -> unsigned {
+        if constexpr (NT % PPC == 0) {
+            if (i < NP - 1 || (CELLS * PPC) % NT == 0) return lst + i * (NT / PPC) * STR;
+        }
+        const unsigned p = tid + i * NT, c = p / PPC;
+        return (c < (unsigned)CELLS ? c : (unsigned)CELLS) * STR + (p % PPC) * 16u;
+    };
+
+    const int chunks = Cp / 64;
+    unsigned arow[RB];   // LDS address of this lane's point of each row block, tap (0, 0)
+#pragma unroll
+    for (int i = 0; i < RB; i++) {
+        const unsigned m = min(m0 + (wr * RB + i) * 16 + (int)(lane & 15), rows - 1);
+        arow[i] = (conv_cell(m) + kCellsPerBoard - 21 - q0) * STR + (lane >> 4) * 16;
+    }
+    const int kb = (tn * WN + wn) * NB;          // first block of 16 output channels
+    unsigned ws = (unsigned)kb * 1024u;
+    const unsigned wstep = (unsigned)Kp * 64u;   // bytes per k-step
+    const unsigned wv = lane * 16u;
+    int4v w[D][NB];
+    auto wload = [&](int slot, int j, unsigned st) {
+        w[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(rW, wv + j * 1024, ws + st * wstep, 0);
+    };
+
+    const int ch0 = (kb >> 1) * 32 + 8 * (int)(lane >> 4) + 4 * (kb & 1);   // first channel
+    unsigned ro[RB];                              // byte offset of this lane's point and channel
+    int4v rr[RB][PR];
+#pragma unroll
+    for (int i = 0; i < RB; i++) {
+        const int m = m0 + (wr * RB + i) * 16 + (int)(lane & 15);
+        ro[i] = m < rows ? (unsigned)((m * Kp + ch0) * 2) : 0xfffff000u;
+    }
+    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, (size_t)rows * Kp * 2);
+    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, (size_t)rows * Kp * 2);
+    auto load_res = [&]() {
+        if (res != nullptr) {
+#pragma unroll
+            for (int i = 0; i < RB; i++)
+#pragma unroll
+                for (int j = 0; j < PR; j++) {
+                    if constexpr (NB >= 2) {
+                        rr[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rR, ro[i] + j * 64, 0, 0);
+                    } else {
+                        const int2v t = __builtin_bit_cast(
+                            int2v, __builtin_amdgcn_raw_buffer_load_b64(rR, ro[i], 0, 0));
+                        rr[i][j] = int4v{t.x, t.y, 0, 0};
+                    }
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < RB; i++)
+#pragma unroll
+                for (int j = 0; j < PR; j++) rr[i][j] = int4v{0, 0, 0, 0};
+        }
+    };
+
+    {
+        int4v stg[NP];
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rX, poff[i], 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) wload(d, j, d);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (EARLY) load_res();
+        for (int i = tid; i < CW; i += NT) {
+            const float s = bn_scale[tn * CW + i];
+            bn[0][i] = s;
+            bn[1][i] = -s * bn_mean[tn * CW + i];
+        }
+#pragma unroll
+        for (int i = 0; i < NP; i++) *reinterpret_cast<int4v*>(lds + laddr(i)) = stg[i];
+    }
+    float4v acc[RB][NB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    // LDS is what the work-group shares: its writes are waited for, the filter loads stay in
+    // flight across the barrier.
+    auto lds_barrier = []() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    lds_barrier();
+
+    int4v a[DA][RB];
+    auto aread = [&](int i, int st) {
+        const int sub = st / KS, tap = (st % KS) / 2, half = st & 1;
+        return *reinterpret_cast<const int4v*>(lds + arow[i] + ((tap / 3) * 20 + tap % 3) * STR +
+                                               sub * 128 + half * 64);
+    };
+    if constexpr (!DB) {
+#pragma unroll
+        for (int d = 0; d < DA; d++)
+#pragma unroll
+            for (int i = 0; i < RB; i++) a[d][i] = aread(i, d);
+    }
+    unsigned other = BUF;   // byte offset of the buffer being filled (CC == 0)
+#pragma unroll 1
+    for (int c = 0; c < chunks; c++) {
+        if constexpr (DB) {
+#pragma unroll
+            for (int d = 0; d < DA; d++)
+#pragma unroll
+                for (int i = 0; i < RB; i++) a[d][i] = aread(i, d);
+        }
+        // the last chunk stages itself again, into the buffer nobody reads any more: loads
+        // and stores without branches keep the count of outstanding loads exact
+        const unsigned next = (unsigned)(c + 1 < chunks ? c + 1 : c) * 128u;
+        int4v sg[SGRP];
+#pragma unroll
+        for (int st = 0; st < KS; st++) {
+            if constexpr (DB) {
+#pragma unroll
+                for (int g = 0; g < NG; g++) {
+                    if (st == g * GS) {
+#pragma unroll
+                        for (int i = 0; i < SGRP; i++)
+                            if (g * SGRP + i < NP)
+                                sg[i] = __builtin_amdgcn_raw_buffer_load_b128(
+                                    rX, poff[g * SGRP + i], next, 0);
+                    }
+                    if (st == (g + 1) * GS - 1) {
+#pragma unroll
+                        for (int i = 0; i < SGRP; i++)
+                            if (g * SGRP + i < NP)
+                                *reinterpret_cast<int4v*>(lds + laddr(g * SGRP + i) + other) = sg[i];
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // The filters of step st + D - 1 go into the slot that step st - 1 has left, and each
+            // row block's next fragment is read behind the instructions that used the last one;
+            // the barriers keep this order.
+#pragma unroll
+            for (int i = 0; i < RB; i++) {
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+                    if (i == (RB >= NB ? j : 0)) wload((st + D - 1) % D, j, st + D - 1);
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        __builtin_bit_cast(half8v, w[st % D][j]),
+                        __builtin_bit_cast(half8v, a[st % DA][i]), acc[i][j], 0, 0, 0);
+                if (!DB || st + DA < KS) a[st % DA][i] = aread(i, st + DA);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        ws += KS * wstep;
+        if constexpr (DB) {
+            lds_barrier();
+            const unsigned flip = (c & 1) ? (unsigned)-BUF : (unsigned)BUF;
+#pragma unroll
+            for (int i = 0; i < RB; i++) arow[i] += flip;
+            other -= flip;
+        } else {
+#pragma unroll
+            for (int i = 0; i < RB; i++) arow[i] += 128;
+        }
+    }
+
+    // max(0, scale * (y - mean) + rfac * res), clamped to the stored range
+    if constexpr (!EARLY) load_res();
+#pragma unroll
+    for (int j = 0; j < PR; j++) {
+        const int cl = ch0 - tn * CW + j * 32;
+        float sc[E], nb[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            sc[e] = bn[0][cl + e];
+            nb[e] = bn[1][cl + e];
+        }
+#pragma unroll
+        for (int i = 0; i < RB; i++) {
+            const half8v rh = __builtin_bit_cast(half8v, rr[i][j]);
+            half8v o;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if (e >= E) { o[e] = (half_t)0.0f; continue; }
+                const float v = acc[i][NB >= 2 ? 2 * j + e / 4 : 0][e % 4];
+                o[e] = (half_t)fminf(
+                    fmaxf(0.0f, fmaf((float)rh[e], rfac, fmaf(v, sc[e % E], nb[e % E]))),
+                    kActStoreMax);
+            }
+            const int4v bits = __builtin_bit_cast(int4v, o);
+            if constexpr (NB >= 2)
+                __builtin_amdgcn_raw_buffer_store_b128(bits, rY, ro[i] + j * 64, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b64(uint2v{(unsigned)bits.x, (unsigned)bits.y},
+                                                      rY, ro[i], 0, 0);
+        }
+    }
+}
+
+template <int RB, int NB, int WR, int WN, int D, int DA, int CC, int OCC>
+static void launch_conv_as(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
+                           const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
+                           int Kp, hipStream_t s, LaunchTimer* t) {
+    constexpr int MT = WR * RB * 16, CW = WN * NB * 16;
+    const int tiles_m = (n * kPts + MT - 1) / MT, tiles_n = Kp / CW;
+    int seg = (tiles_m * tiles_n + 7) / 8;
+    seg = (seg + tiles_n - 1) / tiles_n * tiles_n;   // the channel tiles of a row tile together
+    launch(conv3x3_k<RB, NB, WR, WN, D, DA, CC, OCC>, dim3(8 * seg), dim3(64 * WR * WN), s, t, X,
+           Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, Kp, tiles_n, seg, tiles_m * tiles_n);
+}
+
+// 64 filters have too little arithmetic per point to need it, and from 320 on the Winograd
+// kernels are ahead for some batches (384 filters, 44 boards: 40 against 52 us per layer).
+bool conv3x3_serves(int Kp, int elem_bytes) {
+    return elem_bytes == 2 && (Kp == 128 || Kp == 192 || Kp == 256);
+}
+
+// The tile.  A layer of few boards is a chain of latencies, so its points and channels are
+// spread over the 256 compute units in the smallest tiles that still make no more than one
+// work-group per unit; larger ones reuse each operand more.  Measured at 256 filters, us per
+// layer of a dependent chain with the tile of 32x32 | 32x64 | 48x64 | 96x64 | 192x64 |
+// 192x128 (points x channels), - = not measured:
+//    1 board    6.6 |  7.1 |  8.9 |  9.9 | 14.2 | 20.3
+//    4 boards   7.9 |  7.2 |  8.8 | 10.0 | 14.6 | 20.6
+//    8 boards   9.8 |  9.8 |  8.9 | 10.0 | 14.7 | 20.6
+//   16 boards  17.5 | 13.6 | 11.8 | 10.2 | 14.8 | 20.7
+//   32 boards  30.9 | 23.9 | 16.8 | 16.0 | 15.4 | 21.1
+//   64 boards     - |    - |    - |    - |    - | 22.7
+// (each entry jumps where the tile passes 256 work-groups).  192 filters have no tile of 128
+// channels; there 128 x 192 takes the place of 192 x 128 (64 boards 18.2 against 19.7 us with
+// three tiles of 64 channels).
+void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
+                    const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,
+                    hipStream_t s, LaunchTimer* t) {
+    if (!conv3x3_serves(Kp, 2) || Cp % 64 != 0)
+        throw std::invalid_argument("no direct convolution for this width");
+    const int rows = n * kPts;
+    auto groups = [&](int mt, int cw) { return ((rows + mt - 1) / mt) * (Kp / cw); };
+    constexpr int kUnits = 256;
+#define LZ_CONV(RB, NB, WR, WN, D, DA, CC, OCC)                                                   \
+    launch_conv_as<RB, NB, WR, WN, D, DA, CC, OCC>(X, Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, \
+                                                   Kp, s, t)
+    // whole patches in LDS: the input layer and towers of up to 256 filters
+    const int cc = Cp / 64;
+    if (cc <= 4 && groups(32, 32) <= kUnits) {
+        switch (cc) {
+            case 1: LZ_CONV(2, 1, 1, 2, 18, 6, 1, 1); return;
+            case 2: LZ_CONV(2, 1, 1, 2, 18, 6, 2, 1); return;
+            case 3: LZ_CONV(2, 1, 1, 2, 18, 6, 3, 1); return;
+            default: LZ_CONV(2, 1, 1, 2, 18, 6, 4, 1); return;
+        }
+    }
+    if (cc <= 4 && groups(32, 64) <= kUnits) {
+        switch (cc) {
+            case 1: LZ_CONV(2, 1, 1, 4, 18, 3, 1, 1); return;
+            case 2: LZ_CONV(2, 1, 1, 4, 18, 3, 2, 1); return;
+            case 3: LZ_CONV(2, 1, 1, 4, 18, 3, 3, 1); return;
+            default: LZ_CONV(2, 1, 1, 4, 18, 3, 4, 1); return;
+        }
+    }
+    if (groups(48, 64) <= kUnits) {
+        LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
+        return;
+    }
+    if (groups(96, 64) <= kUnits) {
+        LZ_CONV(3, 2, 2, 2, 6, 3, 0, 2);
+        return;
+    }
+    if (groups(192, 64) <= kUnits) {
+        LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);
+        return;
+    }
+    if (Kp % 128 == 0)
+        LZ_CONV(6, 4, 2, 2, 3, 1, 0, 2);
+    else if (Kp == 192)
+        LZ_CONV(4, 6, 2, 2, 3, 1, 0, 2);
+    else
+        LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);
+#undef LZ_CONV
+}
+
+// ---------------------------------------------------------------------------
+// 3x3 filters from their Winograd form U = G f G^T ([36][C][F], what a pipe is handed): the
+// rows 0 and 5 of G are the unit vectors of f's outer taps and half the difference of rows 2
+// and 1 is sqrt(2)/3 times the middle one, so f = L U L^T with the L below.  Every filter is
+// checked by transforming it forward again: *bad is set if some u is further from G f G^T
+// than rounding explains (such a U is no transform of a 3x3 filter, and only the Winograd
+// kernels can compute with it).
+__device__ constexpr float kG[6][3] = {{1.0f, 0.0f, 0.0f},
+                                       {-2.0f / 3.0f, -0.47140452f, -1.0f / 3.0f},
+                                       {-2.0f / 3.0f, 0.47140452f, -1.0f / 3.0f},
+                                       {1.0f / 6.0f, 0.23570226f, 1.0f / 3.0f},
+                                       {1.0f / 6.0f, -0.23570226f, 1.0f / 3.0f},
+                                       {0.0f, 0.0f, 1.0f}};
+
+__global__ __launch_bounds__(256) void filters_3x3_k(const float* __restrict__ U,
+                                                     half_t* __restrict__ Wf, int C, int F, int Kp,
+                                                     int* __restrict__ bad) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= C * F) return;
+    const int c = i / F, k = i - c * F;
+    float u[6][6], peak = 0.0f;
+#pragma unroll
+    for (int p = 0; p < 36; p++) {
+        u[p / 6][p % 6] = U[((size_t)p * C + c) * F + k];
+        peak = fmaxf(peak, fabsf(u[p / 6][p % 6]));
+    }
+    constexpr float kMid = 1.0606602f;   // 3 / (2 sqrt 2)
+    float t[3][6], f[3][3];
+#pragma unroll
+    for (int x = 0; x < 6; x++) {
+        t[0][x] = u[0][x];
+        t[1][x] = (u[2][x] - u[1][x]) * kMid;
+        t[2][x] = u[5][x];
+    }
+#pragma unroll
+    for (int y = 0; y < 3; y++) {
+        f[y][0] = t[y][0];
+        f[y][1] = (t[y][2] - t[y][1]) * kMid;
+        f[y][2] = t[y][5];
+    }
+    bool ok = true;
+#pragma unroll
+    for (int y = 0; y < 6; y++) {
+        float g[3];
+#pragma unroll
+        for (int x = 0; x < 3; x++) g[x] = kG[y][0] * f[0][x] + kG[y][1] * f[1][x] + kG[y][2] * f[2][x];
+#pragma unroll
+        for (int x = 0; x < 6; x++) {
+            const float v = g[0] * kG[x][0] + g[1] * kG[x][1] + g[2] * kG[x][2];
+            ok = ok && fabsf(v - u[y][x]) <= 1e-4f * peak;
+        }
+    }
+    if (!ok) *bad = 1;
+#pragma unroll
+    for (int tap = 0; tap < 9; tap++)
+        Wf[conv3x3_index(k, c, tap, Kp)] =
+            (half_t)fminf(fmaxf(f[tap / 3][tap % 3], -65504.0f), 65504.0f);
+}
+
+void conv3x3_filters(const float* U, half_t* Wf, int C, int F, int Kp, int* bad, hipStream_t s) {
+    hipLaunchKernelGGL(filters_3x3_k, dim3((unsigned)((C * F + 255) / 256)), dim3(256), 0, s, U, Wf,
+                       C, F, Kp, bad);
+}
+
+void conv3x3_winograd_filters(const half_t* Wf, int C, int Cp, int F, int Kp, half_t* U) {
+    const double s2 = std::sqrt(2.0);
+    const double G[6][3] = {{1, 0, 0},
+                            {-2.0 / 3, -s2 / 3, -1.0 / 3},
+                            {-2.0 / 3, s2 / 3, -1.0 / 3},
+                            {1.0 / 6, s2 / 6, 1.0 / 3},
+                            {1.0 / 6, -s2 / 6, 1.0 / 3},
+                            {0, 0, 1}};
+    for (int k = 0; k < F; k++)
+        for (int c = 0; c < C; c++)
+            for (int p = 0; p < kPos; p++) {
+                double v = 0.0;
+                for (int tap = 0; tap < 9; tap++)
+                    v += G[p / 6][tap / 3] * G[p % 6][tap % 3] *
+                         (double)Wf[conv3x3_index(k, c, tap, Kp)];
+                U[((size_t)p * Kp + k) * Cp + c] = (half_t)v;
+            }
+}
+
+}  // namespace lzhip

@@ -163,7 +163,6 @@ public:
         } unwind{this};
         for (int i = 0; i < m_n_lanes; i++) {
             HIP_CHECK(hipStreamCreate(&m_lane[i].stream));
-            HIP_CHECK(hipEventCreateWithFlags(&m_lane[i].last, hipEventDisableTiming));
         }
         const size_t B = (size_t)max_batch;
         m_din.alloc(B * kInPlanes * kPts);
@@ -184,17 +183,9 @@ public:
             Lane& ln = m_lane[i];
             ln.act0.alloc(B * kPts * m_C0p);
             for (auto& a : ln.act) a.alloc(B * kPts * m_Fp);
-            ln.V.alloc((size_t)kPos * m_Tp * m_Fp);
-            ln.M.alloc((size_t)kPos * m_Tp * m_Fp);
-            ln.flags.alloc(B * kFusedFlagsPerBoard);    // zeroed: no launch has epoch 0
         }
-        m_gave_up.alloc(1);
-        *m_gave_up.p = 0;
-        // measurement knobs.  LZHIP_FUSE: 0 never, 1 where it pays (the default), 2 wherever a
-        // fused launch exists; LZHIP_SLAB=0: tile arrays row by row at every batch
-        if (const char* e = std::getenv("LZHIP_FUSE")) m_fuse = std::atoi(e);
-        if (const char* e = std::getenv("LZHIP_INPLACE")) m_in_place = std::atoi(e) != 0;
-        if (const char* e = std::getenv("LZHIP_SLAB")) m_slab = std::atoi(e) != 0;
+        if (const char* e = std::getenv("LZHIP_INPLACE"))   // measurement knob
+            m_in_place = std::atoi(e) != 0;
         m_scalar.alloc(4);
         for (int i = 0; i < kTimerPool; i++) {
             HIP_CHECK(hipEventCreate(&m_ev_start[i]));
@@ -222,8 +213,6 @@ public:
             sl.done = nullptr;
         }
         for (auto& ln : m_lane) {
-            if (ln.last) (void)hipEventDestroy(ln.last);
-            ln.last = nullptr;
             if (ln.stream) (void)hipStreamDestroy(ln.stream);
             ln.stream = nullptr;
         }
@@ -258,6 +247,7 @@ public:
             m_layers.clear();
             m_w3.release();
             m_s.clear();
+            release_tiles();
             throw;
         }
         m_ready = true;
@@ -268,6 +258,11 @@ public:
         auto& ln = m_lane[0];
         const int F = m_filters;
         m_layers.resize(n_layers);
+        // fp16 towers of the widths conv3x3_serves names are computed by direct convolution,
+        // provided that what was handed over are transforms of 3x3 filters; all else goes
+        // through the Winograd kernels and needs their tile arrays.
+        m_direct = conv3x3_serves(m_Fp, (int)sizeof(P)) && build_direct_filters(n_layers, U);
+        if (!m_direct) alloc_tiles();
         // Filters are laid out on the host in fp32; an fp16 net converts them on the device.
         std::vector<float> tmp;
         DevBuf<float> stage;
@@ -289,14 +284,14 @@ public:
             Layer& L = m_layers[l];
             L.C = l == 0 ? kInPlanes : F;
             L.Cp = l == 0 ? m_C0p : m_Fp;
-            tmp.assign((size_t)kPos * m_Fp * L.Cp, 0.0f);
-            // One copy of the filters, in the order the GEMM of this width and precision
-            // reads them.  Whether that is the streaming kernel does not depend on the batch
-            // of a forward (only on the handle's limit), so a network holds either the
-            // fragment order or the row order, never both.
-            if (gemm_stream_shape(kTilesPerBoard, L.Cp, m_Fp, (int)sizeof(P)) &&
-                gemm_stream_prefers(m_Fp, (int)sizeof(P), m_max_batch)) {
-                build_stream_filters(U[l], L.C, F, L.Cp, m_Fp, (int)sizeof(P), tmp.data());
+            if (!m_direct) tmp.assign((size_t)kPos * m_Fp * L.Cp, 0.0f);
+            // One copy of the filters, in the order the kernel of this width and precision
+            // reads them.  Which kernel that is does not depend on the batch of a forward
+            // (only on the handle's limit), so a network holds one order, never two.
+            if (m_direct) {
+            } else if (gemm_stream_shape(kTilesPerBoard, L.Cp, m_Fp, (int)sizeof(P)) &&
+                       gemm_stream_prefers(m_Fp, m_max_batch)) {
+                build_stream_filters(U[l], L.C, F, L.Cp, m_Fp, tmp.data());
                 upload(L.Uf);
             } else {
                 // reference layout [36][C][F] (F fastest)  ->  [36][Fp][Cp] (C fastest),
@@ -327,6 +322,51 @@ public:
         for (int l = 0; l < n_layers; l++) upload_bn(l);
         if (precision_of<P>() == LZHIP_FP16) calibrate();
         HIP_CHECK(hipStreamSynchronize(ln.stream));
+    }
+
+    // Filters of the direct convolution for every layer; false (and nothing kept) if some layer's
+    // U is not the transform of 3x3 filters.
+    bool build_direct_filters(int n_layers, const float* const* U) {
+        if constexpr (sizeof(P) != 2) {
+            (void)n_layers;
+            (void)U;
+            return false;
+        } else {
+            hipStream_t s = m_lane[0].stream;
+            const int F = m_filters;
+            DevBuf<float> stage;
+            DevBuf<int> bad;
+            stage.alloc((size_t)kPos * F * (F > kInPlanes ? F : kInPlanes));
+            bad.alloc(1);
+            for (int l = 0; l < n_layers; l++) {
+                Layer& L = m_layers[l];
+                const int C = l == 0 ? kInPlanes : F, Cp = l == 0 ? m_C0p : m_Fp;
+                L.W3.alloc(conv3x3_filter_count(Cp, m_Fp));
+                HIP_CHECK(hipMemcpy(stage.p, U[l], sizeof(float) * (size_t)kPos * C * F,
+                                    hipMemcpyHostToDevice));
+                conv3x3_filters(stage.p, L.W3.p, C, F, m_Fp, bad.p, s);
+                HIP_CHECK(hipGetLastError());
+                HIP_CHECK(hipStreamSynchronize(s));
+            }
+            int is_bad = 0;
+            HIP_CHECK(hipMemcpy(&is_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost));
+            if (is_bad)
+                for (auto& L : m_layers) L.W3.release();
+            return !is_bad;
+        }
+    }
+
+    void alloc_tiles() {
+        for (int i = 0; i < m_n_lanes; i++) {
+            m_lane[i].V.alloc((size_t)kPos * m_Tp * m_Fp);
+            m_lane[i].M.alloc((size_t)kPos * m_Tp * m_Fp);
+        }
+    }
+    void release_tiles() {
+        for (int i = 0; i < m_n_lanes; i++) {
+            m_lane[i].V.release();
+            m_lane[i].M.release();
+        }
     }
 
     // -------------------------------------------------------------------
@@ -388,16 +428,6 @@ public:
     void sync() override {
         HIP_CHECK(hipSetDevice(m_device));
         for (int i = 0; i < m_n_lanes; i++) HIP_CHECK(hipStreamSynchronize(m_lane[i].stream));
-        check_waits();
-    }
-
-    // A fused launch whose work-groups gave up waiting for each other has produced nothing
-    // usable; it says so through a word in mapped host memory.
-    void check_waits() {
-        if (__atomic_load_n(m_gave_up.p, __ATOMIC_RELAXED) != 0)
-            throw std::runtime_error(
-                "a fused transform + GEMM launch ran into its wait limit: the results of this "
-                "handle are invalid (LZHIP_FUSE=0 runs the two kernels as separate launches)");
     }
 
     // Host-buffer forward.  Up to kIoSlots callers may be inside at once: each
@@ -491,7 +521,6 @@ public:
             HIP_CHECK(hipEventRecord(sl->done, ln.stream));
         }
         HIP_CHECK(hipEventSynchronize(sl->done));
-        check_waits();
         std::memcpy(out_a, sl->hpol.p, sizeof(float) * (size_t)n * na);
         std::memcpy(out_b, sl->hval.p, sizeof(float) * (size_t)n * nb);
     }
@@ -626,38 +655,39 @@ public:
         d_sc.alloc(m_Fp); d_mn.alloc(m_Fp);
         HIP_CHECK(hipMemcpy(d_sc.p, sc.data(), sizeof(float) * m_Fp, hipMemcpyHostToDevice));
         HIP_CHECK(hipMemcpy(d_mn.p, mn.data(), sizeof(float) * m_Fp, hipMemcpyHostToDevice));
-        launch_in_transform<P>(a_in, ln.V.p, n, Cp, m_Tp, ln.stream, nullptr);
-        // The layout a forward of n boards keeps its tiles in: the GEMM and the output
-        // transform run as they do there.  In a forward a tower layer's V comes slab by slab
-        // from the fused transform; here the input transform's rows are re-laid on the host.
-        int slab = 0;
+        // A direct tower has no Winograd stages of its own: V and M are computed from the
+        // filters it holds by the tiled kernels, Y by the kernel a forward runs.
+        DevBuf<P> d_V, d_M, d_U;
+        P *V = ln.V.p, *M = ln.M.p;
+        const P *U = L.U.p, *Uf = L.Uf.p;
         if constexpr (sizeof(P) == 2) {
-            if (m_slab && L.Uf.p != nullptr && gemm_stream_shape(Tu, Cp, m_Fp, 2))
-                slab = tile_slab(n, m_Fp, 2, true);
+            if (m_direct) {
+                std::vector<P> w3(L.W3.count), u((size_t)kPos * m_Fp * Cp, (P)0.0f);
+                HIP_CHECK(hipMemcpy(w3.data(), L.W3.p, w3.size() * sizeof(P), hipMemcpyDeviceToHost));
+                conv3x3_winograd_filters(w3.data(), C, Cp, F, m_Fp, u.data());
+                d_U.alloc(u.size());
+                HIP_CHECK(hipMemcpy(d_U.p, u.data(), u.size() * sizeof(P), hipMemcpyHostToDevice));
+                d_V.alloc((size_t)kPos * m_Tp * m_Fp);
+                d_M.alloc((size_t)kPos * m_Tp * m_Fp);
+                V = d_V.p; M = d_M.p; U = d_U.p; Uf = nullptr;
+            }
         }
-        std::vector<P> v_rows;
-        if (Vout || (slab != 0 && Cp != 64)) {
-            v_rows.resize((size_t)kPos * m_Tp * Cp);
-            HIP_CHECK(hipStreamSynchronize(ln.stream));
-            HIP_CHECK(hipMemcpy(v_rows.data(), ln.V.p, v_rows.size() * sizeof(P), hipMemcpyDeviceToHost));
+        launch_in_transform<P>(a_in, V, n, Cp, m_Tp, ln.stream, nullptr);
+        launch_gemm<P>(V, U, Uf, M, Tu, m_Tp, Cp, m_Fp, ln.stream, nullptr);
+        if constexpr (sizeof(P) == 2) {
+            if (m_direct)
+                launch_conv3x3(a_in, L.W3.p, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, Cp, m_Fp,
+                               ln.stream, nullptr);
         }
-        if (slab != 0 && Cp != 64) {
-            std::vector<P> g(v_rows.size());
-            for (int p = 0; p < kPos; p++)
-                for (int t = 0; t < m_Tp; t++)
-                    for (int c = 0; c < Cp; c++)
-                        g[(((size_t)p * (Cp / slab) + c / slab) * m_Tp + t) * slab + c % slab] =
-                            v_rows[((size_t)p * m_Tp + t) * Cp + c];
-            HIP_CHECK(hipMemcpy(ln.V.p, g.data(), g.size() * sizeof(P), hipMemcpyHostToDevice));
-        }
-        launch_gemm<P>(ln.V.p, L.U.p, L.Uf.p, ln.M.p, Tu, m_Tp, Cp, m_Fp, ln.stream, nullptr, slab);
-        launch_out_transform<P>(ln.M.p, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, m_Fp, m_Tp,
-                                ln.stream, nullptr, slab);
+        if (!m_direct)
+            launch_out_transform<P>(M, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, m_Fp, m_Tp,
+                                    ln.stream, nullptr);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipStreamSynchronize(ln.stream));
         const int T = n * kTilesPerBoard;
         if (Vout) {
-            const std::vector<P>& h = v_rows;
+            std::vector<P> h((size_t)kPos * m_Tp * Cp);
+            HIP_CHECK(hipMemcpy(h.data(), V, h.size() * sizeof(P), hipMemcpyDeviceToHost));
             for (int t = 0; t < T; t++)
                 for (int p = 0; p < kPos; p++)
                     for (int c = 0; c < C; c++)
@@ -666,13 +696,12 @@ public:
         }
         if (Mout) {
             std::vector<P> h((size_t)kPos * m_Tp * m_Fp);
-            HIP_CHECK(hipMemcpy(h.data(), ln.M.p, h.size() * sizeof(P), hipMemcpyDeviceToHost));
+            HIP_CHECK(hipMemcpy(h.data(), M, h.size() * sizeof(P), hipMemcpyDeviceToHost));
             for (int t = 0; t < T; t++)
                 for (int p = 0; p < kPos; p++)
                     for (int k = 0; k < F; k++)
-                        Mout[(((size_t)(t / 25) * kPos + p) * F + k) * 25 + t % 25] = (float)
-                            (slab != 0 ? h[(((size_t)p * (m_Fp / slab) + k / slab) * m_Tp + t) * slab + k % slab]
-                                       : h[((size_t)p * m_Tp + t) * m_Fp + k]);
+                        Mout[(((size_t)(t / 25) * kPos + p) * F + k) * 25 + t % 25] =
+                            (float)h[((size_t)p * m_Tp + t) * m_Fp + k];
         }
         if (Yout) {
             std::vector<P> h((size_t)n * kPts * m_Fp);
@@ -717,9 +746,6 @@ private:
         hipStream_t stream = nullptr;
         std::mutex mu;  // serialises enqueues on this lane
         DevBuf<P> act0, act[3], V, M;
-        DevBuf<unsigned long long> flags;   // fused launches: one word per (board, channel group)
-        unsigned long long epoch = 0;       // grows by one per fused launch (under mu)
-        hipEvent_t last = nullptr;          // recorded behind the lane's latest forward
         std::map<GraphKey, hipGraphExec_t> graphs;
     };
     static constexpr int kLanes = 3;   // upper bound; m_n_lanes are in use
@@ -730,10 +756,6 @@ private:
         hipStream_t stream = nullptr;
         P *act0 = nullptr, *act[3] = {nullptr, nullptr, nullptr}, *V = nullptr, *M = nullptr;
         int Tp = 0;
-        // what a fused transform + GEMM launch synchronises through; null: separate launches
-        unsigned long long* flags = nullptr;
-        unsigned long long* epoch = nullptr;
-        bool alone = false;   // no other lane had work on the device when this one was enqueued
     };
     Work work_of(Lane& ln) const {
         Work w;
@@ -743,20 +765,15 @@ private:
         w.V = ln.V.p;
         w.M = ln.M.p;
         w.Tp = m_Tp;
-        w.flags = ln.flags.p;
-        w.epoch = &ln.epoch;
-        // (an event that was never recorded reads as complete)
-        w.alone = true;
-        for (int i = 0; i < m_n_lanes; i++)
-            if (&m_lane[i] != &ln && hipEventQuery(m_lane[i].last) != hipSuccess) w.alone = false;
-        (void)hipGetLastError();   // hipErrorNotReady is an answer, not a failure
         return w;
     }
 
     struct Layer {
         int C = 0, Cp = 0;
-        DevBuf<P> U;
-        DevBuf<P> Uf;                         // fragment order (streaming GEMM), may be empty
+        // the filters in one of three orders, the other two empty:
+        DevBuf<P> U;                          // [36][Fp][Cp] (tiled GEMMs)
+        DevBuf<P> Uf;                         // fragment order of the streaming GEMM
+        DevBuf<P> W3;                         // 3x3, fragment order of the direct convolution
         std::vector<float> mean, scale;       // as pushed (unscaled)
         DevBuf<float> d_mean, d_scale;        // with activation scales folded in
         float rfac = 1.0f;
@@ -795,6 +812,13 @@ private:
     // Activation buffer roles rotate: cur = block input, mid, nxt = block output.
     void run_conv(Lane& ln, int l, int n, const P* in, const P* res, P* out, bool timed) {
         Layer& L = m_layers[l];
+        if constexpr (sizeof(P) == 2) {
+            if (m_direct) {
+                launch_conv3x3(in, L.W3.p, res, out, L.d_scale.p, L.d_mean.p, L.rfac, n, L.Cp,
+                               m_Fp, ln.stream, timer(timed, LZHIP_K_GEMM));
+                return;
+            }
+        }
         const int Tu = n * kTilesPerBoard;
         launch_in_transform<P>(in, ln.V.p, n, L.Cp, m_Tp, ln.stream, timer(timed, LZHIP_K_IN));
         launch_gemm<P>(ln.V.p, L.U.p, L.Uf.p, ln.M.p, Tu, m_Tp, L.Cp, m_Fp, ln.stream,
@@ -847,9 +871,6 @@ private:
     void enqueue_forward(Lane& ln, int n, const float* d_in, const uint32_t* d_bits,
                          float* d_pol, float* d_val, bool timed) {
         enqueue_forward(work_of(ln), n, d_in, d_bits, d_pol, d_val, timed);
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        HIP_CHECK(hipStreamIsCapturing(ln.stream, &cap));
-        if (cap == hipStreamCaptureStatusNone) HIP_CHECK(hipEventRecord(ln.last, ln.stream));
     }
     void enqueue_forward(const Work& w, int n, const float* d_in, const uint32_t* d_bits,
                          float* d_pol, float* d_val, bool timed) {
@@ -861,39 +882,24 @@ private:
         else
             launch_pack_input_bits<P>(d_bits, w.act0, n, kInPlanes, m_C0p, w.stream,
                                       timer(timed, LZHIP_K_PACK));
+        if constexpr (sizeof(P) == 2) {
+            if (m_direct) {
+                enqueue_direct(w, n, d_pol, d_val, timed);
+                return;
+            }
+        }
         launch_in_transform<P>(w.act0, w.V, n, m_C0p, w.Tp, w.stream, timer(timed, LZHIP_K_IN));
-        // Small batches of fp16 towers (xform_gemm_shape) keep their tile arrays slab by slab
-        // (tile_slab) from the first GEMM's output to the last transform's input -- nothing
-        // outside this function sees them -- and send the transform of layer l and the GEMM
-        // of layer l + 1 as one launch where xform_gemm_pays says that is faster: the fused
-        // launch shortens a chain of dependent kernels, but its waiting work-groups hold
-        // compute units that another lane's kernels could use, so the answer depends on
-        // whether this forward has the device to itself.  All ways give the same bits.  No
-        // fused launches under graph capture (the launch carries a number that has to differ
-        // from launch to launch), when every launch is timed, or on the static working memory.
-        int slab = 0;
-        if constexpr (sizeof(P) == 2) {
-            if (m_slab && m_layers.size() > 1 && m_layers[1].Uf.p != nullptr &&
-                gemm_stream_shape(Tu, m_Fp, m_Fp, 2))
-                slab = tile_slab(n, m_Fp, 2, w.alone);
-        }
-        bool fused = false;
-        if constexpr (sizeof(P) == 2) {
-            fused = m_fuse > 0 && !timed && !m_use_graph && w.flags != nullptr &&
-                    xform_gemm_shape(n, m_Fp, 2) &&
-                    (m_fuse > 1 || xform_gemm_pays(n, m_Fp, slab, w.alone));
-        }
         // With the streaming GEMM the tower's layers work in place: M_l is written over V_l
         // and V_{l+1} over M_l (see the kernels), so a lane's tiles are one array instead of
         // two and the lanes' working sets (2 or 3 x 33 MB of tiles less at 64 boards) fit the
         // 256 MB memory-side cache.  Layer 0 reads 64 padded planes and keeps its own output.
         P* tiles = w.M;
-        const bool in_place = m_in_place && !fused && m_layers.size() > 1 &&
+        const bool in_place = m_in_place && m_layers.size() > 1 &&
                               gemm_stream_shape(Tu, m_Fp, m_Fp, (int)sizeof(P)) &&
                               m_layers[1].Uf.p != nullptr;
         int cur = 0, nxt = 1;  // block input (skip) / block output
         launch_gemm<P>(w.V, m_layers[0].U.p, m_layers[0].Uf.p, w.M, Tu, w.Tp, m_layers[0].Cp, m_Fp,
-                       w.stream, timer(timed, LZHIP_K_GEMM), slab);
+                       w.stream, timer(timed, LZHIP_K_GEMM));
         for (int l = 0; l < nl; l++) {
             Layer& L = m_layers[l];
             const bool block_end = (l % 2) == 0;      // layer 0 and second convs
@@ -901,30 +907,41 @@ private:
             P* out = l == 0 ? w.act[cur] : w.act[nxt];
             if (l == nl - 1) {
                 launch_out_transform<P>(tiles, res, out, L.d_scale.p, L.d_mean.p, L.rfac, n, m_Fp,
-                                        w.Tp, w.stream, timer(timed, LZHIP_K_OUT), slab);
+                                        w.Tp, w.stream, timer(timed, LZHIP_K_OUT));
                 launch_head_conv<P>(out, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
                                     timer(timed, LZHIP_K_HEAD));
             } else {
                 Layer& N = m_layers[l + 1];
-                bool done = false;
-                if constexpr (sizeof(P) == 2) {
-                    if (fused) {
-                        launch_xform_gemm(w.M, res, block_end ? out : nullptr, w.M, L.d_scale.p,
-                                          L.d_mean.p, L.rfac, n, m_Fp, w.Tp, N.Uf.p, w.flags,
-                                          ++*w.epoch, m_gave_up.p, w.stream, slab);
-                        done = true;
-                    }
-                }
-                if (!done) {
-                    launch_out_in_transform<P>(tiles, res, block_end ? out : nullptr, w.V,
-                                               L.d_scale.p, L.d_mean.p, L.rfac, n, m_Fp, w.Tp,
-                                               w.stream, timer(timed, LZHIP_K_OUTIN), slab);
-                    if (in_place) tiles = w.V;
-                    launch_gemm<P>(w.V, N.U.p, N.Uf.p, tiles, Tu, w.Tp, N.Cp, m_Fp, w.stream,
-                                   timer(timed, LZHIP_K_GEMM), slab);
-                }
+                launch_out_in_transform<P>(tiles, res, block_end ? out : nullptr, w.V, L.d_scale.p,
+                                           L.d_mean.p, L.rfac, n, m_Fp, w.Tp, w.stream,
+                                           timer(timed, LZHIP_K_OUTIN));
+                if (in_place) tiles = w.V;
+                launch_gemm<P>(w.V, N.U.p, N.Uf.p, tiles, Tu, w.Tp, N.Cp, m_Fp, w.stream,
+                               timer(timed, LZHIP_K_GEMM));
             }
             if (block_end && l >= 2) { const int o = cur; cur = nxt; nxt = o; }
+        }
+    }
+
+    // The layer loop of a direct tower: one launch per layer.
+    void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed) {
+        if constexpr (sizeof(P) == 2) {
+            const int nl = (int)m_layers.size();
+            const P* last = w.act[0];
+            int cur = 0, nxt = 2;   // block input (skip) / block output; 1 lies between
+            for (int l = 0; l < nl; l++) {
+                Layer& L = m_layers[l];
+                const bool second = l >= 2 && (l % 2) == 0;
+                const P* in = l == 0 ? w.act0 : second ? w.act[1] : w.act[cur];
+                P* out = l == 0 ? w.act[cur] : second ? w.act[nxt] : w.act[1];
+                launch_conv3x3(in, L.W3.p, second ? w.act[cur] : nullptr, out, L.d_scale.p,
+                               L.d_mean.p, L.rfac, n, L.Cp, m_Fp, w.stream,
+                               timer(timed, LZHIP_K_GEMM));
+                last = out;
+                if (second) { const int o = cur; cur = nxt; nxt = o; }
+            }
+            launch_head_conv<P>(last, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
+                                timer(timed, LZHIP_K_HEAD));
         }
     }
 
@@ -978,7 +995,7 @@ private:
             bool adjusted = false;
             for (int attempt = 0; attempt < 8; attempt++) {
                 upload_bn(l);
-                if (attempt == 0) {
+                if (attempt == 0 || m_direct) {
                     run_conv(ln, l, n, src, res, dst, false);
                 } else {
                     Layer& L = m_layers[l];
@@ -1044,10 +1061,8 @@ private:
         const char* e = std::getenv("LZHIP_GRAPH");
         return e != nullptr && std::atoi(e) != 0;
     }();
-    int m_fuse = 1;                      // fused transform + GEMM launches (see enqueue_forward)
+    bool m_direct = false;               // direct convolutions (set by push_weights)
     bool m_in_place = true;              // tower layers keep V and M in one array (see enqueue_forward)
-    bool m_slab = true;                  // small batches keep the tile arrays slab by slab (tile_slab)
-    PinnedBuf<unsigned> m_gave_up;       // set by a fused launch whose wait ran into its limit
 };
 
 std::unique_ptr<HIPPipe> create_hip_pipe(int device, int precision, int max_batch, int filters) {

@@ -53,58 +53,51 @@ template <typename P> bool gemm_supports_channels(int Cp);
 
 // M[p][t][k] = sum_c V[p][t][c] * U[p][k][c]
 // T = real tile rows (25 per board); Tp = allocated rows, a multiple of kTileRowPad.
-// Uf: the same filters in the fragment order of the streaming kernels (see
+// Uf: the same filters in the fragment order of the streaming kernel (see
 // build_stream_filters), or null; taken when gemm_stream_shape(T, Cp, Kp, sizeof(P)).
-// slab (0, or tile_slab's 16 / 32; streaming shapes only): M is written slab by slab,
-// [36][Kp / slab][Tp][slab], and V read that way too unless it is the first layer's (Cp == 64).
 template <typename P>
 void launch_gemm(const P* V, const P* U, const P* Uf, P* M, int T, int Tp, int Cp, int Kp,
-                 hipStream_t s, LaunchTimer* t, int slab = 0);
+                 hipStream_t s, LaunchTimer* t);
 bool gemm_stream_shape(int T, int Cp, int Kp, int elem_bytes);
-// Whether a handle for batches up to max_batch should hold the streaming kernels' filters
+// Whether a handle for batches up to max_batch should hold the streaming kernel's filters
 // where gemm_stream_shape allows them (measured; see there).
-bool gemm_stream_prefers(int Kp, int elem_bytes, int max_batch);
-// Layout of the tile arrays that suits a forward of n boards: 0 row by row, else the slab width.
-int tile_slab(int n, int Kp, int elem_bytes, bool alone);
-// src [36][C][F] fp32 (F fastest) -> dst in the operand order of the streaming kernel for
-// elements of elem_bytes (2: [36][Kp/32][Cp/16][64][8], 4: [36][Kp/32][Cp/8][64][4]), values
-// in fp32, zero padded; convert_filters turns such an array into fp16 on the device.
-void build_stream_filters(const float* src, int C, int F, int Cp, int Kp, int elem_bytes,
-                          float* dst);
+bool gemm_stream_prefers(int Kp, int max_batch);
+// src [36][C][F] fp32 (F fastest) -> dst in the operand order of the streaming kernel
+// ([36][Kp/32][Cp/8][64][4]), zero padded.
+void build_stream_filters(const float* src, int C, int F, int Cp, int Kp, float* dst);
+// fp32 -> fp16 on the device.
 void convert_filters(const float* src, _Float16* dst, size_t n, hipStream_t s);
 
-// M [36][Tp][Kp] (slab > 0: [36][Kp / slab][Tp][slab]) -> out [n][361][Kp]:
+// M [36][Tp][Kp] -> out [n][361][Kp]:
 // max(0, scale*(A^T m A - mean) + rfac*res)
 template <typename P>
 void launch_out_transform(const P* M, const P* res, P* out, const float* bn_scale,
                           const float* bn_mean, float rfac, int n, int Kp, int Tp,
-                          hipStream_t s, LaunchTimer* t, int slab = 0);
+                          hipStream_t s, LaunchTimer* t);
 
 // Output transform of one layer fused with the input transform of the next:
 // M [36][Tp][Kp] -> V_next [36][Tp][Kp]; the activation [n][361][Kp] is also
-// written to act_out unless that is null.  Needs Kp to be a multiple of 64.  slab (0, 16 or
-// 32): both tile arrays lie slab by slab and a work-group takes `slab` channels.
+// written to act_out unless that is null.  Needs Kp to be a multiple of 64.
 template <typename P>
 void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const float* bn_scale,
                              const float* bn_mean, float rfac, int n, int Kp, int Tp,
-                             hipStream_t s, LaunchTimer* t, int slab = 0);
+                             hipStream_t s, LaunchTimer* t);
 
-// launch_out_in_transform of one layer and launch_gemm of the next (filters Uf, in the
-// streaming kernel's order) as one launch, for the shapes xform_gemm_shape accepts (fp16;
-// 256 filters up to 32 boards, 192 up to 42, 128 up to 64).  M is read by the transform and
-// rewritten by the GEMM; V is M (row by row: slab = 0) or M or a second array (slab by slab).
-// flags: kFusedFlagsPerBoard 64-bit words per board (zero before the first launch); epoch: a
-// value no earlier launch on these flags used; *gave_up is set to 1 if a wait inside the
-// launch ran into its limit (the results are then invalid).
-constexpr int kFusedFlagsPerBoard = 16;
-bool xform_gemm_shape(int n, int Kp, int elem_bytes);
-// Whether the fused launch is the faster way (measured) for a forward of n boards with the tile
-// arrays in slabs of `slab` channels (0: rows) that has the device to itself or not.
-bool xform_gemm_pays(int n, int Kp, int slab, bool alone);
-void launch_xform_gemm(_Float16* M, const _Float16* res, _Float16* act_out, _Float16* V,
-                       const float* bn_scale, const float* bn_mean, float rfac, int n, int Kp,
-                       int Tp, const _Float16* Uf, unsigned long long* flags,
-                       unsigned long long epoch, unsigned* gave_up, hipStream_t s, int slab = 0);
+// Direct 3x3 convolution in fp16 (conv3x3.hip), one launch per layer:
+// X [n][361][Cp] -> Y [n][361][Kp] = min(max(0, scale*(conv - mean) + rfac*res), kActStoreMax);
+// res may be null and is not Y.  Wf: conv3x3_filter_count elements, zero but for what
+// conv3x3_filters writes.
+bool conv3x3_serves(int Kp, int elem_bytes);
+size_t conv3x3_filter_count(int Cp, int Kp);
+void launch_conv3x3(const _Float16* X, const _Float16* Wf, const _Float16* res, _Float16* Y,
+                    const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,
+                    hipStream_t s, LaunchTimer* t);
+// Filters of one layer from U [36][C][F] fp32 on the device; *bad (device) is set if U is not
+// the Winograd transform of 3x3 filters.
+void conv3x3_filters(const float* U, _Float16* Wf, int C, int F, int Kp, int* bad, hipStream_t s);
+// The way back, on the host: Winograd filters [36][Kp][Cp] of the filters as stored (padding of
+// U is left as it is).
+void conv3x3_winograd_filters(const _Float16* Wf, int C, int Cp, int F, int Kp, _Float16* U);
 
 // 1x1 head convolutions: act [n][361][Cp] x w[3][Cp] -> pol [n][2][361], val [n][361],
 // both multiplied by out_scale.

@@ -3,31 +3,18 @@
 // Arithmetic follows the reference CPU pipe (reference src/CPUPipe.cpp:63-284,
 // :352-377) and its OpenCL twins (src/kernels/convolve3.opencl:47-79); the
 // decomposition, layouts and launch shapes are this library's own.
-#include "kernels.h"
-
 #include <cstdlib>
 #include <stdexcept>
 #include <type_traits>
 
-#include <hip/hip_ext.h>
+#include "kernel_util.h"
 
 namespace lzhip {
 
-typedef _Float16 half_t;
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef _Float16 half8v __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
-typedef int int4v __attribute__((ext_vector_type(4)));
 
 #define SQ2 1.4142135623730951f
-// Timeline hook for measurement builds (a harness that includes this file defines it to
-// record a timestamp); expands to nothing in the library.
-#ifndef LZ_STAMP
-#define LZ_STAMP(i)
-#endif
-constexpr int kStoreThrough = 17;  // cache policy of a raw buffer store: sc0 | sc1 (write-through)
-
 // ---------------------------------------------------------------------------
 // Per-lane channel vector: how many consecutive channels one lane owns in the
 // bandwidth-bound kernels (4 bytes per lane and access for both types).
@@ -108,16 +95,6 @@ __device__ __forceinline__ void at6(const float i0, const float i1, const float 
 }
 
 // ---------------------------------------------------------------------------
-template <typename K, typename... Args>
-static inline void launch(K kernel, dim3 grid, dim3 block, hipStream_t s, LaunchTimer* t,
-                          Args... args) {
-    if (t && t->start) {
-        hipExtLaunchKernelGGL(kernel, grid, block, 0, s, t->start, t->stop, 0, args...);
-    } else {
-        hipLaunchKernelGGL(kernel, grid, block, 0, s, args...);
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Planes NCHW fp32 [n][C][361] -> channels-last storage type [n][361][Cp],
 // channels C..Cp-1 zero.
@@ -252,13 +229,10 @@ void launch_in_transform(const P* act, P* V, int n, int Cp, int Tp, hipStream_t 
 // out = max(0, scale*(y - mean) + rfac*res); rfac carries the ratio of the
 // activation scales of the skip connection and of this layer (1 in fp32).
 template <typename P>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const P* base, size_t bytes);
-
-template <typename P>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) void out_transform_k(
     const P* __restrict__ M, const P* __restrict__ res, P* __restrict__ out,
     const float* __restrict__ bn_scale, const float* __restrict__ bn_mean, float rfac, int T,
-    int Kp, int Tp, int slab) {
+    int Kp, int Tp) {
     constexpr int VN = ChanVec<P>::N;
     const int lpt = Kp / VN;
     const int gid = blockIdx.x * 256 + threadIdx.x;
@@ -270,9 +244,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) voi
     const int by = j / 5, bx = j - by * 5;
 
     float m[VN][36];
-    // slab > 0: M lies slab by slab, [36][Kp / slab][Tp][slab]
-    const P* msrc = slab > 0 ? M + ((size_t)(c / slab) * Tp + t) * slab + c % slab
-                             : M + (size_t)t * Kp + c;
+    const P* msrc = M + (size_t)t * Kp + c;
     const size_t pstride = (size_t)Tp * Kp;
 #pragma unroll
     for (int p = 0; p < 36; p++) {
@@ -356,13 +328,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) voi
 template <typename P>
 void launch_out_transform(const P* M, const P* res, P* out, const float* bn_scale,
                           const float* bn_mean, float rfac, int n, int Kp, int Tp,
-                          hipStream_t s, LaunchTimer* t, int slab) {
+                          hipStream_t s, LaunchTimer* t) {
     const int T = n * kTilesPerBoard;
     const int lanes = T * (Kp / ChanVec<P>::N);
-    if (slab != 0 && (slab % ChanVec<P>::N != 0 || Kp % slab != 0))
-        throw std::invalid_argument("out_transform: slab width does not fit");
     launch(out_transform_k<P>, dim3((lanes + 255) / 256), dim3(256), s, t, M, res, out,
-           bn_scale, bn_mean, rfac, T, Kp, Tp, slab);
+           bn_scale, bn_mean, rfac, T, Kp, Tp);
 }
 
 // ---------------------------------------------------------------------------
@@ -450,12 +420,6 @@ template <> struct BufIO2<half_t> {
     }
 };
 
-template <typename P>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const P* base, size_t bytes) {
-    // untyped 32-bit-element descriptor for gfx9-family raw buffer instructions
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<P*>(base), 0, (int)bytes, 0x00020000);
-}
-
 // One workgroup owns one board and 64 channels.  A lane owns two consecutive
 // channels (one 4- or 8-byte access instead of two), a half-wave owns a tile,
 // so a wavefront handles two neighbouring tiles at once and the 13 wavefronts
@@ -499,18 +463,14 @@ constexpr int plane_row_pairs(int cg) {
 constexpr int plane_pairs(int cg) { return kPlane * plane_row_pairs(cg); }
 constexpr int fuse_waves(int cg) { return (kTilesPerBoard + 128 / cg - 1) / (128 / cg); }
 
-// The body of the kernel, for work-group `wg` of the launch's transform work-groups, with
-// the LDS plane handed in (plane_pairs(CG) channel pairs); returns the work item
-// (board * channel groups + channel group) it processed, or -1 if `wg` had none.
-// VPOL = cache policy of the stores of V.  VSLAB / MSLAB: V is written / M is read channel
-// group by channel group, [36][Kp / CG][Tp][CG], instead of [36][Tp][Kp] (tile_slab): the 25
-// tiles of this work-group's board and channel group are then one contiguous run per
-// Winograd position (whole lines, which is also what makes write-through stores cheap).
-template <typename P, int CG, int VPOL, bool VSLAB = false, bool MSLAB = false>
-__device__ __forceinline__ int out_in_transform_body(
-    typename BufIO2<P>::pair_t* ybuf, unsigned wg, const P* M, const P* res, P* act_out, P* Vn,
+// M and Vn may be one array (every value of M is in a register before the same lane writes
+// the value of V that takes its place), so neither is declared free of aliases.
+template <typename P, int CG>
+__global__ __launch_bounds__(fuse_waves(CG) * 64) void out_in_transform_k(
+    const P* M, const P* __restrict__ res, P* __restrict__ act_out, P* Vn,
     const float* __restrict__ bn_scale, const float* __restrict__ bn_mean, float rfac, int n,
     int Kp, int Tp) {
+    __shared__ typename BufIO2<P>::pair_t ybuf[plane_pairs(CG)];
     typedef typename BufIO2<P>::pair_t pair_t;
     constexpr int CP = CG / 2;        // channel pairs per plane cell = lanes per tile
     constexpr int CS = plane_cell_pairs(CG), RS = plane_row_pairs(CG);   // plane strides
@@ -523,8 +483,8 @@ __device__ __forceinline__ int out_in_transform_body(
     // once, instead of once for each die that holds a piece of it.
     const int ncg = Kp / CG;
     const int per_die = (n * ncg + 7) >> 3;
-    const int item = (int)(wg & 7) * per_die + (int)(wg >> 3);
-    if (item >= n * ncg) return -1;
+    const int item = (int)(blockIdx.x & 7) * per_die + (int)(blockIdx.x >> 3);
+    if (item >= n * ncg) return;
     const int b = item / ncg;
     const int cg = item - b * ncg;
 
@@ -570,18 +530,12 @@ __device__ __forceinline__ int out_in_transform_body(
     // for it.  The scheduling barrier keeps the compiler from sinking those loads behind
     // the first arithmetic on M.
     pair_t m[36];   // as stored; converted where used
-    // the same two offsets in the slab layout, [36][Kp / CG][Tp][CG]
-    unsigned voff_s = cl * 2 * esz + (valid ? sub : 0u) * (unsigned)CG * esz;
-    asm volatile("" : "+v"(voff_s));
-    const unsigned soff_s =
-        ((unsigned)cg * (unsigned)Tp + (unsigned)(b * kTilesPerBoard + TPW * wave)) *
-        (unsigned)CG * esz;
 #pragma unroll
     for (int xx = 0; xx < 6; xx++) {
-        unsigned so = (MSLAB ? soff_s : soff_t) + (unsigned)xx * pstride;
+        unsigned so = soff_t + (unsigned)xx * pstride;
 #pragma unroll
         for (int row = 0; row < 6; row++) {
-            m[row * 6 + xx] = BufIO2<P>::load_raw(rM, MSLAB ? voff_s : voff_t, so);
+            m[row * 6 + xx] = BufIO2<P>::load_raw(rM, voff_t, so);
             so += 6u * pstride;
         }
         __builtin_amdgcn_sched_barrier(0);   // keep the columns in this order
@@ -603,7 +557,6 @@ __device__ __forceinline__ int out_in_transform_body(
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    LZ_STAMP(1);
     // zero the halo cells of the plane (rows and columns 0, 20, 21): 3 full rows
     // and 3 cells in each of the 19 rows between them; one cell per tile slot
     {
@@ -665,9 +618,7 @@ __device__ __forceinline__ int out_in_transform_body(
             }
         }
     }
-    LZ_STAMP(2);
     __syncthreads();
-    LZ_STAMP(3);
     // The activation leaves only now: stores issued before the barrier would have to be
     // acknowledged before any wavefront may pass it; here they drain under phase 2.
     if (act_out != nullptr) {
@@ -708,39 +659,21 @@ __device__ __forceinline__ int out_in_transform_body(
                 else outp[q].y = (P)d[q];
             }
         }
-        LZ_STAMP(4);
         if (valid) {
-            unsigned so = VSLAB ? soff_s : soff_t, vo = VSLAB ? voff_s : voff_t;
+            unsigned so = soff_t;
 #pragma unroll
             for (int p = 0; p < 36; p++) {
-                BufIO2<P>::template store<VPOL>(outp[p], rV, vo, so);
+                BufIO2<P>::template store<xform_store_policy<CG>()>(outp[p], rV, voff_t, so);
                 so += pstride;
             }
         }
     }
-    LZ_STAMP(5);
-    return item;
-}
-
-// M and Vn may be one array (every value of M is in a register before the same lane writes
-// the value of V that takes its place), so neither is declared free of aliases.
-// SLAB: M and V lie slab by slab, [36][Kp / CG][Tp][CG] (see tile_slab); V's stores are then
-// whole lines and go out write-through.
-template <typename P, int CG, bool SLAB = false>
-__global__ __launch_bounds__(fuse_waves(CG) * 64) void out_in_transform_k(
-    const P* M, const P* __restrict__ res, P* __restrict__ act_out, P* Vn,
-    const float* __restrict__ bn_scale, const float* __restrict__ bn_mean, float rfac, int n,
-    int Kp, int Tp) {
-    __shared__ typename BufIO2<P>::pair_t ybuf[plane_pairs(CG)];
-    (void)out_in_transform_body<P, CG, SLAB ? kStoreThrough : xform_store_policy<CG>(), SLAB,
-                                SLAB>(ybuf, blockIdx.x, M, res, act_out, Vn, bn_scale, bn_mean,
-                                      rfac, n, Kp, Tp);
 }
 
 template <typename P>
 void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const float* bn_scale,
                              const float* bn_mean, float rfac, int n, int Kp, int Tp,
-                             hipStream_t s, LaunchTimer* t, int slab) {
+                             hipStream_t s, LaunchTimer* t) {
     // With few boards a narrow shape spreads a board's arithmetic over more compute units;
     // the 64-channel shape moves whole lines.  Measured at 256 filters with the layers working
     // in place (transform + GEMM per layer, us, with 16 / 32 / 64 channels per work-group):
@@ -751,15 +684,7 @@ void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const 
     // of it (16 channels at batch 16: 11.2 us per launch against 7.7).
     const int items64 = n * (Kp / 64);
     auto grid = [](int items) { return dim3((unsigned)(8 * ((items + 7) / 8))); };
-    if (slab == 16)
-        launch(out_in_transform_k<P, 16, true>, grid(items64 * 4), dim3(fuse_waves(16) * 64), s,
-               t, M, res, act_out, Vn, bn_scale, bn_mean, rfac, n, Kp, Tp);
-    else if (slab == 32)
-        launch(out_in_transform_k<P, 32, true>, grid(items64 * 2), dim3(fuse_waves(32) * 64), s,
-               t, M, res, act_out, Vn, bn_scale, bn_mean, rfac, n, Kp, Tp);
-    else if (slab != 0)
-        throw std::invalid_argument("out_in_transform: slabs are 16 or 32 channels wide");
-    else if (items64 > 80)
+    if (items64 > 80)
         launch(out_in_transform_k<P, 64>, grid(items64), dim3(fuse_waves(64) * 64), s, t, M, res,
                act_out, Vn, bn_scale, bn_mean, rfac, n, Kp, Tp);
     else if (items64 > 64)
@@ -1486,36 +1411,34 @@ __global__ __launch_bounds__(512) void wino_gemm_split_k(const P* __restrict__ V
 }
 
 // ---------------------------------------------------------------------------
-// Filter-stationary streaming GEMM (fp16 storage).  One work-group of NW wavefronts
-// (8 at 256 filters, 6 / 4 / 2 at 192 / 128 / 64) owns one Winograd position and a run of
-// consecutive 32-row blocks of V; wavefront w owns output channels 32w..32w+31 of a
-// column tile of 32 NW channels and keeps its
-// share of U_p -- 32 channels x Cp input channels -- in registers for the whole
-// kernel (Cp/4 registers per lane), already in the order the matrix instruction
-// wants it.  V streams through: a 32-row block (all Cp input channels, so the
-// contraction of those rows completes in one step) is requested kStreamAhead steps
-// ahead into registers and passes through a three-stage LDS ring, where all
-// wavefronts read it as their column operand.  A step multiplies one block; the
-// fragment reads of the block's second half and of the next block's first half are
-// issued ahead of the matrix instructions that hide them, and one barrier ends the
-// step.  Loads of later blocks, matrix instructions and stores of earlier blocks are
-// in flight together from the first block to the last.
+// Filter-stationary streaming GEMM in fp32 (v_mfma_f32_32x32x2_f32, a sixteenth of the fp16
+// matrix rate: this kernel is bound by the matrix pipe, not by the stream).  One work-group of
+// NW wavefronts (8 at 256 filters, 6 / 4 at 192 / 128) owns one Winograd position and a run of
+// consecutive 32-row blocks of V; wavefront w owns output channels 32w..32w+31 and keeps its
+// share of U_p -- 32 channels x Cp input channels -- in Cp/2 registers per lane for the whole
+// kernel, already in the order the matrix instruction wants it.  V streams through: a 32-row
+// block (all Cp input channels, so the contraction of those rows completes in one step) is
+// requested kStreamAhead steps ahead into registers and passes through a three-stage LDS ring,
+// where all wavefronts read it as their column operand, 4 matrix instructions per 16-byte
+// fragment read.  The contraction index is dealt so that one 16-byte read serves four
+// instructions: in instruction 4j + i, lanes 0..31 hold input channel 8j + i and lanes 32..63
+// channel 8j + 4 + i, of U (rows) and of V (columns) alike.
 //
 // Output: register r of lane l of a 32x32 accumulator holds row 8(r/4) + 4(l/32) + r%4
 // of the row operand.  The row operand is U, and the host stores U's channels permuted
 // (gemm_stream_channel) so that this lane's sixteen registers are the channels
-// 16(r/8) + 8(l/32) + r%8 of the wavefront's 32, i.e. two 16-byte runs.  Those go into
-// an LDS copy of the block's 32 x 32 NW result, and one step later (behind the barrier
-// that is there anyway) every wavefront sends its share of the rows, 1 KiB per store
-// instruction.  The stores are write-through (sc0 sc1): whole lines leave for memory
-// while the kernel runs, instead of collecting as dirty lines in the L2 that the end
-// of the kernel has to flush with nothing else in flight (measured at 64 boards and
-// 256 filters: 14.2 -> 12.3 us per launch; in 32-byte pieces straight from the
-// accumulators write-through is slower than write-back).
+// 16(r/8) + 8(l/32) + r%8 of the wavefront's 32, i.e. two runs of eight.  The block's result
+// goes through a single LDS copy (two barriers per step are little beside 128 matrix
+// instructions) and leaves as whole rows, 1 KiB per store instruction, write-through (sc0 sc1):
+// whole lines leave for memory while the kernel runs, instead of collecting as dirty lines in
+// the L2 that the end of the kernel has to flush with nothing else in flight.  (Stored straight
+// from the accumulators instead, 64 bytes per lane with write-back stores and one barrier per
+// step, the kernel is slower: 87 against 83 us per launch at 64 boards and 256 filters, 28
+// against 24 at 128 filters.)
 //
-// Uf layout ("fragment order"): [36][Kp/32][Cp/16][64 lanes][8 halves]; lane l of
-// fragment (p, wb, kc) holds U_p[32 wb + gemm_stream_channel(l % 32)][16 kc + 8 (l / 32) + 0..7],
-// so every operand load of a wavefront is one contiguous KiB.
+// Uf layout: [36][Kp/32][Cp/8][64 lanes][4 floats]; lane l of fragment (p, wb, j) holds
+// U_p[32 wb + gemm_stream_channel(l % 32)][8 j + 4 (l / 32) + 0..3], so every operand load of a
+// wavefront is one contiguous KiB.
 constexpr int kStreamBlocks = 16;  // most 32-row blocks per work-group (steps of the pipeline)
 constexpr int kStreamAhead = 2;    // blocks requested ahead of the one being multiplied
 
@@ -1523,384 +1446,6 @@ __host__ __device__ constexpr int gemm_stream_channel(int i) {
     // i = 8q + 4h + e  ->  16 (q / 2) + 8 h + 4 (q % 2) + e
     return 16 * (i >> 4) + 8 * ((i >> 2) & 1) + 4 * ((i >> 3) & 1) + (i & 3);
 }
-
-// What a fused launch hands the GEMM's work-groups to wait on (see xform_gemm_k): one
-// 64-bit word per (board, channel group) of the transform that produces V in the same
-// launch, set to `epoch` when that work-group's stores have reached memory.
-struct StreamWait {
-    const unsigned long long* flags;
-    unsigned long long epoch;
-    unsigned* gave_up;     // set to 1 if a wait ran into its spin limit
-    int ncg;               // channel groups per board
-};
-constexpr int kFlagSpinLimit = 1 << 18;   // polls of ~0.3 us each before a wait gives up
-
-// LDS of the streaming GEMM in halves: the ring of V blocks (as many stages as the
-// pipeline can use) and two copies of a block's result.
-template <int NKC, int NBLK, int NW> constexpr int gemm_stream_lds_halves() {
-    return (NBLK < 3 ? NBLK : 3) * 32 * (NKC * 16 + 8) + 2 * 32 * (32 * NW + 8);
-}
-
-// FUSED: the work-group is part of a fused launch (xform_gemm_k): it waits for the producers
-// of its rows.  VSLAB / MSLAB > 0: V is read / M is written slab by slab,
-// [Kp / SLAB][Tp][SLAB] per position, instead of row by row, [Tp][Kp] (the layout the narrow
-// transform shapes work in, where a work-group's 25 tiles are one contiguous run).
-template <int NKC, int NBLK, int NW, bool FUSED, int VSLAB = 0, int MSLAB = 0>
-__device__ __forceinline__ void wino_gemm_stream_body(half_t* smem, unsigned wg, const half_t* V,
-                                                      const half_t* __restrict__ Uf, half_t* M,
-                                                      int T, int Tp, int Kp, int chunks,
-                                                      int nblk_total, int tiles_n, int seg,
-                                                      StreamWait wait) {
-    constexpr int D = kStreamAhead;
-    constexpr int NT = 64 * NW;                  // threads: NW wavefronts of 32 output channels
-    constexpr int CW = 32 * NW;                  // width of the column tile
-    constexpr int Cp = NKC * 16;
-    constexpr int HK = NKC / 2;                  // fragments per half block
-    constexpr int CPRW = Cp / 8;                 // 16-byte chunks per row
-    constexpr int NCH = 32 * CPRW;               // chunks per block
-    constexpr int CH = (NCH + NT - 1) / NT;      // chunk loads per thread and block
-    constexpr bool FULL = NCH % NT == 0;         // every thread has all CH chunks
-    constexpr int ROWE = Cp + 8;                 // padded LDS row (halves): conflict-free 16-byte reads
-    constexpr int STAGE = 32 * ROWE;
-    constexpr int OROW = CW + 8;                 // row of the output copy (halves)
-    constexpr int OSTAGE = 32 * OROW;
-    static_assert(NKC % 2 == 0 && D == 2, "pipeline shape");
-    constexpr int SLAB = VSLAB;
-    static_assert((VSLAB == 0 || VSLAB == 16 || VSLAB == 32) &&
-                      (MSLAB == 0 || MSLAB == 16 || MSLAB == 32),
-                  "slab widths");
-
-    constexpr int NST = NBLK < 3 ? NBLK : 3;     // stages of the ring in use
-    static_assert(NST * STAGE + 2 * OSTAGE == gemm_stream_lds_halves<NKC, NBLK, NW>(), "LDS size");
-    half_t* const obuf = smem + NST * STAGE;
-
-    const int n_items = kPos * chunks * tiles_n;
-    const int xcd = wg & 7;
-    const int item = xcd * seg + (int)(wg >> 3);
-    if ((int)(wg >> 3) >= seg || item >= n_items) return;
-    const int tn = item % tiles_n;
-    const int rest = item / tiles_n;
-    const int ch = rest % chunks;
-    const int p = rest / chunks;
-    // this work-group's real blocks: [blk0, blk1), at most NBLK of them
-    const int blk0 = (ch * nblk_total) / chunks;
-    const int blk1 = ((ch + 1) * nblk_total) / chunks;
-    const int nreal = blk1 - blk0;
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int hh = lane >> 5, jrow = lane & 31;
-
-    // chunk coordinates of this thread's loads within a block
-    int lrow[CH], lcc[CH];
-    bool lval[CH];
-    unsigned lslab[CH];   // slab layout: byte offset of the chunk's slab and place in its row
-#pragma unroll
-    for (int i = 0; i < CH; i++) {
-        const int idx = tid + i * NT;
-        lval[i] = FULL || idx < NCH;
-        if constexpr (SLAB > 0) {
-            // a wavefront's 64 chunks are consecutive rows of one slab: one contiguous KiB
-            constexpr int CPS = SLAB / 8;               // chunks per row of a slab
-            const int g = idx / (32 * CPS), rem = idx % (32 * CPS);
-            lrow[i] = rem / CPS;
-            lcc[i] = g * CPS + rem % CPS;
-            lslab[i] = ((unsigned)g * (unsigned)Tp * SLAB + (unsigned)(rem % CPS) * 8u) * 2u;
-        } else {
-            lrow[i] = (idx / CPRW) & 31;
-            lcc[i] = idx % CPRW;
-            lslab[i] = 0;
-        }
-    }
-    const half_t* Vp = V + (size_t)p * Tp * Cp;
-
-    int4v st[D][CH];
-    // In a fused launch V has just been written by work-groups of the same launch on other
-    // dies: its loads carry the device-scope policy (sc1), which takes them past this
-    // die's caches to where those (written-through) stores went.
-    const __amdgpu_buffer_rsrc_t rV = make_rsrc(Vp, (size_t)Tp * Cp * sizeof(half_t));
-    auto gload = [&](int slot, int s) {
-        // steps past the last real block re-read that block (cache hits, never stored)
-        const int blk = blk0 + (s < nreal ? s : nreal - 1);
-#pragma unroll
-        for (int i = 0; i < CH; i++) {
-            const int row = min(blk * 32 + lrow[i], T - 1);
-            if (lval[i]) {
-                if constexpr (SLAB > 0)
-                    st[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(
-                        rV, lslab[i] + (unsigned)row * (unsigned)(SLAB * 2), 0, FUSED ? 16 : 0);
-                else if constexpr (FUSED)
-                    st[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(
-                        rV, (unsigned)(row * Cp + lcc[i] * 8) * 2u, 0, 16);
-                else
-                    st[slot][i] =
-                        *reinterpret_cast<const int4v*>(Vp + (size_t)row * Cp + lcc[i] * 8);
-            }
-        }
-    };
-    auto lstore = [&](int slot, int buf) {
-        half_t* S = smem + buf * STAGE;
-#pragma unroll
-        for (int i = 0; i < CH; i++)
-            if (lval[i]) *reinterpret_cast<int4v*>(&S[lrow[i] * ROWE + lcc[i] * 8]) = st[slot][i];
-    };
-
-    // The first two blocks of V, then this wavefront's share of U in the order the
-    // multiplication uses it.  (Completion is counted in issue order: the LDS stores below
-    // wait for V only, and each matrix instruction of the first step only for the filter
-    // fragments up to its own, so the first step starts while most of U is still arriving:
-    // -0.5 us per launch at 64 boards against U first.)
-    int4v u[NKC];
-    const half_t* Up =
-        Uf + ((((size_t)p * (Kp / 32) + (size_t)tn * NW + wave) * NKC) * 64 + lane) * 8;
-    if constexpr (FUSED) {
-        // The filters depend on nothing in this launch: they are requested first and
-        // arrive while the transform work-groups are still producing V.  Then wait for the
-        // transform work-groups of every board that has a tile among this work-group's rows.
-#pragma unroll
-        for (int kc = 0; kc < NKC; kc++)
-            u[kc] = *reinterpret_cast<const int4v*>(Up + (size_t)kc * 64 * 8);
-        LZ_STAMP(10);
-        const int row_lo = blk0 * 32, row_hi = min(blk1 * 32, T);
-        const int b_lo = row_lo / kTilesPerBoard, b_hi = (row_hi - 1) / kTilesPerBoard;
-        const int nflags = (b_hi - b_lo + 1) * wait.ncg;
-        const unsigned long long* f = wait.flags + (size_t)b_lo * wait.ncg;
-        for (int i = tid; i < nflags; i += NT) {
-            int polls = 0;
-            while (__hip_atomic_load(f + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
-                   wait.epoch) {
-                __builtin_amdgcn_s_sleep(2);
-                if (++polls > kFlagSpinLimit) {   // never hang: report and go on
-                    __hip_atomic_store(wait.gave_up, 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_SYSTEM);
-                    break;
-                }
-            }
-        }
-        __syncthreads();
-        LZ_STAMP(11);
-        gload(0, 0);
-        if (NBLK > 1) gload(1, 1);
-    } else {
-        gload(0, 0);
-        if (NBLK > 1) gload(1, 1);
-#pragma unroll
-        for (int kc = 0; kc < NKC; kc++)
-            u[kc] = *reinterpret_cast<const int4v*>(Up + (size_t)kc * 64 * 8);
-    }
-    lstore(0, 0);
-    if (NBLK > 1) lstore(1, 1);
-    __syncthreads();
-    LZ_STAMP(12);
-
-    // M goes out through a raw buffer whose extent is the T real rows of this position:
-    // rows past the last tile, and the steps past this work-group's last block, get an
-    // offset outside it and are dropped by the hardware, so the stores are unconditional
-    // straight-line code (a branch around them would make the compiler wait for every
-    // outstanding load behind it).
-    const size_t m_bytes = (size_t)(MSLAB > 0 ? Tp : T) * Kp * sizeof(half_t);
-    const __amdgpu_buffer_rsrc_t rM = make_rsrc(M + (size_t)p * Tp * Kp, m_bytes);
-    const unsigned m_rowb = (unsigned)Kp * 2u;
-    // The 32 x CW result leaves in 16-byte pieces, two per thread.  Eight wavefronts:
-    // wavefront w sends rows 4w..4w+3, two whole 512-byte rows per store instruction.  Fewer:
-    // the pieces are dealt to the threads in memory order (a row holds CW / 8 of them), so
-    // that a store instruction still writes one contiguous KiB when the tile is the whole row.
-    // Slabs: a slab's share of the block (32 rows x MSLAB channels) is contiguous, and the
-    // pieces are dealt in that order, so a store instruction again writes one contiguous KiB.
-    constexpr int PPR = CW / 8;
-    auto send_rows = [&](int s) {
-        const half_t* O = obuf + (s & 1) * OSTAGE;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            int r, cc;
-            if constexpr (MSLAB > 0) {
-                constexpr int PR = MSLAB / 8;              // pieces per row of a slab
-                const int piece = tid + i * NT;
-                const int g = piece / (32 * PR), rem = piece - g * (32 * PR);
-                r = rem / PR;
-                cc = g * PR + (rem - r * PR);
-            } else if constexpr (NW == 8) {
-                r = wave * 4 + hh + 2 * i;
-                cc = jrow;
-            } else {
-                const int piece = tid + i * NT;
-                r = piece / PPR;
-                cc = piece - r * PPR;
-            }
-            const int4v v = *reinterpret_cast<const int4v*>(O + r * OROW + cc * 8);
-            const unsigned row = (unsigned)((blk0 + s) * 32 + r);
-            unsigned vo;
-            if constexpr (MSLAB > 0) {
-                constexpr int PR = MSLAB / 8;
-                const unsigned slab = (unsigned)(tn * (CW / MSLAB) + cc / PR);
-                vo = (s < nreal && row < (unsigned)T)
-                         ? ((slab * (unsigned)Tp + row) * (unsigned)MSLAB + (unsigned)(cc % PR) * 8u) * 2u
-                         : 0x7ffffff0u;
-            } else {
-                vo = s < nreal ? row * m_rowb + (unsigned)(tn * CW + cc * 8) * 2u : 0x7ffffff0u;
-            }
-            __builtin_amdgcn_raw_buffer_store_b128(v, rM, vo, 0, kStoreThrough);
-        }
-    };
-
-    const int frag = jrow * ROWE + hh * 8;
-    int4v alo[HK], ahi[HK];
-#pragma unroll
-    for (int kc = 0; kc < HK; kc++) alo[kc] = *reinterpret_cast<const int4v*>(smem + frag + kc * 16);
-
-    // Every work-group runs all NBLK steps; those past its last block multiply stale data and
-    // store nothing.  (Leaving after nreal steps, with the blocks split evenly over 7
-    // work-groups per position at every batch, was measured and is slower in this kernel,
-    // which the stream bounds: one lane -1 % at 64 boards, -6 % at 96, +5 % at 40.)
-#pragma unroll
-    for (int s = 0; s < NBLK; s++) {
-        if (s + D < NBLK) gload(s % D, s + D);
-        if (s > 0) send_rows(s - 1);
-        const half_t* S = smem + (s % 3) * STAGE + frag;
-#pragma unroll
-        for (int kc = 0; kc < HK; kc++)
-            ahi[kc] = *reinterpret_cast<const int4v*>(S + (HK + kc) * 16);
-        __builtin_amdgcn_sched_barrier(0);
-        float16v acc;
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-#pragma unroll
-        for (int kc = 0; kc < HK; kc++)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, u[kc]),
-                                                         __builtin_bit_cast(half8v, alo[kc]), acc,
-                                                         0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + 1 < NBLK) {
-            const half_t* Sn = smem + ((s + 1) % 3) * STAGE + frag;
-#pragma unroll
-            for (int kc = 0; kc < HK; kc++)
-                alo[kc] = *reinterpret_cast<const int4v*>(Sn + kc * 16);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int kc = 0; kc < HK; kc++)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, u[HK + kc]),
-                                                         __builtin_bit_cast(half8v, ahi[kc]), acc,
-                                                         0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + 2 < NBLK) lstore((s + 2) % D, (s + 2) % 3);
-        half8v o0, o1;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            o0[e] = to_storage<half_t>(acc[e]);
-            o1[e] = to_storage<half_t>(acc[8 + e]);
-        }
-        half_t* O = obuf + (s & 1) * OSTAGE + jrow * OROW + wave * 32 + hh * 8;
-        *reinterpret_cast<half8v*>(O) = o0;
-        *reinterpret_cast<half8v*>(O + 16) = o1;
-        __syncthreads();
-        LZ_STAMP(13 + s);
-    }
-    send_rows(NBLK - 1);
-}
-
-// V and M may be one array when the tile is the whole row of M (tiles_n == 1, as many input
-// as output channels): a work-group has a block of V in LDS before it writes the block of M
-// that takes its place, and no other work-group touches those rows.
-template <int NKC, int NBLK, int NW, int VSLAB = 0, int MSLAB = 0>
-__global__ __launch_bounds__(64 * NW) void wino_gemm_stream_k(const half_t* V,
-                                                          const half_t* __restrict__ Uf,
-                                                          half_t* M, int T, int Tp,
-                                                          int Kp, int chunks, int nblk_total,
-                                                          int tiles_n, int seg) {
-    __shared__ __attribute__((aligned(16))) half_t smem[gemm_stream_lds_halves<NKC, NBLK, NW>()];
-    wino_gemm_stream_body<NKC, NBLK, NW, false, VSLAB, MSLAB>(
-        smem, blockIdx.x, V, Uf, M, T, Tp, Kp, chunks, nblk_total, tiles_n, seg, StreamWait{});
-}
-
-// ---------------------------------------------------------------------------
-// One launch for the fused transform of layer l (M_l -> V_{l+1}) and the GEMM of layer l+1
-// (V_{l+1} -> M_{l+1}), for small batches.  Two dependent launches cost a hand-over of
-// ~2.4 us between them whatever their size, and a GEMM work-group spends its first ~2 us
-// fetching 128 KiB of filters that depend on nothing: at 16 boards those two are a third of
-// a layer.  Here the launch's first work-groups run the transform and the rest the GEMM.
-// The GEMM work-groups request their filters at once, then wait, per board whose tiles
-// they multiply, for a word that each transform work-group sets (to the launch's `epoch`,
-// a number that grows with every fused launch of a lane, so nothing has to be cleared)
-// after its stores of V -- written through, with the device-scope policy -- have been
-// acknowledged; the GEMM work-groups read V with the same policy.  (Release and acquire
-// fences in their place would write back and invalidate a die's whole L2 once per wavefront:
-// measured 60 us per launch at 16 boards.)  With few boards the transform leaves compute
-// units free, and the GEMM work-groups that start there have their filters by the time V
-// is ready; from 16 boards they follow as the transform's work-groups retire, and the
-// launch still saves the hand-over.
-//
-// Waiting is safe because the waiters never hold what the producers need: work-groups are
-// dispatched in the order of their index, so every transform work-group is resident (or
-// done) before the first GEMM work-group starts, and a transform work-group waits for
-// nothing.  A wait is bounded all the same: after kFlagSpinLimit polls it reports through
-// `gave_up` and goes on, so that the launch always ends.
-//
-// The buffers: the transform reads M and writes V, the GEMM reads V and writes M -- the
-// same M.  A GEMM work-group writes rows of M only after every transform work-group of
-// the boards those rows belong to has finished, i.e. after their last read.  V and M are
-// normally one array, each stage overwriting its input, as the separate launches do.
-// SLAB: both lie slab by slab, [36][Kp / CG][Tp][CG] (tile_slab), so that the transform reads
-// and writes whole lines; row by row, its written-through 32- and 64-byte pieces of V land in
-// lines that the die's L2 already holds from reading M.
-template <int CG, int NBLK, int NW, bool SLAB>
-__global__ __launch_bounds__(64 * (NW > fuse_waves(CG) ? NW : fuse_waves(CG))) void xform_gemm_k(
-    half_t* M, const half_t* res, half_t* act_out, half_t* V, const float* __restrict__ bn_scale,
-    const float* __restrict__ bn_mean, float rfac, int n, int Kp, int Tp,
-    const half_t* __restrict__ Uf, int T, int chunks, int nblk_total, int tiles_n, int seg,
-    unsigned n_xform_wg, unsigned long long* flags, unsigned long long epoch, unsigned* gave_up) {
-    typedef BufIO2<half_t>::pair_t pair_t;
-    constexpr int NKC = 2 * NW;      // tower layers: as many input as output channels
-    constexpr int XBYTES = plane_pairs(CG) * (int)sizeof(pair_t);
-    constexpr int GBYTES = gemm_stream_lds_halves<NKC, NBLK, NW>() * 2;
-    // More than half of a compute unit's 160 KiB, whatever the roles need: two work-groups of
-    // this launch never share a unit.  A GEMM work-group beside a transform work-group sends
-    // its 128 KiB of filters through the memory pipeline that the transform -- which the
-    // whole launch waits for -- is using (measured at 16 boards: 16.7 us per launch with
-    // sharing, also with the filter requests spread out in time, 16.1 without).
-    constexpr int ALONE = 82 * 1024;
-    constexpr int NEED = XBYTES > GBYTES ? XBYTES : GBYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NEED > ALONE ? NEED : ALONE];
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    LZ_STAMP(0);
-    if (blockIdx.x < n_xform_wg) {
-        if (wave >= fuse_waves(CG)) return;    // the block is sized for the larger role
-        const int item = out_in_transform_body<half_t, CG, kStoreThrough, SLAB, SLAB>(
-            reinterpret_cast<pair_t*>(lds), blockIdx.x, M, res, act_out, V, bn_scale, bn_mean,
-            rfac, n, Kp, Tp);
-        if (item < 0) return;                  // uniform over the work-group
-        // V was stored write-through: once a wavefront's stores are acknowledged they are in
-        // memory, past every die's cache.  All wavefronts wait for that, then one word says so.
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        LZ_STAMP(6);
-        __syncthreads();
-        if (threadIdx.x == 0)
-            __hip_atomic_store(flags + item, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        LZ_STAMP(7);
-    } else {
-        if (wave >= NW) return;
-        wino_gemm_stream_body<NKC, NBLK, NW, true, SLAB ? CG : 0, SLAB ? CG : 0>(
-            reinterpret_cast<half_t*>(lds), blockIdx.x - n_xform_wg, V, Uf, M, T, Tp, Kp, chunks,
-            nblk_total, tiles_n, seg, StreamWait{flags, epoch, gave_up, Kp / CG});
-    }
-}
-
-// ---------------------------------------------------------------------------
-// The same filter-stationary structure in fp32 (v_mfma_f32_32x32x2_f32, a sixteenth of
-// the fp16 matrix rate: this kernel is bound by the matrix pipe, not by the stream).
-// Wavefront w keeps U_p for its 32 output channels in Cp/2 registers per lane; a step
-// multiplies one 32-row block of V, 4 matrix instructions per 16-byte fragment read, so
-// that nothing but the matrix pipe is busy for long.  The contraction index is dealt so
-// that one 16-byte read serves four instructions: in instruction 4j + i, lanes 0..31
-// hold input channel 8j + i and lanes 32..63 channel 8j + 4 + i, of U (rows) and of V
-// (columns) alike.  The block's result goes through a single LDS copy (two barriers per
-// step are little beside 128 matrix instructions) and leaves as whole rows, written
-// through, as in the fp16 kernel.  (Stored straight from the accumulators instead, 64
-// bytes per lane with write-back stores and one barrier per step, the kernel is slower:
-// 87 against 83 us per launch at 64 boards and 256 filters, 28 against 24 at 128 filters.)
-//
-// Uf layout: [36][Kp/32][Cp/8][64 lanes][4 floats]; lane l of fragment (p, wb, j) holds
-// U_p[32 wb + gemm_stream_channel(l % 32)][8 j + 4 (l / 32) + 0..3].
 
 template <int NK8, int NBLK, int NW>
 __global__ __launch_bounds__(64 * NW) void wino_gemm_stream32_k(const float* V,   // may be M
@@ -2049,14 +1594,10 @@ __global__ __launch_bounds__(64 * NW) void wino_gemm_stream32_k(const float* V, 
     send_rows(last);
 }
 
-// Fragment-order copy of one layer's filters for the streaming kernels, built on the host
-// in fp32 (fp16 nets convert on the device, convert_filters): src is the reference layout
-// [36][C][F] (F fastest); dst is [36][Kp/32][Cp/16][64][8] for wino_gemm_stream_k
-// (elem_bytes 2) and [36][Kp/32][Cp/8][64][4] for wino_gemm_stream32_k (elem_bytes 4), zero
-// padded: a fragment is G consecutive input channels per lane, G = 16 / elem_bytes.
-void build_stream_filters(const float* src, int C, int F, int Cp, int Kp, int elem_bytes,
-                          float* dst) {
-    const int G = 16 / elem_bytes;             // values per lane and fragment
+// Fragment-order copy of one layer's filters for the streaming kernel: src is the reference
+// layout [36][C][F] (F fastest), dst [36][Kp/32][Cp/8][64][4], zero padded.
+void build_stream_filters(const float* src, int C, int F, int Cp, int Kp, float* dst) {
+    constexpr int G = 4;                       // values per lane and fragment
     const int nfr = Cp / (2 * G), nwb = Kp / 32;
     for (int p = 0; p < kPos; p++)
         for (int wb = 0; wb < nwb; wb++)
@@ -2088,18 +1629,7 @@ void convert_filters(const float* src, half_t* dst, size_t n, hipStream_t s) {
                        dim3(256), 0, s, src, dst, n);
 }
 
-// Blocks per work-group for T tile rows in the fp16 kernel: the fewest (a power of two up
-// to kStreamBlocks) with which one round of work-groups covers the 256 compute units, so
-// that a batch of 8 boards runs one block per work-group, 64 boards eight and 128 sixteen.
-static int gemm_stream_blocks(int T, int Kp) {
-    const int nblk = (T + 31) / 32;
-    const int per_pos = 256 / (kPos * ((Kp + 255) / 256));   // work-groups per position in one round
-    int nb = 1;
-    while (nb < kStreamBlocks && (nblk + nb - 1) / nb > per_pos) nb *= 2;
-    return nb;
-}
-
-// The fp32 kernel's split of a position's 32-row blocks over work-groups: as many work-groups per
+// The split of a position's 32-row blocks over work-groups: as many work-groups per
 // position as one round over the 256 compute units allows (7 at one column tile: 252
 // work-groups), fewer when there are fewer blocks, more when a work-group would otherwise
 // get more than kStreamBlocks.  A work-group takes floor or ceil of blocks / chunks and
@@ -2117,215 +1647,21 @@ static StreamSplit gemm_stream_split(int T, int Kp) {
     return {chunks, nb};
 }
 
-// Whether launch_gemm takes a streaming kernel for this shape when it is handed the
-// fragment-order filters: input layer (64 padded planes) and tower layers, any batch, of nets
-// of 128, 192 and 256 filters in both storage types (one column tile of Kp / 32 wavefronts;
-// at 64 filters the tiled kernel is as fast: 3.0 against 3.5 us at 4 boards, 3.5 against 3.5 at
-// 33).  fp32, tiled -> streaming: 256 filters 88 -> 79-83 us per launch at 64 boards, 78 -> 58 at
-// 48, 22 -> 13 at 8; 128 filters 27 -> 23 at 64 boards.  At 192 filters in fp32 six wavefronts
-// sit unevenly on four SIMDs: the streaming kernel is ahead up to 24 boards on one lane (15x192
-// forwards +6 % at 1 board, +11 % at 8, +20 % at 16, +10 % at 24; all lanes +4 % at 8, +2 % at 16,
-// -15 % at 24) and behind beyond (-4 % at 32, -8 % at 64): gemm_stream_prefers says which kernel
-// family a handle of a given batch limit holds the filters for.  One family per handle keeps a
-// position's result independent of the batch it is evaluated in.
+// Whether launch_gemm takes the streaming kernel for this shape when it is handed the
+// fragment-order filters: input layer (64 padded planes) and tower layers, any batch, of fp32
+// nets of 128, 192 and 256 filters (one column tile of Kp / 32 wavefronts).  Tiled -> streaming:
+// 256 filters 88 -> 79-83 us per launch at 64 boards, 78 -> 58 at 48, 22 -> 13 at 8; 128 filters
+// 27 -> 23 at 64 boards.  At 192 filters six wavefronts sit unevenly on four SIMDs: the
+// streaming kernel is ahead up to 24 boards on one lane (15x192 forwards +6 % at 1 board, +11 %
+// at 8, +20 % at 16, +10 % at 24; all lanes +4 % at 8, +2 % at 16, -15 % at 24) and behind beyond
+// (-4 % at 32, -8 % at 64): gemm_stream_prefers says which kernel family a handle of a given
+// batch limit holds the filters for.  One family per handle keeps a position's result
+// independent of the batch it is evaluated in.
 bool gemm_stream_shape(int T, int Cp, int Kp, int elem_bytes) {
-    (void)elem_bytes;
-    if (T < 1 || !(Cp == 64 || Cp == Kp)) return false;
+    if (elem_bytes != 4 || T < 1 || !(Cp == 64 || Cp == Kp)) return false;
     return Kp == 128 || Kp == 256 || Kp == 192;
 }
-bool gemm_stream_prefers(int Kp, int elem_bytes, int max_batch) {
-    return !(Kp == 192 && elem_bytes == 4 && max_batch > 16);
-}
-
-template <int NKC, int NW>
-static void launch_gemm_stream_nkc(const half_t* V, const half_t* Uf, half_t* M, int T, int Tp,
-                                   int Kp, hipStream_t s, LaunchTimer* t, int slab) {
-    const int nblk = (T + 31) / 32;
-    const int nb = gemm_stream_blocks(T, Kp);
-    const int chunks = (nblk + nb - 1) / nb;
-    const int tiles_n = Kp / (32 * NW);
-    const int n_items = kPos * chunks * tiles_n;
-    int seg = (n_items + 7) / 8;
-    seg = (seg + tiles_n - 1) / tiles_n * tiles_n;
-    const dim3 grid(8 * seg), block(64 * NW);
-#define LZ_STREAM(NB, VS, MS)                                                                     \
-    launch(wino_gemm_stream_k<NKC, NB, NW, VS, MS>, grid, block, s, t, V, Uf, M, T, Tp, Kp,      \
-           chunks, nblk, tiles_n, seg)
-    // slabs: the first layer reads its 64 input planes row by row (NKC == 4) and writes slabs;
-    // the pairs (slab width, blocks per work-group) are those tile_slab hands out
-    constexpr bool FIRST = NKC == 4;
-    if (slab == 16) {
-        switch (nb) {
-            case 1: LZ_STREAM(1, FIRST ? 0 : 16, 16); return;
-            case 2: LZ_STREAM(2, FIRST ? 0 : 16, 16); return;
-            case 4: LZ_STREAM(4, FIRST ? 0 : 16, 16); return;
-            default: break;
-        }
-    } else if (slab == 32) {
-        switch (nb) {
-            case 2: LZ_STREAM(2, FIRST ? 0 : 32, 32); return;
-            case 4: LZ_STREAM(4, FIRST ? 0 : 32, 32); return;
-            case 8: LZ_STREAM(8, FIRST ? 0 : 32, 32); return;
-            default: break;
-        }
-    }
-    if (slab != 0) throw std::invalid_argument("no slab-layout GEMM instantiated for this batch");
-    switch (nb) {
-        case 1: LZ_STREAM(1, 0, 0); break;
-        case 2: LZ_STREAM(2, 0, 0); break;
-        case 4: LZ_STREAM(4, 0, 0); break;
-        case 8: LZ_STREAM(8, 0, 0); break;
-        default: LZ_STREAM(16, 0, 0); break;
-    }
-#undef LZ_STREAM
-}
-
-// NW = Kp / 32 wavefronts per work-group; the first layer reads the 64 padded input planes.
-template <int NW>
-static void launch_gemm_stream_nw(const half_t* V, const half_t* Uf, half_t* M, int T, int Tp,
-                                  int Cp, int Kp, hipStream_t s, LaunchTimer* t, int slab) {
-    if (Cp == 64)
-        launch_gemm_stream_nkc<4, NW>(V, Uf, M, T, Tp, Kp, s, t, slab);
-    else
-        launch_gemm_stream_nkc<2 * NW, NW>(V, Uf, M, T, Tp, Kp, s, t, slab);
-}
-
-static void launch_gemm_stream(const half_t* V, const half_t* Uf, half_t* M, int T, int Tp,
-                               int Cp, int Kp, hipStream_t s, LaunchTimer* t, int slab) {
-    switch (Kp) {
-        case 256: launch_gemm_stream_nw<8>(V, Uf, M, T, Tp, Cp, Kp, s, t, slab); break;
-        case 192: launch_gemm_stream_nw<6>(V, Uf, M, T, Tp, Cp, Kp, s, t, slab); break;
-        default: launch_gemm_stream_nw<4>(V, Uf, M, T, Tp, Cp, Kp, s, t, slab); break;
-    }
-}
-
-// The layout of the tile arrays for a forward of n boards: 0 = row by row, [36][Tp][Kp];
-// 16 or 32 = slab by slab, [36][Kp / w][Tp][w], for the batches that take the transform
-// shapes of that many channels per work-group (fp16 towers of 128, 192 and 256 filters).  A
-// transform work-group (one board, w channels) then reads and writes its 25 tiles as one
-// contiguous run of 25 w values per Winograd position instead of 25 pieces of 2 w bytes, and
-// the GEMM reads and writes a slab's share of a 32-row block as one contiguous run: the same
-// bytes in a quarter (an eighth) of the requests to the L2s.  Measured, transform alone at
-// 256 filters, rows / slabs: 16 boards 7.0 / 6.0 us, 24 boards 9.2 (64-channel shape) / 7.3,
-// 32 boards 9.3 / 7.8; from 40 boards the 64-channel shape (whole lines anyway) is level.
-// Forwards, evaluations/s, rows -> slabs (best launch form each):
-//   40x256 one lane: 1 board +6 %, 4 +10 %, 8 +9 %, 12 +8 %, 16 +10 %, 20 +2 %, 24 +3 %,
-//          28 +6 %, 32 +6 %; three lanes: 12 +8 %, 16 +5 %, 20 +4 %, 24 -8 %, 28 -3 %, 32 -2 %
-//   15x192 one lane: 1 to 4 +8 %, 8 +12 %, 16 +15 %, 21 +16 %, 26 +3 %, 32 +8 %, 42 0 %;
-//          three lanes: 8 and 12 -3 %, 16 0 % (two lanes +13 %), 21 +11 %, 26 +14 %, 42 +4 %
-//   10x128 one lane: 1 to 8 +3..6 %, 16 +10 %, 24 +8 %, 32 +15 %, 40 +4 %, 48 0 %, 64 -1 %;
-//          three lanes: 16 -1 % (two lanes +9 %), 32 +2 %, 40 +8 %, 48 0 %, two lanes at 64 -5 %
-// hence: every such batch at 192 filters, up to 44 boards at 128, and at 256 filters up to
-// 20 boards, or up to 32 when the forward has the device to itself (`alone`).
-int tile_slab(int n, int Kp, int elem_bytes, bool alone) {
-    if (!xform_gemm_shape(n, Kp, elem_bytes)) return 0;
-    if (Kp == 256 && n > 20 && !alone) return 0;
-    if (Kp == 128 && n > 44) return 0;
-    return n * (Kp / 64) <= 64 ? 16 : 32;
-}
-
-// Shapes served by the fused transform + GEMM launch: fp16 towers of 128, 192 and 256
-// filters (the widths of the streaming GEMM) at batches that take the narrow transform
-// shapes (up to 32 boards at 256 filters, 42 at 192, 64 at 128).
-bool xform_gemm_shape(int n, int Kp, int elem_bytes) {
-    return elem_bytes == 2 && (Kp == 128 || Kp == 192 || Kp == 256) && n >= 1 &&
-           n * (Kp / 64) <= 128;
-}
-
-// Whether the fused launch is the faster way to run a forward of n boards whose tile arrays
-// lie in slabs of `slab` channels (0: row by row), with the device to itself (`alone`) or
-// shared with other lanes' forwards.  Measured (40x256 / 15x192 / 10x128, evaluations per
-// second against separate launches):
-//   alone, slabs: the launch pays where the transform's work-groups fill the device in one
-//     round (n Kp / slab between 232 and 256), so that GEMM work-groups, which have fetched
-//     their filters meanwhile, start as those retire instead of after a hand-over between
-//     launches: 256 filters +3 % at 16 and 32 boards, 192 filters +4 % at 21 and +6 % at 42,
-//     128 filters +5 % at 32; elsewhere -1..-10 % (256 filters: 8 to 12 boards -3..-6 %, 24
-//     and 28 -4 %).  And at 256 filters up to 7 boards, where most of the device is free for
-//     GEMM work-groups that fetch 128 KiB of filters each while the transform runs: +16 % at
-//     1 board, +14 % at 2, +10 % at 3 and 4, +6 % at 5, +2 % at 6 (192 and 128 filters have a
-//     half and a quarter of those bytes to hide: 0..-7 % up to 8 boards).
-//   not alone, slabs: with few boards the device is mostly idle, and a lane's waiting GEMM
-//     work-groups take nothing from the other lanes: three lanes, 256 filters +35 % at 3
-//     boards, +19 % at 5, 0 % at 6, -17 % at 8; 192 filters +72 % at 1, +46 % at 2, +54 % at 4,
-//     +12 % at 8, -10 % at 16; 128 filters +55 % at 1 to 4, +10 % at 8, -14 % at 16; two lanes
-//     the same up to 4 or 5 boards (+7..37 %) and -1..-10 % at 8: taken up to 5 (256) or 6 boards.
-//   rows (what is left of them: 128 filters from 45 boards, alone): +8 % at 48, +25 % at 64.
-bool xform_gemm_pays(int n, int Kp, int slab, bool alone) {
-    if (slab == 0) return alone && Kp == 128 && n >= 32;
-    if (!alone) return n <= (Kp == 256 ? 5 : 6);
-    const int groups = n * (Kp / slab);
-    return (groups >= 232 && groups <= 256) || (Kp == 256 && n <= 7);
-}
-
-template <int CG, int NBLK, int NW, bool SLAB>
-static void launch_xform_gemm_as(half_t* M, const half_t* res, half_t* act_out, half_t* V,
-                                 const float* bn_scale, const float* bn_mean, float rfac, int n,
-                                 int Kp, int Tp, const half_t* Uf, unsigned long long* flags,
-                                 unsigned long long epoch, unsigned* gave_up, hipStream_t s) {
-    const int T = n * kTilesPerBoard;
-    const int nblk = (T + 31) / 32;
-    const int chunks = (nblk + NBLK - 1) / NBLK;
-    const int tiles_n = Kp / (32 * NW);
-    const int seg = (kPos * chunks * tiles_n + 7) / 8;
-    const unsigned n_xform_wg = 8u * (unsigned)((n * (Kp / CG) + 7) / 8);
-    constexpr int WAVES = NW > fuse_waves(CG) ? NW : fuse_waves(CG);
-    hipLaunchKernelGGL((xform_gemm_k<CG, NBLK, NW, SLAB>),
-                       dim3(n_xform_wg + 8u * (unsigned)seg), dim3(64 * WAVES), 0, s, M, res,
-                       act_out, V, bn_scale, bn_mean, rfac, n, Kp, Tp, Uf, T, chunks, nblk, tiles_n,
-                       seg, n_xform_wg, flags, epoch, gave_up);
-}
-
-template <int NW>
-static void launch_xform_gemm_nw(half_t* M, const half_t* res, half_t* act_out, half_t* V,
-                                 const float* bn_scale, const float* bn_mean, float rfac, int n,
-                                 int Kp, int Tp, const half_t* Uf, unsigned long long* flags,
-                                 unsigned long long epoch, unsigned* gave_up, hipStream_t s,
-                                 int slab) {
-    const int nb = gemm_stream_blocks(n * kTilesPerBoard, Kp);
-    const bool narrow = n * (Kp / 64) <= 64;     // 16-channel transform groups, else 32
-#define LZ_FUSED(CG, NB, SLAB)                                                                  \
-    launch_xform_gemm_as<CG, NB, NW, SLAB>(M, res, act_out, V, bn_scale, bn_mean, rfac, n, Kp,    \
-                                           Tp, Uf, flags, epoch, gave_up, s)
-    // the pairs that occur: 16-channel groups up to 64 / (Kp / 64) boards, i.e. up to 7, 14 or
-    // (128 filters) 25 blocks of 32 rows per position; 32-channel groups up to twice that
-    if (slab != 0) {   // both arrays slab by slab (they may be one)
-        if (slab != (narrow ? 16 : 32))
-            throw std::invalid_argument("fused launch: the slab width follows the batch");
-        if (narrow && nb == 1) LZ_FUSED(16, 1, true);
-        else if (narrow && nb == 2) LZ_FUSED(16, 2, true);
-        else if (narrow && nb == 4) LZ_FUSED(16, 4, true);
-        else if (!narrow && nb == 2) LZ_FUSED(32, 2, true);
-        else if (!narrow && nb == 4) LZ_FUSED(32, 4, true);
-        else if (!narrow && nb == 8) LZ_FUSED(32, 8, true);
-        else throw std::invalid_argument("no fused launch instantiated for this batch");
-        return;
-    }
-    if (V != M) throw std::invalid_argument("fused launch: row by row, V and M are one array");
-    if (narrow && nb == 1) LZ_FUSED(16, 1, false);
-    else if (narrow && nb == 2) LZ_FUSED(16, 2, false);
-    else if (narrow && nb == 4) LZ_FUSED(16, 4, false);
-    else if (!narrow && nb == 2) LZ_FUSED(32, 2, false);
-    else if (!narrow && nb == 4) LZ_FUSED(32, 4, false);
-    else if (!narrow && nb == 8) LZ_FUSED(32, 8, false);
-    else throw std::invalid_argument("no fused launch instantiated for this batch");
-#undef LZ_FUSED
-}
-
-// slab: 0 (V and M one array, row by row) or tile_slab's width (slab by slab; one array or two).
-// flags: kFusedFlagsPerBoard words per board of the largest batch, zero before the first
-// launch; epoch: a number no earlier launch on these flags has used (grows by one per launch).
-void launch_xform_gemm(half_t* M, const half_t* res, half_t* act_out, half_t* V,
-                       const float* bn_scale, const float* bn_mean, float rfac, int n, int Kp,
-                       int Tp, const half_t* Uf, unsigned long long* flags,
-                       unsigned long long epoch, unsigned* gave_up, hipStream_t s, int slab) {
-    if (!xform_gemm_shape(n, Kp, 2)) throw std::invalid_argument("no fused launch for this shape");
-    switch (Kp) {
-        case 256: launch_xform_gemm_nw<8>(M, res, act_out, V, bn_scale, bn_mean, rfac, n, Kp, Tp, Uf, flags, epoch, gave_up, s, slab); break;
-        case 192: launch_xform_gemm_nw<6>(M, res, act_out, V, bn_scale, bn_mean, rfac, n, Kp, Tp, Uf, flags, epoch, gave_up, s, slab); break;
-        default: launch_xform_gemm_nw<4>(M, res, act_out, V, bn_scale, bn_mean, rfac, n, Kp, Tp, Uf, flags, epoch, gave_up, s, slab); break;
-    }
-}
+bool gemm_stream_prefers(int Kp, int max_batch) { return !(Kp == 192 && max_batch > 16); }
 
 template <int NK8, int NW>
 static void launch_gemm_stream32_nk(const float* V, const float* Uf, float* M, int T, int Tp,
@@ -2354,8 +1690,7 @@ static void launch_gemm_stream32_nw(const float* V, const float* Uf, float* M, i
 }
 
 static void launch_gemm_stream(const float* V, const float* Uf, float* M, int T, int Tp, int Cp,
-                               int Kp, hipStream_t s, LaunchTimer* t, int slab) {
-    if (slab != 0) throw std::invalid_argument("the fp32 GEMM works row by row");
+                               int Kp, hipStream_t s, LaunchTimer* t) {
     if (Kp == 256)
         launch_gemm_stream32_nw<8>(V, Uf, M, T, Tp, Cp, Kp, s, t);
     else if (Kp == 192)
@@ -2400,14 +1735,15 @@ template bool gemm_supports_channels<half_t>(int);
 // must be a multiple of 256.
 template <typename P>
 void launch_gemm(const P* V, const P* U, const P* Uf, P* M, int T, int Tp, int Cp, int Kp,
-                 hipStream_t s, LaunchTimer* t, int slab) {
+                 hipStream_t s, LaunchTimer* t) {
     constexpr int BK = 128 / (int)sizeof(P);
     const int nk = Cp / BK;
-    if (Uf != nullptr && gemm_stream_shape(T, Cp, Kp, (int)sizeof(P))) {
-        launch_gemm_stream(V, Uf, M, T, Tp, Cp, Kp, s, t, slab);
-        return;
+    if constexpr (sizeof(P) == 4) {
+        if (Uf != nullptr && gemm_stream_shape(T, Cp, Kp, (int)sizeof(P))) {
+            launch_gemm_stream(V, Uf, M, T, Tp, Cp, Kp, s, t);
+            return;
+        }
     }
-    if (slab != 0) throw std::invalid_argument("only the streaming GEMM works slab by slab");
     // The 256 x 256 tile pays off once its tiles can occupy most of the 256 compute units
     // (measured at 256 filters: from 6 row tiles = 216 work-groups, batch 52; with 5 = 180 the
     // 128 x 128 tiles are 2 % ahead; fp32 keeps the earlier hand-over at 160).
@@ -2711,13 +2047,12 @@ void launch_heads(const float* pol, const float* val, HeadParams hp, float tempe
     template void launch_in_transform<P>(const P*, P*, int, int, int, hipStream_t,             \
                                          LaunchTimer*);                                        \
     template void launch_gemm<P>(const P*, const P*, const P*, P*, int, int, int, int,         \
-                                 hipStream_t, LaunchTimer*, int);                              \
+                                 hipStream_t, LaunchTimer*);                                   \
     template void launch_out_transform<P>(const P*, const P*, P*, const float*, const float*,  \
-                                          float, int, int, int, hipStream_t, LaunchTimer*,     \
-                                          int);                                                \
+                                          float, int, int, int, hipStream_t, LaunchTimer*);    \
     template void launch_out_in_transform<P>(const P*, const P*, P*, P*, const float*,         \
                                              const float*, float, int, int, int, hipStream_t,  \
-                                             LaunchTimer*, int);                               \
+                                             LaunchTimer*);                                    \
     template void launch_head_conv<P>(const P*, const float*, float, float*, float*, int, int, \
                                       hipStream_t, LaunchTimer*);                              \
     template void launch_absmax<P>(const P*, size_t, float*, hipStream_t);

@@ -799,3 +799,53 @@ def test_fp16_range_beyond_the_calibration_positions(pkg, netgen, orc):
         assert rel_l2(Y[i], want) <= 4e-3
     assert clipped > 100, clipped
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,batches", [
+    (256, (1, 2, 3, 5, 6, 8, 9, 17, 18, 34, 35, 71)),
+    (192, (1, 3, 4, 7, 8, 11, 12, 22, 23, 45, 46)),
+    (128, (1, 5, 6, 11, 12, 17, 34, 35, 68, 69)),
+])
+def test_direct_convolution_tiles(pkg, netgen, orc, filters, batches):
+    """fp16 towers of 128, 192 and 256 filters: one layer with a skip connection at batches on
+    both sides of every change of tile, whole batch against a float32 convolution."""
+    import torch
+    import torch.nn.functional as F
+    maxb = max(batches)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 6600 + filters, pkg.FP16, maxb)
+    rng = np.random.default_rng(filters)
+    a = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
+    r = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
+    y = F.conv2d(torch.from_numpy(a.reshape(maxb, filters, 19, 19)), torch.from_numpy(net.conv_w[2]),
+                 padding=1).numpy().reshape(maxb, filters, 361)
+    want = np.maximum(0.0, ref.scale[2][None, :, None] * (y - ref.mean[2][None, :, None]) + r)
+    for n in batches:
+        print("case: direct convolution, %d filters, %d boards" % (filters, n), flush=True)
+        got = pipe.debug_layer(2, a[:n], r[:n])[2]
+        for i in range(n):
+            assert rel_l2(got[i], want[i]) <= 2e-3, (n, i)
+    pipe.close()
+
+
+def test_winograd_filters_of_no_3x3_filter(pkg, netgen, orc):
+    """Winograd-domain filters that are not the transform of any 3x3 filter have no direct
+    form: such a network runs through the Winograd kernels and agrees with the oracle."""
+    net = netgen.make_network(1, 128, 6700)
+    w, h = netgen.prepare(net)
+    w_ref, h_ref = netgen.prepare(net, orc.winograd_transform_f, orc.process_bn_var)
+    rng = np.random.default_rng(6701)
+    for ws in (w, w_ref):
+        ws.m_conv_weights[1] = (rng.standard_normal(36 * 128 * 128) * 0.04).astype(np.float32).reshape(36, 128, 128)
+        rng = np.random.default_rng(6701)
+    ref = orc.OraclePipe()
+    ref.initialize(128)
+    ref.push_weights(6, 18, 128, w_ref)
+    pipe = pkg.HIPScheduler(pkg.FP16, 5)
+    pipe.initialize(128)
+    pipe.push_weights(6, 18, 128, w)
+    x = netgen.synthetic_inputs(5, seed=67)
+    pol, val = pipe.forward_batch(x)
+    for i in range(5):
+        rp, rv = ref.forward(x[i])
+        assert rel_l2(pol[i], rp) <= 2e-2 and rel_l2(val[i], rv) <= 2e-2, i
+    pipe.close()
