@@ -183,8 +183,14 @@ private:
         std::condition_variable cv;
         int state = 0;  // 0 pending, 1 done, 2 halted, 3 failed
     };
+    // A worker's buffers for batches of more than one request.
+    struct Staging {
+        std::vector<float> in, pol, val;
+        std::vector<uint32_t> bits;
+    };
     void start_worker();
     void worker();
+    int execute(const std::shared_ptr<Request>* batch, int n, Staging* st, std::string& why);
     int submit(const std::shared_ptr<Request>& req);
 
     int m_precision = LZHIP_FP32, m_max_batch = 1, m_device = 0;
@@ -199,6 +205,7 @@ private:
     std::atomic<bool> m_draining{false};
     std::atomic<int> m_outstanding{0};  // callers currently inside forward()
     int m_max_wait_us = -1;   // < 0: automatic
+    int m_waiting = 0;        // workers with a batch that wait for a place in the executor
     int m_population = 1;     // callers seen around recent batches
     int m_inflight = 0;       // positions in batches assembled and not yet answered
     int m_lanes = 1;          // batches the executor runs side by side

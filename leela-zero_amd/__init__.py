@@ -151,7 +151,7 @@ def lib():
                                              ctypes.POINTER(ctypes.c_int)]
         L.lzhip_destroy.argtypes = [ctypes.c_void_p]
         L.lzhip_push_weights.argtypes = [ctypes.c_void_p, ctypes.c_int, _fpp, _fpp, _fpp, _fp, _fp]
-        L.lzhip_forward.argtypes = [ctypes.c_void_p, _fp, _fp, _fp]
+        L.lzhip_forward.argtypes = [ctypes.c_void_p] * 4
         L.lzhip_forward_batch.argtypes = [ctypes.c_void_p, ctypes.c_int, _fp, _fp, _fp]
         L.lzhip_forward_batch_device.argtypes = [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 3
         L.lzhip_forward_batch_device_noalloc.argtypes = ([ctypes.c_void_p, ctypes.c_int]
@@ -167,7 +167,8 @@ def lib():
         L.lzhip_process_batch_stats.argtypes = [ctypes.POINTER(ctypes.c_uint64)]
         L.lzhip_push_heads.argtypes = [ctypes.c_void_p] + [_fp] * 10
         L.lzhip_evaluate_batch.argtypes = [ctypes.c_void_p, ctypes.c_int, _fp, ctypes.c_float] + [_fp] * 5
-        L.lzhip_forward_eval.argtypes = [ctypes.c_void_p, _fp, ctypes.c_float, _fp, _fp]
+        L.lzhip_forward_eval.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float,
+                                         ctypes.c_void_p, _fp]
         L.lzhip_timed_evaluations.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, _fp,
                                               ctypes.c_float, _fp, _fp, _fp]
         L.lzhip_winograd_transform_f.argtypes = [_fp, ctypes.c_int, ctypes.c_int, _fp]
@@ -213,6 +214,22 @@ def _check(rc):
 
 def _f32(a):
     return np.ascontiguousarray(a, dtype=np.float32)
+
+
+# A call's own work in Python runs under the interpreter's lock, one thread at a time: 16
+# search threads that each spend 12 us on pointers are 200 us in which the device waits.  The
+# entry points that are called per position take addresses and arrays made the cheap way.
+_pol_t = ctypes.c_float * POL_SIZE
+_val_t = ctypes.c_float * VAL_SIZE
+_policy_t = ctypes.c_float * MOVES
+
+
+def _position(a):
+    """(array to keep, address) of one position's planes."""
+    x = _f32(a)
+    if x.size != INPUT_SIZE:
+        raise ValueError("input must have 18*361 values")
+    return x, x.__array_interface__["data"][0]
 
 
 def _ptr(a):
@@ -381,12 +398,12 @@ class HIPScheduler:
     def forward(self, input):
         """One position through the batching queue: in[6498] -> (pol[722], val[361])."""
         self._need()
-        x = _f32(input).reshape(-1)
-        if x.size != INPUT_SIZE:
-            raise ValueError("input must have 18*361 values")
+        x, at = _position(input)
         pol = np.empty(POL_SIZE, dtype=np.float32)
         val = np.empty(VAL_SIZE, dtype=np.float32)
-        _check(lib().lzhip_forward(self._h, _ptr(x), _ptr(pol), _ptr(val)))
+        rc = _lib.lzhip_forward(self._h, at, _pol_t.from_buffer(pol), _val_t.from_buffer(val))
+        if rc != OK:
+            _check(rc)
         return pol, val
 
     def drain(self):
@@ -473,13 +490,11 @@ class HIPScheduler:
         """One position through the batching queue with the heads computed on the
         device: returns (policy[362] in NN index order, value = tanh output)."""
         self._need()
-        x = _f32(input).reshape(-1)
-        if x.size != INPUT_SIZE:
-            raise ValueError("input must have 18*361 values")
+        x, at = _position(input)
         policy = np.empty(MOVES, dtype=np.float32)
         value = ctypes.c_float()
-        _check(lib().lzhip_forward_eval(self._h, _ptr(x), float(temperature), _ptr(policy),
-                                        ctypes.byref(value)))
+        _check(_lib.lzhip_forward_eval(self._h, at, float(temperature),
+                                       _policy_t.from_buffer(policy), ctypes.byref(value)))
         return policy, value.value
 
     def evaluate_batch(self, inputs, temperature=1.0, want_raw=False):

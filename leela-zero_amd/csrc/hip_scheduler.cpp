@@ -16,6 +16,7 @@
 
 #include "forward_pipe.h"
 #include "hip_pipe.h"
+#include "plane_bits.h"
 
 namespace lzhip {
 
@@ -140,27 +141,6 @@ int HIPScheduler::evaluate_raw(const float* in, float temperature, float* policy
     return submit(req);
 }
 
-// Packs planes that hold only +0.0f and 1.0f, one bit per value; false (and `bits`
-// unspecified) as soon as any other value shows up.
-static bool pack_planes(const float* in, uint32_t* bits) {
-    static_assert(sizeof(float) == sizeof(uint32_t), "float size");
-    constexpr uint32_t kOne = 0x3f800000u;
-    uint32_t word = 0, other = 0;
-    int w = 0;
-    for (int i = 0; i < kInSize; i++) {
-        uint32_t v;
-        std::memcpy(&v, in + i, sizeof(v));
-        other |= (v != 0u && v != kOne) ? 1u : 0u;
-        word |= (uint32_t)(v == kOne) << (i & 31);
-        if ((i & 31) == 31) {
-            bits[w++] = word;
-            word = 0;
-        }
-    }
-    if (kInSize & 31) bits[w] = word;
-    return other == 0;
-}
-
 int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
     if (m_draining.load()) {
         m_halted++;
@@ -168,7 +148,7 @@ int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
     }
     req->packed = m_exec && m_exec->accepts_bits() && pack_planes(req->in, req->bits);
     m_outstanding++;
-    bool wake;
+    bool wake, alone = false;
     {
         std::lock_guard<std::mutex> lk(m_mutex);
         if (!m_running) {
@@ -181,11 +161,29 @@ int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
             m_halted++;
             return LZHIP_EHALT;
         }
-        m_queue.push_back(req);
+        // A caller that is alone evaluates its position itself: handing it to a worker and being
+        // woken by it costs two thread switches (about 15 us of a 200 us evaluation), and there
+        // is nobody to share a batch with.
+        if (m_queue.empty() && !m_collecting && m_exec_busy < m_lanes && m_population <= 1 &&
+            m_outstanding.load() == 1) {
+            alone = true;
+            m_exec_busy++;
+            m_inflight++;
+        } else {
+            m_queue.push_back(req);
+        }
         // The collecting worker sleeps until the queue has the length it waits for (or its
         // grace period ends, or the device comes free: others notify it of those); waking
         // every worker for every request in between only makes them queue up for this mutex.
-        wake = !m_collecting || m_queue.size() >= m_wake_at;
+        wake = !alone && (!m_collecting || m_queue.size() >= m_wake_at);
+    }
+    if (alone) {
+        std::string why;
+        const int state = execute(&req, 1, nullptr, why);
+        m_outstanding--;
+        if (state != 1) throw std::runtime_error(why);
+        m_requests++;
+        return LZHIP_OK;
     }
     if (wake) m_cv.notify_all();  // the collecting worker and an idle one share this condition
     int state;
@@ -211,6 +209,66 @@ int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
     throw std::runtime_error(msg);
 }
 
+// Runs a batch that has its place in the executor and counts it; 1, or 3 and why.  A single
+// request is evaluated in the caller's own buffers and needs no staging.
+int HIPScheduler::execute(const std::shared_ptr<Request>* batch, int n, Staging* st,
+                          std::string& why) {
+    const Request& first = *batch[0];
+    const bool heads = first.heads;
+    bool packed = true;
+    for (int i = 0; i < n; i++) packed = packed && batch[i]->packed;
+    const float* in = first.in;
+    const uint32_t* bits = first.bits;
+    float *pol = first.pol, *val = first.val;
+    if (n > 1) {
+        for (int i = 0; i < n; i++) {
+            if (packed)
+                std::memcpy(st->bits.data() + (size_t)i * BatchExecutor::kInputWords,
+                            batch[i]->bits, sizeof(uint32_t) * BatchExecutor::kInputWords);
+            else
+                std::memcpy(st->in.data() + (size_t)i * kInSize, batch[i]->in,
+                            sizeof(float) * kInSize);
+        }
+        in = st->in.data();
+        bits = st->bits.data();
+        pol = st->pol.data();
+        val = st->val.data();
+    }
+    int outcome = 1;
+    const auto t0 = std::chrono::steady_clock::now();
+    try {
+        if (packed)
+            m_exec->run_bits(n, bits, heads, first.temperature, pol, val);
+        else if (heads)
+            m_exec->evaluate_heads_batch(n, in, first.temperature, pol, val);
+        else
+            m_exec->forward_batch(n, in, pol, val);
+    } catch (const std::exception& e) {
+        outcome = 3;
+        why = e.what();
+    }
+    bool wake;
+    {
+        const double us =
+            std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
+        std::lock_guard<std::mutex> lk(m_mutex);
+        m_exec_us = m_exec_us > 0.0 ? 0.75 * m_exec_us + 0.25 * us : us;
+        // callers in flight plus those that queued up meanwhile; forgets slowly
+        m_population = std::max(m_outstanding.load(), m_population - 1);
+        m_inflight -= n;
+        m_exec_busy--;
+        wake = !st && (m_collecting || m_waiting > 0 || !m_queue.empty());
+    }
+    if (wake) m_cv.notify_all();
+    m_batches++;
+    (n == 1 ? batch_stats.single_evals : batch_stats.batch_evals)++;
+    batch_stats.positions += (size_t)n;
+    batch_stats.slots += (size_t)m_max_batch;
+    uint32_t seen = m_max_seen.load();
+    while ((uint32_t)n > seen && !m_max_seen.compare_exchange_weak(seen, (uint32_t)n)) {}
+    return outcome;
+}
+
 // Batch pickup.  The worker sleeps until a request exists, then grants a
 // grace period for the batch to grow towards the number of callers seen around
 // the previous batches (those that were queued or in flight when a batch
@@ -222,17 +280,21 @@ int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
 // estimate of the callers that is too high costs at most that much per batch
 // and decays by one caller per batch.
 void HIPScheduler::worker() {
-    std::vector<float> in, pol, val;
-    std::vector<uint32_t> bits((size_t)m_max_batch * BatchExecutor::kInputWords);
-    in.resize((size_t)m_max_batch * kInSize);
-    pol.resize((size_t)m_max_batch * kPolSize);
-    val.resize((size_t)m_max_batch * kValSize);
+    Staging staging;
+    staging.bits.resize((size_t)m_max_batch * BatchExecutor::kInputWords);
+    staging.in.resize((size_t)m_max_batch * kInSize);
+    staging.pol.resize((size_t)m_max_batch * kPolSize);
+    staging.val.resize((size_t)m_max_batch * kValSize);
     std::vector<std::shared_ptr<Request>> batch;
     for (;;) {
         batch.clear();
         {
             std::unique_lock<std::mutex> lk(m_mutex);
-            m_cv.wait(lk, [&] { return !m_running || (!m_collecting && !m_queue.empty()); });
+            // (one batch at most is assembled ahead of the executor)
+            m_cv.wait(lk, [&] {
+                return !m_running || (!m_collecting && !m_queue.empty() &&
+                                      m_exec_busy + m_waiting <= m_lanes);
+            });
             if (!m_running) return;
             // Only one worker assembles a batch at a time; it hands the role on
             // when it leaves this block.
@@ -303,64 +365,32 @@ void HIPScheduler::worker() {
         }
         if (batch.empty()) continue;
         const int n = (int)batch.size();  // m_inflight was raised under the lock above
-        bool all_packed = true;
-        for (int i = 0; i < n; i++) all_packed = all_packed && batch[i]->packed;
-        if (all_packed) {
-            for (int i = 0; i < n; i++)
-                std::memcpy(bits.data() + (size_t)i * BatchExecutor::kInputWords, batch[i]->bits,
-                            sizeof(uint32_t) * BatchExecutor::kInputWords);
-        } else {
-            for (int i = 0; i < n; i++)
-                std::memcpy(in.data() + (size_t)i * kInSize, batch[i]->in, sizeof(float) * kInSize);
-        }
         {
             // the executor takes m_lanes batches at a time
             std::unique_lock<std::mutex> lk(m_mutex);
+            m_waiting++;
             m_cv.wait(lk, [&] { return m_exec_busy < m_lanes; });
+            m_waiting--;
             m_exec_busy++;
         }
-        int outcome = 1;
-        const auto t0 = std::chrono::steady_clock::now();
-        try {
-            if (all_packed)
-                m_exec->run_bits(n, bits.data(), batch[0]->heads, batch[0]->temperature,
-                                 pol.data(), val.data());
-            else if (batch[0]->heads)
-                m_exec->evaluate_heads_batch(n, in.data(), batch[0]->temperature, pol.data(),
-                                             val.data());
-            else
-                m_exec->forward_batch(n, in.data(), pol.data(), val.data());
-        } catch (const std::exception& e) {
-            outcome = 3;
+        std::string why;
+        const int outcome = execute(batch.data(), n, &staging, why);
+        if (outcome != 1) {
             std::lock_guard<std::mutex> lk(m_mutex);
             delete m_fail_msg;
-            m_fail_msg = new std::string(e.what());
-        }
-        {
-            const double us =
-                std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
-            std::lock_guard<std::mutex> lk(m_mutex);
-            m_exec_us = m_exec_us > 0.0 ? 0.75 * m_exec_us + 0.25 * us : us;
-            // callers in flight plus those that queued up meanwhile; forgets slowly
-            m_population = std::max(m_outstanding.load(), m_population - 1);
-            m_inflight -= n;
-            m_exec_busy--;
+            m_fail_msg = new std::string(why);
         }
         m_cv.notify_all();  // a collector may be waiting for the device to come free
-        m_batches++;
-        (n == 1 ? batch_stats.single_evals : batch_stats.batch_evals)++;
-        batch_stats.positions += (size_t)n;
-        batch_stats.slots += (size_t)m_max_batch;
-        uint32_t seen = m_max_seen.load();
-        while ((uint32_t)n > seen && !m_max_seen.compare_exchange_weak(seen, (uint32_t)n)) {}
         for (int i = 0; i < n; i++) {
             Request& r = *batch[i];
-            if (outcome == 1 && r.heads) {
-                std::memcpy(r.pol, pol.data() + (size_t)i * 362, sizeof(float) * 362);
-                *r.val = val[i];
-            } else if (outcome == 1) {
-                std::memcpy(r.pol, pol.data() + (size_t)i * kPolSize, sizeof(float) * kPolSize);
-                std::memcpy(r.val, val.data() + (size_t)i * kValSize, sizeof(float) * kValSize);
+            if (outcome == 1 && n > 1 && r.heads) {
+                std::memcpy(r.pol, staging.pol.data() + (size_t)i * 362, sizeof(float) * 362);
+                *r.val = staging.val[i];
+            } else if (outcome == 1 && n > 1) {
+                std::memcpy(r.pol, staging.pol.data() + (size_t)i * kPolSize,
+                            sizeof(float) * kPolSize);
+                std::memcpy(r.val, staging.val.data() + (size_t)i * kValSize,
+                            sizeof(float) * kValSize);
             }
             {
                 std::lock_guard<std::mutex> lk(r.mu);
