@@ -15,6 +15,7 @@
 #include <stdexcept>
 
 #include "kernels.h"
+#include "plane_bits.h"
 
 namespace lzhip {
 
@@ -436,7 +437,11 @@ public:
     // the lock, so that the next batch is queued on the device while this one
     // runs and host-side copies overlap device work.
     void forward_batch(int n, const float* in, float* pol, float* val) override {
-        run_host_batch(n, in, nullptr, false, 1.0f, pol, val);
+        HostCall c;
+        c.in = in;
+        c.pol = pol;
+        c.val = val;
+        run_host_batch(n, c);
     }
 
     // Bit-packed planes: 816 bytes per position travel instead of 26 KB; the first kernel
@@ -444,24 +449,60 @@ public:
     bool accepts_bits() const override { return true; }
     void run_bits(int n, const uint32_t* bits, bool heads, float temperature, float* out_a,
                   float* out_b) override {
-        if (heads && !m_heads_ready) throw std::invalid_argument("push_heads has not been called");
-        if (heads && !(temperature > 0.0f))
-            throw std::invalid_argument("temperature must be positive");
-        run_host_batch(n, nullptr, bits, heads, temperature, out_a, out_b);
+        HostCall c;
+        c.bits = bits;
+        c.heads = heads;
+        c.temperature = temperature;
+        (heads ? c.policy : c.pol) = out_a;
+        (heads ? c.value : c.val) = out_b;
+        run_host_batch(n, c);
     }
 
     // The same path with the heads computed on the device: policy [n][362] and the
     // tanh value [n] come back instead of the raw planes.
     void evaluate_heads_batch(int n, const float* in, float temperature, float* policy,
                               float* value) override {
-        if (!m_heads_ready) throw std::invalid_argument("push_heads has not been called");
-        if (!(temperature > 0.0f)) throw std::invalid_argument("temperature must be positive");
-        run_host_batch(n, in, nullptr, true, temperature, policy, value);
+        evaluate_batch(n, in, temperature, policy, value, nullptr, nullptr, nullptr);
     }
 
-    void run_host_batch(int n, const float* in, const uint32_t* bits, bool heads,
-                        float temperature, float* out_a, float* out_b) {
+    void evaluate_batch(int n, const float* in, float temperature, float* policy, float* value,
+                        float* logits, float* pol, float* val) override {
+        HostCall c;
+        c.in = in;
+        c.heads = true;
+        c.temperature = temperature;
+        c.policy = policy;
+        c.value = value;
+        c.logits = logits;
+        c.pol = pol;
+        c.val = val;
+        run_host_batch(n, c);
+    }
+
+    // One batch with its planes and results in the caller's host memory: the planes as floats
+    // or as bits; the heads or the raw planes; results that are null are not wanted.
+    struct HostCall {
+        const float* in = nullptr;
+        const uint32_t* bits = nullptr;
+        bool heads = false;
+        float temperature = 1.0f;
+        float *policy = nullptr, *value = nullptr, *logits = nullptr;
+        float *pol = nullptr, *val = nullptr;
+    };
+
+    // Pinned host memory is mapped into the device's address space: the first kernel reads the
+    // packed planes and the last ones write the results straight through it, so that no copy
+    // command sits between this batch's kernels and the next batch's (each one is a bubble of
+    // tens of microseconds on the stream, and copies to and from the caller's pageable
+    // memory also wait for one another: they were two thirds of a 37-position call on a
+    // 10x128 network).  Planes that hold only 0 and 1 -- the engine's -- are packed on the way
+    // into pinned memory; other values, 32 times larger, go by copy.
+    void run_host_batch(int n, const HostCall& c) {
         check_ready(n);
+        if (c.heads && !m_heads_ready)
+            throw std::invalid_argument("push_heads has not been called");
+        if (c.heads && !(c.temperature > 0.0f))
+            throw std::invalid_argument("temperature must be positive");
         HIP_CHECK(hipSetDevice(m_device));
         IoSlot* sl = nullptr;
         {
@@ -486,43 +527,58 @@ public:
                 self->m_slot_cv.notify_all();
             }
         } release{this, sl};
-        // sizes of the two results per position, both written by the device into hpol / hval
-        const size_t na = heads ? 362 : 2 * kPts, nb = heads ? 1 : kPts;
-        if (bits)
-            std::memcpy(sl->hbits.p, bits, sizeof(uint32_t) * (size_t)n * kInputWords);
+        const size_t in_size = (size_t)kInPlanes * kPts;
+        bool packed = true;
+        if (c.bits)
+            std::memcpy(sl->hbits.p, c.bits, sizeof(uint32_t) * (size_t)n * kInputWords);
         else
-            std::memcpy(sl->hin.p, in, sizeof(float) * (size_t)n * kInPlanes * kPts);
+            for (int i = 0; i < n && packed; i++)
+                packed = pack_planes(c.in + (size_t)i * in_size,
+                                     sl->hbits.p + (size_t)i * kInputWords);
+        if (!packed) std::memcpy(sl->hin.p, c.in, sizeof(float) * (size_t)n * in_size);
         {
             // each staging slot has a lane of its own: two batches run side by side
             Lane& ln = m_lane[sl - m_slot];
             std::lock_guard<std::mutex> lk(ln.mu);
-            // Pinned host memory is mapped into the device's address space: the first
-            // kernel reads the packed planes and the last ones write the results straight
-            // through it, so that no copy command sits between this batch's kernels and
-            // the next batch's (each one is a bubble of tens of microseconds on the
-            // stream).  Float planes, 32 times larger, still go by copy.
-            float* out_a_dev = heads ? sl->dpol.p : sl->hpol.p;   // raw planes: straight to host
-            float* out_b_dev = heads ? sl->dval.p : sl->hval.p;
-            if (bits) {
-                run_forward(ln, n, nullptr, sl->hbits.p, out_a_dev, out_b_dev);
-            } else {
-                HIP_CHECK(hipMemcpyAsync(sl->din.p, sl->hin.p,
-                                         sizeof(float) * (size_t)n * kInPlanes * kPts,
+            float* pol_dev = c.heads ? sl->dpol.p : sl->hpol.p;   // raw planes: straight to host
+            float* val_dev = c.heads ? sl->dval.p : sl->hval.p;
+            if (!packed)
+                HIP_CHECK(hipMemcpyAsync(sl->din.p, sl->hin.p, sizeof(float) * (size_t)n * in_size,
                                          hipMemcpyHostToDevice, ln.stream));
-                run_forward(ln, n, sl->din.p, nullptr, out_a_dev, out_b_dev);
-            }
-            if (heads) {
-                HeadParams hp{m_h[0].p, m_h[1].p, m_h[2].p, m_h[3].p, m_h[4].p,
-                              m_h[5].p, m_h[6].p, m_h[7].p, m_h[8].p, m_h[9].p};
-                launch_heads(sl->dpol.p, sl->dval.p, hp, temperature, sl->hpol.p, nullptr,
-                             sl->hval.p, sl->dwork.p, n, ln.stream);
+            run_forward(ln, n, packed ? nullptr : sl->din.p, packed ? sl->hbits.p : nullptr,
+                        pol_dev, val_dev);
+            if (c.heads) {
+                launch_heads(pol_dev, val_dev, head_params(), c.temperature, sl->hpol.p,
+                             c.logits ? sl->hlogits.p : nullptr, sl->hval.p, sl->dwork.p, n,
+                             ln.stream);
+                // (rarely asked for)
+                if (c.pol)
+                    HIP_CHECK(hipMemcpyAsync(c.pol, pol_dev, sizeof(float) * (size_t)n * 2 * kPts,
+                                             hipMemcpyDeviceToHost, ln.stream));
+                if (c.val)
+                    HIP_CHECK(hipMemcpyAsync(c.val, val_dev, sizeof(float) * (size_t)n * kPts,
+                                             hipMemcpyDeviceToHost, ln.stream));
             }
             HIP_CHECK(hipGetLastError());
             HIP_CHECK(hipEventRecord(sl->done, ln.stream));
         }
         HIP_CHECK(hipEventSynchronize(sl->done));
-        std::memcpy(out_a, sl->hpol.p, sizeof(float) * (size_t)n * na);
-        std::memcpy(out_b, sl->hval.p, sizeof(float) * (size_t)n * nb);
+        auto fetch = [n](float* dst, const float* src, size_t each) {
+            if (dst) std::memcpy(dst, src, sizeof(float) * (size_t)n * each);
+        };
+        if (c.heads) {
+            fetch(c.policy, sl->hpol.p, 362);
+            fetch(c.value, sl->hval.p, 1);
+            fetch(c.logits, sl->hlogits.p, 362);
+        } else {
+            fetch(c.pol, sl->hpol.p, 2 * kPts);
+            fetch(c.val, sl->hval.p, kPts);
+        }
+    }
+
+    HeadParams head_params() const {
+        return HeadParams{m_h[0].p, m_h[1].p, m_h[2].p, m_h[3].p, m_h[4].p,
+                          m_h[5].p, m_h[6].p, m_h[7].p, m_h[8].p, m_h[9].p};
     }
 
     // -------------------------------------------------------------------
@@ -552,38 +608,13 @@ public:
         up(m_h[9], hw.ip2_val_b, 1);
         const size_t B = (size_t)m_max_batch;
         m_dpolicy.alloc(B * 362);
-        m_dlogits.alloc(B * 362);
         m_dvalue.alloc(B);
         m_dwork.alloc(B * (362 + 256));
-        for (int i = 0; i < m_n_lanes; i++) m_slot[i].dwork.alloc(B * (362 + 256));
+        for (int i = 0; i < m_n_lanes; i++) {
+            m_slot[i].dwork.alloc(B * (362 + 256));
+            m_slot[i].hlogits.alloc(B * 362);
+        }
         m_heads_ready = true;
-    }
-
-    void evaluate_batch(int n, const float* in, float temperature, float* policy, float* value,
-                        float* logits, float* pol, float* val) override {
-        Lane& ln = m_lane[0];
-        std::lock_guard<std::mutex> lk(ln.mu);
-        check_ready(n);
-        if (!m_heads_ready) throw std::invalid_argument("push_heads has not been called");
-        if (!(temperature > 0.0f)) throw std::invalid_argument("temperature must be positive");
-        HIP_CHECK(hipSetDevice(m_device));
-        HIP_CHECK(hipMemcpyAsync(m_din.p, in, sizeof(float) * (size_t)n * kInPlanes * kPts,
-                                 hipMemcpyHostToDevice, ln.stream));
-        run_forward(ln, n, m_din.p, nullptr, m_dpol.p, m_dval.p);
-        HeadParams hp{m_h[0].p, m_h[1].p, m_h[2].p, m_h[3].p, m_h[4].p,
-                      m_h[5].p, m_h[6].p, m_h[7].p, m_h[8].p, m_h[9].p};
-        launch_heads(m_dpol.p, m_dval.p, hp, temperature, m_dpolicy.p, m_dlogits.p, m_dvalue.p,
-                     m_dwork.p, n, ln.stream);
-        HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipStreamSynchronize(ln.stream));
-        HIP_CHECK(hipMemcpy(policy, m_dpolicy.p, sizeof(float) * (size_t)n * 362, hipMemcpyDeviceToHost));
-        HIP_CHECK(hipMemcpy(value, m_dvalue.p, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost));
-        if (logits)
-            HIP_CHECK(hipMemcpy(logits, m_dlogits.p, sizeof(float) * (size_t)n * 362, hipMemcpyDeviceToHost));
-        if (pol)
-            HIP_CHECK(hipMemcpy(pol, m_dpol.p, sizeof(float) * (size_t)n * 2 * kPts, hipMemcpyDeviceToHost));
-        if (val)
-            HIP_CHECK(hipMemcpy(val, m_dval.p, sizeof(float) * (size_t)n * kPts, hipMemcpyDeviceToHost));
     }
 
     float timed_evaluations(int n, int reps, const float* in, float temperature, float* policy,
@@ -601,8 +632,7 @@ public:
         hpolicy.alloc((size_t)n * 362);
         hvalue.alloc((size_t)n);
         std::memcpy(hin.p, in, in_count * sizeof(float));
-        HeadParams hp{m_h[0].p, m_h[1].p, m_h[2].p, m_h[3].p, m_h[4].p,
-                      m_h[5].p, m_h[6].p, m_h[7].p, m_h[8].p, m_h[9].p};
+        const HeadParams hp = head_params();
         HIP_CHECK(hipStreamSynchronize(ln.stream));
         HIP_CHECK(hipEventRecord(m_ev_start[0], ln.stream));
         for (int r = 0; r < reps; r++) {
@@ -1036,7 +1066,7 @@ private:
     // Staging of forward_batch: kIoSlots batches may be between "copied in" and
     // "copied out" at once, slot i on lane i.
     struct IoSlot {
-        PinnedBuf<float> hin, hpol, hval;
+        PinnedBuf<float> hin, hpol, hval, hlogits;
         PinnedBuf<uint32_t> hbits;
         DevBuf<float> din, dpol, dval;
         DevBuf<float> dwork;   // heads: logits and hidden units between the two kernels
@@ -1050,7 +1080,7 @@ private:
     std::vector<Layer> m_layers;
     std::atomic<bool> m_ready{false};   // set by a push_weights that ran to its end
     std::vector<float> m_s;  // activation scales, m_s[0] = input
-    DevBuf<float> m_h[10], m_dpolicy, m_dlogits, m_dvalue, m_dwork;
+    DevBuf<float> m_h[10], m_dpolicy, m_dvalue, m_dwork;
     bool m_heads_ready = false;
     hipEvent_t m_ev_start[kTimerPool] = {}, m_ev_stop[kTimerPool] = {};
     int m_timer_class[kTimerPool] = {};
