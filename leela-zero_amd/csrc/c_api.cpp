@@ -409,7 +409,7 @@ int lzhip_get_output(lzhip_handle* h, const lzhip_head_weights* heads, const uin
     const int frc = h->sched->forward_raw(in.data(), pol.data(), val.data());
     if (frc == LZHIP_EHALT) return fail(LZHIP_EHALT, "halted by drain");
     float p[go::kPoints + 1];
-    heads_on_host(*hw, pol.data(), val.data(), softmax_temp, p, winrate);
+    heads_on_host(*hw, 1, pol.data(), val.data(), softmax_temp, p, winrate);
     for (int i = 0; i < go::kPoints; i++) policy[symmetry_index(symmetry, i)] = p[i];
     policy[go::kPoints] = p[go::kPoints];
     if (h->value_not_stm.load() && to_move == go::WHITE) *winrate = 1.0f - *winrate;
@@ -450,7 +450,7 @@ int lzhip_netbench(lzhip_handle* h, const lzhip_head_weights* heads, const uint8
                         halted++;
                         break;
                     }
-                    heads_on_host(*hw, pol.data(), val.data(), 1.0f, p, &win);
+                    heads_on_host(*hw, 1, pol.data(), val.data(), 1.0f, p, &win);
                 }
             } catch (const std::exception& e) {
                 std::lock_guard<std::mutex> lk(err_mu);
@@ -475,29 +475,30 @@ int lzhip_get_output_average(lzhip_handle* h, const lzhip_head_weights* heads,
     GUARD_BEGIN
     const auto hw = resolve_heads(h, heads);
     constexpr int S = 8;
-    std::vector<float> in((size_t)S * LZHIP_INPUT_SIZE), pol((size_t)S * LZHIP_POL_SIZE),
-        val((size_t)S * LZHIP_VAL_SIZE);
-    for (int sym = 0; sym < S; sym++) {
-        const int rc = lzhip_gather_features(boards, n_boards, to_move, sym,
-                                             in.data() + (size_t)sym * LZHIP_INPUT_SIZE);
-        if (rc != LZHIP_OK) return rc;
-    }
+    if (n_boards < 1 || n_boards > go::kHistory || (to_move != LZHIP_BLACK && to_move != LZHIP_WHITE))
+        return fail(LZHIP_EINVAL, "n_boards in 1..8, to_move 0/1");
+    const uint8_t* ptr[go::kHistory];
+    for (int i = 0; i < n_boards; i++) ptr[i] = boards + (size_t)i * go::kPoints;
+    // The planes go down one bit per value: written as floats (208 KB) they were cleared,
+    // filled, copied to pinned memory and copied to the device, a tenth of an evaluation.
+    uint32_t bits[S * BatchExecutor::kInputWords];
+    std::vector<float> pol((size_t)S * LZHIP_POL_SIZE), val((size_t)S * LZHIP_VAL_SIZE);
+    for (int sym = 0; sym < S; sym++)
+        gather_bits(ptr, n_boards, to_move, sym, bits + sym * BatchExecutor::kInputWords);
     const int step = std::min(S, h->pipe->max_batch());
-    for (int s0 = 0; s0 < S; s0 += step) {
-        const int n = std::min(step, S - s0);
-        h->pipe->forward_batch(n, in.data() + (size_t)s0 * LZHIP_INPUT_SIZE,
-                               pol.data() + (size_t)s0 * LZHIP_POL_SIZE,
-                               val.data() + (size_t)s0 * LZHIP_VAL_SIZE);
-    }
+    for (int s0 = 0; s0 < S; s0 += step)
+        h->pipe->run_bits(std::min(step, S - s0), bits + s0 * BatchExecutor::kInputWords, false,
+                          1.0f, pol.data() + (size_t)s0 * LZHIP_POL_SIZE,
+                          val.data() + (size_t)s0 * LZHIP_VAL_SIZE);
+    float p[S * (go::kPoints + 1)], w[S];
+    heads_on_host(*hw, S, pol.data(), val.data(), softmax_temp, p, w);
     for (int i = 0; i <= go::kPoints; i++) policy[i] = 0.0f;
     float win = 0.0f;
     for (int sym = 0; sym < S; sym++) {
-        float p[go::kPoints + 1], w;
-        heads_on_host(*hw, pol.data() + (size_t)sym * LZHIP_POL_SIZE,
-                      val.data() + (size_t)sym * LZHIP_VAL_SIZE, softmax_temp, p, &w);
-        for (int i = 0; i < go::kPoints; i++) policy[symmetry_index(sym, i)] += p[i] / (float)S;
-        policy[go::kPoints] += p[go::kPoints] / (float)S;
-        win += w / (float)S;
+        const float* ps = p + sym * (go::kPoints + 1);
+        for (int i = 0; i < go::kPoints; i++) policy[symmetry_index(sym, i)] += ps[i] / (float)S;
+        policy[go::kPoints] += ps[go::kPoints] / (float)S;
+        win += w[sym] / (float)S;
     }
     *winrate = (h->value_not_stm.load() && to_move == go::WHITE) ? 1.0f - win : win;
     return LZHIP_OK;

@@ -10,6 +10,10 @@
 #include <stdexcept>
 #include <thread>
 
+#ifdef __SSE2__
+#include <emmintrin.h>
+#endif
+
 namespace lzhip {
 
 using go::kPass;
@@ -77,6 +81,57 @@ void gather_features(const uint8_t* const* boards, int n_boards, int to_move, in
     for (int i = 0; i < kPoints; i++) stm[i] = 1.0f;
 }
 
+void gather_bits(const uint8_t* const* boards, int n_boards, int to_move, int symmetry,
+                 uint32_t* bits) {
+    // 64 values at a time; LZHIP_INPUT_SIZE = 6498 values are 102 words of 64 (203 full words
+    // of 32 and a part)
+    constexpr int kWords = (LZHIP_INPUT_SIZE + 63) / 64, kChunks = (kPoints + 63) / 64;
+    uint64_t out[kWords + 1] = {};
+    auto put = [&](int plane, const uint64_t* mask) {
+        const int bit = plane * kPoints, w = bit >> 6, sh = bit & 63;
+        for (int c = 0; c < kChunks; c++) {
+            out[w + c] |= mask[c] << sh;
+            if (sh) out[w + c + 1] |= mask[c] >> (64 - sh);
+        }
+    };
+    const int16_t* map = sym_table().idx[symmetry];
+    const int n = std::min(n_boards, go::kHistory);
+    for (int h = 0; h < n; h++) {
+        uint8_t c[64 * kChunks];
+        std::memset(c + kPoints, 0xff, sizeof(c) - kPoints);   // no colour
+        for (int i = 0; i < kPoints; i++) c[i] = boards[h][map[i]];
+        uint64_t own[kChunks], opp[kChunks];
+        for (int k = 0; k < kChunks; k++) {
+            uint64_t a = 0, b = 0;
+#ifdef __SSE2__
+            for (int q = 0; q < 4; q++) {
+                const __m128i v =
+                    _mm_loadu_si128(reinterpret_cast<const __m128i*>(c + 64 * k + 16 * q));
+                a |= (uint64_t)_mm_movemask_epi8(_mm_cmpeq_epi8(v, _mm_set1_epi8((char)to_move)))
+                     << (16 * q);
+                b |= (uint64_t)_mm_movemask_epi8(
+                         _mm_cmpeq_epi8(v, _mm_set1_epi8((char)(to_move ^ 1))))
+                     << (16 * q);
+            }
+#else
+            for (int i = 0; i < 64; i++) {
+                a |= (uint64_t)(c[64 * k + i] == to_move) << i;
+                b |= (uint64_t)(c[64 * k + i] == (to_move ^ 1)) << i;
+            }
+#endif
+            own[k] = a;
+            opp[k] = b;
+        }
+        put(h, own);
+        put(go::kHistory + h, opp);
+    }
+    uint64_t all[kChunks];
+    for (int k = 0; k < kChunks; k++) all[k] = ~0ull;
+    all[kChunks - 1] = (1ull << (kPoints - 64 * (kChunks - 1))) - 1;
+    put(2 * go::kHistory + (to_move == go::BLACK ? 0 : 1), all);
+    std::memcpy(bits, out, sizeof(uint32_t) * BatchExecutor::kInputWords);
+}
+
 void gather_features(const go::Position& pos, int symmetry, float* out) {
     const uint8_t* boards[go::kHistory];
     const int n = std::min(pos.movenum() + 1, go::kHistory);
@@ -108,38 +163,112 @@ HeadWeights::HeadWeights(const lzhip_head_weights& w) {
     ip2_val_b = w.ip2_val_b[0];
 }
 
-void heads_on_host(const HeadWeights& w, const float* pol, const float* val, float softmax_temp,
-                   float* policy, float* winrate) {
-    constexpr int pout = kPoints + 1;
-    float logits[pout];
-    for (int o = 0; o < pout; o++) logits[o] = w.ip_pol_b[o];
-    for (int c = 0; c < 2; c++)
-        for (int i = 0; i < kPoints; i++) {
-            const float x = w.bn_pol_scale[c] * (pol[c * kPoints + i] - w.bn_pol_mean[c]);
-            if (x <= 0.0f) continue;
-            const float* row = &w.ip_pol_wt[(size_t)(c * kPoints + i) * pout];
-            for (int o = 0; o < pout; o++) logits[o] += x * row[o];
-        }
-    float alpha = logits[0];
-    for (int o = 1; o < pout; o++) alpha = std::max(alpha, logits[o]);
-    float denom = 0.0f;
-    for (int o = 0; o < pout; o++) {
-        policy[o] = std::exp((logits[o] - alpha) / softmax_temp);
-        denom += policy[o];
-    }
-    for (int o = 0; o < pout; o++) policy[o] /= denom;
+namespace {
 
-    float hid[256];
-    for (int o = 0; o < 256; o++) hid[o] = w.ip1_val_b[o];
-    for (int i = 0; i < kPoints; i++) {
-        const float x = w.bn_val_scale * (val[i] - w.bn_val_mean);
-        if (x <= 0.0f) continue;
-        const float* row = &w.ip1_val_wt[(size_t)i * 256];
-        for (int o = 0; o < 256; o++) hid[o] += x * row[o];
+// y += W^T x over the inputs x that are positive after batch norm (the others add nothing),
+// for n positions at once.  Blocks of 8 rows of W (at most 12 KB) stay in the first-level cache
+// while the positions pass over them, and a pass adds up to four rows per visit of y.
+template <int N>
+__attribute__((always_inline)) inline void fc_rows(const float* wt, const float* x, int inputs,
+                                                   int stride, float* y, int n) {
+    for (int i0 = 0; i0 < inputs; i0 += 8) {
+        const int rows = inputs - i0 < 8 ? inputs - i0 : 8;
+        for (int p = 0; p < n; p++) {
+            const float *r[8], *xp = x + (size_t)p * stride + i0;
+            float v[8];
+            int m = 0;
+            for (int i = 0; i < rows; i++)
+                if (xp[i] > 0.0f) {
+                    v[m] = xp[i];
+                    r[m++] = wt + (size_t)(i0 + i) * N;
+                }
+            float* __restrict yp = y + (size_t)p * N;
+            int k = 0;
+            for (; k + 4 <= m; k += 4) {
+                const float *a = r[k], *b = r[k + 1], *c = r[k + 2], *d = r[k + 3];
+                const float va = v[k], vb = v[k + 1], vc = v[k + 2], vd = v[k + 3];
+                for (int o = 0; o < N; o++)
+                    yp[o] = yp[o] + va * a[o] + vb * b[o] + (vc * c[o] + vd * d[o]);
+            }
+            for (; k < m; k++) {
+                const float* a = r[k];
+                const float va = v[k];
+                for (int o = 0; o < N; o++) yp[o] += va * a[o];
+            }
+        }
     }
-    float out = w.ip2_val_b;
-    for (int o = 0; o < 256; o++) out += std::max(hid[o], 0.0f) * w.ip2_val_w[o];
-    *winrate = (1.0f + std::tanh(out)) / 2.0f;
+}
+
+typedef void FcRows(const float*, const float*, int, int, float*, int);
+template <int N> struct Fc {
+    static void base(const float* wt, const float* x, int k, int s, float* y, int n) {
+        fc_rows<N>(wt, x, k, s, y, n);
+    }
+#if defined(__x86_64__)
+    __attribute__((target("avx2,fma"))) static void avx2(const float* wt, const float* x, int k,
+                                                         int s, float* y, int n) {
+        fc_rows<N>(wt, x, k, s, y, n);
+    }
+    __attribute__((target("avx512f,avx2,fma"))) static void avx512(const float* wt, const float* x,
+                                                                   int k, int s, float* y, int n) {
+        fc_rows<N>(wt, x, k, s, y, n);
+    }
+#endif
+    // the widest version the processor runs
+    static FcRows* best() {
+#if defined(__x86_64__)
+        if (__builtin_cpu_supports("avx512f")) return avx512;
+        if (__builtin_cpu_supports("avx2") && __builtin_cpu_supports("fma")) return avx2;
+#endif
+        return base;
+    }
+};
+
+}  // namespace
+
+void heads_on_host(const HeadWeights& w, int n, const float* pol, const float* val,
+                   float softmax_temp, float* policy, float* winrate) {
+    constexpr int pout = kPoints + 1, pin = 2 * kPoints, kBlock = 8, vout = 256;
+    static FcRows* const fc_pol = Fc<pout>::best();
+    static FcRows* const fc_val = Fc<vout>::best();
+    float x[kBlock * pin], y[kBlock * pout];
+    for (int p0 = 0; p0 < n; p0 += kBlock) {
+        const int m = std::min(kBlock, n - p0);
+        for (int p = 0; p < m; p++) {
+            const float* src = pol + (size_t)(p0 + p) * pin;
+            for (int c = 0; c < 2; c++)
+                for (int i = 0; i < kPoints; i++)
+                    x[p * pin + c * kPoints + i] =
+                        w.bn_pol_scale[c] * (src[c * kPoints + i] - w.bn_pol_mean[c]);
+            for (int o = 0; o < pout; o++) y[p * pout + o] = w.ip_pol_b[o];
+        }
+        fc_pol(w.ip_pol_wt.data(), x, pin, pin, y, m);
+        for (int p = 0; p < m; p++) {
+            const float* logits = y + p * pout;
+            float* out = policy + (size_t)(p0 + p) * pout;
+            float alpha = logits[0];
+            for (int o = 1; o < pout; o++) alpha = std::max(alpha, logits[o]);
+            float denom = 0.0f;
+            for (int o = 0; o < pout; o++) {
+                out[o] = std::exp((logits[o] - alpha) / softmax_temp);
+                denom += out[o];
+            }
+            for (int o = 0; o < pout; o++) out[o] /= denom;
+        }
+        for (int p = 0; p < m; p++) {
+            const float* src = val + (size_t)(p0 + p) * kPoints;
+            for (int i = 0; i < kPoints; i++)
+                x[p * pin + i] = w.bn_val_scale * (src[i] - w.bn_val_mean);
+            for (int o = 0; o < vout; o++) y[p * vout + o] = w.ip1_val_b[o];
+        }
+        fc_val(w.ip1_val_wt.data(), x, kPoints, pin, y, m);
+        for (int p = 0; p < m; p++) {
+            const float* hid = y + p * vout;
+            float out = w.ip2_val_b;
+            for (int o = 0; o < vout; o++) out += std::max(hid[o], 0.0f) * w.ip2_val_w[o];
+            winrate[p0 + p] = (1.0f + std::tanh(out)) / 2.0f;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -201,7 +330,7 @@ Netresult NetworkFacade::get_output_internal(const go::Position& pos, int symmet
         winrate = (1.0f + value) / 2.0f;
     } else {
         m_pipe.forward(in, pol, val);  // may throw NetworkHaltException
-        heads_on_host(*m_heads, pol.data(), val.data(), m_temp, policy, &winrate);
+        heads_on_host(*m_heads, 1, pol.data(), val.data(), m_temp, policy, &winrate);
     }
     Netresult r;
     const int16_t* map = sym_table().idx[symmetry];

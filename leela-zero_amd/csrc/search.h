@@ -46,6 +46,9 @@ int symmetry_index(int symmetry, int idx);
 void gather_features(const uint8_t* const* boards, int n_boards, int to_move, int symmetry,
                      float* out /* [18][361] */);
 void gather_features(const go::Position& pos, int symmetry, float* out);
+// The same planes one bit per value, as BatchExecutor::run_bits takes them.
+void gather_bits(const uint8_t* const* boards, int n_boards, int to_move, int symmetry,
+                 uint32_t* bits /* [BatchExecutor::kInputWords] */);
 
 struct Netresult {
     std::array<float, go::kPoints> policy{};
@@ -67,9 +70,9 @@ struct HeadWeights {
 
 // BN+ReLU, FC, softmax / FC, ReLU, FC, tanh on raw head planes; policy comes
 // back in NN index order (no symmetry un-rotation).
-void heads_on_host(const HeadWeights& w, const float* pol /*[2][361]*/,
-                   const float* val /*[361]*/, float softmax_temp, float* policy /*[362]*/,
-                   float* winrate);
+void heads_on_host(const HeadWeights& w, int n, const float* pol /*[n][2][361]*/,
+                   const float* val /*[n][361]*/, float softmax_temp, float* policy /*[n][362]*/,
+                   float* winrate /*[n]*/);
 
 class EvalCache {
 public:
