@@ -37,6 +37,65 @@ __device__ __forceinline__ unsigned conv_cell(unsigned m) {
     return b * kCellsPerBoard + (y + 1) * 20 + x;
 }
 
+// The patch of a tile (the cells that its points reach) and what lies where in it.  Where it
+// begins is worked out once, in scalar registers; from there on every cell is less than 400 away
+// and every division is a 24-bit multiplication and a shift.  (With full divisions by 400, 20,
+// 361 and 19 and a branch for every kind of border a work-group spent 1400 to 4200 cycles, up to
+// a third of its life, before its first load; so 1000 to 1900.)
+struct PatchStart {
+    unsigned q0, b0, y0, x0;   // first cell, one board on (stays positive), and its parts
+    unsigned mb, mp;           // board and point of the tile's first row
+};
+__device__ __forceinline__ PatchStart patch_start(unsigned m0) {
+    PatchStart s;
+    s.q0 = conv_cell(m0) + kCellsPerBoard - 21;
+    s.b0 = s.q0 / kCellsPerBoard;
+    s.y0 = (s.q0 - s.b0 * kCellsPerBoard) / 20;
+    s.x0 = s.q0 - s.b0 * kCellsPerBoard - s.y0 * 20;
+    s.mb = m0 / kPts;
+    s.mp = m0 - s.mb * kPts;
+    return s;
+}
+// Cell of the patch in which the upper left tap of the tile's row `local` lies.
+__device__ __forceinline__ unsigned patch_cell(const PatchStart& s, unsigned local) {
+    unsigned p = s.mp + local;
+    const unsigned next = p >= kPts ? 1u : 0u;
+    p -= next * kPts;
+    const unsigned y = __umul24(p, 3450u) >> 16;   // p / 19
+    return (s.mb + next) * kCellsPerBoard + 20 + p + y + kCellsPerBoard - 21 - s.q0;
+}
+// Byte offsets in X of a thread's 16-byte pieces (PPC to a cell); cells off the board and
+// boards outside the batch get an offset outside the buffer and read as zero.
+template <int CELLS, int PPC, int NT, int NP>
+__device__ __forceinline__ void patch_offsets(unsigned (&poff)[NP], const PatchStart& s,
+                                              unsigned tid, unsigned Cp) {
+    static_assert(CELLS <= 380 && CELLS * PPC + NT < 16384, "small divisions");
+    // (points of row y1 = 0 of the board before: kept positive by the same distance)
+    const unsigned pt0 = s.b0 * kPts, lead = (kPts + kBoard) * Cp * 2u;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const unsigned piece = tid + i * NT;
+        const unsigned cell = PPC == 24 ? __umul24(piece, 2731u) >> 16 : piece / PPC;
+        const unsigned part = piece - cell * PPC;
+        const unsigned t = s.x0 + cell, dy = __umul24(t, 3277u) >> 16;   // t / 20
+        const unsigned x = t - dy * 20, y = s.y0 + dy;                   // y >= 20: the next board
+        const unsigned pt = pt0 + __umul24(y, 19u) + x - (y >= 20 ? 19u : 0u);
+        unsigned off = __umul24(pt, Cp * 2u) + part * 16u - lead;
+        asm volatile("" : "+v"(off));   // keeps the compiler from branching around it
+        const unsigned bad = (unsigned)(cell >= (unsigned)CELLS) | (unsigned)(x == 19) |
+                             (unsigned)(y == 0) | (unsigned)(y == 20);
+        poff[i] = off | (0u - bad);
+    }
+}
+
+// LDS is what a work-group shares: its writes are waited for, loads from memory stay in flight
+// across the barrier.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Filters: [k-step][Kp / 16][64 lanes][8], k-step = (chunk of 64 input channels, tap, half of
 // the chunk), i.e. the matrix instruction's row operand in the order it is used; every load of
 // a wavefront is one contiguous KiB.  Lane l of block kb holds output channel
@@ -84,11 +143,20 @@ size_t conv3x3_filter_count(int Cp, int Kp) {
 //
 // The sum over taps and channels runs in the same order in every variant, with the same
 // instruction, so a position's result does not depend on the batch it is evaluated in.
+// How the tiles of a layer lie on the 8 dies: 2^split dies side by side over the channel tiles,
+// 8 / 2^split over the row tiles, `cols` x `rows` tiles each.  Every die has an L2 of its own and
+// starts a layer with it empty, so it fetches its share of the filters (all of them / 2^split)
+// and of the planes (all of them / (8 / 2^split)): of the ways that load the dies equally the
+// one that fetches least is taken.
+struct ConvGrid {
+    int split, cols, rows, tiles_m;
+};
+
 template <int RB, int NB, int WR, int WN, int D, int DA, int CC, int OCC>
 __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
     half_t* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
-    float rfac, int n, int Cp, int Kp, int tiles_n, int seg, int n_items) {
+    float rfac, int n, int Cp, int Kp, ConvGrid g) {
     constexpr bool DB = CC == 0;
     constexpr int CH = DB ? 1 : CC;              // chunks of 64 channels staged together
     constexpr int NT = 64 * WR * WN;
@@ -104,7 +172,10 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     constexpr int GS = KS / NG > 0 ? KS / NG : 1;
     constexpr int PR = NB >= 2 ? NB / 2 : 1;     // stores per point: two blocks give 16 bytes
     constexpr int E = NB >= 2 ? 8 : 4;           // channels per store
-    constexpr bool EARLY = RB * NB <= 4;         // skip connection requested before the arithmetic
+    // The skip connection is requested with the planes where its registers (4 RB PR) can wait
+    // through the arithmetic (8 boards of 256 filters: the work-group's last phase 1500 -> 640
+    // cycles).
+    constexpr bool EARLY = RB * PR <= 6;
     static_assert(KS % D == 0 && KS % DA == 0, "rings turn a whole number of times per chunk");
     static_assert(D <= kFilterLookahead, "filter padding");
     static_assert(!DB || NG <= KS, "one group of pieces per k-step at most");
@@ -112,34 +183,43 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     __shared__ __attribute__((aligned(16))) unsigned char lds[DB ? 2 * BUF : BUF + 128 * DA];
     __shared__ __attribute__((aligned(16))) float bn[2][CW];
 
-    // Work-group w runs on die w % 8; the items (row tile, channel tile; channel tile fastest)
-    // are cut into 8 contiguous segments, one per die: the channel tiles of a row tile, and row
-    // tiles next to each other, read the same planes.
-    const int item = (int)(blockIdx.x & 7) * seg + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= seg || item >= n_items) return;
-    const int tn = item % tiles_n, tm = item / tiles_n;
+    // The grid is (8 cols) x rows, so work-group (x, y) runs on die x % 8 (see ConvGrid).
+    const int die = blockIdx.x & 7;
+    const int tn = (die & ((1 << g.split) - 1)) * g.cols + (int)(blockIdx.x >> 3);
+    const int tm = (die >> g.split) * g.rows + (int)blockIdx.y;
+    if (tm >= g.tiles_m) return;
     const int rows = n * kPts, m0 = tm * MT;
     const unsigned tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const int wr = wave / WN, wn = wave % WN;
 
-    // Global offsets of this thread's pieces of the patch; cells off the board (and past the
-    // batch) get an offset outside the buffer and read as zero.
-    const unsigned q0 = conv_cell(m0) + kCellsPerBoard - 21;   // one board on: stays positive
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
+    // First of all what depends on nothing that has to be worked out: batch norm (waited for with
+    // the planes; its loads come first, since loads are waited for in order) and filters.
+    static_assert(CW <= NT, "one thread per channel");
+    const unsigned bnoff = tid < (unsigned)CW ? (tn * CW + tid) * 4u : 0xfffffff0u;
+    const float scale = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                      make_rsrc(bn_scale, Kp * 4), bnoff, 0, 0));
+    const float mean = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                     make_rsrc(bn_mean, Kp * 4), bnoff, 0, 0));
+    const int kb = (tn * WN + wn) * NB;          // first block of 16 output channels
+    unsigned ws = (unsigned)kb * 1024u;
+    const unsigned wstep = (unsigned)Kp * 64u;   // bytes per k-step
+    const unsigned wv = lane * 16u;
     const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wf, ((size_t)9 * Cp + 32 * kFilterLookahead) * Kp * 2);
-    unsigned poff[NP];
+    int4v w[D][NB];
+    auto wload = [&](int slot, int j, unsigned st) {
+        w[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(rW, wv + j * 1024, ws + st * wstep, 0);
+    };
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const unsigned piece = tid + i * NT, cell = piece / PPC, part = piece % PPC;
-        const unsigned q = q0 + cell;
-        const unsigned b1 = q / kCellsPerBoard, r = q - b1 * kCellsPerBoard, y1 = r / 20,
-                       x = r - y1 * 20;
-        const bool ok = (cell < (unsigned)CELLS) & (b1 >= 1) & (b1 <= (unsigned)n) & (y1 >= 1) &
-                        (x < (unsigned)kBoard);
-        poff[i] = ok ? (((b1 - 1) * kPts + (y1 - 1) * kBoard + x) * (unsigned)Cp + part * 8u) * 2u
-                     : 0xfffffff0u;
-    }
+    for (int d = 0; d < D - 1; d++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) wload(d, j, d);
+    __builtin_amdgcn_sched_barrier(0);
+
+    const PatchStart ps = patch_start(m0);
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
+    unsigned poff[NP];
+    patch_offsets<CELLS, PPC, NT>(poff, ps, tid, Cp);
     // LDS address of piece i: a constant distance from piece 0 (but for the last, which may
     // lie past the end, and where a row of threads is no whole number of cells)
     const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 16u;
@@ -153,19 +233,11 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
 
     const int chunks = Cp / 64;
     unsigned arow[RB];   // LDS address of this lane's point of each row block, tap (0, 0)
+    static_assert(MT <= kPts, "a tile touches two boards at most");
 #pragma unroll
-    for (int i = 0; i < RB; i++) {
-        const unsigned m = min(m0 + (wr * RB + i) * 16 + (int)(lane & 15), rows - 1);
-        arow[i] = (conv_cell(m) + kCellsPerBoard - 21 - q0) * STR + (lane >> 4) * 16;
-    }
-    const int kb = (tn * WN + wn) * NB;          // first block of 16 output channels
-    unsigned ws = (unsigned)kb * 1024u;
-    const unsigned wstep = (unsigned)Kp * 64u;   // bytes per k-step
-    const unsigned wv = lane * 16u;
-    int4v w[D][NB];
-    auto wload = [&](int slot, int j, unsigned st) {
-        w[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(rW, wv + j * 1024, ws + st * wstep, 0);
-    };
+    for (int i = 0; i < RB; i++)
+        arow[i] = patch_cell(ps, min((wr * RB + i) * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
+                  (lane >> 4) * 16;
 
     const int ch0 = (kb >> 1) * 32 + 8 * (int)(lane >> 4) + 4 * (kb & 1);   // first channel
     unsigned ro[RB];                              // byte offset of this lane's point and channel
@@ -204,33 +276,19 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
 #pragma unroll
         for (int i = 0; i < NP; i++)
             stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rX, poff[i], 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int d = 0; d < D - 1; d++)
-#pragma unroll
-            for (int j = 0; j < NB; j++) wload(d, j, d);
-        __builtin_amdgcn_sched_barrier(0);
         if constexpr (EARLY) load_res();
-        for (int i = tid; i < CW; i += NT) {
-            const float s = bn_scale[tn * CW + i];
-            bn[0][i] = s;
-            bn[1][i] = -s * bn_mean[tn * CW + i];
-        }
 #pragma unroll
         for (int i = 0; i < NP; i++) *reinterpret_cast<int4v*>(lds + laddr(i)) = stg[i];
+        if (tid < (unsigned)CW) {
+            bn[0][tid] = scale;
+            bn[1][tid] = -scale * mean;
+        }
     }
     float4v acc[RB][NB];
 #pragma unroll
     for (int i = 0; i < RB; i++)
 #pragma unroll
         for (int j = 0; j < NB; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-    // LDS is what the work-group shares: its writes are waited for, the filter loads stay in
-    // flight across the barrier.
-    auto lds_barrier = []() {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
     lds_barrier();
 
     int4v a[DA][RB];
@@ -342,16 +400,32 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     }
 }
 
+static ConvGrid conv_grid(int tiles_m, int tiles_n, int n, int Cp, int Kp) {
+    ConvGrid best{};
+    size_t best_cost = ~(size_t)0;
+    for (int split = 0; split < 4 && tiles_n % (1 << split) == 0; split++) {
+        const int over_rows = 8 >> split;
+        const ConvGrid g{split, tiles_n >> split, (tiles_m + over_rows - 1) / over_rows, tiles_m};
+        const size_t bytes = ((size_t)9 * Cp * Kp >> split) + (size_t)n * kPts * Cp / over_rows;
+        // (32 units a die; rounds of tiles first)
+        const size_t rounds = ((size_t)g.cols * g.rows + 31) / 32;
+        const size_t cost = rounds << 40 | bytes;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = g;
+        }
+    }
+    return best;
+}
+
 template <int RB, int NB, int WR, int WN, int D, int DA, int CC, int OCC>
 static void launch_conv_as(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                            const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
                            int Kp, hipStream_t s, LaunchTimer* t) {
     constexpr int MT = WR * RB * 16, CW = WN * NB * 16;
     const int tiles_m = (n * kPts + MT - 1) / MT, tiles_n = Kp / CW;
-    int seg = (tiles_m * tiles_n + 7) / 8;
-    seg = (seg + tiles_n - 1) / tiles_n * tiles_n;   // the channel tiles of a row tile together
-    launch(conv3x3_k<RB, NB, WR, WN, D, DA, CC, OCC>, dim3(8 * seg), dim3(64 * WR * WN), s, t, X,
-           Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, Kp, tiles_n, seg, tiles_m * tiles_n);
+    const ConvGrid best = conv_grid(tiles_m, tiles_n, n, Cp, Kp);
+    launch(conv3x3_k<RB, NB, WR, WN, D, DA, CC, OCC>, dim3(8 * best.cols, best.rows), dim3(64 * WR * WN), s, t, X, Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, Kp, best);
 }
 
 // 64 filters have too little arithmetic per point to need it, and from 320 on the Winograd
@@ -365,13 +439,16 @@ bool conv3x3_serves(int Kp, int elem_bytes) {
 // work-group per unit; larger ones reuse each operand more.  Measured at 256 filters, us per
 // layer of a dependent chain with the tile of 32x32 | 32x64 | 48x64 | 96x64 | 192x64 |
 // 192x128 (points x channels), - = not measured:
-//    1 board    6.6 |  7.1 |  8.9 |  9.9 | 14.2 | 20.3
-//    4 boards   7.9 |  7.2 |  8.8 | 10.0 | 14.6 | 20.6
-//    8 boards   9.8 |  9.8 |  8.9 | 10.0 | 14.7 | 20.6
-//   16 boards  17.5 | 13.6 | 11.8 | 10.2 | 14.8 | 20.7
-//   32 boards  30.9 | 23.9 | 16.8 | 16.0 | 15.4 | 21.1
-//   64 boards     - |    - |    - |    - |    - | 22.7
-// (each entry jumps where the tile passes 256 work-groups).  192 filters have no tile of 128
+//    1 board    6.4 |  6.8 |  8.3 |  9.4 | 13.8 | 19.5
+//    4 boards   7.8 |  7.3 |  8.5 |  9.6 | 14.3 | 19.8
+//    8 boards   9.6 |  9.7 |  8.8 |  9.8 | 14.4 | 19.9
+//   16 boards  16.0 | 13.5 | 11.9 | 10.6 | 14.9 | 20.3
+//   24 boards  22.4 | 20.7 | 14.7 | 15.8 | 15.7 | 20.9
+//   32 boards  28.5 | 24.0 | 17.0 | 16.2 | 15.7 | 20.7
+//   64 boards  52.4 | 46.2 | 32.1 | 29.1 | 27.0 | 25.1
+// (each entry jumps where the tile passes 256 work-groups; the two wavefronts of a 48x64 tile
+// leave room for three on a unit, and until then it beats a 192x64 tile on half the units: 24
+// boards above, 37 boards of 128 filters 8.8 against 9.9).  192 filters have no tile of 128
 // channels; there 128 x 192 takes the place of 192 x 128 (64 boards 18.2 against 19.7 us with
 // three tiles of 64 channels).
 void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
@@ -409,6 +486,10 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
     }
     if (groups(96, 64) <= kUnits) {
         LZ_CONV(3, 2, 2, 2, 6, 3, 0, 2);
+        return;
+    }
+    if (groups(48, 64) <= 3 * kUnits) {
+        LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
         return;
     }
     if (groups(192, 64) <= kUnits) {
