@@ -409,7 +409,7 @@ int lzhip_get_output(lzhip_handle* h, const lzhip_head_weights* heads, const uin
     const int frc = h->sched->forward_raw(in.data(), pol.data(), val.data());
     if (frc == LZHIP_EHALT) return fail(LZHIP_EHALT, "halted by drain");
     float p[go::kPoints + 1];
-    heads_on_host(*hw, 1, pol.data(), val.data(), softmax_temp, p, winrate);
+    heads_on_host(*hw, pol.data(), val.data(), softmax_temp, p, winrate);
     for (int i = 0; i < go::kPoints; i++) policy[symmetry_index(symmetry, i)] = p[i];
     policy[go::kPoints] = p[go::kPoints];
     if (h->value_not_stm.load() && to_move == go::WHITE) *winrate = 1.0f - *winrate;
@@ -450,7 +450,7 @@ int lzhip_netbench(lzhip_handle* h, const lzhip_head_weights* heads, const uint8
                         halted++;
                         break;
                     }
-                    heads_on_host(*hw, 1, pol.data(), val.data(), 1.0f, p, &win);
+                    heads_on_host(*hw, pol.data(), val.data(), 1.0f, p, &win);
                 }
             } catch (const std::exception& e) {
                 std::lock_guard<std::mutex> lk(err_mu);

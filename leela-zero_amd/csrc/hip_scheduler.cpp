@@ -362,13 +362,14 @@ void HIPScheduler::worker() {
                 m_queue.pop_front();
             }
             m_inflight += (int)batch.size();
+            // (counted before another worker may collect)
+            if (!batch.empty()) m_waiting++;
         }
         if (batch.empty()) continue;
         const int n = (int)batch.size();  // m_inflight was raised under the lock above
         {
             // the executor takes m_lanes batches at a time
             std::unique_lock<std::mutex> lk(m_mutex);
-            m_waiting++;
             m_cv.wait(lk, [&] { return m_exec_busy < m_lanes; });
             m_waiting--;
             m_exec_busy++;

@@ -330,7 +330,7 @@ Netresult NetworkFacade::get_output_internal(const go::Position& pos, int symmet
         winrate = (1.0f + value) / 2.0f;
     } else {
         m_pipe.forward(in, pol, val);  // may throw NetworkHaltException
-        heads_on_host(*m_heads, 1, pol.data(), val.data(), m_temp, policy, &winrate);
+        heads_on_host(*m_heads, pol.data(), val.data(), m_temp, policy, &winrate);
     }
     Netresult r;
     const int16_t* map = sym_table().idx[symmetry];

@@ -73,6 +73,10 @@ struct HeadWeights {
 void heads_on_host(const HeadWeights& w, int n, const float* pol /*[n][2][361]*/,
                    const float* val /*[n][361]*/, float softmax_temp, float* policy /*[n][362]*/,
                    float* winrate /*[n]*/);
+inline void heads_on_host(const HeadWeights& w, const float* pol, const float* val,
+                          float softmax_temp, float* policy, float* winrate) {
+    heads_on_host(w, 1, pol, val, softmax_temp, policy, winrate);
+}
 
 class EvalCache {
 public:
