@@ -64,28 +64,26 @@ __device__ __forceinline__ unsigned patch_cell(const PatchStart& s, unsigned loc
     const unsigned y = __umul24(p, 3450u) >> 16;   // p / 19
     return (s.mb + next) * kCellsPerBoard + 20 + p + y + kCellsPerBoard - 21 - s.q0;
 }
-// Byte offsets in X of a thread's 16-byte pieces (PPC to a cell); cells off the board and
-// boards outside the batch get an offset outside the buffer and read as zero.
-template <int CELLS, int PPC, int NT, int NP>
-__device__ __forceinline__ void patch_offsets(unsigned (&poff)[NP], const PatchStart& s,
-                                              unsigned tid, unsigned Cp) {
-    static_assert(CELLS <= 380 && CELLS * PPC + NT < 16384, "small divisions");
-    // (points of row y1 = 0 of the board before: kept positive by the same distance)
-    const unsigned pt0 = s.b0 * kPts, lead = (kPts + kBoard) * Cp * 2u;
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const unsigned piece = tid + i * NT;
-        const unsigned cell = PPC == 24 ? __umul24(piece, 2731u) >> 16 : piece / PPC;
-        const unsigned part = piece - cell * PPC;
-        const unsigned t = s.x0 + cell, dy = __umul24(t, 3277u) >> 16;   // t / 20
-        const unsigned x = t - dy * 20, y = s.y0 + dy;                   // y >= 20: the next board
-        const unsigned pt = pt0 + __umul24(y, 19u) + x - (y >= 20 ? 19u : 0u);
-        unsigned off = __umul24(pt, Cp * 2u) + part * 16u - lead;
-        asm volatile("" : "+v"(off));   // keeps the compiler from branching around it
-        const unsigned bad = (unsigned)(cell >= (unsigned)CELLS) | (unsigned)(x == 19) |
-                             (unsigned)(y == 0) | (unsigned)(y == 20);
-        poff[i] = off | (0u - bad);
-    }
+// Byte offset in X of a thread's 16-byte piece i (PPC to a cell); cells off the board and boards
+// outside the batch get an offset outside the buffer and read as zero.
+template <int CELLS, int PPC, int NT>
+__device__ __forceinline__ unsigned patch_offset(int i, const PatchStart& s, unsigned tid,
+                                                 unsigned Cp) {
+    static_assert(CELLS <= 380 && (PPC != 24 || CELLS * PPC + NT < 8200), "small divisions");
+    const unsigned piece = tid + i * NT;
+    const unsigned cell = PPC == 24 ? __umul24(piece, 2731u) >> 16 : piece / PPC;
+    const unsigned part = piece - cell * PPC;
+    const unsigned t = s.x0 + cell, dy = __umul24(t, 3277u) >> 16;   // t / 20
+    const unsigned x = t - dy * 20, y = s.y0 + dy;                   // y >= 20: the next board
+    // t - dy = 19 dy + x, in points of the board's rows; row y1 = 0 of the board before is kept
+    // positive by `lead`
+    const unsigned lead = (kPts + kBoard) * Cp * 2u;
+    const unsigned pt = s.b0 * kPts + s.y0 * kBoard + t - dy - (y >= 20 ? 19u : 0u);
+    unsigned off = __umul24(pt, Cp * 2u) + part * 16u - lead;
+    asm volatile("" : "+v"(off));   // keeps the compiler from branching around it
+    const unsigned bad = (unsigned)(cell >= (unsigned)CELLS) | (unsigned)(x == 19) |
+                         (unsigned)(y == 0) | (unsigned)(y == 20);
+    return off | (0u - bad);
 }
 
 // LDS is what a work-group shares: its writes are waited for, loads from memory stay in flight
@@ -143,14 +141,28 @@ size_t conv3x3_filter_count(int Cp, int Kp) {
 //
 // The sum over taps and channels runs in the same order in every variant, with the same
 // instruction, so a position's result does not depend on the batch it is evaluated in.
-// How the tiles of a layer lie on the 8 dies: 2^split dies side by side over the channel tiles,
-// 8 / 2^split over the row tiles, `cols` x `rows` tiles each.  Every die has an L2 of its own and
-// starts a layer with it empty, so it fetches its share of the filters (all of them / 2^split)
-// and of the planes (all of them / (8 / 2^split)): of the ways that load the dies equally the
-// one that fetches least is taken.
+// How the tiles of a layer lie on the 8 dies: 2^split dies side by side over the channel tiles
+// (`cols` of them each), 8 / 2^split over the row tiles: a column of dies deals its tiles, row by
+// row, in equal shares of `share`, which may end within a row (in whole rows, 44 boards of 384
+// filters gave some dies 33 tiles for their 32 units: 52 us per layer, now
+// 36; 44 boards of 192 filters 21.2, now 14.2).  Every die
+// has an L2 of its own and starts a layer with it empty, so it fetches its share of the filters
+// (all of them / 2^split) and of the planes (all of them / (8 / 2^split)): of the ways that load
+// the dies equally the one that fetches least is taken.
 struct ConvGrid {
-    int split, cols, rows, tiles_m;
+    int split, cols, share, tiles_m;
+    unsigned inv;   // ceil(2^31 / cols)
 };
+struct ConvTile {
+    int m, n;
+};
+// Work-group x runs on die x % 8.
+__device__ __forceinline__ ConvTile conv_tile(const ConvGrid& g) {
+    const int die = blockIdx.x & 7;
+    const unsigned i = (die >> g.split) * g.share + (blockIdx.x >> 3);
+    const int m = (int)__umulhi(i * 2u, g.inv);
+    return {m, (die & ((1 << g.split) - 1)) * g.cols + (int)i - m * g.cols};
+}
 
 template <int RB, int NB, int WR, int WN, int D, int DA, int CC, int OCC>
 __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
@@ -183,10 +195,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     __shared__ __attribute__((aligned(16))) unsigned char lds[DB ? 2 * BUF : BUF + 128 * DA];
     __shared__ __attribute__((aligned(16))) float bn[2][CW];
 
-    // The grid is (8 cols) x rows, so work-group (x, y) runs on die x % 8 (see ConvGrid).
-    const int die = blockIdx.x & 7;
-    const int tn = (die & ((1 << g.split) - 1)) * g.cols + (int)(blockIdx.x >> 3);
-    const int tm = (die >> g.split) * g.rows + (int)blockIdx.y;
+    const ConvTile tile = conv_tile(g);
+    const int tn = tile.n, tm = tile.m;
     if (tm >= g.tiles_m) return;
     const int rows = n * kPts, m0 = tm * MT;
     const unsigned tid = threadIdx.x, lane = tid & 63;
@@ -219,7 +229,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     const PatchStart ps = patch_start(m0);
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
     unsigned poff[NP];
-    patch_offsets<CELLS, PPC, NT>(poff, ps, tid, Cp);
+#pragma unroll
+    for (int i = 0; i < NP; i++) poff[i] = patch_offset<CELLS, PPC, NT>(i, ps, tid, Cp);
     // LDS address of piece i: a constant distance from piece 0 (but for the last, which may
     // lie past the end, and where a row of threads is no whole number of cells)
     const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 16u;
@@ -405,10 +416,12 @@ static ConvGrid conv_grid(int tiles_m, int tiles_n, int n, int Cp, int Kp) {
     size_t best_cost = ~(size_t)0;
     for (int split = 0; split < 4 && tiles_n % (1 << split) == 0; split++) {
         const int over_rows = 8 >> split;
-        const ConvGrid g{split, tiles_n >> split, (tiles_m + over_rows - 1) / over_rows, tiles_m};
+        const int cols = tiles_n >> split;
+        const ConvGrid g{split, cols, (tiles_m * cols + over_rows - 1) / over_rows, tiles_m,
+                         ((1u << 31) + cols - 1) / cols};
         const size_t bytes = ((size_t)9 * Cp * Kp >> split) + (size_t)n * kPts * Cp / over_rows;
         // (32 units a die; rounds of tiles first)
-        const size_t rounds = ((size_t)g.cols * g.rows + 31) / 32;
+        const size_t rounds = ((size_t)g.share + 31) / 32;
         const size_t cost = rounds << 40 | bytes;
         if (cost < best_cost) {
             best_cost = cost;
@@ -425,13 +438,16 @@ static void launch_conv_as(const half_t* X, const half_t* Wf, const half_t* res,
     constexpr int MT = WR * RB * 16, CW = WN * NB * 16;
     const int tiles_m = (n * kPts + MT - 1) / MT, tiles_n = Kp / CW;
     const ConvGrid best = conv_grid(tiles_m, tiles_n, n, Cp, Kp);
-    launch(conv3x3_k<RB, NB, WR, WN, D, DA, CC, OCC>, dim3(8 * best.cols, best.rows), dim3(64 * WR * WN), s, t, X, Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, Kp, best);
+    launch(conv3x3_k<RB, NB, WR, WN, D, DA, CC, OCC>, dim3(8 * best.share),
+           dim3(64 * WR * WN), s, t, X, Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, Kp, best);
 }
 
-// 64 filters have too little arithmetic per point to need it, and from 320 on the Winograd
-// kernels are ahead for some batches (384 filters, 44 boards: 40 against 52 us per layer).
+// The published widths and 384.  Measured per forward of 10 blocks, Winograd kernels -> this, us:
+// 64 filters, 1 board 191 -> 73, 64 boards 351 -> 127, 200 boards 488 -> 271; 384 filters, 1 board
+// 263 -> 120, 16 boards 523 -> 468, 44 boards 937 -> 761, 100 boards 1628 -> 1733, 200 boards 3297
+// -> 2923, and with two forwards side by side 44 boards 1407 -> 1271, 100 boards 3314 -> 2711.
 bool conv3x3_serves(int Kp, int elem_bytes) {
-    return elem_bytes == 2 && (Kp == 128 || Kp == 192 || Kp == 256);
+    return elem_bytes == 2 && (Kp == 64 || Kp == 128 || Kp == 192 || Kp == 256 || Kp == 384);
 }
 
 // The tile.  A layer of few boards is a chain of latencies, so its points and channels are
@@ -503,6 +519,232 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
     else
         LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);
 #undef LZ_CONV
+}
+
+// ---------------------------------------------------------------------------
+// The same layer with the sum over input channels dealt to the wavefronts of a work-group.
+//
+// With few boards a unit has one small tile, and what a layer takes is one chain of latencies.  In
+// conv3x3_k the wavefronts of such a tile each own so narrow a part of it that every operand is
+// fetched twice or four times, and all wait for the whole patch.  Here every wavefront owns the
+// whole tile and KW-th of the k-steps (HPW halves of a chunk of 64 channels, all nine taps): each
+// operand is fetched once, a wavefront stages its own input channels and waits for nobody, its
+// filters are in flight all at once (D = 9 HPW; two thirds of them where six wavefronts share
+// the registers), and the partial sums meet in LDS at the end, in the order of the wavefronts.
+// Measured per forward of 10 blocks, conv3x3_k -> this, us: 64 filters see conv3x3_serves; 128
+// filters, 1 board 99 -> 74, 8 boards 113 -> 90; 192 filters, 1 board 121 -> 96, 5 boards 138 ->
+// 115; 256 filters, 1 board 133 -> 107, 5 boards 159 -> 146.
+// Tiles of 96x32, 96x64 and 192x64 points x channels were tried for larger batches and gave
+// nothing (256 filters, 16 boards 215 -> 212, 32 boards 318 -> 324; two forwards side by side
+// lost 10 %): there the partial sums' way through LDS, 2 KW RB NB KiB, costs what it saves.
+// The order of the sum differs from conv3x3_k's, so a network uses one or the other whatever the
+// batch (conv3x3_splits).
+template <int RB, int KW, int HPW, int D>
+__global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
+    const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
+    half_t* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
+    float rfac, int n, int Kp, ConvGrid g) {
+    constexpr int NB = 2, DA = 3;                          // 32 channels; planes read ahead
+    constexpr int CH = KW * HPW / 2, Cp = 64 * CH, NT = 64 * KW;
+    constexpr int MT = RB * 16, CW = NB * 16, CELLS = conv_cells(MT);
+    constexpr int STR = HPW * 64 + 16, SLICE = (CELLS + 1) * STR;   // bytes per cell, wavefront
+    constexpr int PPC = HPW * 4, NP = (CELLS * PPC + 63) / 64;   // 16-byte pieces: a cell's, a lane's
+    constexpr int STEPS = 9 * HPW;
+    constexpr int QP = (RB + KW - 1) / KW;   // blocks of 16 points that a wavefront finishes
+    constexpr int BYTES = KW * (SLICE > RB * NB * 1024 ? SLICE : RB * NB * 1024);
+    static_assert(D <= STEPS && CW <= NT, "tile");
+    static_assert(HPW == 2 || (HPW == 1 && KW % 2 == 0), "whole chunks");
+    __shared__ __attribute__((aligned(16))) unsigned char lds[BYTES];
+    __shared__ __attribute__((aligned(16))) float bn[2][CW];
+
+    const ConvTile tile = conv_tile(g);
+    const int tn = tile.n, tm = tile.m;
+    if (tm >= g.tiles_m) return;
+    const int rows = n * kPts, m0 = tm * MT;
+    const unsigned tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
+
+    const unsigned bnoff = tid < (unsigned)CW ? (tn * CW + tid) * 4u : 0xfffffff0u;
+    const float scale = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                      make_rsrc(bn_scale, Kp * 4), bnoff, 0, 0));
+    const float mean = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                     make_rsrc(bn_mean, Kp * 4), bnoff, 0, 0));
+    // this wavefront's k-steps, nine taps of one half after the other: their places in Wf
+    const unsigned first = HPW == 2 ? wave * kStepsPerChunk
+                                    : (wave >> 1) * kStepsPerChunk + (wave & 1);
+    const unsigned wstep = (unsigned)Kp * 64u;
+    const unsigned ws = first * wstep + (unsigned)(tn * NB) * 1024u;
+    const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wf, ((size_t)9 * Cp + 32 * kFilterLookahead) * Kp * 2);
+    int4v w[D][NB];
+    auto wload = [&](int slot, int j, unsigned st) {
+        w[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(rW, lane * 16u + j * 1024,
+                                                           ws + (st % 9 * 2 + st / 9) * wstep, 0);
+    };
+    // A wavefront reads only its own input channels, so it stages them itself and waits for
+    // nobody.  A few filters, the planes, the other filters: what the L1 delivers is what a tile
+    // waits for at first, so the planes do not stand behind filters that are needed after them,
+    // and each piece is requested as soon as its address is known.
+    constexpr int F0 = D - 1 < 4 ? D - 1 : 4;
+    auto filters = [&](int from, int to) {
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                if (d >= from && d < to) wload(d, j, d);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    filters(0, F0);
+    const PatchStart ps = patch_start(m0);
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
+    int4v stg[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        stg[i] = __builtin_amdgcn_raw_buffer_load_b128(
+            rX, patch_offset<CELLS, PPC, 64>(i, ps, lane, Cp), wave * (HPW * 64), 0);
+        if (i % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    filters(F0, D - 1);
+
+    // the blocks of 16 points that this wavefront finishes: where they lie, and the skip connection
+    unsigned ro[QP];
+    int4v rr[QP];
+    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, (size_t)rows * Kp * 2);
+    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, (size_t)rows * Kp * 2);
+    const int cl = 8 * (int)(lane >> 4);   // first of this lane's 8 channels
+#pragma unroll
+    for (int q = 0; q < QP; q++) {
+        const int i = q * KW + wave, m = m0 + i * 16 + (int)(lane & 15);
+        ro[q] = i < RB && m < rows ? (unsigned)((m * Kp + tn * CW + cl) * 2) : 0xfffffff0u;
+        rr[q] = int4v{0, 0, 0, 0};
+    }
+    if (res != nullptr) {
+#pragma unroll
+        for (int q = 0; q < QP; q++)
+            rr[q] = __builtin_amdgcn_raw_buffer_load_b128(rR, ro[q], 0, 0);
+    }
+    unsigned char* const own = lds + wave * SLICE;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const unsigned piece = lane + i * 64, cell = piece / PPC;
+        *reinterpret_cast<int4v*>(own + (cell < (unsigned)CELLS ? cell : (unsigned)CELLS) * STR +
+                                  piece % PPC * 16u) = stg[i];
+    }
+    if (tid < (unsigned)CW) {
+        bn[0][tid] = scale;
+        bn[1][tid] = -scale * mean;
+    }
+    unsigned arow[RB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+        arow[i] = patch_cell(ps, min(i * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
+                  (lane >> 4) * 16;
+    float4v acc[RB][NB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+
+    int4v a[DA][RB];
+    auto aread = [&](int i, int st) {
+        const int half = st / 9, tap = st % 9;
+        return *reinterpret_cast<const int4v*>(own + arow[i] + ((tap / 3) * 20 + tap % 3) * STR +
+                                               half * 64);
+    };
+#pragma unroll
+    for (int d = 0; d < DA; d++)
+#pragma unroll
+        for (int i = 0; i < RB; i++) a[d][i] = aread(i, d);
+#pragma unroll
+    for (int st = 0; st < STEPS; st++) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < RB; i++) {
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                if (i == (RB >= NB ? j : 0) && st + D - 1 < STEPS)
+                    wload((st + D - 1) % D, j, st + D - 1);
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    __builtin_bit_cast(half8v, w[st % D][j]),
+                    __builtin_bit_cast(half8v, a[st % DA][i]), acc[i][j], 0, 0, 0);
+            if (st + DA < STEPS) a[st % DA][i] = aread(i, st + DA);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    // partial sums through LDS: [wavefront][row block][channel block][64 lanes][4]
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            *reinterpret_cast<float4v*>(lds + ((wave * RB + i) * NB + j) * 1024 + lane * 16) =
+                acc[i][j];
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < QP; q++) {
+        const int i = q * KW + wave;
+        if (i >= RB) continue;
+        float4v part[KW][NB];
+#pragma unroll
+        for (int k = 0; k < KW; k++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                part[k][j] = *reinterpret_cast<const float4v*>(
+                    lds + ((k * RB + i) * NB + j) * 1024 + lane * 16);
+        const half8v rh = __builtin_bit_cast(half8v, rr[q]);
+        half8v o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float v = part[0][e / 4][e % 4];
+#pragma unroll
+            for (int k = 1; k < KW; k++) v += part[k][e / 4][e % 4];
+            o[e] = (half_t)fminf(
+                fmaxf(0.0f, fmaf((float)rh[e], rfac, fmaf(v, bn[0][cl + e], bn[1][cl + e]))),
+                kActStoreMax);
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY, ro[q], 0, 0);
+    }
+}
+
+// The tile, in blocks of 16 points by 32 channels: the smallest whose work-groups are no more
+// than the compute units; 0: none of the three is.
+static int split_blocks(int n, int Kp) {
+    for (int rb = 2; rb <= 4; rb++)
+        if ((n * kPts + rb * 16 - 1) / (rb * 16) * (Kp / 32) <= 256) return rb;
+    return 0;
+}
+
+bool conv3x3_splits(int Kp, int max_batch) {
+    return conv3x3_serves(Kp, 2) && split_blocks(max_batch, Kp) > 0;
+}
+
+void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
+                          const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
+                          int Kp, hipStream_t s, LaunchTimer* t) {
+    const int rb = split_blocks(n, Kp);
+    if (!conv3x3_splits(Kp, n) || Cp != Kp)
+        throw std::invalid_argument("no split convolution for this width or batch");
+    const ConvGrid g = conv_grid((n * kPts + rb * 16 - 1) / (rb * 16), Kp / 32, n, Cp, Kp);
+    auto go = [&](auto kernel, int waves) {
+        launch(kernel, dim3(8 * g.share), dim3(64 * waves), s, t, X, Wf, res, Y, bn_scale,
+               bn_mean, rfac, n, Kp, g);
+    };
+    // KW wavefronts x HPW halves of a chunk
+#define LZ_SPLIT(KW, HPW, D)                                   \
+    if (rb == 2) go(conv3x3_split_k<2, KW, HPW, D>, KW);       \
+    else if (rb == 3) go(conv3x3_split_k<3, KW, HPW, D>, KW);  \
+    else go(conv3x3_split_k<4, KW, HPW, D>, KW)
+    switch (Kp) {
+        case 64: LZ_SPLIT(2, 1, 9); break;
+        case 128: LZ_SPLIT(4, 1, 9); break;
+        case 192: LZ_SPLIT(3, 2, 18); break;
+        case 256: LZ_SPLIT(4, 2, 18); break;
+        default: LZ_SPLIT(6, 2, 12); break;
+    }
+#undef LZ_SPLIT
 }
 
 // ---------------------------------------------------------------------------

@@ -261,8 +261,11 @@ public:
         m_layers.resize(n_layers);
         // fp16 towers of the widths conv3x3_serves names are computed by direct convolution,
         // provided that what was handed over are transforms of 3x3 filters; all else goes
-        // through the Winograd kernels and needs their tile arrays.
-        m_direct = conv3x3_serves(m_Fp, (int)sizeof(P)) && build_direct_filters(n_layers, U);
+        // through the Winograd kernels and needs their tile arrays.  (So do towers of 64 filters
+        // and less than 3 blocks: no network that is played has so few, and they are what holds
+        // the half-precision Winograd kernels, and their launches, to account at little cost.)
+        m_direct = conv3x3_serves(m_Fp, (int)sizeof(P)) && (m_Fp > 64 || n_layers >= 7) &&
+                   build_direct_filters(n_layers, U);
         if (!m_direct) alloc_tiles();
         // Filters are laid out on the host in fp32; an fp16 net converts them on the device.
         std::vector<float> tmp;
@@ -706,8 +709,7 @@ public:
         launch_gemm<P>(V, U, Uf, M, Tu, m_Tp, Cp, m_Fp, ln.stream, nullptr);
         if constexpr (sizeof(P) == 2) {
             if (m_direct)
-                launch_conv3x3(a_in, L.W3.p, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, Cp, m_Fp,
-                               ln.stream, nullptr);
+                conv_direct(L, a_in, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, ln.stream, nullptr);
         }
         if (!m_direct)
             launch_out_transform<P>(M, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, m_Fp, m_Tp,
@@ -844,8 +846,8 @@ private:
         Layer& L = m_layers[l];
         if constexpr (sizeof(P) == 2) {
             if (m_direct) {
-                launch_conv3x3(in, L.W3.p, res, out, L.d_scale.p, L.d_mean.p, L.rfac, n, L.Cp,
-                               m_Fp, ln.stream, timer(timed, LZHIP_K_GEMM));
+                conv_direct(L, in, res, out, L.d_scale.p, L.d_mean.p, L.rfac, n, ln.stream,
+                            timer(timed, LZHIP_K_GEMM));
                 return;
             }
         }
@@ -953,6 +955,16 @@ private:
         }
     }
 
+    // One layer of a direct tower; which of the two kernels depends on the handle, not on n.
+    void conv_direct(const Layer& L, const P* in, const P* res, P* out, const float* scale,
+                     const float* mean, float rfac, int n, hipStream_t s, LaunchTimer* t) {
+        if constexpr (sizeof(P) == 2) {
+            const bool split = L.Cp == m_Fp && conv3x3_splits(m_Fp, m_max_batch);
+            (split ? launch_conv3x3_split : launch_conv3x3)(in, L.W3.p, res, out, scale, mean, rfac,
+                                                            n, L.Cp, m_Fp, s, t);
+        }
+    }
+
     // The layer loop of a direct tower: one launch per layer.
     void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed) {
         if constexpr (sizeof(P) == 2) {
@@ -964,9 +976,8 @@ private:
                 const bool second = l >= 2 && (l % 2) == 0;
                 const P* in = l == 0 ? w.act0 : second ? w.act[1] : w.act[cur];
                 P* out = l == 0 ? w.act[cur] : second ? w.act[nxt] : w.act[1];
-                launch_conv3x3(in, L.W3.p, second ? w.act[cur] : nullptr, out, L.d_scale.p,
-                               L.d_mean.p, L.rfac, n, L.Cp, m_Fp, w.stream,
-                               timer(timed, LZHIP_K_GEMM));
+                conv_direct(L, in, second ? w.act[cur] : nullptr, out, L.d_scale.p, L.d_mean.p,
+                            L.rfac, n, w.stream, timer(timed, LZHIP_K_GEMM));
                 last = out;
                 if (second) { const int o = cur; cur = nxt; nxt = o; }
             }

@@ -827,6 +827,36 @@ def test_direct_convolution_tiles(pkg, netgen, orc, filters, batches):
     pipe.close()
 
 
+@pytest.mark.parametrize("filters,maxb,batches", [
+    (64, 11, (1, 11)), (64, 17, (12, 17)), (64, 22, (1, 18, 22)),
+    (64, 137, (11, 12, 22, 23, 34, 35, 68, 69, 102, 103, 136, 137)),
+    (128, 5, (1, 5)), (128, 8, (6, 8)), (128, 11, (9, 11)),
+    (192, 3, (1, 3)), (192, 5, (4, 5)), (192, 7, (1, 6, 7)), (192, 44, (44,)),
+    (256, 2, (1, 2)), (256, 4, (3, 4)), (256, 5, (1, 5)),
+    (384, 1, (1,)), (384, 2, (2,)), (384, 3, (1, 3)), (384, 45, (1, 5, 6, 11, 12, 17, 18, 22, 23, 44, 45)),
+])
+def test_direct_convolution_of_small_handles_and_other_widths(pkg, netgen, orc, filters, maxb, batches):
+    """fp16 towers whose handle is small enough for the convolution that deals its sum to the
+    wavefronts (three tiles, both ends of each), and the tiles of 64 and 384 filters: one layer
+    with a skip connection against a float32 convolution."""
+    import torch
+    import torch.nn.functional as F
+    blocks = 3 if filters == 64 else 1      # fewer blocks of 64 filters stay with Winograd
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, blocks, filters, 6650 + filters, pkg.FP16, maxb)
+    rng = np.random.default_rng(filters + maxb)
+    a = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
+    r = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
+    y = F.conv2d(torch.from_numpy(a.reshape(maxb, filters, 19, 19)), torch.from_numpy(net.conv_w[2]),
+                 padding=1).numpy().reshape(maxb, filters, 361)
+    want = np.maximum(0.0, ref.scale[2][None, :, None] * (y - ref.mean[2][None, :, None]) + r)
+    for n in batches:
+        print("case: %d filters, %d boards of %d" % (filters, n, maxb), flush=True)
+        got = pipe.debug_layer(2, a[:n], r[:n])[2]
+        for i in range(n):
+            assert rel_l2(got[i], want[i]) <= 2e-3, (n, i)
+    pipe.close()
+
+
 def test_winograd_filters_of_no_3x3_filter(pkg, netgen, orc):
     """Winograd-domain filters that are not the transform of any 3x3 filter have no direct
     form: such a network runs through the Winograd kernels and agrees with the oracle."""
