@@ -82,7 +82,9 @@ int lzhip_create_from_file(const char* path, int precision, int max_batch, int d
                            lzhip_handle** out, int* filters, int* blocks);
 
 /* Destructor of the backend (reference src/OpenCLScheduler.cpp:134-144):
- * wakes and joins the worker, pending requests finish with LZHIP_EHALT. */
+ * wakes and joins the workers, pending requests finish with LZHIP_EHALT, requests already on
+ * the device with their results; returns when the last caller has left lzhip_forward /
+ * lzhip_forward_eval.  No other call may be in progress on the handle. */
 int lzhip_destroy(lzhip_handle* h);
 
 /* ForwardPipe::push_weights (reference src/ForwardPipe.h:65-67; contents of

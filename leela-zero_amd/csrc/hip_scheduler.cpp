@@ -7,7 +7,8 @@
 //    its own buffers (:256-277, :392-403);
 //  * drain() empties the queue and makes every waiting and every later
 //    forward() end with NetworkHaltException until resume() (:411-441);
-//  * the destructor stops the worker and releases waiters (:134-144).
+//  * the destructor stops the worker and releases waiters (:134-144); it returns once the
+//    last caller has left forward(), also one that evaluates its own position.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -35,6 +36,7 @@ HIPScheduler::HIPScheduler(std::unique_ptr<BatchExecutor> exec) : m_exec(std::mo
 }
 
 HIPScheduler::~HIPScheduler() {
+    m_draining.store(true);   // whoever is about to queue a request is halted
     {
         std::lock_guard<std::mutex> lk(m_mutex);
         m_running = false;
@@ -55,6 +57,10 @@ HIPScheduler::~HIPScheduler() {
         }
         r->cv.notify_all();
     }
+    // A caller that was answered still reads members, and a lone one is inside the executor.
+    // Looking again now and then, instead of a condition to wait for, keeps a lock and a
+    // wake-up out of every evaluation.
+    while (m_outstanding.load() > 0) std::this_thread::sleep_for(std::chrono::microseconds(50));
     delete m_fail_msg;
 }
 
@@ -142,25 +148,27 @@ int HIPScheduler::evaluate_raw(const float* in, float temperature, float* policy
 }
 
 int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
+    // The destructor waits for the callers counted here: leaving is the last thing that a call
+    // does to this object.
+    struct Inside {
+        std::atomic<int>& count;
+        explicit Inside(std::atomic<int>& c) : count(c) { count++; }
+        ~Inside() { count--; }
+    } inside(m_outstanding);
     if (m_draining.load()) {
         m_halted++;
         return LZHIP_EHALT;
     }
     req->packed = m_exec && m_exec->accepts_bits() && pack_planes(req->in, req->bits);
-    m_outstanding++;
     bool wake, alone = false;
     {
         std::lock_guard<std::mutex> lk(m_mutex);
-        if (!m_running) {
-            m_outstanding--;
-            throw std::runtime_error("forward: scheduler is not initialised");
-        }
-        // drain() may have started between the check above and here
+        // drain() or the destructor may have started between the check above and here
         if (m_draining.load()) {
-            m_outstanding--;
             m_halted++;
             return LZHIP_EHALT;
         }
+        if (!m_running) throw std::runtime_error("forward: scheduler is not initialised");
         // A caller that is alone evaluates its position itself: handing it to a worker and being
         // woken by it costs two thread switches (about 15 us of a 200 us evaluation), and there
         // is nobody to share a batch with.
@@ -180,7 +188,6 @@ int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
     if (alone) {
         std::string why;
         const int state = execute(&req, 1, nullptr, why);
-        m_outstanding--;
         if (state != 1) throw std::runtime_error(why);
         m_requests++;
         return LZHIP_OK;
@@ -192,7 +199,6 @@ int HIPScheduler::submit(const std::shared_ptr<Request>& req) {
         req->cv.wait(lk, [&] { return req->state != 0; });
         state = req->state;
     }
-    m_outstanding--;
     if (state == 1) {
         m_requests++;
         return LZHIP_OK;

@@ -5,7 +5,8 @@
 //   * a batch never exceeds max_batch;
 //   * drain() releases every waiter with a halt, later calls halt at once,
 //     resume() needs an empty queue and re-opens the pipe;
-//   * destruction with idle and with blocked callers ends cleanly;
+//   * destruction with idle, with blocked and with evaluating callers ends cleanly, and
+//     only after the last caller has left forward();
 //   * an executor failure reaches the caller as an exception;
 //   * with an executor that accepts two or three batches at a time, that many are in
 //     flight together and all of the above still holds;
@@ -290,6 +291,60 @@ static void test_destroy_with_waiters(int concurrency) {
     std::printf("destroy: %d served, %d halted\n", ok.load(), halted.load());
 }
 
+// Notes what is left of the executor and of the scheduler when an evaluation ends.
+class MortalExec : public FakeExec {
+public:
+    struct Fate {
+        std::atomic<bool> dead{false}, outlived{false};
+    };
+    MortalExec(int mb, int delay_us, int concurrency, std::shared_ptr<Fate> f)
+        : FakeExec(mb, 0, concurrency), m_wait(delay_us), m_fate(std::move(f)) {}
+    ~MortalExec() override { m_fate->dead = true; }
+    void forward_batch(int n, const float* in, float* pol, float* val) override {
+        const std::shared_ptr<Fate> fate = m_fate;   // outlives this object
+        started++;
+        std::this_thread::sleep_for(std::chrono::microseconds(m_wait));
+        if (fate->dead) {
+            fate->outlived = true;
+            return;
+        }
+        FakeExec::forward_batch(n, in, pol, val);
+    }
+    std::atomic<int> started{0};
+private:
+    int m_wait;
+    std::shared_ptr<Fate> m_fate;
+};
+
+// The scheduler dies, without a drain() before, while `callers` threads are inside forward():
+// one evaluating its own position (a lone caller), or batches inside the executor and more
+// requests behind them.  Each is answered or halted before the destructor returns.
+static void test_destroy_under_callers(int callers, int concurrency) {
+    auto fate = std::make_shared<MortalExec::Fate>();
+    auto* fe = new MortalExec(2, 20000, concurrency, fate);
+    auto* s = new HIPScheduler{std::unique_ptr<BatchExecutor>(fe)};
+    s->set_max_wait_us(0);
+    std::atomic<int> ok{0}, halted{0};
+    std::vector<std::thread> th;
+    for (int t = 0; t < callers; t++)
+        th.emplace_back([&, t] {
+            try {
+                one_call(*s, (float)t, 1.0f, ok, halted);
+            } catch (const std::runtime_error&) {
+                CHECK(!fate->outlived);
+            }
+        });
+    while (s->outstanding() < callers || fe->started < 1) std::this_thread::yield();
+    delete s;
+    CHECK(fate->dead);
+    for (auto& t : th) t.join();
+    CHECK(!fate->outlived);
+    CHECK(ok + halted == callers);
+    CHECK(ok >= 1);
+    std::printf("destroy under %d callers: %d served, %d halted\n", callers, ok.load(),
+                halted.load());
+}
+
 static void test_executor_failure(int concurrency) {
     auto* fe = new FakeExec(4, 10, concurrency);
     HIPScheduler s{std::unique_ptr<BatchExecutor>(fe)};
@@ -331,6 +386,8 @@ int main() {
     for (int c = 1; c <= 3; c++) {
         test_drain_resume(c);
         test_destroy_with_waiters(c);
+        test_destroy_under_callers(1, c);
+        test_destroy_under_callers(9, c);
         test_executor_failure(c);
     }
     std::printf("scheduler tests passed\n");
