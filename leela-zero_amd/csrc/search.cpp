@@ -165,7 +165,7 @@ HeadWeights::HeadWeights(const lzhip_head_weights& w) {
 
 namespace {
 
-// y += W^T x over the inputs x that are positive after batch norm (the others add nothing),
+// y += W^T x over the inputs x but those ReLU turns to zero after batch norm (they add nothing),
 // for n positions at once.  Blocks of 8 rows of W (at most 12 KB) stay in the first-level cache
 // while the positions pass over them, and a pass adds up to four rows per visit of y.
 template <int N>
@@ -178,7 +178,7 @@ __attribute__((always_inline)) inline void fc_rows(const float* wt, const float*
             float v[8];
             int m = 0;
             for (int i = 0; i < rows; i++)
-                if (xp[i] > 0.0f) {
+                if (!(xp[i] <= 0.0f)) {   // (a NaN must come through)
                     v[m] = xp[i];
                     r[m++] = wt + (size_t)(i0 + i) * N;
                 }

@@ -19,6 +19,7 @@
 //   * with the heads computed behind the pipe (requests of that kind are batched
 //     among themselves) the search plays the same single-thread game as with the
 //     heads on the calling thread;
+//   * a NaN in the raw planes reaches the policy and the win rate;
 //   * an executor failure reaches the caller as an exception.
 #include <atomic>
 #include <chrono>
@@ -502,6 +503,40 @@ static void test_puct_arithmetic() {
     std::printf("puct arithmetic pinned\n");
 }
 
+// A raw plane that holds a NaN (a broken network or kernel) has to show in the policy or the
+// win rate of its own position, wherever it lies, and in no other position of the call.
+static void test_nan_reaches_the_heads() {
+    Heads heads;
+    const HeadWeights w(heads.c);
+    const int n = 9;   // one more than the heads take at a time
+    const float nan = std::nanf("");
+    auto run = [&](int bad, int pol_at, int val_at, std::vector<float>& policy,
+                   std::vector<float>& win) {
+        std::vector<float> pol((size_t)n * LZHIP_POL_SIZE), val((size_t)n * LZHIP_VAL_SIZE);
+        for (size_t i = 0; i < pol.size(); i++) pol[i] = (float)((int)(i * 7 % 13) - 6);
+        for (size_t i = 0; i < val.size(); i++) val[i] = (float)(i * 5 % 11) / 11.0f;
+        if (pol_at >= 0) pol[(size_t)bad * LZHIP_POL_SIZE + pol_at] = nan;
+        if (val_at >= 0) val[(size_t)bad * LZHIP_VAL_SIZE + val_at] = nan;
+        policy.assign((size_t)n * 362, -1.0f);
+        win.assign(n, -1.0f);
+        heads_on_host(w, n, pol.data(), val.data(), 1.0f, policy.data(), win.data());
+    };
+    std::vector<float> p0, w0, p1, w1;
+    run(0, -1, -1, p0, w0);
+    for (float v : p0) CHECK(std::isfinite(v));
+    for (float v : w0) CHECK(std::isfinite(v));
+    for (int bad : {0, 7, 8})
+        for (int at : {0, 5, 360, 361, 721}) {
+            run(bad, at, at % 361, p1, w1);
+            for (int b = 0; b < n; b++) {
+                CHECK(b == bad ? std::isnan(w1[b]) : w1[b] == w0[b]);
+                for (int i = 0; i < 362; i++)
+                    CHECK(b == bad ? std::isnan(p1[(size_t)b * 362 + i])
+                                   : p1[(size_t)b * 362 + i] == p0[(size_t)b * 362 + i]);
+            }
+        }
+}
+
 int main() {
     test_puct_arithmetic();
     std::printf("unrotation\n");
@@ -509,6 +544,8 @@ int main() {
     test_value_head_not_stm();
     std::printf("symmetric cache probe\n");
     test_symmetric_cache_probe();
+    std::printf("NaN through the heads\n");
+    test_nan_reaches_the_heads();
     std::printf("heads behind the pipe\n");
     test_heads_behind_the_pipe();
     std::printf("single thread\n");
