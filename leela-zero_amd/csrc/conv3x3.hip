@@ -411,6 +411,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     }
 }
 
+constexpr int kUnits = 256;   // compute units
+
 static ConvGrid conv_grid(int tiles_m, int tiles_n, int n, int Cp, int Kp) {
     ConvGrid best{};
     size_t best_cost = ~(size_t)0;
@@ -442,12 +444,29 @@ static void launch_conv_as(const half_t* X, const half_t* Wf, const half_t* res,
            dim3(64 * WR * WN), s, t, X, Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, Kp, best);
 }
 
-// The published widths and 384.  Measured per forward of 10 blocks, Winograd kernels -> this, us:
-// 64 filters, 1 board 191 -> 73, 64 boards 351 -> 127, 200 boards 488 -> 271; 384 filters, 1 board
-// 263 -> 120, 16 boards 523 -> 468, 44 boards 937 -> 761, 100 boards 1628 -> 1733, 200 boards 3297
-// -> 2923, and with two forwards side by side 44 boards 1407 -> 1271, 100 boards 3314 -> 2711.
-bool conv3x3_serves(int Kp, int elem_bytes) {
-    return elem_bytes == 2 && (Kp == 64 || Kp == 128 || Kp == 192 || Kp == 256 || Kp == 384);
+// Which handles compute by direct convolution.  Its arithmetic grows with the square of the
+// width, what the Winograd kernels move with the width itself: up to 384 filters the matrix pipe
+// is through with the one before the memory is with the other; above, only where a layer is a
+// chain of latencies, that is where tiles of 96x64 make no more than one work-group per unit.
+// Measured per forward of 5 blocks, Winograd kernels -> this, us (one forward at a time | two | three
+// side by side):
+//   320 filters,  1 board 133 -> 60, 16: 250 -> 171 | 290 -> 260 | 366 -> 371, 64: 495 -> 459 | 856 -> 750
+//   384 filters,  8 boards 200 -> 137 | 237 -> 189 | 289 -> 270, 44: 459 -> 364 | 730 -> 622 | 1087 -> 908,
+//                 100: 842 -> 860 | 1716 -> 1384, 200: 1703 -> 1476 | 3379 -> 2789
+//   448 filters,  8 boards 215 -> 154, 12: 277 -> 225 | 327 -> 362 | 457 -> 565, 64: 716 -> 806 | 1341 -> 1427
+//   512 filters,  8 boards 238 -> 172, 10: 254 -> 240 | 324 -> 373 | 428 -> 545, 64: 784 -> 820 | 1486 -> 1519
+//   640 filters,  6 boards 289 -> 200 | 435 -> 330 | 595 -> 497, 8: 301 -> 293 | 441 -> 471 | 613 -> 743
+//   768 filters,  5 boards 278 -> 228 | 433 -> 381 | 591 -> 567, 16: 514 -> 534 | 857 -> 936
+//  1024 filters,  4 boards 396 -> 305 | 598 -> 525 | 822 -> 777, 64: 2229 -> 2972
+// Left out: 512 filters at 16 to 40 boards gain too (32: 572 -> 446 | 874 -> 780) and lose again
+// beyond.  Taken in: what loses one at a time and gains side by side, 384 filters at 100 boards
+// (567 tiles on 512 places) and 320 at 32 (276 -> 302 | 408 -> 383 | 616 -> 557); and the reverse,
+// 448 filters at 9 boards (214 -> 155 | 258 -> 240 | 336 -> 359).
+// The batch is the handle's largest, so that a network keeps its filters in one order and a
+// position's result does not depend on what it is evaluated with.
+bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
+    if (elem_bytes != 2 || Kp % 64 != 0) return false;
+    return Kp <= 384 || (max_batch * kPts + 95) / 96 * (Kp / 64) <= kUnits;
 }
 
 // The tile.  A layer of few boards is a chain of latencies, so its points and channels are
@@ -470,11 +489,10 @@ bool conv3x3_serves(int Kp, int elem_bytes) {
 void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                     const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,
                     hipStream_t s, LaunchTimer* t) {
-    if (!conv3x3_serves(Kp, 2) || Cp % 64 != 0)
+    if (Kp % 64 != 0 || Cp % 64 != 0)
         throw std::invalid_argument("no direct convolution for this width");
     const int rows = n * kPts;
     auto groups = [&](int mt, int cw) { return ((rows + mt - 1) / mt) * (Kp / cw); };
-    constexpr int kUnits = 256;
 #define LZ_CONV(RB, NB, WR, WN, D, DA, CC, OCC)                                                   \
     launch_conv_as<RB, NB, WR, WN, D, DA, CC, OCC>(X, Wf, res, Y, bn_scale, bn_mean, rfac, n, Cp, \
                                                    Kp, s, t)
@@ -529,11 +547,12 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // fetched twice or four times, and all wait for the whole patch.  Here every wavefront owns the
 // whole tile and KW-th of the k-steps (HPW halves of a chunk of 64 channels, all nine taps): each
 // operand is fetched once, a wavefront stages its own input channels and waits for nobody, its
-// filters are in flight all at once (D = 9 HPW; two thirds of them where six wavefronts share
-// the registers), and the partial sums meet in LDS at the end, in the order of the wavefronts.
-// Measured per forward of 10 blocks, conv3x3_k -> this, us: 64 filters see conv3x3_serves; 128
+// filters are in flight all at once (D = 9 HPW; two thirds of them where five or more wavefronts
+// share the registers), and the partial sums meet in LDS at the end, in the order of the wavefronts.
+// Measured per forward of 10 blocks, conv3x3_k -> this, us: 128
 // filters, 1 board 99 -> 74, 8 boards 113 -> 90; 192 filters, 1 board 121 -> 96, 5 boards 138 ->
-// 115; 256 filters, 1 board 133 -> 107, 5 boards 159 -> 146.
+// 115; 256 filters, 1 board 133 -> 107, 5 boards 159 -> 146; of 5 blocks, 1 board: 320 filters
+// 105 -> 60, 384 116 -> 63, 448 131 -> 70, 512 136 -> 76.
 // Tiles of 96x32, 96x64 and 192x64 points x channels were tried for larger batches and gave
 // nothing (256 filters, 16 boards 215 -> 212, 32 boards 318 -> 324; two forwards side by side
 // lost 10 %): there the partial sums' way through LDS, 2 KW RB NB KiB, costs what it saves.
@@ -713,12 +732,14 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 // than the compute units; 0: none of the three is.
 static int split_blocks(int n, int Kp) {
     for (int rb = 2; rb <= 4; rb++)
-        if ((n * kPts + rb * 16 - 1) / (rb * 16) * (Kp / 32) <= 256) return rb;
+        if ((n * kPts + rb * 16 - 1) / (rb * 16) * (Kp / 32) <= kUnits) return rb;
     return 0;
 }
 
+// A wavefront takes 64 input channels (32 of up to 128): eight wavefronts' planes are what the LDS
+// holds, so 512 filters are the widest.
 bool conv3x3_splits(int Kp, int max_batch) {
-    return conv3x3_serves(Kp, 2) && split_blocks(max_batch, Kp) > 0;
+    return Kp % 64 == 0 && Kp <= 512 && split_blocks(max_batch, Kp) > 0;
 }
 
 void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
@@ -742,7 +763,13 @@ void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, 
         case 128: LZ_SPLIT(4, 1, 9); break;
         case 192: LZ_SPLIT(3, 2, 18); break;
         case 256: LZ_SPLIT(4, 2, 18); break;
-        default: LZ_SPLIT(6, 2, 12); break;
+        // from here on two wavefronts share a SIMD's registers: two thirds of the filters ahead
+        case 320: LZ_SPLIT(5, 2, 12); break;
+        case 384: LZ_SPLIT(6, 2, 12); break;
+        case 448: LZ_SPLIT(7, 2, 12); break;
+        default:   // 512 filters: the third tile is for 3 boards, which they no longer fit in
+            if (rb == 2) go(conv3x3_split_k<2, 8, 2, 12>, 8);
+            else go(conv3x3_split_k<3, 8, 2, 12>, 8);
     }
 #undef LZ_SPLIT
 }

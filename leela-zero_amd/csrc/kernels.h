@@ -87,7 +87,8 @@ void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const 
 // X [n][361][Cp] -> Y [n][361][Kp] = min(max(0, scale*(conv - mean) + rfac*res), kActStoreMax);
 // res may be null and is not Y.  Wf: conv3x3_filter_count elements, zero but for what
 // conv3x3_filters writes.
-bool conv3x3_serves(int Kp, int elem_bytes);
+// Whether a handle for batches of up to max_batch computes by it (measured; see there).
+bool conv3x3_serves(int Kp, int max_batch, int elem_bytes);
 size_t conv3x3_filter_count(int Cp, int Kp);
 void launch_conv3x3(const _Float16* X, const _Float16* Wf, const _Float16* res, _Float16* Y,
                     const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,

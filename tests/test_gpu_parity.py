@@ -834,11 +834,18 @@ def test_direct_convolution_tiles(pkg, netgen, orc, filters, batches):
     (192, 3, (1, 3)), (192, 5, (4, 5)), (192, 7, (1, 6, 7)), (192, 44, (44,)),
     (256, 2, (1, 2)), (256, 4, (3, 4)), (256, 5, (1, 5)),
     (384, 1, (1,)), (384, 2, (2,)), (384, 3, (1, 3)), (384, 45, (1, 5, 6, 11, 12, 17, 18, 22, 23, 44, 45)),
+    (320, 2, (1, 2)), (320, 3, (3,)), (320, 4, (1, 4)), (320, 55, (3, 6, 7, 13, 20, 21, 27, 28, 55)),
+    (448, 1, (1,)), (448, 2, (2,)), (448, 3, (1, 3)), (448, 9, (1, 4, 5, 9)),
+    (512, 1, (1,)), (512, 2, (1, 2)), (512, 8, (1, 4, 5, 8)),
+    (640, 6, (1, 3, 4, 6)), (768, 5, (5,)), (1024, 4, (1, 2, 3, 4)),
+    # widths that are padded to a multiple of 64
+    (24, 12, (1, 12)), (100, 5, (1, 5)), (100, 70, (12, 17, 18, 35, 52, 69, 70)),
+    (200, 2, (1, 2)), (200, 36, (6, 9, 17, 18, 26, 35, 36)), (330, 4, (1, 4)),
 ])
 def test_direct_convolution_of_small_handles_and_other_widths(pkg, netgen, orc, filters, maxb, batches):
     """fp16 towers whose handle is small enough for the convolution that deals its sum to the
-    wavefronts (three tiles, both ends of each), and the tiles of 64 and 384 filters: one layer
-    with a skip connection against a float32 convolution."""
+    wavefronts (three tiles, both ends of each), and the tiles of 64 filters, of more than 256 and
+    of padded widths: one layer with a skip connection against a float32 convolution."""
     import torch
     import torch.nn.functional as F
     blocks = 3 if filters == 64 else 1      # fewer blocks of 64 filters stay with Winograd
@@ -854,6 +861,34 @@ def test_direct_convolution_of_small_handles_and_other_widths(pkg, netgen, orc, 
         got = pipe.debug_layer(2, a[:n], r[:n])[2]
         for i in range(n):
             assert rel_l2(got[i], want[i]) <= 2e-3, (n, i)
+    pipe.close()
+
+
+@pytest.mark.parametrize("filters,maxb,direct", [
+    (64, 200, True), (100, 40, True), (256, 64, True), (320, 64, True), (384, 45, True),
+    (448, 9, True), (448, 10, False), (512, 8, True), (512, 9, False), (640, 6, True),
+    (640, 7, False), (768, 5, True), (768, 6, False), (1024, 4, True), (1024, 5, False)])
+def test_which_handles_convolve_directly(pkg, netgen, orc, filters, maxb, direct):
+    """fp16 handles of up to 384 filters, and wider ones whose largest batch makes no more than
+    one tile of 96 points x 64 filters per compute unit, run one kernel per layer; the others run
+    the Winograd kernels.  Both agree with the oracle, also for one position on the handle."""
+    import torch
+    print("case: kernels of %d filters, handles of %d" % (filters, maxb), flush=True)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1 if filters > 64 else 3, filters,
+                                       6680 + filters, pkg.FP16, maxb)
+    x = netgen.synthetic_inputs(maxb, seed=6681)
+    d_in = torch.from_numpy(x).cuda()
+    pol, val = torch.zeros(maxb, 722, device="cuda"), torch.zeros(maxb, 361, device="cuda")
+    torch.cuda.synchronize()
+    _, cnt = pipe.profile_forward(maxb, d_in.data_ptr(), pol.data_ptr(), val.data_ptr())
+    assert (cnt[pkg.K_IN] == 0) == direct, list(cnt)
+    one_pol, one_val = pipe.forward_batch(x[:1])
+    assert np.array_equal(pol.cpu().numpy()[0], one_pol[0])
+    assert np.array_equal(val.cpu().numpy()[0], one_val[0])
+    for i in {0, maxb - 1}:
+        rp, rv = ref.forward(x[i])
+        assert rel_l2(pol.cpu().numpy()[i], rp) <= 2e-2, i
+        assert rel_l2(val.cpu().numpy()[i], rv) <= 2e-2, i
     pipe.close()
 
 
