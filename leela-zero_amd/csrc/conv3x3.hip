@@ -483,7 +483,12 @@ bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
 //   64 boards  52.4 | 46.2 | 32.1 | 29.1 | 27.0 | 25.1
 // (each entry jumps where the tile passes 256 work-groups; the two wavefronts of a 48x64 tile
 // leave room for three on a unit, and until then it beats a 192x64 tile on half the units: 24
-// boards above, 37 boards of 128 filters 8.8 against 9.9).  192 filters have no tile of 128
+// boards above, 37 boards of 128 filters 8.8 against 9.9.  It fetches every filter four times as
+// often, which the wider layers feel and so do forwards side by side: above 256 filters the
+// 192x64 tile is taken.  Per forward of 5 blocks, 48x64 | 192x64, us: 384 filters, 16 boards 210 |
+// 210, two side by side 358 | 302, three 518 | 419; 12 boards 191 | 207, 278 | 266, 395 | 346; 320
+// filters, 20 boards 185 | 183, 319 | 273, 464 | 368.  At 256 filters, 24 boards: 158 | 167, 252 |
+// 228, 364 | 301).  192 filters have no tile of 128
 // channels; there 128 x 192 takes the place of 192 x 128 (64 boards 18.2 against 19.7 us with
 // three tiles of 64 channels).
 void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
@@ -522,7 +527,7 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
         LZ_CONV(3, 2, 2, 2, 6, 3, 0, 2);
         return;
     }
-    if (groups(48, 64) <= 3 * kUnits) {
+    if (Kp <= 256 && groups(48, 64) <= 3 * kUnits) {
         LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
         return;
     }
