@@ -261,10 +261,8 @@ public:
         m_layers.resize(n_layers);
         // fp16 towers that conv3x3_serves names are computed by direct convolution,
         // provided that what was handed over are transforms of 3x3 filters; all else goes
-        // through the Winograd kernels and needs their tile arrays.  (So do towers of 64 filters
-        // and less than 3 blocks: no network that is played has so few, and they are what holds
-        // the half-precision Winograd kernels, and their launches, to account at little cost.)
-        m_direct = conv3x3_serves(m_Fp, m_max_batch, (int)sizeof(P)) && (m_Fp > 64 || n_layers >= 7) &&
+        // through the Winograd kernels and needs their tile arrays.
+        m_direct = conv3x3_serves(m_Fp, m_max_batch, (int)sizeof(P)) &&
                    build_direct_filters(n_layers, U);
         if (!m_direct) alloc_tiles();
         // Filters are laid out on the host in fp32; an fp16 net converts them on the device.

@@ -15,10 +15,17 @@ from helpers import max_abs, rel_l2
 pytestmark = pytest.mark.gpu
 
 
-def make_pipes(pkg, netgen, orc, blocks, filters, seed, precision, max_batch):
+def make_pipes(pkg, netgen, orc, blocks, filters, seed, precision, max_batch, winograd=False):
+    """winograd: one Winograd position of layer 1 is scaled, which no 3x3 filter can express, so
+    that an fp16 network runs the Winograd kernels whatever its width."""
     net = netgen.make_network(blocks, filters, seed)
     w, h = netgen.prepare(net)
     w_ref, h_ref = netgen.prepare(net, orc.winograd_transform_f, orc.process_bn_var)
+    if winograd:
+        for ws in (w, w_ref):
+            u = np.array(ws.m_conv_weights[1], np.float32).reshape(36, filters, filters)
+            u[14] *= 1.25
+            ws.m_conv_weights[1] = u
     ref = orc.OraclePipe()
     ref.initialize(filters)
     ref.push_weights(6, 18, filters, w_ref)
@@ -409,11 +416,12 @@ def test_drain_and_resume(pkg, netgen, orc):
     pipe.close()
 
 
-def test_device_resident_forward_and_profile(pkg, netgen, orc):
+@pytest.mark.parametrize("winograd", [False, True])
+def test_device_resident_forward_and_profile(pkg, netgen, orc, winograd):
     """The device-pointer entry point (what the bench times) gives the same planes as
     the host entry point, and the per-kernel timing hook reports every launch."""
     import torch
-    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, 64, 80, pkg.FP16, 4)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, 64, 80, pkg.FP16, 4, winograd)
     x = netgen.synthetic_inputs(4, seed=8)
     pol_h, val_h = pipe.forward_batch(x)
     d_in = torch.from_numpy(x).cuda()
@@ -424,9 +432,12 @@ def test_device_resident_forward_and_profile(pkg, netgen, orc):
     pipe.sync()
     assert np.array_equal(d_pol.cpu().numpy(), pol_h) and np.array_equal(d_val.cpu().numpy(), val_h)
     ms, cnt = pipe.profile_forward(4, d_in.data_ptr(), d_pol.data_ptr(), d_val.data_ptr())
-    # 2 blocks = 5 conv layers: 5 GEMMs, 4 fused out->in transforms, 1 plain of each
-    assert list(cnt) == [1, 1, 5, 1, 1, 4]
-    assert np.all(ms > 0) and np.all(ms < 50)
+    # 2 blocks = 5 conv layers: 5 GEMMs, 4 fused out->in transforms, 1 plain of each; as direct
+    # convolutions (counted with the GEMMs) one launch a layer
+    assert list(cnt) == ([1, 1, 5, 1, 1, 4] if winograd else [1, 0, 5, 0, 1, 0])
+    assert np.array_equal(ms > 0, cnt > 0) and np.all(ms < 50)
+    rp, rv = ref.forward(x[3])
+    assert rel_l2(pol_h[3], rp) <= 2e-2 and rel_l2(val_h[3], rv) <= 2e-2
     assert np.array_equal(d_pol.cpu().numpy(), pol_h)
     pipe.close()
 
@@ -848,8 +859,7 @@ def test_direct_convolution_of_small_handles_and_other_widths(pkg, netgen, orc, 
     of padded widths: one layer with a skip connection against a float32 convolution."""
     import torch
     import torch.nn.functional as F
-    blocks = 3 if filters == 64 else 1      # fewer blocks of 64 filters stay with Winograd
-    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, blocks, filters, 6650 + filters, pkg.FP16, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 6650 + filters, pkg.FP16, maxb)
     rng = np.random.default_rng(filters + maxb)
     a = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
     r = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
@@ -874,8 +884,7 @@ def test_which_handles_convolve_directly(pkg, netgen, orc, filters, maxb, direct
     the Winograd kernels.  Both agree with the oracle, also for one position on the handle."""
     import torch
     print("case: kernels of %d filters, handles of %d" % (filters, maxb), flush=True)
-    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1 if filters > 64 else 3, filters,
-                                       6680 + filters, pkg.FP16, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 6680 + filters, pkg.FP16, maxb)
     x = netgen.synthetic_inputs(maxb, seed=6681)
     d_in = torch.from_numpy(x).cuda()
     pol, val = torch.zeros(maxb, 722, device="cuda"), torch.zeros(maxb, 361, device="cuda")
