@@ -350,23 +350,11 @@ void HIPScheduler::worker() {
                 // system_clock: waits on it map to pthread_cond_timedwait, which thread
                 // sanitizers model; the grace period is far too short for clock steps
                 // to matter.
-                // Requests that still come in the last quarter of the grace period promise the
-                // rest: it goes on, quarter by quarter, while they do, at most to twice its
-                // length.  (16 Python callers take 400 to 500 us to come back one after the
-                // other, as long as half a 40x256 forward: without this every fourth batch left
-                // without some of them, and those took a
-                // forward of their own: 16 callers, four positions each, 5.4 -> 5.0 ms.)
-                const auto part = std::chrono::microseconds((cap_us + 3) / 4);
-                auto deadline = std::chrono::system_clock::now();
-                const int most = m_max_wait_us >= 0 ? 4 : 8;
-                for (int i = 1; i <= most; i++) {
-                    const size_t before = m_queue.size();
-                    deadline += part;
-                    const bool ended = m_cv.wait_until(lk, deadline, [&] {
-                        return !m_running || m_queue.empty() || m_queue.size() >= target;
-                    });
-                    if (ended || (i >= 4 && m_queue.size() == before)) break;
-                }
+                const auto deadline =
+                    std::chrono::system_clock::now() + std::chrono::microseconds(cap_us);
+                m_cv.wait_until(lk, deadline, [&] {
+                    return !m_running || m_queue.empty() || m_queue.size() >= target;
+                });
                 if (!m_running) return;
             }
             // drain() may have emptied the queue while we waited
