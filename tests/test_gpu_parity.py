@@ -36,22 +36,21 @@ def make_pipes(pkg, netgen, orc, blocks, filters, seed, precision, max_batch, wi
     return net, pipe, ref, h_ref
 
 
-@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("precision,winograd", [(0, False), (1, False), (1, True)])
 @pytest.mark.parametrize("filters,n", [(8, 3), (64, 3), (192, 3), (192, 30), (128, 3), (128, 40),
                                        (256, 3), (256, 16), (256, 20), (256, 40)])
-def test_single_layer_stages(pkg, netgen, orc, precision, filters, n):
+def test_single_layer_stages(pkg, netgen, orc, precision, winograd, filters, n):
     """V, M and Y of one convolution layer against the oracle's stages, for the input
     layer (18 planes) and a residual-tower layer with a skip connection.  The M stage is
     the check the reference's tuner makes of every GEMM it times, against a plain sgemm
-    (reference src/Tuner.cpp:262-301); 128 and 256 filters put the streaming GEMMs of both
-    storage types under it, at 3 boards (one 32-row block per work-group) and at 40 (several
-    blocks per work-group, a last block of 8 rows).  The fp16 GEMM and output transform run
-    in the layout a forward of that many boards keeps its tiles in: slabs of 16 channels at
-    3 and 16 boards, of 32 at 20 (256 filters), 30 (192) and 40 (128), rows at 40 boards of
-    256 filters."""
+    (reference src/Tuner.cpp:262-301); in fp32, 128 and 256 filters put the streaming GEMM
+    under it, at 3 boards (one 32-row block per work-group) and at 40 (several
+    blocks per work-group, a last block of 8 rows).  An fp16 layer is a direct convolution: Y is
+    what a forward computes, V and M come from its filters by the tiled kernels.  With filters that
+    are no 3x3 ones (winograd) all three are the stages of such a network's forward."""
     print("case: single_layer precision=%d filters=%d n=%d" % (precision, filters, n), flush=True)
     net, pipe, ref, _ = make_pipes(pkg, netgen, orc, 1, filters, 40 + filters, precision,
-                                   max(4, n))
+                                   max(4, n), winograd)
     rng = np.random.default_rng(filters)
     tol = 1e-5 if precision == 0 else 4e-3
     # layer 0 on real input planes
@@ -171,11 +170,9 @@ def test_forward_parity(pkg, netgen, orc, blocks, filters, batch, precision):
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("batch", [72, 64, 52, 41, 36, 35, 33, 32, 24, 21, 18, 17, 16, 10, 9, 8, 2, 1])
 def test_forward_parity_wide_batches(pkg, netgen, orc, precision, batch):
-    """256 filters at batch sizes on both sides of every change of kernel shape (GEMM, fp16:
-    the streaming kernel with 1, 2, 4, 8 and 16 blocks of 32 tile rows per work-group, which
-    change at 9, 18, 36 and 72 boards; fp32:
-    256x256 tiles from 41 boards, 128x128 from 21, 128x64 with padded rows below; fused
-    transform: 64 channels per work-group from 21 boards, 32 from 17, 16 below), in both
+    """256 filters at batch sizes on both sides of changes of kernel shape (fp32: the streaming
+    GEMM with 1 to 8 blocks of 32 tile rows per work-group; fused transform: 64 channels per
+    work-group from 21 boards, 32 from 17, 16 below; fp16: the direct convolution's tiles), in both
     precisions, including batches whose tile count is not a multiple of any tile height."""
     print("case: wide 3x256 b%d precision=%d" % (batch, precision), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 3, 256, 3000, precision, batch)
@@ -189,9 +186,8 @@ def test_forward_parity_wide_batches(pkg, netgen, orc, precision, batch):
                                                   (10, 128, 24)])
 def test_forward_parity_deep_fp16(pkg, netgen, orc, blocks, filters, batch):
     """Deep fp16 towers: the two large fp16 benchmark configurations (20x256 batch 32, 40x256
-    batch 64) at full size, and 15x192 and 10x128 (the streaming GEMM with 6 and 4 wavefronts
-    under per-layer activation scales): raw planes of every position of the batch against the oracle, head outputs of
-    three of them."""
+    batch 64) at full size, and 15x192 and 10x128, under per-layer activation scales: raw planes of
+    every position of the batch against the oracle, head outputs of three of them."""
     print("case: deep fp16 %dx%d b%d" % (blocks, filters, batch), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, blocks, filters, 2000 + blocks,
                                        pkg.FP16, batch)
@@ -548,86 +544,68 @@ def test_graph_replays_match_stream_launches(pkg, netgen, orc):
     plain.close()
 
 
-@pytest.mark.parametrize("filters,maxb,batches", [
-    (256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
-    (192, 42, (1, 7, 10, 15, 21, 22, 37, 42)),
-    (128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
+@pytest.mark.parametrize("precision,filters,maxb,batches", [
+    (1, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
+    (1, 192, 42, (1, 7, 10, 15, 21, 22, 37, 42)),
+    (1, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
+    (0, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
+    (0, 192, 16, (1, 5, 9, 15, 16)),
+    (0, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
 ])
-def test_fused_launches_match_separate_launches(pkg, netgen, orc, filters, maxb, batches):
-    """An fp16 tower of 128, 192 or 256 filters sends the transform of a layer and the GEMM of
-    the next as one launch where that is faster and the forward has the device to itself, up
-    to the batch where the transform changes to its 64-channel shape, and up to that batch it
-    keeps its tile arrays slab by slab instead of row by row.  Handles that always fuse
-    (LZHIP_FUSE=2), that never fuse (0) and that decide per forward (the default), each with
-    the slab layout and (LZHIP_SLAB=0) without,
-    must give the same bits, at batches that take each of the shapes (1, 2, 4 or 8 blocks of 32
-    rows per GEMM work-group, 16- or 32-channel transform groups), on one lane and with all
-    lanes busy; and the result agrees with the oracle."""
+def test_busy_lanes_and_tile_layouts_give_the_same_bits(pkg, netgen, orc, precision, filters, maxb,
+                                                        batches):
+    """Every batch on one lane alone, and on all lanes at once with many forwards in a row and no
+    synchronisation, gives the same bits; so does an fp32 handle that keeps V and M of the tower's
+    layers in two arrays (LZHIP_INPLACE=0) beside the default that keeps them in one; and the
+    result agrees with the oracle."""
     import os
     import torch
-    print("case: fused launches, %d filters" % filters, flush=True)
-    pipes = {}
-    for slab in ("0", None):
-        for mode in ("2", "0", None):
-            for key, v in (("LZHIP_FUSE", mode), ("LZHIP_SLAB", slab)):
-                if v is None:
-                    os.environ.pop(key, None)
-                else:
-                    os.environ[key] = v
-            try:
-                net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 4, filters, 3100, pkg.FP16, maxb)
-            finally:
-                os.environ.pop("LZHIP_FUSE", None)
-                os.environ.pop("LZHIP_SLAB", None)
-            pipes[(mode, slab)] = pipe
+    print("case: busy lanes, %d filters precision=%d" % (filters, precision), flush=True)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 4, filters, 3100, precision, maxb)
+    pipes = [pipe]
+    if precision == 0:
+        os.environ["LZHIP_INPLACE"] = "0"
+        try:
+            pipes.append(make_pipes(pkg, netgen, orc, 4, filters, 3100, precision, maxb)[1])
+        finally:
+            del os.environ["LZHIP_INPLACE"]
     x = netgen.synthetic_inputs(maxb, seed=3101)
-    base = pipes[("0", "0")]                      # separate launches, row layout
     for n in batches:
-        want = base.forward_batch(x[:n])
-        for key, pipe in pipes.items():
-            if pipe is base:
-                continue
-            got = pipe.forward_batch(x[:n])
-            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), (n, key)
-    rp, rv = ref.forward(x[7])
+        want = pipe.forward_batch(x[:n])
+        for other in pipes[1:]:
+            got = other.forward_batch(x[:n])
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), n
     nb = batches[4]
-    want = base.forward_batch(x[:nb])
-    assert rel_l2(want[0][7], rp) <= 2e-2 and rel_l2(want[1][7], rv) <= 2e-2
-    # every lane at once, many forwards in a row without synchronisation, always fused
+    want = pipe.forward_batch(x[:nb])
+    tol = 1e-5 if precision == 0 else 2e-2
+    rp, rv = ref.forward(x[7])
+    assert rel_l2(want[0][7], rp) <= tol and rel_l2(want[1][7], rv) <= tol
+    # every lane at once, many forwards in a row without synchronisation
     d_in = torch.from_numpy(x).cuda()
-    for key in (("2", None), ("2", "0"), ("0", None)):
-        pipe = pipes[key]
+    for p in pipes:
         outs = [(torch.zeros(nb, 722, device="cuda"), torch.zeros(nb, 361, device="cuda"))
-                for _ in range(pipe.lanes())]
+                for _ in range(p.lanes())]
         torch.cuda.synchronize()
         for rep in range(8):
             for k, (pol, val) in enumerate(outs):
-                pipe.forward_batch_device(nb, d_in.data_ptr(), pol.data_ptr(), val.data_ptr(), lane=k)
-        pipe.sync()
+                p.forward_batch_device(nb, d_in.data_ptr(), pol.data_ptr(), val.data_ptr(), lane=k)
+        p.sync()
         for pol, val in outs:
-            assert np.array_equal(pol.cpu().numpy(), want[0]), key
-            assert np.array_equal(val.cpu().numpy(), want[1]), key
-    for pipe in pipes.values():
-        pipe.close()
+            assert np.array_equal(pol.cpu().numpy(), want[0])
+            assert np.array_equal(val.cpu().numpy(), want[1])
+    for p in pipes:
+        p.close()
 
 
 def test_random_batches_on_all_lanes_match_the_plain_forward(pkg, netgen, orc):
     """A seeded sequence of 400 forwards of random batches (1 to 32 boards, 256 filters) dealt to
     random lanes with no synchronisation between them -- so that consecutive forwards of a lane
-    change between the slab widths and the row layout, between fused and separate launches,
-    and between having the device alone and sharing it -- gives, forward by forward, the bits
-    of a handle that never fuses and keeps its tiles row by row."""
-    import os
+    change between tiles, and between having the device alone and sharing it -- gives, forward by
+    forward, the bits of another handle that runs one batch at a time."""
     import torch
     print("case: random batches on all lanes", flush=True)
     maxb = 32
-    os.environ["LZHIP_FUSE"] = "0"
-    os.environ["LZHIP_SLAB"] = "0"
-    try:
-        net, plain, ref, h_ref = make_pipes(pkg, netgen, orc, 3, 256, 3300, pkg.FP16, maxb)
-    finally:
-        os.environ.pop("LZHIP_FUSE", None)
-        os.environ.pop("LZHIP_SLAB", None)
+    net, plain, ref, h_ref = make_pipes(pkg, netgen, orc, 3, 256, 3300, pkg.FP16, maxb)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 3, 256, 3300, pkg.FP16, maxb)
     x = netgen.synthetic_inputs(maxb, seed=3301)
     want = {}
@@ -711,13 +689,14 @@ def test_error_behaviour_on_device(pkg, netgen):
 @pytest.mark.parametrize("filters,batch", [(128, 1), (128, 9), (128, 30), (128, 52), (128, 72),
                                            (192, 2), (192, 16), (192, 17), (192, 40), (192, 64)])
 def test_streaming_gemm_at_narrower_widths(pkg, netgen, orc, filters, batch, precision):
-    """Nets of 128 and 192 filters run the streaming GEMM with 4 and 6 wavefronts per
-    work-group (256 filters: 8); in fp32 only the 128-filter ones do, 192 filters stay on the
-    tiled kernels there.  The batches take every number of blocks per work-group (1, 2, 4, 8,
-    16), with tile counts that are not multiples of the 32-row block."""
+    """fp32 nets of 128 filters, and of 192 in handles of up to 16 positions, run the streaming
+    GEMM with 4 and 6 wavefronts per work-group (256 filters: 8); larger handles of 192 filters the
+    tiled one.  fp16 nets whose filters are no 3x3 ones run the tiled GEMM at the same sizes.  The
+    batches take different numbers of blocks per work-group, with tile counts that are not
+    multiples of the 32-row block."""
     print("case: streaming width %d b%d precision=%d" % (filters, batch, precision), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 5100 + filters, precision,
-                                       batch)
+                                       batch, winograd=precision == 1)
     x = netgen.synthetic_inputs(batch, seed=filters + batch)
     check_outputs(pkg, orc, pipe, ref, h_ref, x, precision,
                   idx=sorted({0, batch // 2, batch - 1}))
@@ -727,13 +706,13 @@ def test_streaming_gemm_at_narrower_widths(pkg, netgen, orc, filters, batch, pre
 @pytest.mark.parametrize("filters,batch", [(640, 4), (768, 3), (896, 2), (1024, 12), (1024, 8),
                                            (384, 28), (448, 30), (320, 52)])
 def test_fp16_widths_on_the_tiled_gemm(pkg, netgen, orc, filters, batch):
-    """fp16 widths served by the tiled GEMM kernels (above 256 filters; 64-filter nets are in
-    the small-network cases): the widest ones -- 10, 12, 14 and 16 k-slices, at 1024 filters
-    the one-pass 256x256 tile (from 11 boards) and the 128x64 tile below it -- and widths
-    at batches that take the 128x128 persistent and the 128x64 tiles."""
+    """fp16 widths on the tiled GEMM kernels, where a network's filters are no 3x3 ones or its
+    handle is too large for direct convolution: the widest ones -- 10, 12, 14 and 16 k-slices, at
+    1024 filters the one-pass 256x256 tile (from 11 boards) and the 128x64 tile below it -- and
+    widths at batches that take the 128x128 persistent and the 128x64 tiles."""
     print("case: fp16 width %d b%d" % (filters, batch), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 5000 + filters, pkg.FP16,
-                                       batch)
+                                       batch, winograd=True)
     x = netgen.synthetic_inputs(batch, seed=filters + batch)
     check_outputs(pkg, orc, pipe, ref, h_ref, x, pkg.FP16, idx=[0, batch - 1])
     pipe.close()
@@ -742,8 +721,9 @@ def test_fp16_widths_on_the_tiled_gemm(pkg, netgen, orc, filters, batch):
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("filters,batch", [(384, 6), (512, 44), (320, 3)])
 def test_other_widths(pkg, netgen, orc, precision, filters, batch):
-    """Widths other than the benchmark's: 6, 8 and 5 k-slices in fp16 (12, 16, 10 in fp32),
-    with the large-tile GEMM at 512 filters."""
+    """Widths other than the benchmark's: 12, 16 and 10 k-slices of the tiled GEMM in fp32, with
+    its large tile at 512 filters; in fp16 direct convolution at 384 and 320 filters and the
+    tiled GEMM's 8 k-slices at 512."""
     print("case: width %d b%d precision=%d" % (filters, batch, precision), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 4000 + filters, precision,
                                        batch)
