@@ -6,9 +6,9 @@ A step is one forward pass (residual tower + 1x1 heads) over one batch of 64
 synthetic positions that already sit in device memory; `value` is measured over exactly
 --steps such steps.  The same JSON line also carries the rate through host buffers (PCIe
 inside the timed region), the figure repeated over five blocks of --steps forwards, the
-roofline of the GEMM and of the transforms from per-launch device timestamps, what a plain
-copy of the same bytes takes on this box, the CPU baseline, the same network in fp32 and
-the three smaller configurations.
+roofline of the convolutions (fp32: of the Winograd GEMM and transforms) from per-launch device
+timestamps, what a plain copy of a Winograd layer's bytes takes on this box, the CPU baseline, the
+same network in fp32 and the three smaller configurations.
 """
 import argparse
 import json
@@ -26,20 +26,20 @@ PEAK_MFMA_F16 = 2.5e15   # dense fp16 matrix FLOP/s, MI355X
 PEAK_MFMA_F32 = 157.3e12
 PEAK_HBM = 8.0e12        # bytes/s
 
-# HBM bytes per launch of the Winograd GEMM come from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE
+# HBM bytes per launch of the direct convolution come from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE
 # (KiB per dispatch, scaled by what the same counters read for a plain copy kernel of known
 # size).  Counters cannot be read from inside this process: the figure is read from the
 # tracked summary of those runs, which states it for the workload it was measured on.
-PMC_SUMMARY = os.path.join(ROOT, "profiles", "gemm_and_transform_40x256_fp16_b64_pmc.txt")
+PMC_SUMMARY = os.path.join(ROOT, "profiles", "conv3x3_40x256_fp16_b64_pmc.txt")
 
 
-def measured_gemm_traffic(blocks, filters, precision, batch):
-    """`gemm_traffic_bytes_per_launch = N` of the PMC summary, for its own workload only."""
+def measured_conv_traffic(blocks, filters, precision, batch):
+    """`conv_traffic_bytes_per_launch = N` of the PMC summary, for its own workload only."""
     if (blocks, filters, precision, batch) != (40, 256, "fp16", 64):
         return None
     try:
         for line in open(PMC_SUMMARY):
-            if "gemm_traffic_bytes_per_launch" in line and "=" in line:
+            if "conv_traffic_bytes_per_launch" in line and "=" in line:
                 return float(line.split("=")[1].split()[0])
     except OSError:
         pass
@@ -214,7 +214,7 @@ def netbench_workload(args, pkg, netgen):
 
 def gemm_kernel_name(fp16, Fp, B):
     """The GEMM kernel the library launches for this precision, padded width and batch."""
-    if not fp16 and Fp in (128, 256):
+    if not fp16 and (Fp in (128, 256) or (Fp == 192 and B <= 16)):
         return "wino_gemm_stream32_k (36-way batched Winograd GEMM)"
     return "wino_gemm_k / wino_gemm_big_k family (36-way batched Winograd GEMM)"
 
@@ -361,11 +361,12 @@ def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, 
     gemm_rate = gf / (ms[pkg.K_GEMM] * 1e-3)
     Fp = (F + 63) // 64 * 64
     roofline = {
-        "kernel": ("conv3x3_k (direct convolution + batch norm + skip + ReLU)" if direct
+        "kernel": ("conv3x3_k / conv3x3_split_k (direct convolution + batch norm + skip + ReLU)"
+                   if direct
                    else gemm_kernel_name(prec == pkg.FP16, Fp, B)),
         "bound": "mfma", "achieved": gemm_rate / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
         "frac": gemm_rate / peak,
-        "traffic": None if direct else measured_gemm_traffic(blocks, F, precision, B),
+        "traffic": measured_conv_traffic(blocks, F, precision, B) if direct else None,
         # planes in and out and filters of a tower layer (V, M and U of a Winograd one)
         "algorithmic_bytes_per_launch": (e * (361.0 * B * F * 2 + 9 * F * F) if direct
                                          else 36.0 * e * (25 * B * F * 2 + F * F)),
@@ -373,6 +374,10 @@ def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, 
         "launches_per_forward": int(cnt[pkg.K_GEMM]),
         "flops_per_launch": gf / cnt[pkg.K_GEMM],
     }
+    if direct:
+        # not to be read beside a Winograd GEMM's share: the direct form has 3.6 times the products
+        roofline["frac_of_winograd_products"] = (gemm_flops(B, F, nl) / (ms[pkg.K_GEMM] * 1e-3)
+                                                 / peak)
     roofline["launch_context"] = ("launches that run alone (event-timed forward on one lane, "
                                   "nothing else enqueued)")
     # The events bracket a launch's own execution; what lies between two launches of a chain
@@ -394,8 +399,9 @@ def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, 
             "frac": gf / (ms2[pkg.K_GEMM] * 1e-3) / peak,
             "note": "the same launches while another lane's forward shares the device: each "
                     "lasts longer, two are in progress"}
-    # the same launch against the HBM roof: at this batch the GEMM's flop-per-byte ratio is below
-    # the machine's (peak flops / peak bytes), so HBM, not MFMA, is the roof above it
+    # the same launch against the HBM roof: the roof above a Winograd GEMM, whose flop-per-byte
+    # ratio at this batch is below the machine's (peak flops / peak bytes); a direct convolution's
+    # is above it
     alg_bytes = roofline["algorithmic_bytes_per_launch"]
     roofline["flop_per_byte"] = roofline["flops_per_launch"] / alg_bytes
     roofline["machine_flop_per_byte"] = peak / PEAK_HBM
@@ -629,8 +635,7 @@ def main():
         "hbm_copy_floor": copy_floor(torch, B, F, 2 if args.precision == "fp16" else 4),
         "cpu_baseline": cpu,
     }
-    # what this GEMM launch is against the copy rates measured above: the roof that applies
-    # to one lane is the cache-resident one (V, M and the activations of a lane are ~100 MB)
+    # what this launch's algorithmic bytes are against the copy rates measured above
     floor = out["hbm_copy_floor"]
     alg = out["roofline"]["algorithmic_bytes_per_launch"]
     us = out["roofline"]["avg_launch_us"]
