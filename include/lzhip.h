@@ -241,7 +241,9 @@ int lzhip_get_act_scales(lzhip_handle* h, float* out, int n);
 /* Kernel classes of the tower, for timing. */
 #define LZHIP_K_PACK 0      /* NCHW fp32 input -> channels-last storage type   */
 #define LZHIP_K_IN 1        /* Winograd input transform                        */
-#define LZHIP_K_GEMM 2      /* 36-way batched MFMA GEMM                        */
+#define LZHIP_K_GEMM 2      /* 36-way batched MFMA GEMM; in fp16 the direct convolution
+                             * (batch norm, skip and ReLU included) that is the only
+                             * class of a layer where 3x3 filters were handed over */
 #define LZHIP_K_OUT 3       /* output transform + BN + residual + ReLU         */
 #define LZHIP_K_HEAD 4      /* 1x1 policy/value convolutions                   */
 #define LZHIP_K_OUTIN 5     /* output transform fused with the next input one  */

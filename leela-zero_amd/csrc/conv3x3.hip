@@ -6,10 +6,11 @@
 // directions, and at 256 filters that traffic, not the matrix pipe, is what a layer takes.
 // As an implicit GEMM a layer reads its planes once and its filters once per die, and the
 // fp16 matrix rate is high enough (v_mfma_f32_16x16x32_f16, fp32 accumulate) to do the
-// whole sum.  Measured per layer of a chain of dependent 256-filter layers, Winograd GEMM +
-// fused transform -> this kernel: 64 boards 26.5 -> 22.7 us one forward at a time, 24.2 -> 17.7
-// with two side by side; 200 boards 83 -> 54 (1.57 PFLOP/s; two side by side 1.71; torch.mm of
-// 8192 x 8192 fp16 matrices reached 1.33 on that card); 16 boards 12.8 -> 10.2; 1 board 9.2 -> 6.6.
+// whole sum.  Measured per layer, a forward of 40 blocks of 256 filters divided by its 81 layers,
+// Winograd GEMM + fused transform -> this file: 64 boards 28.6 -> 25.2 us one forward at a time,
+// 24.5 -> 20.6 with two side by side; 200 boards 83 -> 65 (1.30 PFLOP/s; two side by side 1.41;
+// torch.mm of 8192 x 8192 fp16 matrices 1.19 to 1.33 on such cards); 16 boards 13.2 -> 10.3; 1 board
+// 9.1 -> 4.8.
 // It also rounds less: planes and 3x3 filters are the only values kept in half precision.
 #include <cmath>
 #include <stdexcept>
@@ -130,8 +131,10 @@ size_t conv3x3_filter_count(int Cp, int Kp) {
 // the L1 delivers.  RB = 6, NB = 4 (50 % of one, 67 % of the other) is the tile for full
 // batches.  The planes pass through LDS because every value is used nine times: the cells a
 // tile reaches are staged once per chunk of input channels, in rows padded to an odd number
-// of 16-byte pieces (conflict-free fragment reads), and the nine taps and two halves are
-// immediate offsets of one address per 16 points.
+// of 16-byte pieces, and the nine taps and two halves are immediate offsets of one address per 16
+// points.  The padding does not keep the fragment reads free of bank conflicts: counted at 64
+// boards of 256 filters, the LDS is busy for 42 % of a launch, conflicts are 24 %, and the matrix
+// pipes are busy for 57 % of it (32 boards: 61, 35 and 42 %).
 //
 // CC == 0: chunks of 64 input channels in two LDS buffers; the next chunk's pieces are loaded
 // and stored in small groups between the matrix instructions (SGRP at a time: kept whole they

@@ -135,9 +135,12 @@ public:
         if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0)
             throw std::runtime_error(std::string("device is ") + prop.gcnArchName +
                                      ", this library contains gfx950 code only");
-        // Small batches leave more of the device idle at every kernel boundary: a third
-        // lane pays up to batch 48 (40x256 fp16: +1..30 % up to 32, +7 % at 40, +4 % at 48) and
-        // no longer from 52 (-2 % there, -6 % at 64).
+        // Small batches leave more of the device idle at every kernel boundary.  Evaluations of
+        // all lanes, a third lane against two: 20x256 fp16, batch 16 to 32 -2..0 %, 40 and 48
+        // +10 %, 52 +7 %, 64 +2 %; 20x384 fp16, batch 16 to 48 +4..7 %; 20x192 fp32, batch 8 +30 %, 32
+        // +4 %, 48 -3 %, 64 -6 %; 20x256 fp32, batch 8 +24 %, 48 and 64 +3 %.  (At batches below 8 one
+        // host thread cannot feed three lanes.)  The line lies where it did for fp16 Winograd
+        // kernels; of today's only 192 filters in fp32 ask for it.
         m_n_lanes = max_batch <= 48 ? 3 : 2;
         if (const char* e = std::getenv("LZHIP_LANES")) {   // measurement knob: 1..3 lanes
             const int v = std::atoi(e);
@@ -432,11 +435,10 @@ public:
         for (int i = 0; i < m_n_lanes; i++) HIP_CHECK(hipStreamSynchronize(m_lane[i].stream));
     }
 
-    // Host-buffer forward.  Up to kIoSlots callers may be inside at once: each
-    // copies into its own pinned staging, enqueues copy-in, forward and copy-out
-    // on the stream under the pipe lock, and waits for its own event outside
-    // the lock, so that the next batch is queued on the device while this one
-    // runs and host-side copies overlap device work.
+    // Host-buffer forward.  Up to kIoSlots callers may be inside at once: each packs its planes
+    // into its own pinned staging, enqueues the forward on the lane of that slot under the
+    // lane's lock, and waits for its own event outside the lock, so that packing and copies on the
+    // host overlap the other callers' device work (see run_host_batch).
     void forward_batch(int n, const float* in, float* pol, float* val) override {
         HostCall c;
         c.in = in;
@@ -668,7 +670,6 @@ public:
         Layer& L = m_layers[layer];
         const int F = m_filters, C = L.C, Cp = L.Cp;
         const int Tu = n * kTilesPerBoard;
-        // stage fp32 NCHW planes through the V buffer's tail?  No: use a scratch buffer.
         DevBuf<float> d_planes, d_res, d_sc, d_mn;
         d_planes.alloc((size_t)n * C * kPts);
         HIP_CHECK(hipMemcpy(d_planes.p, act_in, sizeof(float) * (size_t)n * C * kPts, hipMemcpyHostToDevice));
@@ -857,12 +858,13 @@ private:
                                 ln.stream, timer(timed, LZHIP_K_OUT));
     }
 
-    // With LZHIP_GRAPH=1 the 165 launches of a forward are captured once per
-    // (batch size, buffers) into a HIP graph and replayed, which takes the launch
-    // work off the host thread.  Only kernel nodes are captured (no memsets or
-    // copies).  On the device the replay measured no faster than stream launches
-    // (the gaps between these kernels are drain and cache write-back, not launch
-    // latency), so plain stream launches are the default.
+    // With LZHIP_GRAPH=1 the launches of a forward (2 + one per layer of a direct tower; 2 + two
+    // per layer with Winograd kernels) are captured once per (batch size, buffers) into a HIP
+    // graph and replayed, which takes the launch work off the host thread.  Only kernel
+    // nodes are captured (no memsets or copies).  On the device the replay measured no faster
+    // than stream launches (40x256 fp16 at batch 16: 0.84 against 0.83 ms; the gaps between
+    // these kernels are drain and cache write-back, not launch latency), so plain stream
+    // launches are the default.
     void clear_graphs(Lane& ln) {
         for (auto& kv : ln.graphs) (void)hipGraphExecDestroy(kv.second);
         ln.graphs.clear();
@@ -894,8 +896,9 @@ private:
         HIP_CHECK(hipGraphLaunch(it->second, ln.stream));
     }
 
-    // Layer loop.  Every layer but the last ends in the fused kernel that turns
-    // M_l straight into V_{l+1}; the spatial activation is written only where a
+    // Layer loop; a direct tower has its own (enqueue_direct).  With the Winograd kernels every
+    // layer but the last ends in the fused kernel that turns M_l straight into V_{l+1}; the
+    // spatial activation is written only where a
     // later layer adds it back as a skip connection (layer 0 and every block
     // output), and by the last layer for the 1x1 heads.
     void enqueue_forward(Lane& ln, int n, const float* d_in, const uint32_t* d_bits,
@@ -919,9 +922,9 @@ private:
             }
         }
         launch_in_transform<P>(w.act0, w.V, n, m_C0p, w.Tp, w.stream, timer(timed, LZHIP_K_IN));
-        // With the streaming GEMM the tower's layers work in place: M_l is written over V_l
-        // and V_{l+1} over M_l (see the kernels), so a lane's tiles are one array instead of
-        // two and the lanes' working sets (2 or 3 x 33 MB of tiles less at 64 boards) fit the
+        // With the streaming GEMM (fp32) the tower's layers work in place: M_l is written over
+        // V_l and V_{l+1} over M_l (see the kernels), so a lane's tiles are one array instead of
+        // two (59 MB less per lane at 64 boards of 256 filters), of which more stays in the
         // 256 MB memory-side cache.  Layer 0 reads 64 padded planes and keeps its own output.
         P* tiles = w.M;
         const bool in_place = m_in_place && m_layers.size() > 1 &&

@@ -443,7 +443,7 @@ template <> struct BufIO2<half_t> {
 // store instruction writes whole 128-byte lines (64 channels of one tile row or board
 // point), and nothing in the kernel reads them again: written through (sc0 sc1) they leave
 // for memory while the kernel runs instead of staying behind as dirty lines that the end
-// of the kernel has to flush (measured at 64 boards, 256 filters: 15.2 -> 14.0 us per
+// of the kernel has to flush (measured in fp16 at 64 boards, 256 filters: 15.2 -> 14.0 us per
 // launch).  The narrower work-groups write half and quarter lines, which written through
 // cost twice the time (32 channels at 64 boards: 16.4 us against 12.9): they stay write-back.
 template <int CG> constexpr int xform_store_policy() { return CG == 64 ? kStoreThrough : 0; }
@@ -675,10 +675,13 @@ void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const 
                              const float* bn_mean, float rfac, int n, int Kp, int Tp,
                              hipStream_t s, LaunchTimer* t) {
     // With few boards a narrow shape spreads a board's arithmetic over more compute units;
-    // the 64-channel shape moves whole lines.  Measured at 256 filters with the layers working
-    // in place (transform + GEMM per layer, us, with 16 / 32 / 64 channels per work-group):
-    // 8 boards 11.7 / 12.8 / 14.0, 16 boards 14.6 / 15.3 / 15.4, 20 boards 17.3 / 16.5 / 16.6,
-    // 24 boards 18.4 / 17.5 / 16.8, 32 boards 21.9 / 20.5 / 19.9, 40 boards 24.7 / 24.8 / 20.8.
+    // the 64-channel shape moves whole lines.  Measured per forward of 10 blocks of 256 filters,
+    // us, with 16 / 32 / 64 channels per work-group.  fp16 (filters that are no 3x3 ones): 8
+    // boards 307 / 324 / 356, 16 boards 415 / 425 / 443, 20 boards 478 / 468 / 478, 24 boards 507 / 494 /
+    // 504, 32 boards 487 / 469 / 489, 64 boards 709 / 680 / 645.  fp32: 8 boards 477 / 504 / 586, 17
+    // boards 692 / 667 / 802, 24 boards 908 / 878 / 990, 32 boards 1094 / 1079 / 1169, 40 boards 1354 /
+    // 1384 / 1371, 64 boards 1954 / 1972 / 1974: there the 64-channel shape is no better at any batch,
+    // and the line below, drawn in fp16, gives away up to a tenth from 21 to 32 boards.
     // The narrow shapes only pay with the die-aware item order of the kernel: dealt round-robin
     // over the dies, their work-groups fetch every line of M once per die that holds a piece
     // of it (16 channels at batch 16: 11.2 us per launch against 7.7).
