@@ -557,10 +557,10 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // operand is fetched once, a wavefront stages its own input channels and waits for nobody, its
 // filters are in flight all at once (D = 9 HPW; two thirds of them where five or more wavefronts
 // share the registers), and the partial sums meet in LDS at the end, in the order of the wavefronts.
-// Measured per forward of 10 blocks, conv3x3_k -> this, us: 128
-// filters, 1 board 99 -> 74, 8 boards 113 -> 90; 192 filters, 1 board 121 -> 96, 5 boards 138 ->
-// 115; 256 filters, 1 board 133 -> 107, 5 boards 159 -> 146; of 5 blocks, 1 board: 320 filters
-// 105 -> 60, 384 116 -> 63, 448 131 -> 70, 512 136 -> 76.
+// Measured per forward of 10 blocks, conv3x3_k -> this, us: 128 filters, 1 board 99 -> 82, 8 boards
+// 110 -> 92; 192 filters, 1 board 120 -> 98, 5 boards 134 -> 114; 256 filters, 1 board 132 -> 104, 5
+// boards 150 -> 138; of 5 blocks, 1 board: 320 filters 105 -> 60, 384 116 -> 63, 448 131 -> 70, 512
+// 136 -> 76.
 // Tiles of 96x32, 96x64 and 192x64 points x channels were tried for larger batches and gave
 // nothing (256 filters, 16 boards 215 -> 212, 32 boards 318 -> 324; two forwards side by side
 // lost 10 %): there the partial sums' way through LDS, 2 KW RB NB KiB, costs what it saves.
