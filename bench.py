@@ -220,14 +220,19 @@ def gemm_kernel_name(fp16, Fp, B):
 
 
 def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, lanes_arg,
-                    profile_reps, host_buffers=False, blocks_of_k=0, min_block=200):
-    """One network on the device: evaluations/s of `steps` forwards of B device-resident
+                    profile_reps, host_buffers=False, blocks_of_k=0, min_block=200, winograd=False):
+    """winograd: one Winograd position of layer 1 is scaled, which no 3x3 filter can express, so
+    that the network runs the Winograd kernels.  One network on the device: evaluations/s of `steps` forwards of B device-resident
     positions (all lanes, and one lane), optionally the same through host buffers, and the
     per-kernel-class durations with the roofline figures derived from them."""
     prec = pkg.FP16 if precision == "fp16" else pkg.FP32
     net = netgen.make_network(blocks, F, seed=2025)
     x = netgen.synthetic_inputs(B, seed=2026)
     w, h = netgen.prepare(net)
+    if winograd:
+        u = np.array(w.m_conv_weights[1], np.float32).reshape(36, F, F)
+        u[14] *= 1.25
+        w.m_conv_weights[1] = u
     pipe = pkg.HIPScheduler(prec, B, device=0)
     pipe.initialize(F)
     pipe.push_weights(6, 18, F, w)
@@ -358,11 +363,15 @@ def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, 
     gf = conv_flops(B, F, nl) if direct else gemm_flops(B, F, nl)
     in_b, out_b, fused_b = transform_bytes(B, F, nl, e)
     peak = PEAK_MFMA_F16 if prec == pkg.FP16 else PEAK_MFMA_F32
+    if direct and prec == pkg.FP32:   # three products of half-precision parts each
+        gf *= 3
+        peak = PEAK_MFMA_F16
     gemm_rate = gf / (ms[pkg.K_GEMM] * 1e-3)
     Fp = (F + 63) // 64 * 64
     roofline = {
-        "kernel": ("conv3x3_k / conv3x3_split_k (direct convolution + batch norm + skip + ReLU)"
-                   if direct
+        "kernel": ("%s (direct convolution + batch norm + skip + ReLU)"
+                   % ("conv3x3_k / conv3x3_split_k" if prec == pkg.FP16 else
+                      "conv3x3_f32_k / conv3x3_f32_split_k") if direct
                    else gemm_kernel_name(prec == pkg.FP16, Fp, B)),
         "bound": "mfma", "achieved": gemm_rate / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
         "frac": gemm_rate / peak,
@@ -374,7 +383,7 @@ def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, 
         "launches_per_forward": int(cnt[pkg.K_GEMM]),
         "flops_per_launch": gf / cnt[pkg.K_GEMM],
     }
-    if direct:
+    if direct and prec == pkg.FP16:
         # not to be read beside a Winograd GEMM's share: the direct form has 3.6 times the products
         roofline["frac_of_winograd_products"] = (gemm_flops(B, F, nl) / (ms[pkg.K_GEMM] * 1e-3)
                                                  / peak)
@@ -477,6 +486,10 @@ def side_config(pkg, netgen, torch, blocks, F, precision, B, args, cpu=False):
     net, x = r.pop("_net"), r.pop("_x")
     r.pop("_pol")
     t = r["roofline_transforms"]["out_in_transform"]
+    if t is None and precision == "fp32":
+        # the transforms of a network of the same size whose filters are no 3x3 ones
+        t = measure_forward(pkg, netgen, torch, blocks, F, precision, B, 10, 2, 0, 2,
+                            winograd=True)["roofline_transforms"]["out_in_transform"]
     out = {"value": r["value"], "unit": "evals/s", "lanes": r["lanes"],
            "one_lane": r["one_lane"]["value"], "ms_per_batch_one_lane": r["one_lane"]["ms_per_step"],
            "gemm_frac_of_mfma_peak": r["roofline"]["frac"],

@@ -249,6 +249,8 @@ public:
         } catch (...) {
             (void)hipStreamSynchronize(ln.stream);
             m_layers.clear();
+            m_direct = false;
+            for (auto& l : m_lane) l.peaks.release();
             m_w3.release();
             m_s.clear();
             release_tiles();
@@ -262,11 +264,12 @@ public:
         auto& ln = m_lane[0];
         const int F = m_filters;
         m_layers.resize(n_layers);
-        // fp16 towers that conv3x3_serves names are computed by direct convolution,
+        // fp32 towers, and fp16 towers that conv3x3_serves names, are computed by direct convolution,
         // provided that what was handed over are transforms of 3x3 filters; all else goes
         // through the Winograd kernels and needs their tile arrays.
-        m_direct = conv3x3_serves(m_Fp, m_max_batch, (int)sizeof(P)) &&
-                   build_direct_filters(n_layers, U);
+        m_direct = (sizeof(P) == 2 ? conv3x3_serves(m_Fp, m_max_batch, (int)sizeof(P))
+                                   : conv3x3_f32_serves(m_Fp)) &&
+                   build_direct_filters(n_layers, U, bn_mean, bn_scale);
         if (!m_direct) alloc_tiles();
         // Filters are laid out on the host in fp32; an fp16 net converts them on the device.
         std::vector<float> tmp;
@@ -331,34 +334,57 @@ public:
 
     // Filters of the direct convolution for every layer; false (and nothing kept) if some layer's
     // U is not the transform of 3x3 filters.
-    bool build_direct_filters(int n_layers, const float* const* U) {
-        if constexpr (sizeof(P) != 2) {
-            (void)n_layers;
-            (void)U;
-            return false;
-        } else {
-            hipStream_t s = m_lane[0].stream;
-            const int F = m_filters;
-            DevBuf<float> stage;
-            DevBuf<int> bad;
-            stage.alloc((size_t)kPos * F * (F > kInPlanes ? F : kInPlanes));
-            bad.alloc(1);
-            for (int l = 0; l < n_layers; l++) {
-                Layer& L = m_layers[l];
-                const int C = l == 0 ? kInPlanes : F, Cp = l == 0 ? m_C0p : m_Fp;
+    bool build_direct_filters(int n_layers, const float* const* U, const float* const* bn_mean,
+                              const float* const* bn_scale) {
+        hipStream_t s = m_lane[0].stream;
+        const int F = m_filters;
+        DevBuf<float> stage;
+        DevBuf<uint32_t> peak;
+        DevBuf<int> bad;
+        stage.alloc((size_t)kPos * F * (F > kInPlanes ? F : kInPlanes));
+        bad.alloc(1);
+        bool good = true;
+        for (int l = 0; l < n_layers && good; l++) {
+            Layer& L = m_layers[l];
+            const int C = l == 0 ? kInPlanes : F, Cp = l == 0 ? m_C0p : m_Fp;
+            HIP_CHECK(hipMemcpy(stage.p, U[l], sizeof(float) * (size_t)kPos * C * F,
+                                hipMemcpyHostToDevice));
+            if constexpr (sizeof(P) == 2) {
                 L.W3.alloc(conv3x3_filter_count(Cp, m_Fp));
-                HIP_CHECK(hipMemcpy(stage.p, U[l], sizeof(float) * (size_t)kPos * C * F,
-                                    hipMemcpyHostToDevice));
                 conv3x3_filters(stage.p, L.W3.p, C, F, m_Fp, bad.p, s);
-                HIP_CHECK(hipGetLastError());
-                HIP_CHECK(hipStreamSynchronize(s));
+            } else {
+                L.W3.alloc(conv3x3_f32_filter_count(Cp, m_Fp));
+                peak.alloc(F);
+                conv3x3_f32_filters(stage.p, L.W3.p, peak.p, C, Cp, F, m_Fp, bad.p, s);
             }
-            int is_bad = 0;
-            HIP_CHECK(hipMemcpy(&is_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost));
-            if (is_bad)
-                for (auto& L : m_layers) L.W3.release();
-            return !is_bad;
+            HIP_CHECK(hipGetLastError());
+            HIP_CHECK(hipStreamSynchronize(s));
+            if constexpr (sizeof(P) == 4) {
+                L.peak.resize(F);
+                HIP_CHECK(hipMemcpy(L.peak.data(), peak.p, sizeof(uint32_t) * F, hipMemcpyDeviceToHost));
+                // the filters' scales have to fit into the batch norm's numbers
+                for (int k = 0; k < F && good; k++) {
+                    const float u = conv3x3_f32_unscale(L.peak[k]);
+                    good = fits(bn_scale[l][k], u) && fits(bn_mean[l][k], 1.0f / u);
+                }
+            }
         }
+        int is_bad = 0;
+        HIP_CHECK(hipMemcpy(&is_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost));
+        good = good && !is_bad;
+        if (!good)
+            for (auto& L : m_layers) {
+                L.W3.release();
+                L.peak.clear();
+            }
+        else if (sizeof(P) == 4)
+            for (int i = 0; i < m_n_lanes; i++)
+                m_lane[i].peaks.alloc(2 * conv3x3_f32_slots(m_Fp, m_max_batch) + 2 * (size_t)m_max_batch);
+        return good;
+    }
+    // Whether v times a power of two is exact: v is no number, zero, or stays a normal one.
+    static bool fits(float v, float power) {
+        return !std::isfinite(v) || v == 0.0f || std::isnormal(v * power);
     }
 
     void alloc_tiles() {
@@ -415,6 +441,10 @@ public:
         w.Tp = kStaticTp;
         w.V = reinterpret_cast<P*>(base);
         w.M = reinterpret_cast<P*>(base + kStaticTileBytes);
+        // (a direct tower has no tiles: the peaks of its layers take their place)
+        w.peaks = m_direct && sizeof(P) == 4 ? reinterpret_cast<uint32_t*>(base) : nullptr;
+        if (w.peaks && peak_words(n) * sizeof(uint32_t) > 2 * kStaticTileBytes)
+            throw std::invalid_argument("no room for the peaks");
         w.act0 = reinterpret_cast<P*>(base + 2 * kStaticTileBytes);
         for (int i = 0; i < 3; i++)
             w.act[i] = reinterpret_cast<P*>(base + 2 * kStaticTileBytes + kStaticAct0Bytes +
@@ -674,7 +704,13 @@ public:
         d_planes.alloc((size_t)n * C * kPts);
         HIP_CHECK(hipMemcpy(d_planes.p, act_in, sizeof(float) * (size_t)n * C * kPts, hipMemcpyHostToDevice));
         P* a_in = (layer == 0) ? ln.act0.p : ln.act[0].p;
-        launch_pack_input<P>(d_planes.p, a_in, n, C, Cp, ln.stream, nullptr);
+        PeakMap peaks{ln.peaks.p, kPts, 1};
+        if constexpr (sizeof(P) == 4) {
+            if (m_direct)
+                launch_pack_input_peaks(d_planes.p, a_in, n, C, Cp, peaks.slots, ln.stream, nullptr);
+        }
+        if (sizeof(P) == 2 || !m_direct)
+            launch_pack_input<P>(d_planes.p, a_in, n, C, Cp, ln.stream, nullptr);
         const P* r = nullptr;
         if (res) {
             d_res.alloc((size_t)n * F * kPts);
@@ -683,7 +719,11 @@ public:
             r = ln.act[1].p;
         }
         std::vector<float> sc(m_Fp, 0.0f), mn(m_Fp, 0.0f);
-        for (int k = 0; k < F; k++) { sc[k] = L.scale[k]; mn[k] = L.mean[k]; }
+        for (int k = 0; k < F; k++) {
+            const float u = L.peak.empty() ? 1.0f : conv3x3_f32_unscale(L.peak[k]);
+            sc[k] = L.scale[k] * u;
+            mn[k] = L.mean[k] / u;
+        }
         d_sc.alloc(m_Fp); d_mn.alloc(m_Fp);
         HIP_CHECK(hipMemcpy(d_sc.p, sc.data(), sizeof(float) * m_Fp, hipMemcpyHostToDevice));
         HIP_CHECK(hipMemcpy(d_mn.p, mn.data(), sizeof(float) * m_Fp, hipMemcpyHostToDevice));
@@ -692,25 +732,26 @@ public:
         DevBuf<P> d_V, d_M, d_U;
         P *V = ln.V.p, *M = ln.M.p;
         const P *U = L.U.p, *Uf = L.Uf.p;
-        if constexpr (sizeof(P) == 2) {
-            if (m_direct) {
-                std::vector<P> w3(L.W3.count), u((size_t)kPos * m_Fp * Cp, (P)0.0f);
-                HIP_CHECK(hipMemcpy(w3.data(), L.W3.p, w3.size() * sizeof(P), hipMemcpyDeviceToHost));
+        if (m_direct) {
+            std::vector<half_t> w3(L.W3.count);
+            std::vector<P> u((size_t)kPos * m_Fp * Cp, (P)0.0f);
+            HIP_CHECK(hipMemcpy(w3.data(), L.W3.p, w3.size() * sizeof(half_t), hipMemcpyDeviceToHost));
+            if constexpr (sizeof(P) == 2)
                 conv3x3_winograd_filters(w3.data(), C, Cp, F, m_Fp, u.data());
-                d_U.alloc(u.size());
-                HIP_CHECK(hipMemcpy(d_U.p, u.data(), u.size() * sizeof(P), hipMemcpyHostToDevice));
-                d_V.alloc((size_t)kPos * m_Tp * m_Fp);
-                d_M.alloc((size_t)kPos * m_Tp * m_Fp);
-                V = d_V.p; M = d_M.p; U = d_U.p; Uf = nullptr;
-            }
+            else
+                conv3x3_f32_winograd_filters(w3.data(), L.peak.data(), C, Cp, F, m_Fp, u.data());
+            d_U.alloc(u.size());
+            HIP_CHECK(hipMemcpy(d_U.p, u.data(), u.size() * sizeof(P), hipMemcpyHostToDevice));
+            d_V.alloc((size_t)kPos * m_Tp * m_Fp);
+            d_M.alloc((size_t)kPos * m_Tp * m_Fp);
+            V = d_V.p; M = d_M.p; U = d_U.p; Uf = nullptr;
         }
         launch_in_transform<P>(a_in, V, n, Cp, m_Tp, ln.stream, nullptr);
         launch_gemm<P>(V, U, Uf, M, Tu, m_Tp, Cp, m_Fp, ln.stream, nullptr);
-        if constexpr (sizeof(P) == 2) {
-            if (m_direct)
-                conv_direct(L, a_in, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, ln.stream, nullptr);
-        }
-        if (!m_direct)
+        if (m_direct)
+            conv_direct(L, a_in, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, peaks,
+                        peak_slots(peaks.slots, n, 0), n, ln.stream, nullptr);
+        else
             launch_out_transform<P>(M, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, m_Fp, m_Tp,
                                     ln.stream, nullptr);
         HIP_CHECK(hipGetLastError());
@@ -777,6 +818,7 @@ private:
         hipStream_t stream = nullptr;
         std::mutex mu;  // serialises enqueues on this lane
         DevBuf<P> act0, act[3], V, M;
+        DevBuf<uint32_t> peaks;   // direct fp32 towers: peak_words
         std::map<GraphKey, hipGraphExec_t> graphs;
     };
     static constexpr int kLanes = 3;   // upper bound; m_n_lanes are in use
@@ -787,7 +829,14 @@ private:
         hipStream_t stream = nullptr;
         P *act0 = nullptr, *act[3] = {nullptr, nullptr, nullptr}, *V = nullptr, *M = nullptr;
         int Tp = 0;
+        uint32_t* peaks = nullptr;   // (direct fp32 towers)
     };
+    // Slots of the input planes, then two sets that the layers write in turn.
+    size_t peak_words(int n) const { return 2 * (size_t)n + 2 * conv3x3_f32_slots(m_Fp, n); }
+    // Where layer l, of n boards, leaves its peaks; -1: the input planes.
+    uint32_t* peak_slots(uint32_t* peaks, int n, int l) const {
+        return l < 0 || !peaks ? peaks : peaks + 2 * n + (l & 1) * conv3x3_f32_slots(m_Fp, n);
+    }
     Work work_of(Lane& ln) const {
         Work w;
         w.stream = ln.stream;
@@ -796,6 +845,7 @@ private:
         w.V = ln.V.p;
         w.M = ln.M.p;
         w.Tp = m_Tp;
+        w.peaks = m_direct ? ln.peaks.p : nullptr;
         return w;
     }
 
@@ -804,7 +854,8 @@ private:
         // the filters in one of three orders, the other two empty:
         DevBuf<P> U;                          // [36][Fp][Cp] (tiled GEMMs)
         DevBuf<P> Uf;                         // fragment order of the streaming GEMM
-        DevBuf<P> W3;                         // 3x3, fragment order of the direct convolution
+        DevBuf<half_t> W3;                    // 3x3, fragment order of the direct convolution
+        std::vector<uint32_t> peak;           // (fp32) largest of each output channel's W3
         std::vector<float> mean, scale;       // as pushed (unscaled)
         DevBuf<float> d_mean, d_scale;        // with activation scales folded in
         float rfac = 1.0f;
@@ -822,8 +873,9 @@ private:
         const float s_in = m_s[l], s_out = m_s[l + 1];
         std::vector<float> sc(m_Fp, 0.0f), mn(m_Fp, 0.0f);
         for (int k = 0; k < m_filters; k++) {
-            sc[k] = L.scale[k] * (s_in / s_out);
-            mn[k] = L.mean[k] / s_in;
+            const float u = L.peak.empty() ? 1.0f : conv3x3_f32_unscale(L.peak[k]);
+            sc[k] = L.scale[k] * (s_in / s_out) * u;
+            mn[k] = L.mean[k] / s_in / u;
         }
         const bool second = l >= 2 && (l % 2) == 0;
         L.rfac = second ? m_s[l - 1] / s_out : 1.0f;
@@ -843,12 +895,11 @@ private:
     // Activation buffer roles rotate: cur = block input, mid, nxt = block output.
     void run_conv(Lane& ln, int l, int n, const P* in, const P* res, P* out, bool timed) {
         Layer& L = m_layers[l];
-        if constexpr (sizeof(P) == 2) {
-            if (m_direct) {
-                conv_direct(L, in, res, out, L.d_scale.p, L.d_mean.p, L.rfac, n, ln.stream,
-                            timer(timed, LZHIP_K_GEMM));
-                return;
-            }
+        if (m_direct) {
+            PeakMap none;
+            conv_direct(L, in, res, out, L.d_scale.p, L.d_mean.p, L.rfac, none, nullptr, n, ln.stream,
+                        timer(timed, LZHIP_K_GEMM));
+            return;
         }
         const int Tu = n * kTilesPerBoard;
         launch_in_transform<P>(in, ln.V.p, n, L.Cp, m_Tp, ln.stream, timer(timed, LZHIP_K_IN));
@@ -909,17 +960,14 @@ private:
                          float* d_pol, float* d_val, bool timed) {
         const int nl = (int)m_layers.size();
         const int Tu = n * kTilesPerBoard;
-        if (d_in)
-            launch_pack_input<P>(d_in, w.act0, n, kInPlanes, m_C0p, w.stream,
-                                 timer(timed, LZHIP_K_PACK));
-        else
-            launch_pack_input_bits<P>(d_bits, w.act0, n, kInPlanes, m_C0p, w.stream,
-                                      timer(timed, LZHIP_K_PACK));
-        if constexpr (sizeof(P) == 2) {
-            if (m_direct) {
-                enqueue_direct(w, n, d_pol, d_val, timed);
-                return;
-            }
+        LaunchTimer* pack = timer(timed, LZHIP_K_PACK);
+        if (!d_in)
+            launch_pack_input_bits<P>(d_bits, w.act0, n, kInPlanes, m_C0p, w.peaks, w.stream, pack);
+        else if (!pack_with_peaks(w, d_in, n, pack))
+            launch_pack_input<P>(d_in, w.act0, n, kInPlanes, m_C0p, w.stream, pack);
+        if (m_direct) {
+            enqueue_direct(w, n, d_pol, d_val, timed);
+            return;
         }
         launch_in_transform<P>(w.act0, w.V, n, m_C0p, w.Tp, w.stream, timer(timed, LZHIP_K_IN));
         // With the streaming GEMM (fp32) the tower's layers work in place: M_l is written over
@@ -956,35 +1004,50 @@ private:
         }
     }
 
+    bool pack_with_peaks(const Work& w, const float* d_in, int n, LaunchTimer* t) {
+        if constexpr (sizeof(P) == 4) {
+            if (w.peaks) {
+                launch_pack_input_peaks(d_in, w.act0, n, kInPlanes, m_C0p, w.peaks, w.stream, t);
+                return true;
+            }
+        }
+        return false;
+    }
+
     // One layer of a direct tower; which of the two kernels depends on the handle, not on n.
+    // fp32: peaks are those of `in` and become those of `out`, which go to `slots`.
     void conv_direct(const Layer& L, const P* in, const P* res, P* out, const float* scale,
-                     const float* mean, float rfac, int n, hipStream_t s, LaunchTimer* t) {
+                     const float* mean, float rfac, PeakMap& peaks, uint32_t* slots, int n,
+                     hipStream_t s, LaunchTimer* t) {
         if constexpr (sizeof(P) == 2) {
             const bool split = L.Cp == m_Fp && conv3x3_splits(m_Fp, m_max_batch);
             (split ? launch_conv3x3_split : launch_conv3x3)(in, L.W3.p, res, out, scale, mean, rfac,
                                                             n, L.Cp, m_Fp, s, t);
+        } else {
+            const bool split = L.Cp == m_Fp && conv3x3_f32_splits(m_Fp, m_max_batch);
+            peaks = (split ? launch_conv3x3_f32_split : launch_conv3x3_f32)(
+                in, L.W3.p, res, out, scale, mean, rfac, peaks, slots, n, L.Cp, m_Fp, s, t);
         }
     }
 
     // The layer loop of a direct tower: one launch per layer.
     void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed) {
-        if constexpr (sizeof(P) == 2) {
-            const int nl = (int)m_layers.size();
-            const P* last = w.act[0];
-            int cur = 0, nxt = 2;   // block input (skip) / block output; 1 lies between
-            for (int l = 0; l < nl; l++) {
-                Layer& L = m_layers[l];
-                const bool second = l >= 2 && (l % 2) == 0;
-                const P* in = l == 0 ? w.act0 : second ? w.act[1] : w.act[cur];
-                P* out = l == 0 ? w.act[cur] : second ? w.act[nxt] : w.act[1];
-                conv_direct(L, in, second ? w.act[cur] : nullptr, out, L.d_scale.p, L.d_mean.p,
-                            L.rfac, n, w.stream, timer(timed, LZHIP_K_GEMM));
-                last = out;
-                if (second) { const int o = cur; cur = nxt; nxt = o; }
-            }
-            launch_head_conv<P>(last, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
-                                timer(timed, LZHIP_K_HEAD));
+        const int nl = (int)m_layers.size();
+        const P* last = w.act[0];
+        PeakMap peaks{w.peaks, kPts, 1};
+        int cur = 0, nxt = 2;   // block input (skip) / block output; 1 lies between
+        for (int l = 0; l < nl; l++) {
+            Layer& L = m_layers[l];
+            const bool second = l >= 2 && (l % 2) == 0;
+            const P* in = l == 0 ? w.act0 : second ? w.act[1] : w.act[cur];
+            P* out = l == 0 ? w.act[cur] : second ? w.act[nxt] : w.act[1];
+            conv_direct(L, in, second ? w.act[cur] : nullptr, out, L.d_scale.p, L.d_mean.p, L.rfac,
+                        peaks, peak_slots(w.peaks, n, l), n, w.stream, timer(timed, LZHIP_K_GEMM));
+            last = out;
+            if (second) { const int o = cur; cur = nxt; nxt = o; }
         }
+        launch_head_conv<P>(last, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
+                            timer(timed, LZHIP_K_HEAD));
     }
 
     float absmax(const P* x, size_t count) {

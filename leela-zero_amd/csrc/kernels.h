@@ -36,12 +36,23 @@ struct LaunchTimer {
 // 32-bit words of one position's 18 x 361 input planes packed one bit per value.
 constexpr int kInputWords = (18 * 361 + 31) / 32;
 
+// Largest magnitudes (bits of a float) of a layer's planes on every board, what the direct fp32
+// convolution scales its operands by: slots[row][2][column] of the tiles of mt points that wrote
+// them, for the first and the second board that a tile meets.
+struct PeakMap {
+    uint32_t* slots = nullptr;
+    int mt = 0, tiles_n = 0;
+};
+// (peaks: null, or 2 n slots of input planes, one tile a board)
 template <typename P>
-void launch_pack_input_bits(const uint32_t* bits, P* act, int n, int C, int Cp, hipStream_t s,
-                            LaunchTimer* t);
+void launch_pack_input_bits(const uint32_t* bits, P* act, int n, int C, int Cp, uint32_t* peaks,
+                            hipStream_t s, LaunchTimer* t);
 template <typename P>
 void launch_pack_input(const float* in, P* act, int n, int C, int Cp, hipStream_t s,
                        LaunchTimer* t);
+// The same with the peaks.
+void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
+                             hipStream_t s, LaunchTimer* t);
 
 // act [n][361][Cp] -> V [36][Tp][Cp]
 template <typename P>
@@ -106,6 +117,31 @@ void conv3x3_filters(const float* U, _Float16* Wf, int C, int F, int Kp, int* ba
 // The way back, on the host: Winograd filters [36][Kp][Cp] of the filters as stored (padding of
 // U is left as it is).
 void conv3x3_winograd_filters(const _Float16* Wf, int C, int Cp, int F, int Kp, _Float16* U);
+
+// Direct 3x3 convolution of fp32 towers (conv3x3_f32.hip), one launch per layer:
+// X [n][361][Cp] -> Y [n][361][Kp] = max(0, scale*(conv - mean) + rfac*res) in fp32, every operand split in
+// two half-precision numbers.  Wf holds the filters of output channel k times 2^e(k):
+// conv3x3_f32_unscale(peak[k]) = 2^-e(k) belongs into scale, 2^e(k) into mean.  peaks: of X; those of Y
+// go to `slots` (conv3x3_f32_slots words) and are returned.
+bool conv3x3_f32_serves(int Kp);
+size_t conv3x3_f32_filter_count(int Cp, int Kp);
+size_t conv3x3_f32_slots(int Kp, int max_batch);
+PeakMap launch_conv3x3_f32(const float* X, const _Float16* Wf, const float* res, float* Y,
+                           const float* bn_scale, const float* bn_mean, float rfac,
+                           const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
+                           hipStream_t s, LaunchTimer* t);
+// The same layer with its sum dealt to the wavefronts of a work-group (conv3x3_splits).
+bool conv3x3_f32_splits(int Kp, int max_batch);
+PeakMap launch_conv3x3_f32_split(const float* X, const _Float16* Wf, const float* res, float* Y,
+                                 const float* bn_scale, const float* bn_mean, float rfac,
+                                 const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
+                                 hipStream_t s, LaunchTimer* t);
+// Filters of one layer and their peaks (F values, zero before) from U [36][C][F]; *bad as above.
+void conv3x3_f32_filters(const float* U, _Float16* Wf, uint32_t* peak, int C, int Cp, int F, int Kp,
+                         int* bad, hipStream_t s);
+float conv3x3_f32_unscale(uint32_t peak_bits);
+void conv3x3_f32_winograd_filters(const _Float16* Wf, const uint32_t* peak, int C, int Cp, int F, int Kp,
+                                  float* U);
 
 // 1x1 head convolutions: act [n][361][Cp] x w[3][Cp] -> pol [n][2][361], val [n][361],
 // both multiplied by out_scale.

@@ -126,10 +126,11 @@ void launch_pack_input(const float* in, P* act, int n, int C, int Cp, hipStream_
 template <typename P>
 __global__ __launch_bounds__(256) void pack_input_bits_k(const uint32_t* __restrict__ bits,
                                                          P* __restrict__ act, int n, int C,
-                                                         int Cp) {
+                                                         int Cp, uint32_t* __restrict__ peaks) {
     const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t total = (size_t)n * kPts * Cp;
     if (gid >= total) return;
+    if (peaks && gid < 2 * (size_t)n) peaks[gid] = 0x3f800000u;
     const int c = (int)(gid % Cp);
     const size_t bp = gid / Cp;
     const int pt = (int)(bp % kPts);
@@ -143,11 +144,50 @@ __global__ __launch_bounds__(256) void pack_input_bits_k(const uint32_t* __restr
 }
 
 template <typename P>
-void launch_pack_input_bits(const uint32_t* bits, P* act, int n, int C, int Cp, hipStream_t s,
-                            LaunchTimer* t) {
+void launch_pack_input_bits(const uint32_t* bits, P* act, int n, int C, int Cp, uint32_t* peaks,
+                            hipStream_t s, LaunchTimer* t) {
     const size_t total = (size_t)n * kPts * Cp;
     launch(pack_input_bits_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, bits, act,
-           n, C, Cp);
+           n, C, Cp, peaks);
+}
+
+// Planes and peaks from float planes: one work-group per board reads all of it (26 KB); the packing
+// is spread over eight.
+constexpr int kPackParts = 8;
+__global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restrict__ in,
+                                                          float* __restrict__ act, int C, int Cp,
+                                                          uint32_t* __restrict__ peaks) {
+    const int b = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
+    const float* planes = in + (size_t)b * C * kPts;
+    float top = 0.0f;
+    if (part == 0) {
+#pragma unroll 8
+        for (int i = tid; i < C * kPts; i += 512) {
+            const float v = fabsf(planes[i]);
+            top = fmaxf(top, v < __builtin_inff() ? v : 0.0f);
+        }
+    }
+    const int from = part * kPts / kPackParts, to = (part + 1) * kPts / kPackParts;
+    float* out = act + (size_t)b * kPts * Cp;
+    for (int i = tid; i < (to - from) * Cp; i += 512) {
+        const int pt = from + i / Cp, c = i % Cp;
+        out[(size_t)pt * Cp + c] = c < C ? planes[(size_t)c * kPts + pt] : 0.0f;
+    }
+    if (part != 0) return;
+    __shared__ float tops[8];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
+    if ((tid & 63) == 0) tops[tid >> 6] = top;
+    __syncthreads();
+    if (tid == 0) {
+        for (int i = 1; i < 8; i++) top = fmaxf(top, tops[i]);
+        peaks[2 * b] = __builtin_bit_cast(uint32_t, top);
+    }
+}
+
+void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
+                             hipStream_t s, LaunchTimer* t) {
+    launch(pack_input_peaks_k, dim3(n, kPackParts), dim3(512), s, t, in, act, C, Cp, peaks);
 }
 
 // ---------------------------------------------------------------------------
@@ -2045,8 +2085,8 @@ void launch_heads(const float* pol, const float* val, HeadParams hp, float tempe
 #define INSTANTIATE(P)                                                                         \
     template void launch_pack_input<P>(const float*, P*, int, int, int, hipStream_t,           \
                                        LaunchTimer*);                                          \
-    template void launch_pack_input_bits<P>(const uint32_t*, P*, int, int, int, hipStream_t,   \
-                                            LaunchTimer*);                                     \
+    template void launch_pack_input_bits<P>(const uint32_t*, P*, int, int, int, uint32_t*,     \
+                                            hipStream_t, LaunchTimer*);                        \
     template void launch_in_transform<P>(const P*, P*, int, int, int, hipStream_t,             \
                                          LaunchTimer*);                                        \
     template void launch_gemm<P>(const P*, const P*, const P*, P*, int, int, int, int,         \

@@ -903,3 +903,79 @@ def test_winograd_filters_of_no_3x3_filter(pkg, netgen, orc):
         rp, rv = ref.forward(x[i])
         assert rel_l2(pol[i], rp) <= 2e-2 and rel_l2(val[i], rv) <= 2e-2, i
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,maxb,batches", [
+    # sums dealt to the wavefronts: the tiles of 16 and of 32 channels, both ends of each
+    (64, 45, (1, 22, 23, 33, 34, 45)), (128, 11, (1, 5, 6, 8, 9, 11)), (192, 7, (1, 2, 3, 5, 6, 7)),
+    (256, 5, (1, 2, 3, 4, 5)), (320, 4, (1, 2, 3, 4)), (384, 3, (1, 2, 3)), (448, 3, (1, 2, 3)),
+    (512, 2, (1, 2)),
+    # the other tiles on both sides of every change
+    (64, 137, (1, 22, 23, 34, 68, 69, 136, 137)), (128, 70, (1, 11, 12, 17, 34, 35, 68, 69, 70)),
+    (192, 46, (1, 7, 8, 11, 22, 23, 45, 46)), (256, 36, (1, 5, 6, 8, 9, 17, 34, 35, 36)),
+    (384, 24, (1, 3, 6, 11, 12, 23, 24)), (512, 18, (1, 4, 5, 9, 17, 18)),
+    # widths that are padded to a multiple of 64
+    (24, 46, (1, 46)), (100, 12, (1, 12)), (200, 6, (1, 6)),
+])
+def test_fp32_direct_convolution(pkg, netgen, orc, filters, maxb, batches):
+    """fp32 towers of 3x3 filters: one layer with a skip connection against a float64 convolution.
+    The bound is what fp32 sums of 9 * filters products show (rounding of a partial sum per 32
+    products and part: 2^-24 sqrt(9 * filters * 3 / 32) at most, times two for what the matrix
+    instruction drops); boards of very different magnitude side by side keep their own scale."""
+    import torch
+    import torch.nn.functional as F
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 6900 + filters, pkg.FP32, maxb)
+    rng = np.random.default_rng(filters + maxb)
+    a = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float32)
+    r = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float32)
+    size = 10.0 ** rng.integers(-12, 13, maxb).astype(np.float32)   # one magnitude a board
+    size[0] = 1.0
+    a *= size[:, None, None]
+    r *= size[:, None, None]
+    y = F.conv2d(torch.from_numpy(a.reshape(maxb, filters, 19, 19)).double(),
+                 torch.from_numpy(net.conv_w[2]).double(), padding=1).numpy().reshape(maxb, filters, 361)
+    scale, mean = ref.scale[2].astype(np.float64), ref.mean[2].astype(np.float64)
+    want = np.maximum(0.0, scale[None, :, None] * (y - mean[None, :, None]) + r)
+    bound = 2.0 * 2.0 ** -24 * (9 * filters * 3 / 32) ** 0.5 + 2.0 ** -22
+    for n in batches:
+        print("case: fp32, %d filters, %d boards of %d" % (filters, n, maxb), flush=True)
+        got = pipe.debug_layer(2, a[:n], r[:n])[2]
+        for i in range(n):
+            assert rel_l2(got[i], want[i]) <= bound, (n, i, rel_l2(got[i], want[i]), bound)
+    pipe.close()
+
+
+@pytest.mark.parametrize("filters,maxb", [(128, 40), (192, 16), (192, 40), (256, 9), (384, 28), (512, 44)])
+def test_fp32_filters_of_no_3x3_filter(pkg, netgen, orc, filters, maxb):
+    """fp32 networks whose filters are no 3x3 ones run the Winograd kernels: the streaming GEMM, the
+    tiled ones, and one position on the handle with the same bits."""
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 6950 + filters, pkg.FP32, maxb,
+                                       winograd=True)
+    x = netgen.synthetic_inputs(maxb, seed=6951)
+    check_outputs(pkg, orc, pipe, ref, h_ref, x, 0, idx=[0, maxb - 1])
+    pol, val = pipe.forward_batch(x)
+    one_pol, one_val = pipe.forward_batch(x[:1])
+    assert np.array_equal(pol[0], one_pol[0]) and np.array_equal(val[0], one_val[0])
+    pipe.close()
+
+
+def test_fp32_range_and_values_that_are_no_numbers(pkg, netgen, orc):
+    """fp32 planes of any magnitude, an infinity and a NaN among them: planes 1e30 and 1e-30 times
+    the engine's agree with the oracle's at the same magnitudes, and an infinity or a NaN in one
+    position leaves the other positions of the batch as they are."""
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, 64, 6960, pkg.FP32, 4)
+    x = netgen.synthetic_inputs(4, seed=6961)
+    want = pipe.forward_batch(x)
+    for factor in (1e30, 1e-30, 3e-3):
+        big = (factor * x).astype(np.float32)
+        pol, val = pipe.forward_batch(big)
+        for i in range(4):
+            rp, rv = ref.forward(big[i])
+            assert rel_l2(pol[i], rp) <= 1e-5 and rel_l2(val[i], rv) <= 1e-5, (factor, i)
+    for bad in (np.inf, np.nan, -np.inf):
+        y = x.copy()
+        y[1].reshape(-1)[5] = bad
+        pol, val = pipe.forward_batch(y)
+        for i in (0, 2, 3):
+            assert np.array_equal(pol[i], want[0][i]) and np.array_equal(val[i], want[1][i]), (bad, i)
+    pipe.close()
