@@ -80,8 +80,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     constexpr int CELLS = conv_cells(MT);
     constexpr int STR = CH * 128 + 16;           // bytes per cell
     constexpr int BUF = (CELLS + 1) * STR;       // one more cell takes the pieces past the end
-    constexpr int PPC = CH * 8;                  // 16-byte pieces per cell
-    constexpr int NP = (CELLS * PPC + NT - 1) / NT;
+    constexpr int PPC = 8;                       // 16-byte pieces per cell and chunk
+    constexpr int NP = (CELLS * PPC + NT - 1) / NT;   // a thread's, per chunk
     constexpr int KS = kStepsPerChunk;
     constexpr int SGRP = 3;
     constexpr int NG = (NP + SGRP - 1) / SGRP;   // groups of pieces per chunk (CC == 0)
@@ -131,39 +131,37 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     __builtin_amdgcn_sched_barrier(0);
 
     const PatchStart ps = patch_start(m0);
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
-    unsigned poff[NP];
-#pragma unroll
-    for (int i = 0; i < NP; i++) poff[i] = patch_offset<CELLS, PPC, NT>(i, ps, tid, Cp * 2);
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 2);
+    const unsigned xrow = (unsigned)Cp * 2u;     // bytes of a cell in memory
+    const unsigned xoff = (ps.q0 + tid / PPC) * xrow + (tid % PPC) * 16u;
+    // piece i, `at` bytes into the cells' channels
+    auto xload = [&](int i, unsigned at) {
+        return __builtin_amdgcn_raw_buffer_load_b128(rX, xoff, i * (NT / PPC) * xrow + at, 0);
+    };
     // LDS address of piece i: a constant distance from piece 0 (but for the last, which may
-    // lie past the end, and where a row of threads is no whole number of cells)
+    // lie past the end)
     const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 16u;
     auto laddr = [&](int i) -> unsigned {
-        if constexpr (NT % PPC == 0) {
-            if (i < NP - 1 || (CELLS * PPC) % NT == 0) return lst + i * (NT / PPC) * STR;
-        }
-        const unsigned p = tid + i * NT, c = p / PPC;
-        return (c < (unsigned)CELLS ? c : (unsigned)CELLS) * STR + (p % PPC) * 16u;
+        if (i < NP - 1 || (CELLS * PPC) % NT == 0) return lst + i * (NT / PPC) * STR;
+        return min(tid / PPC + i * (NT / PPC), (unsigned)CELLS) * STR + (tid % PPC) * 16u;
     };
 
     const int chunks = Cp / 64;
+    const int ch0 = (kb >> 1) * 32 + 8 * (int)(lane >> 4) + 4 * (kb & 1);   // first channel
     unsigned arow[RB];   // LDS address of this lane's point of each row block, tap (0, 0)
+    unsigned ro[RB];     // byte offset of this lane's point and channel
+    int4v rr[RB][PR];
     static_assert(MT <= kPts, "a tile touches two boards at most");
 #pragma unroll
-    for (int i = 0; i < RB; i++)
-        arow[i] = patch_cell(ps, min((wr * RB + i) * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
-                  (lane >> 4) * 16;
-
-    const int ch0 = (kb >> 1) * 32 + 8 * (int)(lane >> 4) + 4 * (kb & 1);   // first channel
-    unsigned ro[RB];                              // byte offset of this lane's point and channel
-    int4v rr[RB][PR];
-#pragma unroll
     for (int i = 0; i < RB; i++) {
-        const int m = m0 + (wr * RB + i) * 16 + (int)(lane & 15);
-        ro[i] = m < rows ? (unsigned)((m * Kp + ch0) * 2) : 0xfffff000u;
+        const int local = (wr * RB + i) * 16 + (int)(lane & 15);
+        const unsigned cell = patch_cell(ps, min(local, rows - 1 - m0));
+        arow[i] = cell * STR + (lane >> 4) * 16;
+        ro[i] = m0 + local < rows ? ((ps.q0 + kPointCell + cell) * Kp + ch0) * 2u : 0xfffff000u;
     }
-    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, (size_t)rows * Kp * 2);
-    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, (size_t)rows * Kp * 2);
+    const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
+    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
+    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
     auto load_res = [&]() {
         if (res != nullptr) {
 #pragma unroll
@@ -187,13 +185,17 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     };
 
     {
-        int4v stg[NP];
+        int4v stg[CH][NP];
 #pragma unroll
-        for (int i = 0; i < NP; i++)
-            stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rX, poff[i], 0, 0);
+        for (int c = 0; c < CH; c++)
+#pragma unroll
+            for (int i = 0; i < NP; i++) stg[c][i] = xload(i, c * 128);
         if constexpr (EARLY) load_res();
 #pragma unroll
-        for (int i = 0; i < NP; i++) *reinterpret_cast<int4v*>(lds + laddr(i)) = stg[i];
+        for (int c = 0; c < CH; c++)
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+                *reinterpret_cast<int4v*>(lds + laddr(i) + c * 128) = stg[c][i];
         if (tid < (unsigned)CW) {
             bn[0][tid] = scale;
             bn[1][tid] = -scale * mean;
@@ -240,8 +242,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
 #pragma unroll
                         for (int i = 0; i < SGRP; i++)
                             if (g * SGRP + i < NP)
-                                sg[i] = __builtin_amdgcn_raw_buffer_load_b128(
-                                    rX, poff[g * SGRP + i], next, 0);
+                                sg[i] = xload(g * SGRP + i, next);
                     }
                     if (st == (g + 1) * GS - 1) {
 #pragma unroll
@@ -501,27 +502,30 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     };
     filters(0, F0);
     const PatchStart ps = patch_start(m0);
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 2);
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 2);
+    constexpr unsigned xrow = Cp * 2;   // bytes of a cell in memory
+    const unsigned xoff = (ps.q0 + lane / PPC) * xrow + (lane % PPC) * 16u;
     int4v stg[NP];
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
+    for (int i = 0; i < NP; i++)
         stg[i] = __builtin_amdgcn_raw_buffer_load_b128(
-            rX, patch_offset<CELLS, PPC, 64>(i, ps, lane, Cp * 2), wave * (HPW * 64), 0);
-        if (i % 2) __builtin_amdgcn_sched_barrier(0);
-    }
+            rX, xoff, i * (64 / PPC) * xrow + wave * (HPW * 64), 0);
     __builtin_amdgcn_sched_barrier(0);
     filters(F0, D - 1);
 
     // the blocks of 16 points that this wavefront finishes: where they lie, and the skip connection
     unsigned ro[QP];
     int4v rr[QP];
-    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, (size_t)rows * Kp * 2);
-    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, (size_t)rows * Kp * 2);
+    const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
+    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
+    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
     const int cl = 8 * (int)(lane >> 4);   // first of this lane's 8 channels
 #pragma unroll
     for (int q = 0; q < QP; q++) {
-        const int i = q * KW + wave, m = m0 + i * 16 + (int)(lane & 15);
-        ro[q] = i < RB && m < rows ? (unsigned)((m * Kp + tn * CW + cl) * 2) : 0xfffffff0u;
+        const int i = q * KW + wave, local = i * 16 + (int)(lane & 15);
+        ro[q] = i < RB && m0 + local < rows
+                    ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + tn * CW + cl) * 2u
+                    : 0xfffffff0u;
         rr[q] = int4v{0, 0, 0, 0};
     }
     if (res != nullptr) {

@@ -139,11 +139,14 @@ struct BoardPeak {
     }
 };
 
-// Scales of a tile: of its patch's cells (rows below 20 of the patch, the others) and of its results
-// (first board of the tile, the next one).
+// Scales of a tile's first board and of the next one, and their reciprocals.
 struct TileScales {
-    float in0, in1, out0, out1;
+    float s0, s1, u0, u1;
 };
+// First cell of the patch that lies on the tile's second board (or past the patch).
+__device__ __forceinline__ unsigned second_board(const PatchStart& s) {
+    return (s.mb + 2) * kCellsPerBoard - s.q0;
+}
 struct TilePeaks {
     BoardPeak a, b;
     bool two;   // the tile reaches a second board
@@ -154,11 +157,9 @@ struct TilePeaks {
         a.load(p, s.mb, lane);
         if (two) b.load(p, s.mb + 1, lane);
     }
-    __device__ __forceinline__ TileScales scales(const PatchStart& s) const {
+    __device__ __forceinline__ TileScales scales() const {
         const unsigned p0 = a.get(), p1 = two ? b.get() : p0;
-        // (a patch that begins on the board before has nothing but border there)
-        const bool whole = s.b0 == s.mb;
-        return {plane_scale(p0), plane_scale(whole ? p0 : p1), plane_unscale(p0), plane_unscale(p1)};
+        return {plane_scale(p0), plane_scale(p1), plane_unscale(p0), plane_unscale(p1)};
     }
 };
 // What a wavefront leaves in red[wavefront] and, after a barrier, the work-group in its slots.
@@ -242,10 +243,13 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     const PatchStart ps = patch_start(m0);
     TilePeaks tp;
     tp.load(peaks, ps, m0, MT, rows, lane);
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 4);
-    unsigned poff[NP];
-#pragma unroll
-    for (int i = 0; i < NP; i++) poff[i] = patch_offset<CELLS, PPC, NT>(i, ps, tid, Cp * 4);
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 4);
+    const unsigned xrow = (unsigned)Cp * 4u;     // bytes of a cell in memory
+    const unsigned xoff = (ps.q0 + tid / PPC) * xrow + (tid % PPC) * 16u;
+    // piece i, `at` bytes into the cells' channels
+    auto xload = [&](int i, unsigned at) {
+        return __builtin_amdgcn_raw_buffer_load_b128(rX, xoff, i * (NT / PPC) * xrow + at, 0);
+    };
     // LDS address of piece i: a constant distance from piece 0 (the last may lie past the end)
     const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 8u;
     TileScales ts;
@@ -254,27 +258,24 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
         const unsigned at = i < NP - 1 || (CELLS * PPC) % NT == 0
                                 ? lst + i * (NT / PPC) * STR
                                 : min(cell, (unsigned)CELLS) * STR + (tid % PPC) * 8u;
-        const unsigned y = ps.y0 + (__umul24(ps.x0 + cell, 3277u) >> 16);
-        store_split(lds + buffer + at, bits, y >= 20 ? ts.in1 : ts.in0);
+        store_split(lds + buffer + at, bits, cell < second_board(ps) ? ts.s0 : ts.s1);
     };
 
     const int chunks = Cp / kF32Chunk;
-    unsigned arow[RB];   // LDS address of this lane's point of each row block, tap (0, 0)
-#pragma unroll
-    for (int i = 0; i < RB; i++)
-        arow[i] = patch_cell(ps, min((wr * RB + i) * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
-                  (lane >> 4) * 16;
-
     const int ch0 = kb * 16 + 4 * (int)(lane >> 4);   // first channel
-    unsigned ro[RB];                                   // byte offset of this lane's point and channel
+    unsigned arow[RB];   // LDS address of this lane's point of each row block, tap (0, 0)
+    unsigned ro[RB];     // byte offset of this lane's point and channel
     int4v rr[RQ][NB];
 #pragma unroll
     for (int i = 0; i < RB; i++) {
-        const int m = m0 + (wr * RB + i) * 16 + (int)(lane & 15);
-        ro[i] = m < rows ? (unsigned)((m * Kp + ch0) * 4) : 0xfffff000u;
+        const int local = (wr * RB + i) * 16 + (int)(lane & 15);
+        const unsigned cell = patch_cell(ps, min(local, rows - 1 - m0));
+        arow[i] = cell * STR + (lane >> 4) * 16;
+        ro[i] = m0 + local < rows ? ((ps.q0 + kPointCell + cell) * Kp + ch0) * 4u : 0xfffff000u;
     }
-    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, (size_t)rows * Kp * 4);
-    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, (size_t)rows * Kp * 4);
+    const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 4;
+    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
+    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
     auto load_res = [&](int i) {
 #pragma unroll
         for (int j = 0; j < NB; j++)
@@ -290,10 +291,9 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     if constexpr (DB) {
         int4v stg[NP];
 #pragma unroll
-        for (int i = 0; i < NP; i++)
-            stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rX, poff[i], 0, 0);
+        for (int i = 0; i < NP; i++) stg[i] = xload(i, 0);
         if constexpr (EARLY) first_res();
-        ts = tp.scales(ps);
+        ts = tp.scales();
 #pragma unroll
         for (int i = 0; i < NP; i++) put(i, 0, stg[i]);
     } else {
@@ -301,11 +301,9 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
         int4v stg[FLY];
 #pragma unroll
         for (int p = 0; p < ALL + FLY; p++) {
-            if (p == FLY) ts = tp.scales(ps);
+            if (p == FLY) ts = tp.scales();
             if (p >= FLY) put((p - FLY) % NP, (p - FLY) / NP * BUF, stg[p % FLY]);
-            if (p < ALL)
-                stg[p % FLY] =
-                    __builtin_amdgcn_raw_buffer_load_b128(rX, poff[p % NP], p / NP * 128, 0);
+            if (p < ALL) stg[p % FLY] = xload(p % NP, p / NP * 128);
         }
         if constexpr (EARLY) first_res();
     }
@@ -351,8 +349,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
 #pragma unroll
                         for (int i = 0; i < SGRP; i++)
                             if (gr * SGRP + i < NP)
-                                sg[i] = __builtin_amdgcn_raw_buffer_load_b128(
-                                    rX, poff[gr * SGRP + i], next, 0);
+                                sg[i] = xload(gr * SGRP + i, next);
                     }
                     if (st == (gr + 1) * GS - 1) {
 #pragma unroll
@@ -405,7 +402,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
 #pragma unroll
     for (int i = 0; i < RB; i++) {
         const int m = m0 + (wr * RB + i) * 16 + (int)(lane & 15);
-        const float unscale = m < m1 ? -ts.out0 : -ts.out1;   // (the sum ends negated)
+        const float unscale = m < m1 ? -ts.u0 : -ts.u1;   // (the sum ends negated)
         float top = 0.0f;
 #pragma unroll
         for (int j = 0; j < NB; j++) {
@@ -537,31 +534,33 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     const PatchStart ps = patch_start(m0);
     TilePeaks tp;
     tp.load(peaks, ps, m0, MT, rows, lane);
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)rows * Cp * 4);
-    unsigned poff[NP];
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 4);
+    constexpr unsigned xrow = Cp * 4;   // bytes of a cell in memory
+    const unsigned xoff = (ps.q0 + lane / PPC) * xrow + (lane % PPC) * 16u;
+    auto xload = [&](int i, int h) {   // piece i of the wavefront's chunk h
+        return __builtin_amdgcn_raw_buffer_load_b128(
+            rX, xoff, i * (64 / PPC) * xrow + (wave * HPW + h) * 128, 0);
+    };
     int4v stg[NP];
-    const unsigned first = wave * (HPW * 128);   // bytes of a point before this wavefront's channels
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-        poff[i] = patch_offset<CELLS, PPC, 64>(i, ps, lane, Cp * 4);
-        stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rX, poff[i], first, 0);
-        if (i % 2) __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int i = 0; i < NP; i++) stg[i] = xload(i, 0);
     __builtin_amdgcn_sched_barrier(0);
     filters(F0, D - 1);
-    const TileScales ts = tp.scales(ps);
+    const TileScales ts = tp.scales();
 
     // the blocks that this wavefront finishes: where they lie, and the skip connection
     unsigned ro[QB];
     int4v rr[QB];
-    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, (size_t)rows * Kp * 4);
-    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, (size_t)rows * Kp * 4);
+    const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 4;
+    const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
+    const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
     const int cl = 4 * (int)(lane >> 4);   // first of this lane's 4 channels of a block
 #pragma unroll
     for (int q = 0; q < QB; q++) {
-        const int id = q * KW + wave, m = m0 + id / NB * 16 + (int)(lane & 15);
-        ro[q] = id < BLOCKS && m < rows
-                    ? (unsigned)((m * Kp + tn * CW + id % NB * 16 + cl) * 4) : 0xfffffff0u;
+        const int id = q * KW + wave, local = id / NB * 16 + (int)(lane & 15);
+        ro[q] = id < BLOCKS && m0 + local < rows
+                    ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + tn * CW + id % NB * 16 + cl) * 4u
+                    : 0xfffffff0u;
         rr[q] = int4v{0, 0, 0, 0};
     }
     if (res != nullptr) {
@@ -574,16 +573,14 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
 #pragma unroll
         for (int i = 0; i < NP; i++) {
             const unsigned cell = lane / PPC + i * (64 / PPC);
-            const unsigned y = ps.y0 + (__umul24(ps.x0 + cell, 3277u) >> 16);
             store_split(own + (i < NP - 1 ? cell : min(cell, (unsigned)CELLS)) * STR + lane % PPC * 8u,
-                        stg[i], y >= 20 ? ts.in1 : ts.in0);
+                        stg[i], cell < second_board(ps) ? ts.s0 : ts.s1);
         }
     };
     stage();
     if constexpr (HPW > 1) {
 #pragma unroll
-        for (int i = 0; i < NP; i++)
-            stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rX, poff[i], first + 128, 0);
+        for (int i = 0; i < NP; i++) stg[i] = xload(i, 1);
         __builtin_amdgcn_sched_barrier(0);
     }
     if (tid < (unsigned)CW) {
@@ -666,7 +663,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
             part[k] = *reinterpret_cast<const float4v*>(lds + (k * BLOCKS + id) * 1024 + lane * 16);
         const float4v r = __builtin_bit_cast(float4v, rr[q]);
         const int m = m0 + id / NB * 16 + (int)(lane & 15), c = id % NB * 16 + cl;
-        const float unscale = m < m1 ? ts.out0 : ts.out1;
+        const float unscale = m < m1 ? ts.u0 : ts.u1;
         float top = 0.0f;
         float4v o;
 #pragma unroll

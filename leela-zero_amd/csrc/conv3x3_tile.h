@@ -9,68 +9,44 @@ typedef int int2v __attribute__((ext_vector_type(2)));
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------------------
-// Geometry.  Row m of the implicit GEMM is point (b, y, x) of the batch.  In LDS the planes
-// stand with a zero border: cell q(m) = 400 b + 20 (y + 1) + x, one zero column between board
-// rows (right border of one row and left border of the next) and one zero row between
-// boards.  A tap (r, s) is then the constant offset 20 (r - 1) + (s - 1), without bounds logic.
-constexpr int kCellsPerBoard = 400;
+// Geometry.  Row m of the implicit GEMM is point (b, y, x) of the batch.  The planes stand with a zero
+// border, in memory (kernels.h: padded planes) as in LDS: point (b, y, x) is cell 400 (b + 1) + 20 (y + 1) + x,
+// with one zero column between board rows (right border of one row and left border of the next) and
+// one zero row between boards.  A tap (r, s) is then the constant offset 20 (r - 1) + (s - 1), without
+// bounds logic, and the patch of a tile is one run of consecutive cells: every piece that a
+// thread fetches lies a constant distance from its first.  (With dense planes in memory and the border
+// made on the way to LDS an address took some 25 instructions, and up to 13 of them per thread came
+// before the first load: 10x128 fp16 batch 5, 86.8 -> 82.8 us a forward, 15x192 batch 8, 218 -> 209,
+// 20x256 batch 32, 676 -> 664; fp32, with more pieces, 6x128 batch 1, 83 -> 75.)
+constexpr int kCellsPerBoard = kPadCells;
+constexpr int kRowCells = 20;
 // Cells that a tile of mt consecutive rows can reach: its own span (a cell more per board
 // row ended, 20 more per board ended) and 21 on either side.
 constexpr int conv_cells(int mt) {
-    return mt - 1 + (mt - 1 + 18) / 19 + 20 * ((mt - 1 + 360) / 361) + 43;
-}
-__device__ __forceinline__ unsigned conv_cell(unsigned m) {
-    const unsigned b = m / kPts, p = m - b * kPts, y = p / kBoard, x = p - y * kBoard;
-    return b * kCellsPerBoard + (y + 1) * 20 + x;
+    return mt - 1 + (mt - 1 + 18) / 19 + kRowCells * ((mt - 1 + 360) / 361) + 2 * (kRowCells + 1) + 1;
 }
 
-// The patch of a tile (the cells that its points reach) and what lies where in it.  Where it
-// begins is worked out once, in scalar registers; from there on every cell is less than 400 away
-// and every division is a 24-bit multiplication and a shift.  (With full divisions by 400, 20,
-// 361 and 19 and a branch for every kind of border a work-group spent 1400 to 4200 cycles, up to
-// a third of its life, before its first load; so 1000 to 1900.)
+// The patch of a tile: the cells that its points reach.
 struct PatchStart {
-    unsigned q0, b0, y0, x0;   // first cell, one board on (stays positive), and its parts
-    unsigned mb, mp;           // board and point of the tile's first row
+    unsigned q0;       // first cell: the upper left tap of the tile's first row
+    unsigned mb, mp;   // board and point of the tile's first row
 };
 __device__ __forceinline__ PatchStart patch_start(unsigned m0) {
     PatchStart s;
-    s.q0 = conv_cell(m0) + kCellsPerBoard - 21;
-    s.b0 = s.q0 / kCellsPerBoard;
-    s.y0 = (s.q0 - s.b0 * kCellsPerBoard) / 20;
-    s.x0 = s.q0 - s.b0 * kCellsPerBoard - s.y0 * 20;
     s.mb = m0 / kPts;
     s.mp = m0 - s.mb * kPts;
+    s.q0 = (s.mb + 1) * kCellsPerBoard + s.mp + s.mp / kBoard - 1;
     return s;
 }
-// Cell of the patch in which the upper left tap of the tile's row `local` lies.
+// Cell of the patch in which the upper left tap of the tile's row `local` lies; the point itself is
+// kPointCell further on.
+constexpr unsigned kPointCell = kRowCells + 1;
 __device__ __forceinline__ unsigned patch_cell(const PatchStart& s, unsigned local) {
     unsigned p = s.mp + local;
     const unsigned next = p >= kPts ? 1u : 0u;
     p -= next * kPts;
     const unsigned y = __umul24(p, 3450u) >> 16;   // p / 19
-    return (s.mb + next) * kCellsPerBoard + 20 + p + y + kCellsPerBoard - 21 - s.q0;
-}
-// Byte offset in X (row_bytes a point) of a thread's 16-byte piece i (PPC to a cell); cells off the board and boards
-// outside the batch get an offset outside the buffer and read as zero.
-template <int CELLS, int PPC, int NT>
-__device__ __forceinline__ unsigned patch_offset(int i, const PatchStart& s, unsigned tid,
-                                                 unsigned row_bytes) {
-    static_assert(CELLS <= 380 && (PPC != 24 || CELLS * PPC + NT < 8200), "small divisions");
-    const unsigned piece = tid + i * NT;
-    const unsigned cell = PPC == 24 ? __umul24(piece, 2731u) >> 16 : piece / PPC;
-    const unsigned part = piece - cell * PPC;
-    const unsigned t = s.x0 + cell, dy = __umul24(t, 3277u) >> 16;   // t / 20
-    const unsigned x = t - dy * 20, y = s.y0 + dy;                   // y >= 20: the next board
-    // t - dy = 19 dy + x, in points of the board's rows; row y1 = 0 of the board before is kept
-    // positive by `lead`
-    const unsigned lead = (kPts + kBoard) * row_bytes;
-    const unsigned pt = s.b0 * kPts + s.y0 * kBoard + t - dy - (y >= 20 ? 19u : 0u);
-    unsigned off = __umul24(pt, row_bytes) + part * 16u - lead;
-    asm volatile("" : "+v"(off));   // keeps the compiler from branching around it
-    const unsigned bad = (unsigned)(cell >= (unsigned)CELLS) | (unsigned)(x == 19) |
-                         (unsigned)(y == 0) | (unsigned)(y == 20);
-    return off | (0u - bad);
+    return (s.mb + 1 + next) * kCellsPerBoard + p + y - 1 - s.q0;
 }
 
 // LDS is what a work-group shares: its writes are waited for, loads from memory stay in flight

@@ -185,8 +185,9 @@ public:
         }
         for (int i = 0; i < m_n_lanes; i++) {
             Lane& ln = m_lane[i];
-            ln.act0.alloc(B * kPts * m_C0p);
-            for (auto& a : ln.act) a.alloc(B * kPts * m_Fp);
+            // (padded planes of a direct tower; the dense ones of another take less)
+            ln.act0.alloc(padded_cells(max_batch) * m_C0p);
+            for (auto& a : ln.act) a.alloc(padded_cells(max_batch) * m_Fp);
         }
         if (const char* e = std::getenv("LZHIP_INPLACE"))   // measurement knob
             m_in_place = std::atoi(e) != 0;
@@ -377,7 +378,14 @@ public:
                 L.W3.release();
                 L.peak.clear();
             }
-        else if (sizeof(P) == 4)
+        else
+            // the planes' borders are zero, whatever a push that failed has left there
+            for (int i = 0; i < m_n_lanes; i++) {
+                Lane& ln = m_lane[i];
+                HIP_CHECK(hipMemset(ln.act0.p, 0, ln.act0.count * sizeof(P)));
+                for (auto& a : ln.act) HIP_CHECK(hipMemset(a.p, 0, a.count * sizeof(P)));
+            }
+        if (good && sizeof(P) == 4)
             for (int i = 0; i < m_n_lanes; i++)
                 m_lane[i].peaks.alloc(2 * conv3x3_f32_slots(m_Fp, m_max_batch) + 2 * (size_t)m_max_batch);
         return good;
@@ -419,9 +427,10 @@ public:
     // handles or threads of this process run one after the other on the device.  While
     // the stream is being captured into a graph no event is recorded or waited for (the
     // captured launches are then ordered by the graph's own dependencies, and replays
-    // that overlap with other users of the array race).  Nothing in the array has to
-    // start at zero: every element a kernel reads for a real tile is written earlier in
-    // the same call (rows of V past the last tile feed only rows of M that no kernel reads).
+    // that overlap with other users of the array race).  The borders of a direct tower's planes are
+    // cleared by each call (another handle's may lie elsewhere); nothing else has to start at
+    // zero: every element a kernel reads for a real tile is written earlier in the same call (rows
+    // of V past the last tile feed only rows of M that no kernel reads).
     void forward_device_static(int n, const float* d_in, float* d_pol, float* d_val) override {
         Lane& ln = m_lane[0];
         std::lock_guard<std::mutex> lk(ln.mu);
@@ -439,22 +448,37 @@ public:
         Work w;
         w.stream = ln.stream;
         w.Tp = kStaticTp;
-        w.V = reinterpret_cast<P*>(base);
-        w.M = reinterpret_cast<P*>(base + kStaticTileBytes);
-        // (a direct tower has no tiles: the peaks of its layers take their place)
-        w.peaks = m_direct && sizeof(P) == 4 ? reinterpret_cast<uint32_t*>(base) : nullptr;
-        if (w.peaks && peak_words(n) * sizeof(uint32_t) > 2 * kStaticTileBytes)
-            throw std::invalid_argument("no room for the peaks");
-        w.act0 = reinterpret_cast<P*>(base + 2 * kStaticTileBytes);
-        for (int i = 0; i < 3; i++)
-            w.act[i] = reinterpret_cast<P*>(base + 2 * kStaticTileBytes + kStaticAct0Bytes +
-                                            (size_t)i * kStaticActBytes);
+        size_t clear = 0;
+        if (m_direct) {
+            // a direct tower has no tiles: its planes, padded and one after the other, are all
+            // there is, and in fp32 the peaks behind them
+            const size_t cells = padded_cells(n) * sizeof(P);
+            w.act0 = reinterpret_cast<P*>(base);
+            for (int i = 0; i < 3; i++)
+                w.act[i] = reinterpret_cast<P*>(base + cells * (m_C0p + i * m_Fp));
+            clear = cells * (m_C0p + 3 * m_Fp);
+            size_t need = clear;
+            if (sizeof(P) == 4) {
+                w.peaks = reinterpret_cast<uint32_t*>(base + clear);
+                need += peak_words(n) * sizeof(uint32_t);
+            }
+            if (need > kStaticBytes)
+                throw std::invalid_argument("no room in the static working memory");
+        } else {
+            w.V = reinterpret_cast<P*>(base);
+            w.M = reinterpret_cast<P*>(base + kStaticTileBytes);
+            w.act0 = reinterpret_cast<P*>(base + 2 * kStaticTileBytes);
+            for (int i = 0; i < 3; i++)
+                w.act[i] = reinterpret_cast<P*>(base + 2 * kStaticTileBytes + kStaticAct0Bytes +
+                                                (size_t)i * kStaticActBytes);
+        }
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         HIP_CHECK(hipStreamIsCapturing(ln.stream, &cap));
         const bool ordered = cap == hipStreamCaptureStatusNone;
         std::lock_guard<std::mutex> order(g_scratch_order_mu);
         hipEvent_t ev = g_scratch_event[m_device];
         if (ordered) HIP_CHECK(hipStreamWaitEvent(ln.stream, ev, 0));
+        if (clear) launch_clear(base, clear, ln.stream);
         enqueue_forward(w, n, d_in, nullptr, d_pol, d_val, false);
         HIP_CHECK(hipGetLastError());
         if (ordered) HIP_CHECK(hipEventRecord(ev, ln.stream));
@@ -710,12 +734,12 @@ public:
                 launch_pack_input_peaks(d_planes.p, a_in, n, C, Cp, peaks.slots, ln.stream, nullptr);
         }
         if (sizeof(P) == 2 || !m_direct)
-            launch_pack_input<P>(d_planes.p, a_in, n, C, Cp, ln.stream, nullptr);
+            launch_pack_input<P>(d_planes.p, a_in, m_direct, n, C, Cp, ln.stream, nullptr);
         const P* r = nullptr;
         if (res) {
             d_res.alloc((size_t)n * F * kPts);
             HIP_CHECK(hipMemcpy(d_res.p, res, sizeof(float) * (size_t)n * F * kPts, hipMemcpyHostToDevice));
-            launch_pack_input<P>(d_res.p, ln.act[1].p, n, F, m_Fp, ln.stream, nullptr);
+            launch_pack_input<P>(d_res.p, ln.act[1].p, m_direct, n, F, m_Fp, ln.stream, nullptr);
             r = ln.act[1].p;
         }
         std::vector<float> sc(m_Fp, 0.0f), mn(m_Fp, 0.0f);
@@ -746,7 +770,14 @@ public:
             d_M.alloc((size_t)kPos * m_Tp * m_Fp);
             V = d_V.p; M = d_M.p; U = d_U.p; Uf = nullptr;
         }
-        launch_in_transform<P>(a_in, V, n, Cp, m_Tp, ln.stream, nullptr);
+        const P* dense = a_in;   // (V is computed from dense planes)
+        DevBuf<P> d_dense;
+        if (m_direct) {
+            d_dense.alloc((size_t)n * kPts * Cp);
+            launch_pack_input<P>(d_planes.p, d_dense.p, false, n, C, Cp, ln.stream, nullptr);
+            dense = d_dense.p;
+        }
+        launch_in_transform<P>(dense, V, n, Cp, m_Tp, ln.stream, nullptr);
         launch_gemm<P>(V, U, Uf, M, Tu, m_Tp, Cp, m_Fp, ln.stream, nullptr);
         if (m_direct)
             conv_direct(L, a_in, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, peaks,
@@ -776,13 +807,13 @@ public:
                             (float)h[((size_t)p * m_Tp + t) * m_Fp + k];
         }
         if (Yout) {
-            std::vector<P> h((size_t)n * kPts * m_Fp);
+            std::vector<P> h((m_direct ? padded_cells(n) : (size_t)n * kPts) * m_Fp);
             HIP_CHECK(hipMemcpy(h.data(), ln.act[2].p, h.size() * sizeof(P), hipMemcpyDeviceToHost));
             for (int b = 0; b < n; b++)
                 for (int pt = 0; pt < kPts; pt++)
                     for (int k = 0; k < F; k++)
                         Yout[((size_t)b * F + k) * kPts + pt] =
-                            (float)h[((size_t)b * kPts + pt) * m_Fp + k];
+                            (float)h[plane_index(m_direct, b, pt) * m_Fp + k];
         }
     }
 
@@ -962,9 +993,9 @@ private:
         const int Tu = n * kTilesPerBoard;
         LaunchTimer* pack = timer(timed, LZHIP_K_PACK);
         if (!d_in)
-            launch_pack_input_bits<P>(d_bits, w.act0, n, kInPlanes, m_C0p, w.peaks, w.stream, pack);
+            launch_pack_input_bits<P>(d_bits, w.act0, m_direct, n, kInPlanes, m_C0p, w.peaks, w.stream, pack);
         else if (!pack_with_peaks(w, d_in, n, pack))
-            launch_pack_input<P>(d_in, w.act0, n, kInPlanes, m_C0p, w.stream, pack);
+            launch_pack_input<P>(d_in, w.act0, m_direct, n, kInPlanes, m_C0p, w.stream, pack);
         if (m_direct) {
             enqueue_direct(w, n, d_pol, d_val, timed);
             return;
@@ -989,7 +1020,7 @@ private:
             if (l == nl - 1) {
                 launch_out_transform<P>(tiles, res, out, L.d_scale.p, L.d_mean.p, L.rfac, n, m_Fp,
                                         w.Tp, w.stream, timer(timed, LZHIP_K_OUT));
-                launch_head_conv<P>(out, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
+                launch_head_conv<P>(out, false, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
                                     timer(timed, LZHIP_K_HEAD));
             } else {
                 Layer& N = m_layers[l + 1];
@@ -1046,7 +1077,7 @@ private:
             last = out;
             if (second) { const int o = cur; cur = nxt; nxt = o; }
         }
-        launch_head_conv<P>(last, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
+        launch_head_conv<P>(last, true, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
                             timer(timed, LZHIP_K_HEAD));
     }
 
@@ -1088,11 +1119,11 @@ private:
             for (int pt = 0; pt < kPts; pt++) x[16 * kPts + pt] = 1.0f;
         }
         HIP_CHECK(hipMemcpy(m_din.p, in.data(), in.size() * sizeof(float), hipMemcpyHostToDevice));
-        launch_pack_input<P>(m_din.p, ln.act0.p, n, kInPlanes, m_C0p, ln.stream, nullptr);
+        launch_pack_input<P>(m_din.p, ln.act0.p, m_direct, n, kInPlanes, m_C0p, ln.stream, nullptr);
 
         const float target = 16.0f;
         const int nl = (int)m_layers.size();
-        const size_t cnt = (size_t)n * kPts * m_Fp;
+        const size_t cnt = (m_direct ? padded_cells(n) : (size_t)n * kPts) * m_Fp;
         int cur = 0, mid = 1, nxt = 2;
         auto settle = [&](int l, const P* src, const P* res, P* dst) {
             // provisional: keep the incoming scale, then correct from the measured range

@@ -1,7 +1,9 @@
 // Launch interface of the gfx950 kernels of the residual tower.
 //
 // Device data layouts (P = storage type: float or _Float16):
-//   act  [n][361][Cp]        activations, channels fastest ("channels-last")
+//   act  [n][361][Cp]        activations, channels fastest ("channels-last"); for direct
+//                            convolutions padded: [n + 2][400][Cp], point (y, x) of board b at
+//                            cell 400 (b + 1) + 20 (y + 1) + x, every other cell zero
 //   V    [36][Tp][Cp]        Winograd-domain input tiles, t = board*25 + by*5 + bx
 //   U    [36][Kp][Cp]        Winograd-domain filters, input channel fastest
 //   M    [36][Tp][Kp]        per-position GEMM results, output channel fastest
@@ -17,6 +19,7 @@ namespace lzhip {
 
 constexpr int kBoard = 19;
 constexpr int kPts = 361;
+constexpr int kPadCells = 400;   // cells of a board in padded planes
 constexpr int kTilesPerBoard = 25;
 constexpr int kPos = 36;       // 6x6 Winograd positions
 constexpr int kInPlanes = 18;
@@ -32,6 +35,14 @@ struct LaunchTimer {
     hipEvent_t start = nullptr, stop = nullptr;
 };
 
+// Index of point pt of board b: cell of padded planes, or point of dense ones.
+__host__ __device__ static inline size_t plane_index(bool padded, int b, int pt) {
+    return padded ? (size_t)(b + 1) * kPadCells + pt + pt / kBoard + 20 : (size_t)b * kPts + pt;
+}
+static inline size_t padded_cells(int n) { return (size_t)(n + 2) * kPadCells; }
+// Clears device memory (a multiple of 16 bytes) by a kernel.
+void launch_clear(void* p, size_t bytes, hipStream_t s);
+
 // NCHW fp32 planes [n][C][361] -> act [n][361][Cp] (channels >= C zero).
 // 32-bit words of one position's 18 x 361 input planes packed one bit per value.
 constexpr int kInputWords = (18 * 361 + 31) / 32;
@@ -45,12 +56,12 @@ struct PeakMap {
 };
 // (peaks: null, or 2 n slots of input planes, one tile a board)
 template <typename P>
-void launch_pack_input_bits(const uint32_t* bits, P* act, int n, int C, int Cp, uint32_t* peaks,
-                            hipStream_t s, LaunchTimer* t);
+void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, int C, int Cp,
+                            uint32_t* peaks, hipStream_t s, LaunchTimer* t);
 template <typename P>
-void launch_pack_input(const float* in, P* act, int n, int C, int Cp, hipStream_t s,
+void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int Cp, hipStream_t s,
                        LaunchTimer* t);
-// The same with the peaks.
+// The same with the peaks; padded.
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
                              hipStream_t s, LaunchTimer* t);
 
@@ -95,7 +106,7 @@ void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const 
                              hipStream_t s, LaunchTimer* t);
 
 // Direct 3x3 convolution in fp16 (conv3x3.hip), one launch per layer:
-// X [n][361][Cp] -> Y [n][361][Kp] = min(max(0, scale*(conv - mean) + rfac*res), kActStoreMax);
+// X [Cp] -> Y [Kp] = min(max(0, scale*(conv - mean) + rfac*res), kActStoreMax), padded planes all three;
 // res may be null and is not Y.  Wf: conv3x3_filter_count elements, zero but for what
 // conv3x3_filters writes.
 // Whether a handle for batches of up to max_batch computes by it (measured; see there).
@@ -119,7 +130,7 @@ void conv3x3_filters(const float* U, _Float16* Wf, int C, int F, int Kp, int* ba
 void conv3x3_winograd_filters(const _Float16* Wf, int C, int Cp, int F, int Kp, _Float16* U);
 
 // Direct 3x3 convolution of fp32 towers (conv3x3_f32.hip), one launch per layer:
-// X [n][361][Cp] -> Y [n][361][Kp] = max(0, scale*(conv - mean) + rfac*res) in fp32, every operand split in
+// X [Cp] -> Y [Kp] = max(0, scale*(conv - mean) + rfac*res) in fp32, padded planes, every operand split in
 // two half-precision numbers.  Wf holds the filters of output channel k times 2^e(k):
 // conv3x3_f32_unscale(peak[k]) = 2^-e(k) belongs into scale, 2^e(k) into mean.  peaks: of X; those of Y
 // go to `slots` (conv3x3_f32_slots words) and are returned.
@@ -146,8 +157,8 @@ void conv3x3_f32_winograd_filters(const _Float16* Wf, const uint32_t* peak, int 
 // 1x1 head convolutions: act [n][361][Cp] x w[3][Cp] -> pol [n][2][361], val [n][361],
 // both multiplied by out_scale.
 template <typename P>
-void launch_head_conv(const P* act, const float* w3, float out_scale, float* pol, float* val,
-                      int n, int Cp, hipStream_t s, LaunchTimer* t);
+void launch_head_conv(const P* act, bool padded, const float* w3, float out_scale, float* pol,
+                      float* val, int n, int Cp, hipStream_t s, LaunchTimer* t);
 
 // max |x| over count elements -> *out (float, must be zeroed before).
 template <typename P>

@@ -100,7 +100,8 @@ __device__ __forceinline__ void at6(const float i0, const float i1, const float 
 // channels C..Cp-1 zero.
 template <typename P>
 __global__ __launch_bounds__(256) void pack_input_k(const float* __restrict__ in,
-                                                    P* __restrict__ act, int n, int C, int Cp) {
+                                                    P* __restrict__ act, bool padded, int n, int C,
+                                                    int Cp) {
     const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t total = (size_t)n * kPts * Cp;
     if (gid >= total) return;
@@ -110,23 +111,23 @@ __global__ __launch_bounds__(256) void pack_input_k(const float* __restrict__ in
     const size_t b = bp / kPts;
     float v = 0.0f;
     if (c < C) v = in[(b * C + c) * kPts + pt];
-    act[gid] = to_storage<P>(v);
+    act[plane_index(padded, (int)b, pt) * Cp + c] = to_storage<P>(v);
 }
 
 template <typename P>
-void launch_pack_input(const float* in, P* act, int n, int C, int Cp, hipStream_t s,
+void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int Cp, hipStream_t s,
                        LaunchTimer* t) {
     const size_t total = (size_t)n * kPts * Cp;
-    launch(pack_input_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, in, act, n, C,
-           Cp);
+    launch(pack_input_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, in, act,
+           padded, n, C, Cp);
 }
 
 // The same from bit-packed planes: bit (c*361 + pt) of a board's kInputWords words is
 // plane c at point pt (planes that hold only 0 and 1, which is what the engine feeds).
 template <typename P>
 __global__ __launch_bounds__(256) void pack_input_bits_k(const uint32_t* __restrict__ bits,
-                                                         P* __restrict__ act, int n, int C,
-                                                         int Cp, uint32_t* __restrict__ peaks) {
+                                                         P* __restrict__ act, bool padded, int n,
+                                                         int C, int Cp, uint32_t* __restrict__ peaks) {
     const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t total = (size_t)n * kPts * Cp;
     if (gid >= total) return;
@@ -140,15 +141,15 @@ __global__ __launch_bounds__(256) void pack_input_bits_k(const uint32_t* __restr
         const int bit = c * kPts + pt;
         v = (float)((bits[b * kInputWords + (bit >> 5)] >> (bit & 31)) & 1u);
     }
-    act[gid] = to_storage<P>(v);
+    act[plane_index(padded, (int)b, pt) * Cp + c] = to_storage<P>(v);
 }
 
 template <typename P>
-void launch_pack_input_bits(const uint32_t* bits, P* act, int n, int C, int Cp, uint32_t* peaks,
-                            hipStream_t s, LaunchTimer* t) {
+void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, int C, int Cp,
+                            uint32_t* peaks, hipStream_t s, LaunchTimer* t) {
     const size_t total = (size_t)n * kPts * Cp;
     launch(pack_input_bits_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, bits, act,
-           n, C, Cp, peaks);
+           padded, n, C, Cp, peaks);
 }
 
 // Planes and peaks from float planes: one work-group per board reads all of it (26 KB); the packing
@@ -168,10 +169,9 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
         }
     }
     const int from = part * kPts / kPackParts, to = (part + 1) * kPts / kPackParts;
-    float* out = act + (size_t)b * kPts * Cp;
     for (int i = tid; i < (to - from) * Cp; i += 512) {
         const int pt = from + i / Cp, c = i % Cp;
-        out[(size_t)pt * Cp + c] = c < C ? planes[(size_t)c * kPts + pt] : 0.0f;
+        act[plane_index(true, b, pt) * Cp + c] = c < C ? planes[(size_t)c * kPts + pt] : 0.0f;
     }
     if (part != 0) return;
     __shared__ float tops[8];
@@ -188,6 +188,16 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
                              hipStream_t s, LaunchTimer* t) {
     launch(pack_input_peaks_k, dim3(n, kPackParts), dim3(512), s, t, in, act, C, Cp, peaks);
+}
+
+__global__ __launch_bounds__(256) void clear_k(int4v* p, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
+        p[i] = int4v{0, 0, 0, 0};
+}
+void launch_clear(void* p, size_t bytes, hipStream_t s) {
+    const size_t n = bytes / 16;
+    hipLaunchKernelGGL(clear_k, dim3((unsigned)(n < 256 * 1024 ? (n + 255) / 256 : 1024)), dim3(256), 0, s,
+                       (int4v*)p, n);
 }
 
 // ---------------------------------------------------------------------------
@@ -1816,7 +1826,7 @@ void launch_gemm(const P* V, const P* U, const P* Uf, P* M, int T, int Tp, int C
 // last activation (reference src/CPUPipe.cpp:424-427).  One wavefront per
 // board point; lanes stride over channels, then a butterfly reduction.
 template <typename P>
-__global__ __launch_bounds__(256) void head_conv_k(const P* __restrict__ act,
+__global__ __launch_bounds__(256) void head_conv_k(const P* __restrict__ act, bool padded,
                                                    const float* __restrict__ w3,
                                                    float out_scale, float* __restrict__ pol,
                                                    float* __restrict__ val, int n, int Cp) {
@@ -1824,7 +1834,7 @@ __global__ __launch_bounds__(256) void head_conv_k(const P* __restrict__ act,
     const int lane = threadIdx.x & 63;
     if (gw >= n * kPts) return;
     const int b = gw / kPts, pt = gw - b * kPts;
-    const P* a = act + (size_t)gw * Cp;
+    const P* a = act + plane_index(padded, b, pt) * Cp;
     float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
     for (int c = lane; c < Cp; c += 64) {
         const float x = (float)a[c];
@@ -1846,11 +1856,11 @@ __global__ __launch_bounds__(256) void head_conv_k(const P* __restrict__ act,
 }
 
 template <typename P>
-void launch_head_conv(const P* act, const float* w3, float out_scale, float* pol, float* val,
-                      int n, int Cp, hipStream_t s, LaunchTimer* t) {
+void launch_head_conv(const P* act, bool padded, const float* w3, float out_scale, float* pol,
+                      float* val, int n, int Cp, hipStream_t s, LaunchTimer* t) {
     const int waves = n * kPts;
-    launch(head_conv_k<P>, dim3((waves + 3) / 4), dim3(256), s, t, act, w3, out_scale, pol, val,
-           n, Cp);
+    launch(head_conv_k<P>, dim3((waves + 3) / 4), dim3(256), s, t, act, padded, w3, out_scale,
+           pol, val, n, Cp);
 }
 
 // ---------------------------------------------------------------------------
@@ -2083,10 +2093,10 @@ void launch_heads(const float* pol, const float* val, HeadParams hp, float tempe
 
 // ---------------------------------------------------------------------------
 #define INSTANTIATE(P)                                                                         \
-    template void launch_pack_input<P>(const float*, P*, int, int, int, hipStream_t,           \
+    template void launch_pack_input<P>(const float*, P*, bool, int, int, int, hipStream_t,     \
                                        LaunchTimer*);                                          \
-    template void launch_pack_input_bits<P>(const uint32_t*, P*, int, int, int, uint32_t*,     \
-                                            hipStream_t, LaunchTimer*);                        \
+    template void launch_pack_input_bits<P>(const uint32_t*, P*, bool, int, int, int,          \
+                                            uint32_t*, hipStream_t, LaunchTimer*);             \
     template void launch_in_transform<P>(const P*, P*, int, int, int, hipStream_t,             \
                                          LaunchTimer*);                                        \
     template void launch_gemm<P>(const P*, const P*, const P*, P*, int, int, int, int,         \
@@ -2096,8 +2106,8 @@ void launch_heads(const float* pol, const float* val, HeadParams hp, float tempe
     template void launch_out_in_transform<P>(const P*, const P*, P*, P*, const float*,         \
                                              const float*, float, int, int, int, hipStream_t,  \
                                              LaunchTimer*);                                    \
-    template void launch_head_conv<P>(const P*, const float*, float, float*, float*, int, int, \
-                                      hipStream_t, LaunchTimer*);                              \
+    template void launch_head_conv<P>(const P*, bool, const float*, float, float*, float*,     \
+                                      int, int, hipStream_t, LaunchTimer*);                    \
     template void launch_absmax<P>(const P*, size_t, float*, hipStream_t);
 INSTANTIATE(float)
 INSTANTIATE(half_t)
