@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
 #pragma unroll
     for (int h = 0; h < HPW; h++) {
         if (h > 0) stage();
-        if (h > 0 && (wave * HPW + h) * 2 == KW * HPW) {   // an odd number of wavefronts: the middle one
+        if (h > 0 && (wave * HPW + h) * 2 == KW * HPW) {   // KW is odd: the middle one
 #pragma unroll
             for (int i = 0; i < RB; i++)
 #pragma unroll
@@ -682,15 +682,24 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     leave_peaks<KW>(red, slots, tm, tn, Kp / CW, wave, top0, top1);
 }
 
-// The tile: blocks of 16 points and of 16 channels; points 0 if no tile makes at most one
-// work-group per unit.
+// The tile, in blocks of 16 points and of 16 channels: the smallest that makes at most one work-group per
+// unit; points 0 if none does.  The tiles of 64 channels are where conv3x3_f32_k's of the same size are
+// bound by the L1 (each of its wavefronts fetches every other one's filters or planes too).  Measured
+// per forward of 4 blocks, conv3x3_f32_k -> 48x64 or 64x64 here, us (one forward at a time | two side by
+// side): 128 filters, 12 boards 116 -> 86 | 134 -> 105, 22: 116 -> 93 | 148 -> 126; 192 filters, 8: 140 -> 103 |
+// 169 -> 147, 15: 143 -> 128 | 194 -> 199; 256 filters, 6: 175 -> 114 | 210 -> 160, 11: 176 -> 132 | 235 -> 227;
+// 320 filters, 6: 201 -> 152 | 254 -> 252; 384 filters, 4: 231 -> 150 | 293 -> 222; 512 filters, 4: 293 -> 179 |
+// 385 -> 320.  Left out: 64x64 for 64 filters, whose two wavefronts leave half a unit idle (40 boards 87 ->
+// 96), and above 256, where the registers do not hold it (320 filters, 8 boards 199 -> 245); 96x64 (256
+// filters, 16 boards 191 -> 193 | 299 -> 324).
 struct SplitTile {
     int rb, nb;
 };
 static SplitTile f32_split_tile(int n, int Kp) {
-    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}};
+    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}, {3, 4}, {4, 4}};
     for (const SplitTile& t : kTiles)
-        if ((n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
+        if ((t.rb * t.nb < 16 || (Kp >= 128 && Kp <= 256)) &&
+            (n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
     return {0, 0};
 }
 
@@ -713,7 +722,10 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
     };
     // KW wavefronts x HPW chunks
 #define LZ_SPLIT(KW, HPW, D)                                                                  \
-    if (tile.nb == 1) {                                                                       \
+    if (tile.nb == 4) {                                                                       \
+        if (tile.rb == 3) go(conv3x3_f32_split_k<3, 4, KW, HPW, (HPW == 2 ? 3 : 5)>, KW);     \
+        else if constexpr (HPW == 1) go(conv3x3_f32_split_k<4, 4, KW, HPW, 4>, KW);           \
+    } else if (tile.nb == 1) {                                                                \
         if (tile.rb == 2) go(conv3x3_f32_split_k<2, 1, KW, HPW, D>, KW);                      \
         else go(conv3x3_f32_split_k<3, 1, KW, HPW, D>, KW);                                   \
     } else if (tile.rb == 2) go(conv3x3_f32_split_k<2, 2, KW, HPW, D>, KW);                   \

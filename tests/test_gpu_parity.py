@@ -910,6 +910,10 @@ def test_winograd_filters_of_no_3x3_filter(pkg, netgen, orc):
     (64, 45, (1, 22, 23, 33, 34, 45)), (128, 11, (1, 5, 6, 8, 9, 11)), (192, 7, (1, 2, 3, 5, 6, 7)),
     (256, 5, (1, 2, 3, 4, 5)), (320, 4, (1, 2, 3, 4)), (384, 3, (1, 2, 3)), (448, 3, (1, 2, 3)),
     (512, 2, (1, 2)),
+    # ... and of 64 channels
+    (64, 34, (24, 34)), (128, 22, (11, 12, 17, 18, 22)), (192, 15, (7, 8, 11, 12, 15)),
+    (256, 11, (5, 6, 8, 9, 11)), (320, 6, (4, 5, 6)), (384, 5, (3, 4, 5)), (448, 4, (3, 4)),
+    (512, 4, (3, 4)),
     # the other tiles on both sides of every change
     (64, 137, (1, 22, 23, 34, 68, 69, 136, 137)), (128, 70, (1, 11, 12, 17, 34, 35, 68, 69, 70)),
     (192, 46, (1, 7, 8, 11, 22, 23, 45, 46)), (256, 36, (1, 5, 6, 8, 9, 17, 34, 35, 36)),
