@@ -54,11 +54,9 @@ size_t conv3x3_filter_count(int Cp, int Kp) {
 // instructions of 16 cycles, 256 / NB of its 128 bytes per cycle, against 256 / RB of the 64 that
 // the L1 delivers.  RB = 6, NB = 4 (50 % of one, 67 % of the other) is the tile for full
 // batches.  The planes pass through LDS because every value is used nine times: the cells a
-// tile reaches are staged once per chunk of input channels, in rows padded to an odd number
-// of 16-byte pieces, and the nine taps and two halves are immediate offsets of one address per 16
-// points.  The padding does not keep the fragment reads free of bank conflicts: counted at 64
-// boards of 256 filters, the LDS is busy for 42 % of a launch, conflicts are 24 %, and the matrix
-// pipes are busy for 57 % of it (32 boards: 61, 35 and 42 %).
+// tile reaches are staged once per chunk of input channels, in an order that the fragment reads
+// take without bank conflicts (CellPitch), and the nine taps and two halves are immediate offsets of
+// one address per 16 points.
 //
 // CC == 0: chunks of 64 input channels in two LDS buffers; the next chunk's pieces are loaded
 // and stored in small groups between the matrix instructions (SGRP at a time: kept whole they
@@ -79,7 +77,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     constexpr int MT = WR * RB * 16, CW = WN * NB * 16;
     constexpr int CELLS = conv_cells(MT);
     constexpr int STR = CH * 128 + 16;           // bytes per cell
-    constexpr int BUF = (CELLS + 1) * STR;       // one more cell takes the pieces past the end
+    constexpr int ROW = CellPitch<STR>::kRow;
+    constexpr int BUF = patch_bytes<STR>(CELLS);
     constexpr int PPC = 8;                       // 16-byte pieces per cell and chunk
     constexpr int NP = (CELLS * PPC + NT - 1) / NT;   // a thread's, per chunk
     constexpr int KS = kStepsPerChunk;
@@ -138,13 +137,11 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     auto xload = [&](int i, unsigned at) {
         return __builtin_amdgcn_raw_buffer_load_b128(rX, xoff, i * (NT / PPC) * xrow + at, 0);
     };
-    // LDS address of piece i: a constant distance from piece 0 (but for the last, which may
-    // lie past the end)
-    const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 16u;
-    auto laddr = [&](int i) -> unsigned {
-        if (i < NP - 1 || (CELLS * PPC) % NT == 0) return lst + i * (NT / PPC) * STR;
-        return min(tid / PPC + i * (NT / PPC), (unsigned)CELLS) * STR + (tid % PPC) * 16u;
-    };
+    unsigned laddr[NP];                          // LDS address of piece i
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        laddr[i] = patch_at<STR>(ps, min(tid / PPC + i * (NT / PPC), (unsigned)CELLS)) +
+                   conv_slot(tid & 3, tid >> 2 & 1) * 16u;
 
     const int chunks = Cp / 64;
     const int ch0 = (kb >> 1) * 32 + 8 * (int)(lane >> 4) + 4 * (kb & 1);   // first channel
@@ -154,9 +151,9 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     static_assert(MT <= kPts, "a tile touches two boards at most");
 #pragma unroll
     for (int i = 0; i < RB; i++) {
-        const int local = (wr * RB + i) * 16 + (int)(lane & 15);
+        const int local = (wr * RB + i) * 16 + conv_point(lane);
         const unsigned cell = patch_cell(ps, min(local, rows - 1 - m0));
-        arow[i] = cell * STR + (lane >> 4) * 16;
+        arow[i] = patch_at<STR>(ps, cell) + conv_slot(lane >> 4, 0) * 16;
         ro[i] = m0 + local < rows ? ((ps.q0 + kPointCell + cell) * Kp + ch0) * 2u : 0xfffff000u;
     }
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
@@ -184,6 +181,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
         }
     };
 
+    clear_gaps<STR, CELLS, NT, DB ? 2 : 1>(lds, ps, tid);
     {
         int4v stg[CH][NP];
 #pragma unroll
@@ -195,7 +193,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
         for (int c = 0; c < CH; c++)
 #pragma unroll
             for (int i = 0; i < NP; i++)
-                *reinterpret_cast<int4v*>(lds + laddr(i) + c * 128) = stg[c][i];
+                *reinterpret_cast<int4v*>(lds + laddr[i] + c * 128) = stg[c][i];
         if (tid < (unsigned)CW) {
             bn[0][tid] = scale;
             bn[1][tid] = -scale * mean;
@@ -211,8 +209,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     int4v a[DA][RB];
     auto aread = [&](int i, int st) {
         const int sub = st / KS, tap = (st % KS) / 2, half = st & 1;
-        return *reinterpret_cast<const int4v*>(lds + arow[i] + ((tap / 3) * 20 + tap % 3) * STR +
-                                               sub * 128 + half * 64);
+        return *reinterpret_cast<const int4v*>(lds + arow[i] + tap / 3 * ROW + tap % 3 * STR +
+                                               sub * 128 + half * 16);
     };
     if constexpr (!DB) {
 #pragma unroll
@@ -248,7 +246,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
 #pragma unroll
                         for (int i = 0; i < SGRP; i++)
                             if (g * SGRP + i < NP)
-                                *reinterpret_cast<int4v*>(lds + laddr(g * SGRP + i) + other) = sg[i];
+                                *reinterpret_cast<int4v*>(lds + laddr[g * SGRP + i] + other) = sg[i];
                     }
                 }
             }

@@ -28,7 +28,7 @@ constexpr int conv_cells(int mt) {
 
 // The patch of a tile: the cells that its points reach.
 struct PatchStart {
-    unsigned q0;       // first cell: the upper left tap of the tile's first row
+    unsigned q0, x0;   // first cell: the upper left tap of the tile's first row; its place in a row of LDS
     unsigned mb, mp;   // board and point of the tile's first row
 };
 __device__ __forceinline__ PatchStart patch_start(unsigned m0) {
@@ -36,6 +36,7 @@ __device__ __forceinline__ PatchStart patch_start(unsigned m0) {
     s.mb = m0 / kPts;
     s.mp = m0 - s.mb * kPts;
     s.q0 = (s.mb + 1) * kCellsPerBoard + s.mp + s.mp / kBoard - 1;
+    s.x0 = (s.q0 + 1) % kRowCells;
     return s;
 }
 // Cell of the patch in which the upper left tap of the tile's row `local` lies; the point itself is
@@ -47,6 +48,60 @@ __device__ __forceinline__ unsigned patch_cell(const PatchStart& s, unsigned loc
     p -= next * kPts;
     const unsigned y = __umul24(p, 3450u) >> 16;   // p / 19
     return (s.mb + 1 + next) * kCellsPerBoard + p + y - 1 - s.q0;
+}
+
+// Where the cells of conv3x3_k's patch lie in LDS, and who reads them.  A fragment read (16 bytes a lane) is
+// served 16 lanes at a time, 256 bytes a cycle: lanes 0-3, 12-15 and 20-27 first, that is eight points of
+// one quarter of the k-step (lane / 16) and the eight other points of the next quarter.  Three
+// things make these 16 meet all 16 slots of 16 bytes, with addresses that are constants from one
+// read to the next:
+//   - a cell takes an odd number of slots (STR bytes), and the pieces of quarters 2 i and 2 i + 1 stand 4
+//     slots apart: conv_slot;
+//   - lanes 4-11 have the even points of a block of 16, the others the odd ones: conv_point;
+//   - a row of 20 cells, left border first, is as long, modulo 256 bytes, as one of 19: the end of a
+//     board row, where the cells of 16 points skip one, does not show.  What lies between two rows
+//     is read as the right border of the first: zeros, which clear_gaps writes.
+// Counted in a loop of reads: 4 cycles each; 8 with the pieces and points in their natural order, 12
+// where 16 points end a board row.  It shows where 192x64 tiles load the LDS most: 20x256 batch 32 640 ->
+// 614 us a forward, two side by side 979 -> 924; 16 boards 830 -> 820 of 40 blocks, the others within 1 %.
+// conv3x3_split_k and the fp32 kernels keep the natural order: they wait for other things, and the
+// addresses cost them more (10x128 fp16 batch 5 84 -> 93, 10x256 fp32 batch 64 1280 -> 1292).
+template <int STR>
+struct CellPitch {
+    static_assert(STR % 32 == 16, "an odd number of slots");
+    static constexpr int kAdd = (256 - STR % 256) % 256;   // bytes more per row
+    static constexpr int kRow = kRowCells * STR + kAdd;
+};
+// Bytes of a patch, with one more cell that takes the pieces past the end.
+template <int STR>
+constexpr int patch_bytes(int cells) {
+    return (cells + 1) * STR + (cells + kRowCells - 1) / kRowCells * CellPitch<STR>::kAdd;
+}
+template <int STR>
+__device__ __forceinline__ unsigned patch_at(const PatchStart& s, unsigned cell) {
+    return cell * STR + (__umul24(s.x0 + cell, 3277u) >> 16) * CellPitch<STR>::kAdd;   // (/ 20)
+}
+// Threads 0 .. NT - 1 clear what lies between the rows of COPIES patches.
+template <int STR, int CELLS, int NT, int COPIES>
+__device__ __forceinline__ void clear_gaps(unsigned char* patches, const PatchStart& s, unsigned tid) {
+    constexpr int GAPS = (CELLS + kRowCells - 1) / kRowCells, PIECES = CellPitch<STR>::kAdd / 16;
+#pragma unroll
+    for (int p = 0; p < (COPIES * GAPS * PIECES + NT - 1) / NT; p++) {
+        const unsigned i = tid + p * NT, gap = i / PIECES % GAPS, copy = i / (PIECES * GAPS);
+        const unsigned end = (gap + 1) * kRowCells - s.x0;   // cells before it
+        if (copy < COPIES && end <= (unsigned)CELLS)
+            *reinterpret_cast<int4v*>(patches + copy * patch_bytes<STR>(CELLS) + end * STR +
+                                      gap * CellPitch<STR>::kAdd + i % PIECES * 16) = int4v{0, 0, 0, 0};
+    }
+}
+// Slot of quarter q of half h of a cell.
+__device__ __forceinline__ unsigned conv_slot(unsigned q, unsigned h) {
+    return 4 * (q & 1) + 2 * (q >> 1) + h;
+}
+// The point of a block of 16 that a lane owns.
+__device__ __forceinline__ int conv_point(unsigned lane) {
+    const unsigned t = (lane + 4) & 15;
+    return (int)(2 * (t & 7) + 1 - (t >> 3));
 }
 
 // LDS is what a work-group shares: its writes are waited for, loads from memory stay in flight
