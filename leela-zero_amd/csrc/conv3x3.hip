@@ -14,6 +14,7 @@
 // It also rounds less: planes and 3x3 filters are the only values kept in half precision.
 #include <cmath>
 #include <stdexcept>
+#include <type_traits>
 
 #include "conv3x3_tile.h"
 
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     static_assert(D <= kFilterLookahead, "filter padding");
     static_assert(!DB || NG <= KS, "one group of pieces per k-step at most");
     static_assert(NB == 1 || NB % 2 == 0, "blocks are stored in pairs");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[DB ? 2 * BUF : BUF + 128 * DA];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[DB ? 2 * BUF : BUF];
     __shared__ __attribute__((aligned(16))) float bn[2][CW];
 
     const ConvTile tile = conv_tile(g);
@@ -159,10 +160,10 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
     const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
     const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
-    auto load_res = [&]() {
+    auto load_res = [&](int from, int to) {
         if (res != nullptr) {
 #pragma unroll
-            for (int i = 0; i < RB; i++)
+            for (int i = from; i < to; i++)
 #pragma unroll
                 for (int j = 0; j < PR; j++) {
                     if constexpr (NB >= 2) {
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
                 }
         } else {
 #pragma unroll
-            for (int i = 0; i < RB; i++)
+            for (int i = from; i < to; i++)
 #pragma unroll
                 for (int j = 0; j < PR; j++) rr[i][j] = int4v{0, 0, 0, 0};
         }
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
         for (int c = 0; c < CH; c++)
 #pragma unroll
             for (int i = 0; i < NP; i++) stg[c][i] = xload(i, c * 128);
-        if constexpr (EARLY) load_res();
+        if constexpr (EARLY) load_res(0, RB);
 #pragma unroll
         for (int c = 0; c < CH; c++)
 #pragma unroll
@@ -219,21 +220,25 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
             for (int i = 0; i < RB; i++) a[d][i] = aread(i, d);
     }
     unsigned other = BUF;   // byte offset of the buffer being filled (CC == 0)
-#pragma unroll 1
-    for (int c = 0; c < chunks; c++) {
+    // Chunk c; the last one stages nothing and fetches no filters past its end, and the skip connection
+    // comes into the registers that this leaves.
+    auto chunk = [&](int c, auto is_last) {
+        constexpr bool LAST = decltype(is_last)::value;
         if constexpr (DB) {
 #pragma unroll
             for (int d = 0; d < DA; d++)
 #pragma unroll
                 for (int i = 0; i < RB; i++) a[d][i] = aread(i, d);
         }
-        // the last chunk stages itself again, into the buffer nobody reads any more: loads
-        // and stores without branches keep the count of outstanding loads exact
-        const unsigned next = (unsigned)(c + 1 < chunks ? c + 1 : c) * 128u;
+        const unsigned next = (unsigned)(c + 1) * 128u;
         int4v sg[SGRP];
 #pragma unroll
         for (int st = 0; st < KS; st++) {
-            if constexpr (DB) {
+            if constexpr (LAST && !EARLY) {
+                if (st == KS - 2) load_res(0, RB / 3);
+                if (st == KS - 1) load_res(RB / 3, RB);
+            }
+            if constexpr (DB && !LAST) {
 #pragma unroll
                 for (int g = 0; g < NG; g++) {
                     if (st == g * GS) {
@@ -258,16 +263,18 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
             for (int i = 0; i < RB; i++) {
 #pragma unroll
                 for (int j = 0; j < NB; j++)
-                    if (i == (RB >= NB ? j : 0)) wload((st + D - 1) % D, j, st + D - 1);
+                    if (i == (RB >= NB ? j : 0) && (!LAST || st + D - 1 < KS))
+                        wload((st + D - 1) % D, j, st + D - 1);
 #pragma unroll
                 for (int j = 0; j < NB; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                         __builtin_bit_cast(half8v, w[st % D][j]),
                         __builtin_bit_cast(half8v, a[st % DA][i]), acc[i][j], 0, 0, 0);
-                if (!DB || st + DA < KS) a[st % DA][i] = aread(i, st + DA);
+                if (st + DA < KS || (!DB && !LAST)) a[st % DA][i] = aread(i, st + DA);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (LAST) return;
         ws += KS * wstep;
         if constexpr (DB) {
             lds_barrier();
@@ -279,10 +286,12 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
 #pragma unroll
             for (int i = 0; i < RB; i++) arow[i] += 128;
         }
-    }
+    };
+#pragma unroll 1
+    for (int c = 0; c < chunks - 1; c++) chunk(c, std::false_type{});
+    chunk(chunks - 1, std::true_type{});
 
     // max(0, scale * (y - mean) + rfac * res), clamped to the stored range
-    if constexpr (!EARLY) load_res();
 #pragma unroll
     for (int j = 0; j < PR; j++) {
         const int cl = ch0 - tn * CW + j * 32;
@@ -306,10 +315,10 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_k(
             }
             const int4v bits = __builtin_bit_cast(int4v, o);
             if constexpr (NB >= 2)
-                __builtin_amdgcn_raw_buffer_store_b128(bits, rY, ro[i] + j * 64, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(bits, rY, ro[i] + j * 64, 0, kStoreThrough);
             else
                 __builtin_amdgcn_raw_buffer_store_b64(uint2v{(unsigned)bits.x, (unsigned)bits.y},
-                                                      rY, ro[i], 0, 0);
+                                                      rY, ro[i], 0, kStoreThrough);
         }
     }
 }
@@ -613,7 +622,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
                 fmaxf(0.0f, fmaf((float)rh[e], rfac, fmaf(v, bn[0][cl + e], bn[1][cl + e]))),
                 kActStoreMax);
         }
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY, ro[q], 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY, ro[q], 0, kStoreThrough);
     }
 }
 

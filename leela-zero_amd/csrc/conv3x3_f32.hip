@@ -253,8 +253,9 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     // LDS address of piece i: a constant distance from piece 0 (the last may lie past the end)
     const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 8u;
     TileScales ts;
+    unsigned tv = tid;   // (opaque in every chunk: the scales of the pieces are not held)
     auto put = [&](int i, unsigned buffer, int4v bits) {
-        const unsigned cell = tid / PPC + i * (NT / PPC);
+        const unsigned cell = tv / PPC + i * (NT / PPC);
         const unsigned at = i < NP - 1 || (CELLS * PPC) % NT == 0
                                 ? lst + i * (NT / PPC) * STR
                                 : min(cell, (unsigned)CELLS) * STR + (tid % PPC) * 8u;
@@ -324,8 +325,11 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
                                                part * 64);
     };
     unsigned other = BUF;   // byte offset of the buffer being filled (CC == 0)
-#pragma unroll 1
-    for (int c = 0; c < chunks; c++) {
+    // Chunk c; the last one stages nothing and fetches no filters past its end, and the skip connection
+    // comes into the registers that this leaves.
+    auto chunk = [&](int c, auto is_last) {
+        constexpr bool LAST = decltype(is_last)::value;
+        asm volatile("" : "+v"(tv));
         if (2 * c == chunks) {
 #pragma unroll
             for (int i = 0; i < RB; i++)
@@ -337,12 +341,14 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
             hi[i] = aread(i, 0, 0);
             if (i < LO) lo[i] = aread(i, 1, 0);
         }
-        // (the last chunk stages itself again, into the buffer nobody reads any more)
-        const unsigned next = (unsigned)(c + 1 < chunks ? c + 1 : c) * 128u;
+        const unsigned next = (unsigned)(c + 1) * 128u;
         int4v sg[SGRP];
 #pragma unroll
         for (int st = 0; st < KS; st++) {
-            if constexpr (DB) {
+            if constexpr (LAST && !EARLY) {
+                if (st == KS - 1) first_res();
+            }
+            if constexpr (DB && !LAST) {
 #pragma unroll
                 for (int gr = 0; gr < NG; gr++) {
                     if (st == gr * GS) {
@@ -364,7 +370,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
             for (int i = 0; i < RB; i++) {
 #pragma unroll
                 for (int j = 0; j < NB; j++)
-                    if (i == (RB >= NB ? j : 0)) wload((st + D - 1) % D, j, st + D - 1);
+                    if (i == (RB >= NB ? j : 0) && (!LAST || st + D - 1 < KS))
+                        wload((st + D - 1) % D, j, st + D - 1);
 #pragma unroll
                 for (int j = 0; j < NB; j++) acc[i][j] = mfma(w[st % D][j], hi[i], acc[i][j]);
                 // (fragments are read behind the instructions that used their registers last)
@@ -382,6 +389,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (LAST) return;
         ws += KS * wstep;
         if constexpr (DB) {
             lds_barrier();
@@ -393,10 +401,12 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
 #pragma unroll
             for (int i = 0; i < RB; i++) arow[i] += BUF;
         }
-    }
+    };
+#pragma unroll 1
+    for (int c = 0; c < chunks - 1; c++) chunk(c, std::false_type{});
+    chunk(chunks - 1, std::true_type{});
 
     // max(0, scale * (y - mean) + rfac * res)
-    if constexpr (!EARLY) first_res();
     float top0 = 0.0f, top1 = 0.0f;
     const int m1 = ((int)ps.mb + 1) * kPts;   // first row of the tile's second board
 #pragma unroll
@@ -416,7 +426,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
                 top = fmaxf(top, finite(o[e]));
             }
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY,
-                                                   ro[i] + j * 64, 0, 0);
+                                                   ro[i] + j * 64, 0, kStoreThrough);
         }
         if (i + RQ < RB) load_res(i + RQ);
         top0 = fmaxf(top0, m < m1 ? top : 0.0f);
