@@ -362,25 +362,30 @@ bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
 // The tile.  A layer of few boards is a chain of latencies, so its points and channels are
 // spread over the 256 compute units in the smallest tiles that still make no more than one
 // work-group per unit; larger ones reuse each operand more.  Measured at 256 filters, us per
-// layer of a dependent chain with the tile of 32x32 | 32x64 | 48x64 | 96x64 | 192x64 |
-// 192x128 (points x channels), - = not measured:
-//    1 board    6.4 |  6.8 |  8.3 |  9.4 | 13.8 | 19.5
-//    4 boards   7.8 |  7.3 |  8.5 |  9.6 | 14.3 | 19.8
-//    8 boards   9.6 |  9.7 |  8.8 |  9.8 | 14.4 | 19.9
-//   16 boards  16.0 | 13.5 | 11.9 | 10.6 | 14.9 | 20.3
-//   24 boards  22.4 | 20.7 | 14.7 | 15.8 | 15.7 | 20.9
-//   32 boards  28.5 | 24.0 | 17.0 | 16.2 | 15.7 | 20.7
-//   64 boards  52.4 | 46.2 | 32.1 | 29.1 | 27.0 | 25.1
-// (each entry jumps where the tile passes 256 work-groups; the two wavefronts of a 48x64 tile
-// leave room for three on a unit, and until then it beats a 192x64 tile on half the units: 24
-// boards above, 37 boards of 128 filters 8.8 against 9.9.  It fetches every filter four times as
-// often, which the wider layers feel and so do forwards side by side: above 256 filters the
-// 192x64 tile is taken.  Per forward of 5 blocks, 48x64 | 192x64, us: 384 filters, 16 boards 210 |
-// 210, two side by side 358 | 302, three 518 | 419; 12 boards 191 | 207, 278 | 266, 395 | 346; 320
-// filters, 20 boards 185 | 183, 319 | 273, 464 | 368.  At 256 filters, 24 boards: 158 | 167, 252 |
-// 228, 364 | 301).  192 filters have no tile of 128
-// channels; there 128 x 192 takes the place of 192 x 128 (64 boards 18.2 against 19.7 us with
-// three tiles of 64 channels).
+// layer of a dependent chain with tiles of points x channels, * where a tile makes more than 256
+// work-groups, that is two or more on some unit:
+//               48x64   96x64  128x64  192x64 128x128 192x128
+//    8 boards    8.2     8.9     9.6    12.3    17.2    19.2
+//   16 boards   11.7*    9.9    10.5    13.1    17.3    19.4
+//   20 boards   13.7*   14.4*   11.0    13.5    17.6    20.0
+//   24 boards   14.3*   14.9*   16.2*   14.1    17.8    20.1
+//   32 boards   17.3*   15.5*   16.6*   14.4    18.2    20.1
+//   40 boards   22.8*   21.5*   17.7*   21.5*   19.1    21.2
+//   64 boards   32.0*   29.2*   26.4*   25.1*   28.5*   24.1
+//   80 boards   40.1*   35.6*   32.2*   33.1*   30.2*   37.6*
+//  128 boards   61.0*   54.2*   47.6*   45.6*   44.9*   42.9*
+// Two chains side by side want larger tiles (us per layer and chain): 20 boards 128x64 8.5, 192x64
+// 8.9, 96x64 9.6; 40 boards 192x64 13.3, 128x128 13.4, 128x64 14.3, 192x128 14.8; 64 boards 192x128 19.1,
+// 192x64 20.2; 80 boards 192x128 23.7, 128x128 25.3.  So 128x128 is taken up to one work-group per unit,
+// where it gains either way, and not up to two (72 to 90 boards of 256 filters one chain at a time
+// 37 -> 30, two side by side 4 to 8 % slower).  At other widths the order is the same: 128 filters, 44
+// boards 48x64 7.9, 128x64 6.7 (two chains 5.9 | 4.9), 70 boards 128x128 10.7, 192x128 12.1 (7.2 | 7.9);
+// 384 filters, 13 boards 192x64 16.8, 128x64 13.7 (13.4 | 12.0), 26 boards 128x128 24.0, 192x128 26.2 (19.4 |
+// 19.8).  64 and 192 filters have no tile of 128 channels; there 128x64 is taken up to two work-groups
+// per unit (192 filters, 52 boards 128x192 15.9, 128x64 13.6, two chains 12.7 | 12.0; 64 filters, 150 boards
+// 192x64 8.7, 128x64 7.1), and beyond, 128x192 takes the place of 192x128 (192 filters, 70 boards 192x64
+// 17.9, 128x192 16.5).  64 filters, whose one chunk is over soon, keep 48x64 up to three work-groups
+// (96 boards 5.8 against 6.4 with 192x64).
 void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                     const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,
                     hipStream_t s, LaunchTimer* t) {
@@ -417,12 +422,24 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
         LZ_CONV(3, 2, 2, 2, 6, 3, 0, 2);
         return;
     }
-    if (Kp <= 256 && groups(48, 64) <= 3 * kUnits) {
+    if (groups(128, 64) <= kUnits) {
+        LZ_CONV(4, 2, 2, 2, 6, 1, 0, 2);
+        return;
+    }
+    if (Kp == 64 && groups(48, 64) <= 3 * kUnits) {
         LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
         return;
     }
     if (groups(192, 64) <= kUnits) {
         LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);
+        return;
+    }
+    if (Kp % 128 == 0 && groups(128, 128) <= kUnits) {
+        LZ_CONV(4, 4, 2, 2, 3, 1, 0, 2);
+        return;
+    }
+    if ((Kp == 64 || Kp == 192) && groups(128, 64) <= 2 * kUnits) {
+        LZ_CONV(4, 2, 2, 2, 6, 1, 0, 2);
         return;
     }
     if (Kp % 128 == 0)

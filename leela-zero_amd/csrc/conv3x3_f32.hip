@@ -448,6 +448,11 @@ static PeakMap launch_f32_as(const float* X, const half_t* Wf, const float* res,
     return {slots, MT, Kp / CW};
 }
 
+// The tiles and their order are conv3x3_k's (launch_conv3x3).  Measured, us per layer of a chain (two chains
+// side by side, per chain): 256 filters, 20 boards 192x64 31.8, 128x64 24.5 (21.9 | 20.2), 40 boards 192x128
+// 50.5, 128x128 42.2 (37.8 | 36.6); 192 filters, 28 boards 192x64 25.1, 128x64 19.7 (30 boards 19.5 | 17.3), 46 boards
+// 128x192 40.0, 128x64 32.4 (28.1 | 25.3); 384 filters, 13 boards 192x64 44.7, 128x64 33.5 (32.1 | 29.1), 26 boards
+// 192x128 72.0, 128x128 58.7.
 PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, float* Y,
                            const float* bn_scale, const float* bn_mean, float rfac,
                            const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
@@ -474,8 +479,17 @@ PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, f
     if (groups(96, 64) <= kUnits) {
         return LZ_F32(3, 2, 2, 2, 6, 0, 2);
     }
+    if (groups(128, 64) <= kUnits) {
+        return LZ_F32(4, 2, 2, 2, 6, 0, 2);
+    }
     if (groups(192, 64) <= kUnits) {
         return LZ_F32(6, 2, 2, 2, 6, 0, 2);
+    }
+    if (Kp % 128 == 0 && groups(128, 128) <= kUnits) {
+        return LZ_F32(4, 4, 2, 2, 3, 0, 2);
+    }
+    if ((Kp == 64 || Kp == 192) && groups(128, 64) <= 2 * kUnits) {
+        return LZ_F32(4, 2, 2, 2, 6, 0, 2);
     }
     if (Kp % 128 == 0) return LZ_F32(6, 4, 2, 2, 3, 0, 2);
     if (Kp == 192) return LZ_F32(4, 6, 2, 2, 3, 0, 2);

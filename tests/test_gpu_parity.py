@@ -918,6 +918,9 @@ def test_winograd_filters_of_no_3x3_filter(pkg, netgen, orc):
     (64, 137, (1, 22, 23, 34, 68, 69, 136, 137)), (128, 70, (1, 11, 12, 17, 34, 35, 68, 69, 70)),
     (192, 46, (1, 7, 8, 11, 22, 23, 45, 46)), (256, 36, (1, 5, 6, 8, 9, 17, 34, 35, 36)),
     (384, 24, (1, 3, 6, 11, 12, 23, 24)), (512, 18, (1, 4, 5, 9, 17, 18)),
+    # 128 points: 64 and 128 channels
+    (64, 103, (90, 91, 102, 103)), (128, 91, (44, 46, 90, 91)), (192, 61, (16, 30, 31, 60, 61)),
+    (256, 46, (20, 22, 23, 45, 46)), (384, 31, (13, 14, 15, 30, 31)),
     # widths that are padded to a multiple of 64
     (24, 46, (1, 46)), (100, 12, (1, 12)), (200, 6, (1, 6)),
 ])
@@ -946,6 +949,34 @@ def test_fp32_direct_convolution(pkg, netgen, orc, filters, maxb, batches):
         got = pipe.debug_layer(2, a[:n], r[:n])[2]
         for i in range(n):
             assert rel_l2(got[i], want[i]) <= bound, (n, i, rel_l2(got[i], want[i]), bound)
+    pipe.close()
+
+
+@pytest.mark.parametrize("filters,batches", [
+    (64, (90, 91, 103, 136, 137, 181, 182)), (128, (45, 46, 90, 91)), (192, (22, 23, 30, 31, 60, 61)),
+    (256, (20, 22, 23, 45, 46)), (384, (12, 14, 15, 30, 31)), (320, (14, 17, 18, 25)),
+])
+def test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches):
+    """fp16 tiles of 128 points by 64 and by 128 channels on both sides of every change: one layer with a
+    skip connection, whole batch against a float32 convolution, and a position's bits in the
+    smallest and in the largest batch."""
+    import torch
+    import torch.nn.functional as F
+    maxb = max(batches)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 6620 + filters, pkg.FP16, maxb)
+    rng = np.random.default_rng(filters)
+    a = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
+    r = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float16).astype(np.float32)
+    y = F.conv2d(torch.from_numpy(a.reshape(maxb, filters, 19, 19)), torch.from_numpy(net.conv_w[2]),
+                 padding=1).numpy().reshape(maxb, filters, 361)
+    want = np.maximum(0.0, ref.scale[2][None, :, None] * (y - ref.mean[2][None, :, None]) + r)
+    one = pipe.debug_layer(2, a[:1], r[:1])[2]
+    for n in batches:
+        print("case: direct convolution, %d filters, %d boards" % (filters, n), flush=True)
+        got = pipe.debug_layer(2, a[:n], r[:n])[2]
+        assert np.array_equal(got[0], one[0])
+        for i in range(n):
+            assert rel_l2(got[i], want[i]) <= 2e-3, (n, i)
     pipe.close()
 
 
