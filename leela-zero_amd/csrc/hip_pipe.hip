@@ -666,9 +666,9 @@ public:
         const size_t B = (size_t)m_max_batch;
         m_dpolicy.alloc(B * 362);
         m_dvalue.alloc(B);
-        m_dwork.alloc(B * (362 + 256));
+        m_dwork.alloc(head_work_count(m_max_batch));
         for (int i = 0; i < m_n_lanes; i++) {
-            m_slot[i].dwork.alloc(B * (362 + 256));
+            m_slot[i].dwork.alloc(head_work_count(m_max_batch));
             m_slot[i].hlogits.alloc(B * 362);
         }
         m_heads_ready = true;

@@ -175,8 +175,9 @@ struct HeadParams {
 // its construction from W [outputs][inputs] row-major.
 size_t head_fc_fragment_count(bool policy);
 void head_fc_fragments(const float* W, bool policy, float* dst);
-// work: device scratch of n * (362 + 256) floats (logits and hidden units between the two
-// kernels).  logits may be null.
+// work: device scratch of head_work_count(n) floats (partial sums of the logits and of the hidden
+// units between the two kernels).  logits may be null.
+size_t head_work_count(int n);
 void launch_heads(const float* pol, const float* val, HeadParams hp, float temperature,
                   float* policy, float* logits, float* value, float* work, int n,
                   hipStream_t s);

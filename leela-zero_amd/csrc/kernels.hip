@@ -1907,61 +1907,70 @@ __device__ __forceinline__ float wave_max(float v) {
 // The two large fully connected layers -- policy 722 -> 362 and value 361 -> 256 -- are
 // matrix products over the batch, [n x K] . [K x N], and run on the matrix cores in fp32
 // (v_mfma_f32_32x32x2_f32: fp32 operands, fp32 accumulate).  One work-group computes a
-// 32-position x 32-output tile: the 32 input rows (batch norm and ReLU applied on the way)
-// are staged in LDS once, the four wavefronts split the contraction index four ways, and
-// their partial tiles meet in LDS.  The weights are held in the operand order of the
-// instruction (head_fc_fragments): lane l of k-step s supplies W^T[2s + l/32][32 cb + l%32],
-// four consecutive steps per 16-byte load, so a wavefront's load is one contiguous KiB.
-// A second, small kernel finishes: softmax over the 362 logits, and FC 256 -> 1 + tanh.
-constexpr int kHeadStepsPol = 92;   // k-steps (of 2) per wavefront: 4 * 92 * 2 = 736 >= 722
-constexpr int kHeadStepsVal = 48;   // 4 * 48 * 2 = 384 >= 361
+// 32-position x 32-output tile over a quarter of the contraction index: its share of the 32
+// input rows (batch norm and ReLU applied on the way) is staged in LDS once, the four
+// wavefronts split the quarter four ways, and their partial tiles meet in LDS.  The quarters
+// meet in the second kernel, which adds them and finishes: softmax over the 362 logits, and FC
+// 256 -> 1 + tanh.  What bounds it is latency, not work: one round trip for the operands, then
+// 24 dependent matrix instructions of 64 cycles.  With the whole index in one work-group these
+// were 92, behind 92 values of the planes per thread with a division each; a call of up to 37
+// positions took 13.2 us for this kernel, now 4.2 to 4.7, and one of 200 now takes 6.4.
+// The weights are held in the operand order of the instruction (head_fc_fragments): lane l of
+// k-step s supplies W^T[2s + l/32][32 cb + l%32], four consecutive steps per 16-byte load, so a
+// wavefront's load is one contiguous KiB.
+constexpr int kHeadQuarters = 4;    // work-groups that share a tile's contraction index
+constexpr int kHeadStepsPol = 24;   // k-steps (of 2) per wavefront: 16 * 24 * 2 = 768 >= 722
+constexpr int kHeadStepsVal = 12;   // 16 * 12 * 2 = 384 >= 361
 constexpr int kHeadColsPol = 12;    // 32-wide output blocks: 384 >= 362
 constexpr int kHeadColsVal = 8;     // 256
-constexpr int kHeadKPad = 4 * kHeadStepsPol * 2;   // staged row length of the wider layer
+
+size_t head_work_count(int n) { return (size_t)kHeadQuarters * n * (362 + 256); }
 
 size_t head_fc_fragment_count(bool policy) {
     return (size_t)(policy ? kHeadColsPol * kHeadStepsPol : kHeadColsVal * kHeadStepsVal) * 4 *
-           64;
+           kHeadQuarters * 64;
 }
 
 // W [N][K] row-major (as the network facade holds it) -> fragment order
-// [col block][wavefront 4][steps/4][lane 64][4 consecutive steps], zero padded.
+// [col block][quarter][wavefront 4][steps/4][lane 64][4 consecutive steps], zero padded.
 void head_fc_fragments(const float* W, bool policy, float* dst) {
     const int K = policy ? 2 * kPts : kPts, N = policy ? 362 : 256;
     const int steps = policy ? kHeadStepsPol : kHeadStepsVal;
     const int cols = policy ? kHeadColsPol : kHeadColsVal;
     for (int cb = 0; cb < cols; cb++)
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < 4 * kHeadQuarters; q++)
             for (int g = 0; g < steps / 4; g++)
                 for (int l = 0; l < 64; l++)
                     for (int e = 0; e < 4; e++) {
                         const int step = q * steps + g * 4 + e;
                         const int k = 2 * step + (l >> 5), j = cb * 32 + (l & 31);
                         const float v = (k < K && j < N) ? W[(size_t)j * K + k] : 0.0f;
-                        dst[((((size_t)cb * 4 + q) * (steps / 4) + g) * 64 + l) * 4 + e] = v;
+                        const size_t share = (size_t)cb * 4 * kHeadQuarters + q;
+                        dst[((share * (steps / 4) + g) * 64 + l) * 4 + e] = v;
                     }
 }
 
 // One layer's share of heads_fc_k.  Everything a work-group reads has been out of the caches
 // since the last call (a tower of 81 layers ran in between) and the planes have just been
 // written on other dies, so a round trip to memory takes ~2 us here: the wavefront's whole
-// share of the weights (23 or 12 KiB) and, per thread, its 92 or 48 values of the planes are
-// requested before the first is used.
+// share of the weights and, per thread, its 24 or 16 values of the planes are requested before the
+// first is used.  out: [kHeadQuarters][n][N] partial sums.
 template <bool POL>
 __device__ __forceinline__ void heads_fc_body(float* xs, const float* __restrict__ src,
                                               const HeadParams& hp, float* __restrict__ out,
-                                              int cb, int r0, int n) {
+                                              int cb, int quarter, int r0, int n) {
     constexpr int STEPS = POL ? kHeadStepsPol : kHeadStepsVal;
     constexpr int G = STEPS / 4;             // 16-byte weight loads per lane
-    constexpr int KP = 4 * STEPS * 2;        // padded contraction length
+    constexpr int KQ = 4 * STEPS * 2;        // contraction length of a quarter
     constexpr int KK = POL ? 2 * kPts : kPts;
     constexpr int N = POL ? 362 : 256;
-    constexpr int ROW = kHeadKPad + 1;       // odd row length: conflict-free column reads
+    constexpr int ROW = KQ + 1;              // odd row length: conflict-free column reads
+    constexpr int J = (KQ + 63) / 64, R = 8; // a lane's values per row, a wavefront's rows
     const int tid = threadIdx.x, lane = tid & 63;
     const int q = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     const float4v* wf = reinterpret_cast<const float4v*>(POL ? hp.ip_pol_wf : hp.ip1_val_wf) +
-                        (((size_t)cb * 4 + q) * G) * 64 + lane;
+                        ((((size_t)cb * kHeadQuarters + quarter) * 4 + q) * G) * 64 + lane;
     float4v w[G];
 #pragma unroll
     for (int g = 0; g < G; g++) w[g] = wf[(size_t)g * 64];
@@ -1971,26 +1980,25 @@ __device__ __forceinline__ void heads_fc_body(float* xs, const float* __restrict
     const float m0 = POL ? hp.bn_pol_mean[0] : hp.bn_val_mean[0];
     const float s1 = POL ? hp.bn_pol_scale[1] : s0;
     const float m1 = POL ? hp.bn_pol_mean[1] : m0;
-    constexpr int U = KP / 8;                // 32 * KP values on 256 threads: all in one go
-    for (int i0 = tid; i0 < 32 * KP; i0 += 256 * U) {
-        float x[U];
+    float x[R][J];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = i0 + u * 256;
-            const int r = i / KP, k = i - r * KP;
-            x[u] = (i < 32 * KP && r0 + r < n && k < KK) ? src[(size_t)(r0 + r) * KK + k] : 0.0f;
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const int row = r0 + q * R + r, c = lane + 64 * j, k = quarter * KQ + c;
+            x[r][j] = row < n && c < KQ && k < KK ? src[(size_t)row * KK + k] : 0.0f;
         }
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = i0 + u * 256;
-            const int r = i / KP, k = i - r * KP;
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const int row = r0 + q * R + r, c = lane + 64 * j, k = quarter * KQ + c;
             const bool second = POL && k >= kPts;
             float y = 0.0f;
-            if (r0 + r < n && k < KK)
-                y = fmaxf(0.0f, (second ? s1 : s0) * (x[u] - (second ? m1 : m0)));
-            if (i < 32 * KP) xs[r * ROW + k] = y;
+            if (row < n && k < KK)
+                y = fmaxf(0.0f, (second ? s1 : s0) * (x[r][j] - (second ? m1 : m0)));
+            if (c < KQ) xs[(q * R + r) * ROW + c] = y;
         }
-    }
     __syncthreads();
 
     float16v acc;
@@ -2013,15 +2021,14 @@ __device__ __forceinline__ void heads_fc_body(float* xs, const float* __restrict
     for (int r = 0; r < 16; r++)
         red[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * 33 + (lane & 31)] = acc[r];
     __syncthreads();
-    const float* bias = POL ? hp.ip_pol_b : hp.ip1_val_b;
+    out += (size_t)quarter * n * N;
     for (int i = tid; i < 32 * 32; i += 256) {
         const int r = i >> 5, j = i & 31;
         const int col = cb * 32 + j;
-        if (r0 + r < n && col < N) {
-            const float v = xs[r * 33 + j] + xs[32 * 33 + r * 33 + j] +
-                            xs[2 * 32 * 33 + r * 33 + j] + xs[3 * 32 * 33 + r * 33 + j];
-            out[(size_t)(r0 + r) * N + col] = POL ? v + bias[col] : fmaxf(0.0f, v + bias[col]);
-        }
+        if (r0 + r < n && col < N)
+            out[(size_t)(r0 + r) * N + col] =
+                xs[r * 33 + j] + xs[32 * 33 + r * 33 + j] + xs[2 * 32 * 33 + r * 33 + j] +
+                xs[3 * 32 * 33 + r * 33 + j];
     }
 }
 
@@ -2029,13 +2036,15 @@ __global__ __launch_bounds__(256) void heads_fc_k(const float* __restrict__ pol,
                                                   const float* __restrict__ val, HeadParams hp,
                                                   float* __restrict__ logits,
                                                   float* __restrict__ hidden, int n) {
-    __shared__ float xs[32 * (kHeadKPad + 1)];
+    constexpr int STAGE = 32 * (8 * kHeadStepsPol + 1), MEET = 4 * 32 * 33;
+    __shared__ float xs[STAGE > MEET ? STAGE : MEET];
     const int tasks = kHeadColsPol + kHeadColsVal;
-    const int rb = blockIdx.x / tasks, task = blockIdx.x - rb * tasks;
+    const int tile = blockIdx.x / kHeadQuarters, quarter = blockIdx.x % kHeadQuarters;
+    const int rb = tile / tasks, task = tile - rb * tasks;
     if (task < kHeadColsPol)
-        heads_fc_body<true>(xs, pol, hp, logits, task, rb * 32, n);
+        heads_fc_body<true>(xs, pol, hp, logits, task, quarter, rb * 32, n);
     else
-        heads_fc_body<false>(xs, val, hp, hidden, task - kHeadColsPol, rb * 32, n);
+        heads_fc_body<false>(xs, val, hp, hidden, task - kHeadColsPol, quarter, rb * 32, n);
 }
 
 // One wavefront per position: softmax over the logits at `temperature`, and the value
@@ -2053,7 +2062,13 @@ __global__ __launch_bounds__(256) void heads_finish_k(const float* __restrict__ 
 #pragma unroll
     for (int qq = 0; qq < 6; qq++) {
         const int i = lane + 64 * qq;
-        l[qq] = i < 362 ? logits_in[(size_t)pos * 362 + i] : -INFINITY;
+        l[qq] = -INFINITY;
+        if (i < 362) {
+            float v = 0.0f;
+#pragma unroll
+            for (int k = 0; k < kHeadQuarters; k++) v += logits_in[((size_t)k * n + pos) * 362 + i];
+            l[qq] = v + hp.ip_pol_b[i];
+        }
         m = fmaxf(m, l[qq]);
     }
     m = wave_max(m);
@@ -2073,7 +2088,14 @@ __global__ __launch_bounds__(256) void heads_finish_k(const float* __restrict__ 
         }
     }
     float acc = 0.0f;
-    for (int i = lane; i < 256; i += 64) acc += hidden[(size_t)pos * 256 + i] * hp.ip2_val_w[i];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = lane + 64 * j;
+        float v = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kHeadQuarters; k++) v += hidden[((size_t)k * n + pos) * 256 + i];
+        acc += fmaxf(0.0f, v + hp.ip1_val_b[i]) * hp.ip2_val_w[i];
+    }
     acc = wave_sum(acc);
     if (lane == 0) value[pos] = tanhf(hp.ip2_val_b[0] + acc);
 }
@@ -2081,12 +2103,13 @@ __global__ __launch_bounds__(256) void heads_finish_k(const float* __restrict__ 
 void launch_heads(const float* pol, const float* val, HeadParams hp, float temperature,
                   float* policy, float* logits, float* value, float* work, int n,
                   hipStream_t s) {
-    // work: [n][362] logits followed by [n][256] hidden units
+    // work: [kHeadQuarters][n][362] of the logits followed by [kHeadQuarters][n][256] of the
+    // hidden units
     float* wl = work;
-    float* wh = work + (size_t)n * 362;
+    float* wh = work + (size_t)kHeadQuarters * n * 362;
     const int rbs = (n + 31) / 32;
-    hipLaunchKernelGGL(heads_fc_k, dim3(rbs * (kHeadColsPol + kHeadColsVal)), dim3(256), 0, s, pol,
-                       val, hp, wl, wh, n);
+    hipLaunchKernelGGL(heads_fc_k, dim3(rbs * (kHeadColsPol + kHeadColsVal) * kHeadQuarters),
+                       dim3(256), 0, s, pol, val, hp, wl, wh, n);
     hipLaunchKernelGGL(heads_finish_k, dim3((n + 3) / 4), dim3(256), 0, s, wl, wh, hp, temperature,
                        policy, logits, value, n);
 }

@@ -1014,3 +1014,39 @@ def test_fp32_range_and_values_that_are_no_numbers(pkg, netgen, orc):
         for i in (0, 2, 3):
             assert np.array_equal(pol[i], want[0][i]) and np.array_equal(val[i], want[1][i]), (bad, i)
     pipe.close()
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 100])
+def test_heads_at_the_edges_of_their_tiles(pkg, netgen, orc, n):
+    """The fully connected heads work on tiles of 32 positions by 32 outputs, and sixteen
+    partial sums meet for each output.  Against float64 from the raw planes of the same call; a
+    sum of K products and a bias in fp32, in any order, is within (K + 4) 2^-24 of the sum of
+    the magnitudes (two of the four roundings are the batch norm's)."""
+    print("case: heads n=%d" % n, flush=True)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, 32, 7100, pkg.FP32, 100)
+    x = netgen.synthetic_inputs(n, seed=71)
+    policy, value, logits, pol, val = pipe.evaluate_batch(x, want_raw=True)
+
+    def fc(a, w, b):
+        w = np.asarray(w, np.float64).reshape(len(b), -1)
+        bound = (a.shape[1] + 4) * 2.0 ** -24 * (np.abs(a) @ np.abs(w).T + np.abs(b))
+        return a @ w.T + b, bound
+
+    def bn(a, mean, scale, per):
+        mean, scale = (np.repeat(np.asarray(v, np.float64), per) for v in (mean, scale))
+        return np.maximum(0.0, scale * (a.astype(np.float64) - mean))
+
+    h = h_ref
+    p = bn(pol, h.bn_pol_mean, h.bn_pol_scale, 361)
+    want, bound = fc(p, h.ip_pol_w, np.asarray(h.ip_pol_b, np.float64))
+    assert (np.abs(logits - want) <= bound).all(), (np.abs(logits - want) / bound).max()
+    e = np.exp(logits.astype(np.float64) - logits.max(axis=1, keepdims=True))
+    assert np.abs(policy - e / e.sum(axis=1, keepdims=True)).max() <= 1e-5
+    v = bn(val, h.bn_val_mean, h.bn_val_scale, 361)
+    hid, hb = fc(v, h.ip1_val_w, np.asarray(h.ip1_val_b, np.float64))
+    hid = np.maximum(0.0, hid)
+    out, ob = fc(hid, h.ip2_val_w, np.asarray(h.ip2_val_b, np.float64))
+    ob = ob + hb @ np.abs(np.asarray(h.ip2_val_w, np.float64)).reshape(-1, 1)
+    # (tanh has slope at most 1; its own error is a few units of the last place of 1)
+    assert (np.abs(value - np.tanh(out[:, 0])) <= ob[:, 0] + 4 * 2.0 ** -24).all()
+    pipe.close()
