@@ -12,6 +12,7 @@
 namespace lzhip {
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float8v __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 
 #define SQ2 1.4142135623730951f
@@ -97,83 +98,97 @@ __device__ __forceinline__ void at6(const float i0, const float i1, const float 
 // ---------------------------------------------------------------------------
 // ---------------------------------------------------------------------------
 // Planes NCHW fp32 [n][C][361] -> channels-last storage type [n][361][Cp],
-// channels C..Cp-1 zero.
+// channels C..Cp-1 zero.  A thread takes one point and every fourth group of eight channels of
+// it: the reads of sixteen points are 64 bytes of a plane, the writes of four threads 64 or 128
+// bytes of a point.  (With a value per thread, channels first, 64 lanes read 64 planes: 200 boards
+// took 13 us, now 6, and from packed planes in host memory, each word fetched by many, 28, now 9;
+// 37 boards 8.2 and 5.3; one board takes the 4 us of a trip across the bus either way.)
+constexpr int kPackThreads = 4 * kPts;   // of a board
+template <typename P, typename Value>
+__device__ __forceinline__ void pack_point(P* __restrict__ cell, int g, int C, int Cp,
+                                           Value value) {
+    typedef P P8 __attribute__((ext_vector_type(8)));
+    for (int c0 = g * 8; c0 < Cp; c0 += 32) {
+        P8 v = {};
+        if (c0 < C) {   // (read past C without a branch to each, so that all eight are in flight)
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = value(min(c0 + e, C - 1));
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = c0 + e < C ? to_storage<P>(x[e]) : (P)0.0f;
+        }
+        *reinterpret_cast<P8*>(cell + c0) = v;
+    }
+}
+
 template <typename P>
 __global__ __launch_bounds__(256) void pack_input_k(const float* __restrict__ in,
                                                     P* __restrict__ act, bool padded, int n, int C,
                                                     int Cp) {
     const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t total = (size_t)n * kPts * Cp;
-    if (gid >= total) return;
-    const int c = (int)(gid % Cp);
-    const size_t bp = gid / Cp;
-    const int pt = (int)(bp % kPts);
-    const size_t b = bp / kPts;
-    float v = 0.0f;
-    if (c < C) v = in[(b * C + c) * kPts + pt];
-    act[plane_index(padded, (int)b, pt) * Cp + c] = to_storage<P>(v);
+    if (gid >= (size_t)n * kPackThreads) return;
+    const int b = (int)(gid / kPackThreads), i = (int)(gid % kPackThreads), pt = i >> 2;
+    const float* planes = in + (size_t)b * C * kPts + pt;
+    pack_point(act + plane_index(padded, b, pt) * Cp, i & 3, C, Cp,
+               [&](int c) { return planes[(size_t)c * kPts]; });
 }
 
 template <typename P>
 void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int Cp, hipStream_t s,
                        LaunchTimer* t) {
-    const size_t total = (size_t)n * kPts * Cp;
+    const size_t total = (size_t)n * kPackThreads;
     launch(pack_input_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, in, act,
            padded, n, C, Cp);
 }
 
 // The same from bit-packed planes: bit (c*361 + pt) of a board's kInputWords words is
-// plane c at point pt (planes that hold only 0 and 1, which is what the engine feeds).
+// plane c at point pt (planes that hold only 0 and 1, which is what the engine feeds).  The
+// words may lie in host memory, across the bus: a work-group fetches its board's once, in one
+// load, and there are three of them to a board.
 template <typename P>
-__global__ __launch_bounds__(256) void pack_input_bits_k(const uint32_t* __restrict__ bits,
-                                                         P* __restrict__ act, bool padded, int n,
-                                                         int C, int Cp, uint32_t* __restrict__ peaks) {
-    const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t total = (size_t)n * kPts * Cp;
-    if (gid >= total) return;
-    if (peaks && gid < 2 * (size_t)n) peaks[gid] = 0x3f800000u;
-    const int c = (int)(gid % Cp);
-    const size_t bp = gid / Cp;
-    const int pt = (int)(bp % kPts);
-    const size_t b = bp / kPts;
-    float v = 0.0f;
-    if (c < C) {
+__global__ __launch_bounds__(512) void pack_input_bits_k(const uint32_t* __restrict__ bits,
+                                                         P* __restrict__ act, bool padded, int C,
+                                                         int Cp, uint32_t* __restrict__ peaks) {
+    __shared__ uint32_t words[kInputWords];
+    const int b = blockIdx.x, i = blockIdx.y * 512 + threadIdx.x, pt = i >> 2;
+    if (threadIdx.x < kInputWords)
+        words[threadIdx.x] = bits[(size_t)b * kInputWords + threadIdx.x];
+    if (peaks && i < 2) peaks[2 * (size_t)b + i] = 0x3f800000u;
+    __syncthreads();
+    if (pt >= kPts) return;
+    pack_point(act + plane_index(padded, b, pt) * Cp, i & 3, C, Cp, [&](int c) {
         const int bit = c * kPts + pt;
-        v = (float)((bits[b * kInputWords + (bit >> 5)] >> (bit & 31)) & 1u);
-    }
-    act[plane_index(padded, (int)b, pt) * Cp + c] = to_storage<P>(v);
+        return (float)((words[bit >> 5] >> (bit & 31)) & 1u);
+    });
 }
 
 template <typename P>
 void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, int C, int Cp,
                             uint32_t* peaks, hipStream_t s, LaunchTimer* t) {
-    const size_t total = (size_t)n * kPts * Cp;
-    launch(pack_input_bits_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, bits, act,
-           padded, n, C, Cp, peaks);
+    launch(pack_input_bits_k<P>, dim3(n, (kPackThreads + 511) / 512), dim3(512), s, t, bits, act,
+           padded, C, Cp, peaks);
 }
 
-// Planes and peaks from float planes: one work-group per board reads all of it (26 KB); the packing
-// is spread over eight.
-constexpr int kPackParts = 8;
+// Planes and peaks from float planes: the first work-group of a board packs nothing and reads all
+// of it (26 KB); three pack.
 __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restrict__ in,
                                                           float* __restrict__ act, int C, int Cp,
                                                           uint32_t* __restrict__ peaks) {
-    const int b = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
+    const int b = blockIdx.x, tid = threadIdx.x;
     const float* planes = in + (size_t)b * C * kPts;
+    if (blockIdx.y > 0) {
+        const int i = (blockIdx.y - 1) * 512 + tid, pt = i >> 2;
+        if (pt < kPts)
+            pack_point(act + plane_index(true, b, pt) * Cp, i & 3, C, Cp,
+                       [&](int c) { return planes[(size_t)c * kPts + pt]; });
+        return;
+    }
     float top = 0.0f;
-    if (part == 0) {
-#pragma unroll 8
-        for (int i = tid; i < C * kPts; i += 512) {
-            const float v = fabsf(planes[i]);
-            top = fmaxf(top, v < __builtin_inff() ? v : 0.0f);
-        }
+#pragma unroll 13
+    for (int i = tid; i < C * kPts; i += 512) {
+        const float v = fabsf(planes[i]);
+        top = fmaxf(top, v < __builtin_inff() ? v : 0.0f);
     }
-    const int from = part * kPts / kPackParts, to = (part + 1) * kPts / kPackParts;
-    for (int i = tid; i < (to - from) * Cp; i += 512) {
-        const int pt = from + i / Cp, c = i % Cp;
-        act[plane_index(true, b, pt) * Cp + c] = c < C ? planes[(size_t)c * kPts + pt] : 0.0f;
-    }
-    if (part != 0) return;
     __shared__ float tops[8];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
@@ -187,7 +202,8 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
 
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
                              hipStream_t s, LaunchTimer* t) {
-    launch(pack_input_peaks_k, dim3(n, kPackParts), dim3(512), s, t, in, act, C, Cp, peaks);
+    launch(pack_input_peaks_k, dim3(n, 1 + (kPackThreads + 511) / 512), dim3(512), s, t, in, act, C,
+           Cp, peaks);
 }
 
 __global__ __launch_bounds__(256) void clear_k(int4v* p, size_t n) {
@@ -1823,27 +1839,36 @@ void launch_gemm(const P* V, const P* U, const P* Uf, P* M, int T, int Tp, int C
 
 // ---------------------------------------------------------------------------
 // 1x1 policy (2 planes) and value (1 plane) convolutions in one pass over the
-// last activation (reference src/CPUPipe.cpp:424-427).  One wavefront per
-// board point; lanes stride over channels, then a butterfly reduction.
-template <typename P>
+// last activation (reference src/CPUPipe.cpp:424-427).  Sixteen lanes to a
+// board point up to 128 channels and 32 beyond, eight channels a lane and load, then a butterfly
+// reduction.  (With a wavefront to a point and a channel a lane the number of wavefronts was the
+// bound: 256 filters, 200 boards 25 us, now 13; 128 filters, 37 boards 5.4 and 3.5.)
+template <typename P, int LP>
 __global__ __launch_bounds__(256) void head_conv_k(const P* __restrict__ act, bool padded,
                                                    const float* __restrict__ w3,
                                                    float out_scale, float* __restrict__ pol,
                                                    float* __restrict__ val, int n, int Cp) {
-    const int gw = (blockIdx.x * 256 + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    if (gw >= n * kPts) return;
-    const int b = gw / kPts, pt = gw - b * kPts;
+    typedef P P8 __attribute__((ext_vector_type(8)));
+    const int gp = (blockIdx.x * 256 + threadIdx.x) / LP;
+    const int lane = threadIdx.x % LP;
+    if (gp >= n * kPts) return;
+    const int b = gp / kPts, pt = gp - b * kPts;
     const P* a = act + plane_index(padded, b, pt) * Cp;
     float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-    for (int c = lane; c < Cp; c += 64) {
-        const float x = (float)a[c];
-        s0 += x * w3[c];
-        s1 += x * w3[Cp + c];
-        s2 += x * w3[2 * Cp + c];
+    for (int c = lane * 8; c < Cp; c += LP * 8) {
+        const P8 x = *reinterpret_cast<const P8*>(a + c);
+        const float8v w0 = *reinterpret_cast<const float8v*>(w3 + c);
+        const float8v w1 = *reinterpret_cast<const float8v*>(w3 + Cp + c);
+        const float8v w2 = *reinterpret_cast<const float8v*>(w3 + 2 * Cp + c);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            s0 += (float)x[e] * w0[e];
+            s1 += (float)x[e] * w1[e];
+            s2 += (float)x[e] * w2[e];
+        }
     }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = LP / 2; off > 0; off >>= 1) {
         s0 += __shfl_xor(s0, off);
         s1 += __shfl_xor(s1, off);
         s2 += __shfl_xor(s2, off);
@@ -1858,9 +1883,13 @@ __global__ __launch_bounds__(256) void head_conv_k(const P* __restrict__ act, bo
 template <typename P>
 void launch_head_conv(const P* act, bool padded, const float* w3, float out_scale, float* pol,
                       float* val, int n, int Cp, hipStream_t s, LaunchTimer* t) {
-    const int waves = n * kPts;
-    launch(head_conv_k<P>, dim3((waves + 3) / 4), dim3(256), s, t, act, padded, w3, out_scale,
-           pol, val, n, Cp);
+    const int points = n * kPts;
+    if (Cp > 128)
+        launch(head_conv_k<P, 32>, dim3((points + 7) / 8), dim3(256), s, t, act, padded, w3,
+               out_scale, pol, val, n, Cp);
+    else
+        launch(head_conv_k<P, 16>, dim3((points + 15) / 16), dim3(256), s, t, act, padded, w3,
+               out_scale, pol, val, n, Cp);
 }
 
 // ---------------------------------------------------------------------------
