@@ -470,12 +470,15 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // lost 10 %): there the partial sums' way through LDS, 2 KW RB NB KiB, costs what it saves.
 // The order of the sum differs from conv3x3_k's, so a network uses one or the other whatever the
 // batch (conv3x3_splits).
-template <int RB, int KW, int HPW, int D>
+template <int RB, int NB, int KW, int HPW, int D>
 __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
     half_t* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
     float rfac, int n, int Kp, ConvGrid g) {
-    constexpr int NB = 2, DA = 3;                          // 32 channels; planes read ahead
+    constexpr int DA = 3;                                  // planes read ahead
+    constexpr int E = 4 * NB;                              // channels that a lane finishes
+    typedef std::conditional_t<NB == 2, int4v, int2v> Piece;
+    typedef half_t HalfE __attribute__((ext_vector_type(E)));
     constexpr int CH = KW * HPW / 2, Cp = 64 * CH, NT = 64 * KW;
     constexpr int MT = RB * 16, CW = NB * 16, CELLS = conv_cells(MT);
     constexpr int STR = HPW * 64 + 16, SLICE = (CELLS + 1) * STR;   // bytes per cell, wavefront
@@ -495,7 +498,9 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const unsigned tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
 
-    const unsigned bnoff = tid < (unsigned)CW ? (tn * CW + tid) * 4u : 0xfffffff0u;
+    // channels in the order of the lanes that finish them
+    auto channel = [&](int c) { return NB == 2 ? tn * CW + c : conv_channel(tn, c); };
+    const unsigned bnoff = tid < (unsigned)CW ? channel(tid) * 4u : 0xfffffff0u;
     const float scale = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                                                       make_rsrc(bn_scale, Kp * 4), bnoff, 0, 0));
     const float mean = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
@@ -539,23 +544,24 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 
     // the blocks of 16 points that this wavefront finishes: where they lie, and the skip connection
     unsigned ro[QP];
-    int4v rr[QP];
+    Piece rr[QP];
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
     const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
     const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
-    const int cl = 8 * (int)(lane >> 4);   // first of this lane's 8 channels
+    const int cl = E * (int)(lane >> 4);   // first of this lane's channels
 #pragma unroll
     for (int q = 0; q < QP; q++) {
         const int i = q * KW + wave, local = i * 16 + (int)(lane & 15);
         ro[q] = i < RB && m0 + local < rows
-                    ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + tn * CW + cl) * 2u
+                    ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + channel(cl)) * 2u
                     : 0xfffffff0u;
-        rr[q] = int4v{0, 0, 0, 0};
+        rr[q] = Piece{};
     }
     if (res != nullptr) {
 #pragma unroll
         for (int q = 0; q < QP; q++)
-            rr[q] = __builtin_amdgcn_raw_buffer_load_b128(rR, ro[q], 0, 0);
+            if constexpr (NB == 2) rr[q] = __builtin_amdgcn_raw_buffer_load_b128(rR, ro[q], 0, 0);
+            else rr[q] = __builtin_amdgcn_raw_buffer_load_b64(rR, ro[q], 0, 0);
     }
     unsigned char* const own = lds + wave * SLICE;
 #pragma unroll
@@ -628,10 +634,10 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
             for (int j = 0; j < NB; j++)
                 part[k][j] = *reinterpret_cast<const float4v*>(
                     lds + ((k * RB + i) * NB + j) * 1024 + lane * 16);
-        const half8v rh = __builtin_bit_cast(half8v, rr[q]);
-        half8v o;
+        const HalfE rh = __builtin_bit_cast(HalfE, rr[q]);
+        HalfE o;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
+        for (int e = 0; e < E; e++) {
             float v = part[0][e / 4][e % 4];
 #pragma unroll
             for (int k = 1; k < KW; k++) v += part[k][e / 4][e % 4];
@@ -639,41 +645,58 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
                 fmaxf(0.0f, fmaf((float)rh[e], rfac, fmaf(v, bn[0][cl + e], bn[1][cl + e]))),
                 kActStoreMax);
         }
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY, ro[q], 0, kStoreThrough);
+        if constexpr (NB == 2)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY, ro[q], 0,
+                                                   kStoreThrough);
+        else
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(int2v, o), rY, ro[q], 0,
+                                                  kStoreThrough);
     }
 }
 
-// The tile, in blocks of 16 points by 32 channels: the smallest whose work-groups are no more
-// than the compute units; 0: none of the three is.
-static int split_blocks(int n, int Kp) {
-    for (int rb = 2; rb <= 4; rb++)
-        if ((n * kPts + rb * 16 - 1) / (rb * 16) * (Kp / 32) <= kUnits) return rb;
-    return 0;
+// The tile, in blocks of 16 points by 16 channels: the smallest whose work-groups are no more
+// than the compute units; {0, 0}: none is.  One block of channels halves the filters that the L1
+// has to deliver to a work-group, which is what a layer of one board waits for: against 32 x 32
+// tiles 128 filters 3.8 -> 3.3 us, 192 4.4 -> 3.8, 256 4.9 -> 4.3, 320 5.3 -> 4.7.  48 x 16 is worth
+// 2 to 4 % up to 256 filters (192 filters, 2 boards 4.4 -> 4.3 us) and no longer beyond (384
+// filters, 1 board 5.5 -> 5.7).
+struct SplitTile {
+    int rb, nb;
+};
+static SplitTile split_tile(int n, int Kp) {
+    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}};
+    for (const SplitTile& t : kTiles)
+        if ((t.rb * t.nb != 3 || Kp <= 256) &&
+            (n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
+    return {0, 0};
 }
 
 // A wavefront takes 64 input channels (32 of up to 128): eight wavefronts' planes are what the LDS
 // holds, so 512 filters are the widest.
 bool conv3x3_splits(int Kp, int max_batch) {
-    return Kp % 64 == 0 && Kp <= 512 && split_blocks(max_batch, Kp) > 0;
+    return Kp % 64 == 0 && Kp <= 512 && split_tile(max_batch, Kp).rb > 0;
 }
 
 void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                           const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
                           int Kp, hipStream_t s, LaunchTimer* t) {
-    const int rb = split_blocks(n, Kp);
+    const SplitTile tile = split_tile(n, Kp);
     if (!conv3x3_splits(Kp, n) || Cp != Kp)
         throw std::invalid_argument("no split convolution for this width or batch");
-    const ConvGrid g = conv_grid((n * kPts + rb * 16 - 1) / (rb * 16), Kp / 32,
+    const ConvGrid g = conv_grid((n * kPts + tile.rb * 16 - 1) / (tile.rb * 16), Kp / (16 * tile.nb),
                                  (size_t)18 * Cp * Kp, (size_t)n * kPts * Cp * 2);
     auto go = [&](auto kernel, int waves) {
         launch(kernel, dim3(8 * g.share), dim3(64 * waves), s, t, X, Wf, res, Y, bn_scale,
                bn_mean, rfac, n, Kp, g);
     };
     // KW wavefronts x HPW halves of a chunk
-#define LZ_SPLIT(KW, HPW, D)                                   \
-    if (rb == 2) go(conv3x3_split_k<2, KW, HPW, D>, KW);       \
-    else if (rb == 3) go(conv3x3_split_k<3, KW, HPW, D>, KW);  \
-    else go(conv3x3_split_k<4, KW, HPW, D>, KW)
+#define LZ_SPLIT(KW, HPW, D)                                               \
+    if (tile.nb == 1) {                                                    \
+        if (tile.rb == 2) go(conv3x3_split_k<2, 1, KW, HPW, D>, KW);       \
+        else if constexpr (KW < 5) go(conv3x3_split_k<3, 1, KW, HPW, D>, KW); \
+    } else if (tile.rb == 2) go(conv3x3_split_k<2, 2, KW, HPW, D>, KW);    \
+    else if (tile.rb == 3) go(conv3x3_split_k<3, 2, KW, HPW, D>, KW);      \
+    else if constexpr (KW < 8) go(conv3x3_split_k<4, 2, KW, HPW, D>, KW)
     switch (Kp) {
         case 64: LZ_SPLIT(2, 1, 9); break;
         case 128: LZ_SPLIT(4, 1, 9); break;
@@ -683,9 +706,7 @@ void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, 
         case 320: LZ_SPLIT(5, 2, 12); break;
         case 384: LZ_SPLIT(6, 2, 12); break;
         case 448: LZ_SPLIT(7, 2, 12); break;
-        default:   // 512 filters: the third tile is for 3 boards, which they no longer fit in
-            if (rb == 2) go(conv3x3_split_k<2, 8, 2, 12>, 8);
-            else go(conv3x3_split_k<3, 8, 2, 12>, 8);
+        default: LZ_SPLIT(8, 2, 12); break;   // (the largest is for 3 boards, which no longer fit)
     }
 #undef LZ_SPLIT
 }

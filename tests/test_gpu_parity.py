@@ -980,6 +980,17 @@ def test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batch
     pipe.close()
 
 
+@pytest.mark.parametrize("filters,batches", [
+    (64, (1, 5, 6, 8, 9)), (128, (1, 2, 3, 4, 5)), (192, (1, 2, 3)), (256, (1, 2, 3)),
+    (320, (1, 2)), (384, (1, 2)), (448, (1, 2)), (512, (1, 2)),
+    (24, (1, 5, 6)), (200, (1, 2)),           # padded to 64 and 256
+])
+def test_direct_convolution_tiles_of_16_channels(pkg, netgen, orc, filters, batches):
+    """The same for small handles, whose smallest tiles have 16 channels: both sides of every
+    change to the next one."""
+    test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches)
+
+
 @pytest.mark.parametrize("filters,maxb", [(128, 40), (192, 16), (192, 40), (256, 9), (384, 28), (512, 44)])
 def test_fp32_filters_of_no_3x3_filter(pkg, netgen, orc, filters, maxb):
     """fp32 networks whose filters are no 3x3 ones run the Winograd kernels: the streaming GEMM, the
