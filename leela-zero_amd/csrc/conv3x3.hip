@@ -388,7 +388,7 @@ bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
 // (96 boards 5.8 against 6.4 with 192x64).
 void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                     const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,
-                    hipStream_t s, LaunchTimer* t) {
+                    int lanes, hipStream_t s, LaunchTimer* t) {
     if (Kp % 64 != 0 || Cp % 64 != 0)
         throw std::invalid_argument("no direct convolution for this width");
     const int rows = n * kPts;
@@ -414,8 +414,20 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
             default: LZ_CONV(2, 1, 1, 4, 18, 3, 4, 1); return;
         }
     }
+    // One small tile to a unit: four wavefronts of 16 channels, so that every SIMD has one (with two of
+    // 32 the tile waited for its 54 steps of 96 cycles; the planes are now read from LDS twice as
+    // often, which the pipe has room for).  Against 48x64 on two wavefronts and 96x64 on four, a
+    // layer of 256 filters, 7 boards 7.8 -> 6.7 us, 9 boards 8.8 -> 7.4; 192 filters, 8 boards 6.4 ->
+    // 5.8, 13 boards 7.4 -> 6.4; two forwards side by side 0 to 7 % faster, three 1 to 8 % slower.  Not
+    // beyond: 96x64 on eight wavefronts, or with 16 channels to a wavefront, is 10 to 14 % slower than as below (16 boards of
+    // 256 filters), and 80x64 no faster.
     if (groups(48, 64) <= kUnits) {
-        LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
+        if (lanes <= 2) LZ_CONV(3, 1, 1, 4, 9, 3, 0, 2);
+        else LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
+        return;
+    }
+    if (groups(64, 64) <= kUnits && lanes <= 2) {
+        LZ_CONV(4, 1, 1, 4, 9, 3, 0, 2);
         return;
     }
     if (groups(96, 64) <= kUnits) {
@@ -442,9 +454,25 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
         LZ_CONV(4, 2, 2, 2, 6, 1, 0, 2);
         return;
     }
+    // More than a round of every tile.  What a forward with the device to itself takes is rounds times
+    // tile, whether the last round is full or nearly empty: 10 blocks of 256 filters, 69 to 90 boards
+    // 763 - 791 us on 192x128 and 588 - 649 on 128x128; of 384 filters, 46 to 60 boards 1059 - 1087 and
+    // 821 - 909; of 192 filters, 91 to 120 boards 637 - 659 on 128x192, 527 - 566 on 128x64, 135 boards
+    // 678 and 590 on 192x64.  Side by side with another forward, which fills the gaps, the tile
+    // that reads least is the best one.
+    auto rounds = [&](int mt, int cw) { return (groups(mt, cw) + kUnits - 1) / kUnits * mt * cw; };
+    if (lanes == 1 && Kp % 128 == 0 && rounds(128, 128) < rounds(192, 128)) {
+        LZ_CONV(4, 4, 2, 2, 3, 1, 0, 2);
+        return;
+    }
+    if (lanes == 1 && Kp % 128 != 0 && rounds(128, 64) < rounds(192, 64) &&
+        (Kp != 192 || rounds(128, 64) < rounds(128, 192))) {
+        LZ_CONV(4, 2, 2, 2, 6, 1, 0, 2);
+        return;
+    }
     if (Kp % 128 == 0)
         LZ_CONV(6, 4, 2, 2, 3, 1, 0, 2);
-    else if (Kp == 192)
+    else if (Kp == 192 && (lanes > 1 || rounds(128, 192) <= rounds(192, 64)))
         LZ_CONV(4, 6, 2, 2, 3, 1, 0, 2);
     else
         LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);

@@ -456,7 +456,7 @@ static PeakMap launch_f32_as(const float* X, const half_t* Wf, const float* res,
 PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, float* Y,
                            const float* bn_scale, const float* bn_mean, float rfac,
                            const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
-                           hipStream_t s, LaunchTimer* t) {
+                           int lanes, hipStream_t s, LaunchTimer* t) {
     if (Kp % 64 != 0 || Cp % 64 != 0)
         throw std::invalid_argument("no direct convolution for this width");
     const int rows = n * kPts;
@@ -473,8 +473,16 @@ PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, f
             default: return LZ_F32(2, 1, 1, 4, 9, 8, 1);
         }
     }
+    // Four wavefronts of 16 channels for up to two forwards side by side: a layer of 256 filters, 8
+    // boards 19.0 -> 15.5 us, 192 filters, 11 boards 15.0 -> 12.4 against two wavefronts of 32
+    // channels, and three forwards side by side 4 to 7 % slower.  64x64 gains 2 to 5 % on 96x64 for a
+    // forward with the device to itself and loses 14 % with three.
     if (groups(48, 64) <= kUnits) {
+        if (lanes <= 2) return LZ_F32(3, 1, 1, 4, 6, 0, 2);
         return LZ_F32(3, 2, 1, 2, 6, 0, 2);
+    }
+    if (lanes == 1 && groups(64, 64) <= kUnits) {
+        return LZ_F32(4, 1, 1, 4, 6, 0, 2);
     }
     if (groups(96, 64) <= kUnits) {
         return LZ_F32(3, 2, 2, 2, 6, 0, 2);
@@ -491,8 +499,17 @@ PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, f
     if ((Kp == 64 || Kp == 192) && groups(128, 64) <= 2 * kUnits) {
         return LZ_F32(4, 2, 2, 2, 6, 0, 2);
     }
+    // (launch_conv3x3's rule: 10 blocks of 256 filters, 70 boards 2002 us on 192x128 and 1518 on 128x128;
+    // of 384 filters, 47 boards 2889 and 2218; of 192 filters, 91 boards 1597 on 128x192 and 1306 on 128x64)
+    auto rounds = [&](int mt, int cw) { return (groups(mt, cw) + kUnits - 1) / kUnits * mt * cw; };
+    if (lanes == 1 && Kp % 128 == 0 && rounds(128, 128) < rounds(192, 128))
+        return LZ_F32(4, 4, 2, 2, 3, 0, 2);
+    if (lanes == 1 && Kp % 128 != 0 && rounds(128, 64) < rounds(192, 64) &&
+        (Kp != 192 || rounds(128, 64) < rounds(128, 192)))
+        return LZ_F32(4, 2, 2, 2, 6, 0, 2);
     if (Kp % 128 == 0) return LZ_F32(6, 4, 2, 2, 3, 0, 2);
-    if (Kp == 192) return LZ_F32(4, 6, 2, 2, 3, 0, 2);
+    if (Kp == 192 && (lanes > 1 || rounds(128, 192) <= rounds(192, 64)))
+        return LZ_F32(4, 6, 2, 2, 3, 0, 2);
     return LZ_F32(6, 2, 2, 2, 6, 0, 2);
 #undef LZ_F32
 }

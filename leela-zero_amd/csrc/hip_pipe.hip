@@ -781,7 +781,7 @@ public:
         launch_gemm<P>(V, U, Uf, M, Tu, m_Tp, Cp, m_Fp, ln.stream, nullptr);
         if (m_direct)
             conv_direct(L, a_in, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, peaks,
-                        peak_slots(peaks.slots, n, 0), n, ln.stream, nullptr);
+                        peak_slots(peaks.slots, n, 0), n, 1, ln.stream, nullptr);
         else
             launch_out_transform<P>(M, r, ln.act[2].p, d_sc.p, d_mn.p, 1.0f, n, m_Fp, m_Tp,
                                     ln.stream, nullptr);
@@ -861,6 +861,7 @@ private:
         P *act0 = nullptr, *act[3] = {nullptr, nullptr, nullptr}, *V = nullptr, *M = nullptr;
         int Tp = 0;
         uint32_t* peaks = nullptr;   // (direct fp32 towers)
+        int lanes = 2;               // forwards that may be running side by side (lanes_in_use)
     };
     // Slots of the input planes, then two sets that the layers write in turn.
     size_t peak_words(int n) const { return 2 * (size_t)n + 2 * conv3x3_f32_slots(m_Fp, n); }
@@ -928,7 +929,7 @@ private:
         Layer& L = m_layers[l];
         if (m_direct) {
             PeakMap none;
-            conv_direct(L, in, res, out, L.d_scale.p, L.d_mean.p, L.rfac, none, nullptr, n, ln.stream,
+            conv_direct(L, in, res, out, L.d_scale.p, L.d_mean.p, L.rfac, none, nullptr, n, 1, ln.stream,
                         timer(timed, LZHIP_K_GEMM));
             return;
         }
@@ -953,6 +954,15 @@ private:
     }
     void clear_graphs() {
         for (auto& ln : m_lane) clear_graphs(ln);
+    }
+    // On how many lanes this forward and the two before it were put: how much of the device it
+    // can expect for itself, which the direct convolutions' tiles depend on (the results do not).
+    int lanes_in_use(const Lane& ln) {
+        const uint32_t id = (uint32_t)(&ln - m_lane);
+        const uint32_t h = (m_recent.load(std::memory_order_relaxed) << 8 | id) & 0xffffffu;
+        m_recent.store(h, std::memory_order_relaxed);
+        const uint32_t b = h >> 8 & 255, c = h >> 16;
+        return 1 + (b != 255 && b != id) + (c != 255 && c != id && c != b);
     }
     // d_in: fp32 planes, or, when null, d_bits: the planes one bit per value
     void run_forward(Lane& ln, int n, const float* d_in, const uint32_t* d_bits, float* d_pol,
@@ -985,7 +995,9 @@ private:
     // output), and by the last layer for the 1x1 heads.
     void enqueue_forward(Lane& ln, int n, const float* d_in, const uint32_t* d_bits,
                          float* d_pol, float* d_val, bool timed) {
-        enqueue_forward(work_of(ln), n, d_in, d_bits, d_pol, d_val, timed);
+        Work w = work_of(ln);
+        w.lanes = timed ? 1 : lanes_in_use(ln);
+        enqueue_forward(w, n, d_in, d_bits, d_pol, d_val, timed);
     }
     void enqueue_forward(const Work& w, int n, const float* d_in, const uint32_t* d_bits,
                          float* d_pol, float* d_val, bool timed) {
@@ -1049,15 +1061,19 @@ private:
     // fp32: peaks are those of `in` and become those of `out`, which go to `slots`.
     void conv_direct(const Layer& L, const P* in, const P* res, P* out, const float* scale,
                      const float* mean, float rfac, PeakMap& peaks, uint32_t* slots, int n,
-                     hipStream_t s, LaunchTimer* t) {
+                     int lanes, hipStream_t s, LaunchTimer* t) {
         if constexpr (sizeof(P) == 2) {
             const bool split = L.Cp == m_Fp && conv3x3_splits(m_Fp, m_max_batch);
-            (split ? launch_conv3x3_split : launch_conv3x3)(in, L.W3.p, res, out, scale, mean, rfac,
-                                                            n, L.Cp, m_Fp, s, t);
+            if (split)
+                launch_conv3x3_split(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, s, t);
+            else
+                launch_conv3x3(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, lanes, s, t);
         } else {
             const bool split = L.Cp == m_Fp && conv3x3_f32_splits(m_Fp, m_max_batch);
-            peaks = (split ? launch_conv3x3_f32_split : launch_conv3x3_f32)(
-                in, L.W3.p, res, out, scale, mean, rfac, peaks, slots, n, L.Cp, m_Fp, s, t);
+            peaks = split ? launch_conv3x3_f32_split(in, L.W3.p, res, out, scale, mean, rfac, peaks,
+                                                     slots, n, L.Cp, m_Fp, s, t)
+                          : launch_conv3x3_f32(in, L.W3.p, res, out, scale, mean, rfac, peaks, slots,
+                                               n, L.Cp, m_Fp, lanes, s, t);
         }
     }
 
@@ -1073,7 +1089,8 @@ private:
             const P* in = l == 0 ? w.act0 : second ? w.act[1] : w.act[cur];
             P* out = l == 0 ? w.act[cur] : second ? w.act[nxt] : w.act[1];
             conv_direct(L, in, second ? w.act[cur] : nullptr, out, L.d_scale.p, L.d_mean.p, L.rfac,
-                        peaks, peak_slots(w.peaks, n, l), n, w.stream, timer(timed, LZHIP_K_GEMM));
+                        peaks, peak_slots(w.peaks, n, l), n, w.lanes, w.stream,
+                        timer(timed, LZHIP_K_GEMM));
             last = out;
             if (second) { const int o = cur; cur = nxt; nxt = o; }
         }
@@ -1198,6 +1215,7 @@ private:
         return e != nullptr && std::atoi(e) != 0;
     }();
     bool m_direct = false;               // direct convolutions (set by push_weights)
+    std::atomic<uint32_t> m_recent{0xffffffu};   // lanes of the last three forwards, a byte each
     bool m_in_place = true;              // tower layers keep V and M in one array (see enqueue_forward)
 };
 

@@ -108,13 +108,13 @@ void launch_out_in_transform(const P* M, const P* res, P* act_out, P* Vn, const 
 // Direct 3x3 convolution in fp16 (conv3x3.hip), one launch per layer:
 // X [Cp] -> Y [Kp] = min(max(0, scale*(conv - mean) + rfac*res), kActStoreMax), padded planes all three;
 // res may be null and is not Y.  Wf: conv3x3_filter_count elements, zero but for what
-// conv3x3_filters writes.
+// conv3x3_filters writes.  lanes: how many forwards may be running side by side.
 // Whether a handle for batches of up to max_batch computes by it (measured; see there).
 bool conv3x3_serves(int Kp, int max_batch, int elem_bytes);
 size_t conv3x3_filter_count(int Cp, int Kp);
 void launch_conv3x3(const _Float16* X, const _Float16* Wf, const _Float16* res, _Float16* Y,
                     const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp, int Kp,
-                    hipStream_t s, LaunchTimer* t);
+                    int lanes, hipStream_t s, LaunchTimer* t);
 // The same layer with its sum dealt to the wavefronts of a work-group: for batches that leave a
 // compute unit one tile.  It sums in another order, so a network takes one or the other for
 // all its batches: this one where conv3x3_splits(Kp, largest batch).  Cp == Kp.
@@ -140,7 +140,7 @@ size_t conv3x3_f32_slots(int Kp, int max_batch);
 PeakMap launch_conv3x3_f32(const float* X, const _Float16* Wf, const float* res, float* Y,
                            const float* bn_scale, const float* bn_mean, float rfac,
                            const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
-                           hipStream_t s, LaunchTimer* t);
+                           int lanes, hipStream_t s, LaunchTimer* t);
 // The same layer with its sum dealt to the wavefronts of a work-group (conv3x3_splits).
 bool conv3x3_f32_splits(int Kp, int max_batch);
 PeakMap launch_conv3x3_f32_split(const float* X, const _Float16* Wf, const float* res, float* Y,

@@ -918,6 +918,11 @@ def test_winograd_filters_of_no_3x3_filter(pkg, netgen, orc):
     (64, 137, (1, 22, 23, 34, 68, 69, 136, 137)), (128, 70, (1, 11, 12, 17, 34, 35, 68, 69, 70)),
     (192, 46, (1, 7, 8, 11, 22, 23, 45, 46)), (256, 36, (1, 5, 6, 8, 9, 17, 34, 35, 36)),
     (384, 24, (1, 3, 6, 11, 12, 23, 24)), (512, 18, (1, 4, 5, 9, 17, 18)),
+    # more than a round of every tile
+    (192, 121, (91, 121)), (256, 69, (69,)), (320, 28, (28,)),
+    # 64 points by 64 channels
+    (64, 46, (34, 35, 45, 46)), (128, 24, (17, 18, 22, 23, 24)), (192, 17, (11, 12, 15, 16, 17)),
+    (256, 13, (8, 9, 11, 12, 13)), (384, 8, (5, 6, 7, 8)),
     # 128 points: 64 and 128 channels
     (64, 103, (90, 91, 102, 103)), (128, 91, (44, 46, 90, 91)), (192, 61, (16, 30, 31, 60, 61)),
     (256, 46, (20, 22, 23, 45, 46)), (384, 31, (13, 14, 15, 30, 31)),
@@ -984,10 +989,16 @@ def test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batch
     (64, (1, 5, 6, 8, 9)), (128, (1, 2, 3, 4, 5)), (192, (1, 2, 3)), (256, (1, 2, 3)),
     (320, (1, 2)), (384, (1, 2)), (448, (1, 2)), (512, (1, 2)),
     (24, (1, 5, 6)), (200, (1, 2)),           # padded to 64 and 256
+    # a wavefront's 16 channels of tiles of 48 and of 64 points
+    (64, (34, 35, 45, 46)), (128, (17, 18, 22, 23)), (192, (11, 12, 15, 16)), (256, (8, 9, 11, 12)),
+    (384, (5, 6, 7, 8)), (512, (4, 5, 6)),
+    # more than a round of every tile, for a forward with the device to itself
+    (128, (136, 137, 181, 182)), (192, (90, 91, 120, 121, 136, 137)), (256, (68, 69, 90, 91, 137)),
+    (384, (45, 46, 60, 61)), (320, (27, 28, 36, 37)),
 ])
 def test_direct_convolution_tiles_of_16_channels(pkg, netgen, orc, filters, batches):
-    """The same for small handles, whose smallest tiles have 16 channels: both sides of every
-    change to the next one."""
+    """The same for the tiles of 16 channels, of small handles and of a wavefront: both sides of
+    every change to the next one."""
     test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches)
 
 
