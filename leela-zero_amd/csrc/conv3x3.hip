@@ -7,10 +7,12 @@
 // As an implicit GEMM a layer reads its planes once and its filters once per die, and the
 // fp16 matrix rate is high enough (v_mfma_f32_16x16x32_f16, fp32 accumulate) to do the
 // whole sum.  Measured per layer, a forward of 40 blocks of 256 filters divided by its 81 layers,
-// Winograd GEMM + fused transform -> this file: 64 boards 28.6 -> 25.2 us one forward at a time,
-// 24.5 -> 20.6 with two side by side; 200 boards 83 -> 65 (1.30 PFLOP/s; two side by side 1.41;
-// torch.mm of 8192 x 8192 fp16 matrices 1.19 to 1.33 on such cards); 16 boards 13.2 -> 10.3; 1 board
-// 9.1 -> 4.8.
+// Winograd GEMM + fused transform -> this file: 64 boards 28.6 -> 22.4 us one forward at a time,
+// 24.5 -> 19.8 with two side by side; 200 boards 83 -> 63 (1.36 PFLOP/s; torch.mm of 8192 x 8192 fp16
+// matrices 1.19 to 1.33 on such cards); 16 boards 13.2 -> 9.8; 1 board, on conv3x3_split_k, 9.1 -> 4.2.
+// What bounds it: with full tiles the matrix pipe, busy 56 % of a launch of 64 boards at the clock that
+// the card's power allows (2.1 GHz); with one round of small tiles a chain of latencies, the first
+// planes and filters, the tail, and the hand-over to the next layer.
 // It also rounds less: planes and 3x3 filters are the only values kept in half precision.
 #include <cmath>
 #include <stdexcept>
@@ -50,11 +52,10 @@ size_t conv3x3_filter_count(int Cp, int Kp) {
 //
 // Operands.  The filters are read once per work-group row of wavefronts straight from the
 // die's L2 into registers (a ring of D k-steps, so that D - 1 steps of matrix instructions
-// cover the latency); no two wavefronts of a work-group column share them through LDS because
-// the LDS pipe is the busier one: it delivers RB KiB per k-step and wavefront for RB * NB
-// instructions of 16 cycles, 256 / NB of its 128 bytes per cycle, against 256 / RB of the 64 that
-// the L1 delivers.  RB = 6, NB = 4 (50 % of one, 67 % of the other) is the tile for full
-// batches.  The planes pass through LDS because every value is used nine times: the cells a
+// cover the latency).  Per k-step a wavefront has RB KiB of planes from LDS and NB KiB of filters from
+// the L1 for RB * NB instructions of 16 cycles: 256 / NB of the LDS pipe's 256 bytes per cycle and 256 /
+// RB of the 64 that the L1 delivers.  RB = 6, NB = 4 (25 % of one, 67 % of the other) is the
+// tile for full batches.  The planes pass through LDS because every value is used nine times: the cells a
 // tile reaches are staged once per chunk of input channels, in an order that the fragment reads
 // take without bank conflicts (CellPitch), and the nine taps and two halves are immediate offsets of
 // one address per 16 points.
@@ -340,18 +341,18 @@ static void launch_conv_as(const half_t* X, const half_t* Wf, const half_t* res,
 // chain of latencies, that is where tiles of 96x64 make no more than one work-group per unit.
 // Measured per forward of 5 blocks, Winograd kernels -> this, us (one forward at a time | two | three
 // side by side):
-//   320 filters,  1 board 133 -> 60, 16: 250 -> 171 | 290 -> 260 | 366 -> 371, 64: 495 -> 459 | 856 -> 750
-//   384 filters,  8 boards 200 -> 137 | 237 -> 189 | 289 -> 270, 44: 459 -> 364 | 730 -> 622 | 1087 -> 908,
-//                 100: 842 -> 860 | 1716 -> 1384, 200: 1703 -> 1476 | 3379 -> 2789
-//   448 filters,  8 boards 215 -> 154, 12: 277 -> 225 | 327 -> 362 | 457 -> 565, 64: 716 -> 806 | 1341 -> 1427
-//   512 filters,  8 boards 238 -> 172, 10: 254 -> 240 | 324 -> 373 | 428 -> 545, 64: 784 -> 820 | 1486 -> 1519
-//   640 filters,  6 boards 289 -> 200 | 435 -> 330 | 595 -> 497, 8: 301 -> 293 | 441 -> 471 | 613 -> 743
-//   768 filters,  5 boards 278 -> 228 | 433 -> 381 | 591 -> 567, 16: 514 -> 534 | 857 -> 936
-//  1024 filters,  4 boards 396 -> 305 | 598 -> 525 | 822 -> 777, 64: 2229 -> 2972
+//   320 filters,  1 board 133 -> 52, 16: 250 -> 126 | 290 -> 202 | 366 -> 289, 64: 495 -> 406 | 856 -> 669
+//   384 filters,  8 boards 200 -> 126 | 237 -> 177 | 289 -> 257, 44: 459 -> 333 | 730 -> 604 | 1087 -> 905,
+//                 100: 842 -> 821 | 1716 -> 1365, 200: 1703 -> 1505 | 3379 -> 2833
+//   448 filters,  8 boards 215 -> 141, 12: 277 -> 225 | 327 -> 362 | 457 -> 565, 64: 716 -> 806 | 1341 -> 1427
+//   512 filters,  8 boards 238 -> 165, 10: 254 -> 240 | 324 -> 373 | 428 -> 545, 64: 784 -> 820 | 1486 -> 1519
+//   640 filters,  6 boards 289 -> 189 | 435 -> 322 | 595 -> 515, 8: 301 -> 293 | 441 -> 471 | 613 -> 743
+//   768 filters,  5 boards 278 -> 217 | 433 -> 373 | 591 -> 597, 16: 514 -> 534 | 857 -> 936
+//  1024 filters,  4 boards 396 -> 294 | 598 -> 516 | 822 -> 810, 64: 2229 -> 2972
 // Left out: 512 filters at 16 to 40 boards gain too (32: 572 -> 446 | 874 -> 780) and lose again
-// beyond.  Taken in: what loses one at a time and gains side by side, 384 filters at 100 boards
-// (567 tiles on 512 places) and 320 at 32 (276 -> 302 | 408 -> 383 | 616 -> 557); and the reverse,
-// 448 filters at 9 boards (214 -> 155 | 258 -> 240 | 336 -> 359).
+// beyond.  (The batches beyond each line were measured when the line was drawn.)  Taken in: what gains
+// one and two at a time and loses three side by side, 448 filters at 9 boards (214 -> 146 | 258 -> 242 |
+// 336 -> 388).
 // The batch is the handle's largest, so that a network keeps its filters in one order and a
 // position's result does not depend on what it is evaluated with.
 bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
@@ -489,13 +490,13 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // operand is fetched once, a wavefront stages its own input channels and waits for nobody, its
 // filters are in flight all at once (D = 9 HPW; two thirds of them where five or more wavefronts
 // share the registers), and the partial sums meet in LDS at the end, in the order of the wavefronts.
-// Measured per forward of 10 blocks, conv3x3_k -> this, us: 128 filters, 1 board 99 -> 82, 8 boards
+// Measured per forward of 10 blocks, conv3x3_k -> this with tiles of 32 channels, us: 128 filters, 1 board 99 -> 82, 8 boards
 // 110 -> 92; 192 filters, 1 board 120 -> 98, 5 boards 134 -> 114; 256 filters, 1 board 132 -> 104, 5
 // boards 150 -> 138; of 5 blocks, 1 board: 320 filters 105 -> 60, 384 116 -> 63, 448 131 -> 70, 512
 // 136 -> 76.
-// Tiles of 96x32, 96x64 and 192x64 points x channels were tried for larger batches and gave
-// nothing (256 filters, 16 boards 215 -> 212, 32 boards 318 -> 324; two forwards side by side
-// lost 10 %): there the partial sums' way through LDS, 2 KW RB NB KiB, costs what it saves.
+// Tiles of 80x32 and 96x32 points x channels for larger batches take 5 to 13 % off a forward
+// alone (20 blocks of 256 filters, 6 boards 322 -> 285 us) and add 10 to 24 % to two or three side by side,
+// of whose work-groups a unit then holds one; 96x64 and 192x64 gave nothing either way.
 // The order of the sum differs from conv3x3_k's, so a network uses one or the other whatever the
 // batch (conv3x3_splits).
 template <int RB, int NB, int KW, int HPW, int D>

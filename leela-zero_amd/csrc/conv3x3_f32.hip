@@ -786,7 +786,7 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
     return {slots, tile.rb * 16, Kp / (16 * tile.nb)};
 }
 
-// Tiles of up to 48 points come in grids of at most three work-groups per unit, larger ones have
+// Tiles of up to 64 points come in grids of at most three work-groups per unit, larger ones have
 // at least 96 points and 64 channels.
 size_t conv3x3_f32_slots(int Kp, int max_batch) {
     const size_t large = (size_t)(max_batch * kPts / 96 + 1) * (Kp / 64);
@@ -795,12 +795,12 @@ size_t conv3x3_f32_slots(int Kp, int max_batch) {
 
 // Which fp32 handles compute directly: all widths an fp32 network may have.  Measured per forward of
 // 4 blocks, Winograd kernels -> this, us (one forward at a time | two side by side):
-//    64 filters, 1 board 108 -> 46 | 130 -> 79, 8: 119 -> 56, 32: 173 -> 86, 64: 251 -> 94
-//   128 filters, 1 board 106 -> 54 | 131 -> 78, 8: 123 -> 71, 12: 142 -> 119, 32: 198 -> 121, 64: 351 -> 206
-//   192 filters, 1 board 140 -> 66, 8: 166 -> 142 | 236 -> 170, 32: 379 -> 240 | 543 -> 333, 64: 577 -> 378
-//   256 filters, 1 board 164 -> 73, 8: 203 -> 177 | 312 -> 217, 32: 479 -> 313 | 783 -> 503, 64: 818 -> 516
-//   384 filters, 1 board 211 -> 101, 4: 229 -> 231, 8: 353 -> 229, 32: 868 -> 636, 64: 1667 -> 1206
-//   512 filters, 1 board 392 -> 115, 8: 555 -> 314, 32: 2370 -> 921, 64: 2744 -> 1761
+//    64 filters, 1 board 108 -> 43 | 130 -> 80, 8: 119 -> 52, 32: 173 -> 80, 64: 251 -> 83
+//   128 filters, 1 board 106 -> 53 | 131 -> 85, 8: 123 -> 69, 12: 142 -> 83, 32: 198 -> 113, 64: 351 -> 184
+//   192 filters, 1 board 140 -> 66, 8: 166 -> 98 | 236 -> 130, 32: 379 -> 222 | 543 -> 328, 64: 577 -> 363
+//   256 filters, 1 board 164 -> 70, 8: 203 -> 116 | 312 -> 186, 32: 479 -> 300 | 783 -> 498, 64: 818 -> 503
+//   384 filters, 1 board 211 -> 99, 4: 229 -> 150, 8: 353 -> 226, 32: 868 -> 625, 64: 1667 -> 1204
+//   512 filters, 1 board 392 -> 116, 8: 555 -> 313, 32: 2370 -> 939, 64: 2744 -> 1749
 // Relative error of the raw policy | value planes against a float64 network, 8 boards: 6x128 8.7e-7 -> 4.2e-7 |
 // 6.6e-7 -> 3.2e-7 (handles of up to 11 positions 3.2e-7 | 2.4e-7), 15x192 4.4e-7 -> 2.7e-7 | 9.5e-7 ->
 // 6.0e-7, 40x256 5.5e-7 -> 5.2e-7 | 2.6e-6 -> 2.2e-6, 40x64 6.5e-7 -> 4.7e-7 | 6.9e-7 -> 5.0e-7, 30x384

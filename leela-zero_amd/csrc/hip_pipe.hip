@@ -39,6 +39,7 @@ typedef _Float16 half_t;
 //   V, M   2 x 36 x 256 x 256 x 4 B = 18 874 368
 //   act0   8 x 361 x 64 x 4 B       =    739 328
 //   act[3] 3 x 8 x 361 x 256 x 4 B  =  8 871 936      total 28 485 632 B (27.2 MiB)
+// (a direct tower lays its padded planes and the peaks there instead, 13.5 MB at most).
 // Every GPU the library runs on holds its own copy from module load to process end.
 // In host code `scratch` is only a handle for hipGetSymbolAddress: the address kernels
 // may use is the one resolved per device in static_scratch().
@@ -1013,10 +1014,11 @@ private:
             return;
         }
         launch_in_transform<P>(w.act0, w.V, n, m_C0p, w.Tp, w.stream, timer(timed, LZHIP_K_IN));
-        // With the streaming GEMM (fp32) the tower's layers work in place: M_l is written over
-        // V_l and V_{l+1} over M_l (see the kernels), so a lane's tiles are one array instead of
-        // two (59 MB less per lane at 64 boards of 256 filters), of which more stays in the
-        // 256 MB memory-side cache.  Layer 0 reads 64 padded planes and keeps its own output.
+        // With the streaming GEMM (fp32 networks whose filters are no 3x3 ones) the tower's layers
+        // work in place: M_l is written over V_l and V_{l+1} over M_l (see the kernels), so a
+        // lane's tiles are one array instead of two (59 MB less per lane at 64 boards of 256
+        // filters), of which more stays in the 256 MB memory-side cache.  Layer 0 reads 64
+        // padded planes and keeps its own output.
         P* tiles = w.M;
         const bool in_place = m_in_place && m_layers.size() > 1 &&
                               gemm_stream_shape(Tu, m_Fp, m_Fp, (int)sizeof(P)) &&
