@@ -10,6 +10,7 @@
 #include <cstdlib>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <tuple>
 #include <stdexcept>
@@ -842,6 +843,10 @@ public:
 
 private:
     typedef std::tuple<int, const void*, float*, float*> GraphKey;
+    struct LayersGraph {
+        int uses = 0;
+        hipGraphExec_t exec = nullptr;
+    };
     // A lane is a stream with the working buffers of one forward.  Two batches on two
     // lanes run side by side on the device: each kernel's start-up and tail overlap with
     // the other lane's work, which a single chain of dependent kernels cannot do.
@@ -852,6 +857,7 @@ private:
         DevBuf<P> act0, act[3], V, M;
         DevBuf<uint32_t> peaks;   // direct fp32 towers: peak_words
         std::map<GraphKey, hipGraphExec_t> graphs;
+        std::map<int, LayersGraph> layers;   // by 4 n + lanes in use
     };
     static constexpr int kLanes = 3;   // upper bound; m_n_lanes are in use
 
@@ -863,6 +869,7 @@ private:
         int Tp = 0;
         uint32_t* peaks = nullptr;   // (direct fp32 towers)
         int lanes = 2;               // forwards that may be running side by side (lanes_in_use)
+        std::map<int, LayersGraph>* layers = nullptr;   // the lane's (none: plain launches)
     };
     // Slots of the input planes, then two sets that the layers write in turn.
     size_t peak_words(int n) const { return 2 * (size_t)n + 2 * conv3x3_f32_slots(m_Fp, n); }
@@ -945,13 +952,17 @@ private:
     // With LZHIP_GRAPH=1 the launches of a forward (2 + one per layer of a direct tower; 2 + two
     // per layer with Winograd kernels) are captured once per (batch size, buffers) into a HIP
     // graph and replayed, which takes the launch work off the host thread.  Only kernel
-    // nodes are captured (no memsets or copies).  On the device the replay measured no faster
+    // nodes are captured (no memsets or copies).  On one lane the replay measured no faster
     // than stream launches (40x256 fp16 at batch 16: 0.84 against 0.83 ms; the gaps between
     // these kernels are drain and cache write-back, not launch latency), so plain stream
-    // launches are the default.
+    // launches are the default, but for small direct towers on several lanes
+    // (launch_layers_graph).
     void clear_graphs(Lane& ln) {
         for (auto& kv : ln.graphs) (void)hipGraphExecDestroy(kv.second);
         ln.graphs.clear();
+        for (auto& kv : ln.layers)
+            if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
+        ln.layers.clear();
     }
     void clear_graphs() {
         for (auto& ln : m_lane) clear_graphs(ln);
@@ -998,6 +1009,7 @@ private:
                          float* d_pol, float* d_val, bool timed) {
         Work w = work_of(ln);
         w.lanes = timed ? 1 : lanes_in_use(ln);
+        if (!m_use_graph) w.layers = &ln.layers;
         enqueue_forward(w, n, d_in, d_bits, d_pol, d_val, timed);
     }
     void enqueue_forward(const Work& w, int n, const float* d_in, const uint32_t* d_bits,
@@ -1080,7 +1092,8 @@ private:
     }
 
     // The layer loop of a direct tower: one launch per layer.
-    void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed) {
+    // All layers of a direct tower, from the packed planes to the last activation, which is returned.
+    const P* enqueue_layers(const Work& w, int n, bool timed) {
         const int nl = (int)m_layers.size();
         const P* last = w.act[0];
         PeakMap peaks{w.peaks, kPts, 1};
@@ -1096,6 +1109,77 @@ private:
             last = out;
             if (second) { const int o = cur; cur = nxt; nxt = o; }
         }
+        return last;
+    }
+    const P* last_activation(const Work& w) const {
+        return w.act[((int)m_layers.size() / 2) % 2 ? 2 : 0];
+    }
+    // The layers as one launch, of a graph that holds them for this lane and batch size: nothing but
+    // kernels, and between the lane's own buffers only, so that it is good for any caller's planes
+    // and results.  It takes the host thread off the layers' 3.5 us a launch, which is what bounds small
+    // networks on several lanes; on one lane, where the kernels are as long as their launches, plain
+    // launches are 3 to 8 % faster.  A graph is made the eighth time that a lane is given a batch size
+    // beside another lane, for eight batch sizes a lane at most.
+    bool launch_layers_graph(const Work& w, int n) {
+        if (!w.layers || w.lanes < 2 || !launch_bound(n)) return false;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(w.stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+            return false;
+        const int key = 4 * n + w.lanes;
+        auto it = w.layers->find(key);
+        if (it == w.layers->end()) {
+            if (w.layers->size() >= 8) return false;
+            it = w.layers->emplace(key, LayersGraph()).first;
+        }
+        LayersGraph& g = it->second;
+        if (!g.exec && ++g.uses == 8) g.exec = layers_graph(w, n);
+        if (!g.exec) return false;
+        HIP_CHECK(hipGraphLaunch(g.exec, w.stream));
+        return true;
+    }
+    // Recorded on a stream of its own that no other work is ordered against, so that a call of
+    // another thread on the default stream cannot meet the recording; null if the runtime declines.
+    hipGraphExec_t layers_graph(Work w, int n) {
+        hipGraph_t graph = nullptr;
+        hipGraphExec_t exec = nullptr;
+        hipStream_t s = nullptr;
+        HIP_CHECK(hipGetLastError());   // (the caller's own, before any of this)
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return nullptr;
+        w.stream = s;
+        if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+            std::exception_ptr failed;
+            try {
+                enqueue_layers(w, n, false);
+            } catch (...) {
+                failed = std::current_exception();
+            }
+            if (hipStreamEndCapture(s, &graph) != hipSuccess) graph = nullptr;
+            if (failed) {
+                if (graph) (void)hipGraphDestroy(graph);
+                (void)hipStreamDestroy(s);
+                std::rethrow_exception(failed);
+            }
+        }
+        if (graph && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess)
+            exec = nullptr;
+        if (graph) (void)hipGraphDestroy(graph);
+        (void)hipStreamDestroy(s);
+        if (!exec) (void)hipGetLastError();   // (what was declined is not the caller's error)
+        return exec;
+    }
+    // Whether the layers of two lanes take the device no longer than their launches take the host.
+    // 20 blocks on two lanes, plain launches -> graph, us for both forwards: fp16 64 filters 1 board 302 ->
+    // 114, 34: 314 -> 200, 90: 316 -> 268; 128 filters 1 board 296 -> 146, 12: 322 -> 249, 25: 318 -> 305, 35:
+    // 338 -> 343; 192 filters 8 boards 315 -> 287, 14: 351 -> 356; 256 filters 1 board 314 -> 190, 5: 326 ->
+    // 292, 8: 376 -> 373; 384 filters 1 board 324 -> 272, 3: 412 -> 415.  fp32 64 filters 1 board 312 -> 188, 16:
+    // 313 -> 299; 128 filters 1 board 236 to 301 -> 246, 8: 326 -> 333; 192 filters 1 board 325 -> 336.
+    bool launch_bound(int n) const {
+        return (size_t)n * m_Fp * m_Fp <= (sizeof(P) == 2 ? 5u * 256 * 256 : 8u * 64 * 64);
+    }
+    void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed) {
+        const int nl = (int)m_layers.size();
+        const P* last = last_activation(w);
+        if (timed || !launch_layers_graph(w, n)) last = enqueue_layers(w, n, timed);
         launch_head_conv<P>(last, true, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
                             timer(timed, LZHIP_K_HEAD));
     }

@@ -1072,3 +1072,55 @@ def test_heads_at_the_edges_of_their_tiles(pkg, netgen, orc, n):
     # (tanh has slope at most 1; its own error is a few units of the last place of 1)
     assert (np.abs(value - np.tanh(out[:, 0])) <= ob[:, 0] + 4 * 2.0 ** -24).all()
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,precision,sizes", [
+    (64, 1, (1, 3, 20)), (128, 1, (2, 20, 21)), (192, 1, (8, 9)), (256, 1, (1, 5, 6)), (64, 0, (1, 8, 9)),
+    (64, 1, tuple(range(1, 13))),
+])
+def test_layers_replayed_on_several_lanes(pkg, netgen, orc, filters, precision, sizes):
+    """Small forwards on two and on three lanes in turn: their layers are one launch of a graph from
+    the eighth use of a batch size on.  Every forward, with new planes each and work of the
+    program's own between them, gives the bits of another handle that runs one batch at a time; so do
+    more batch sizes than a lane keeps graphs of, and calls from three threads."""
+    import threading
+    import torch
+    print("case: replayed layers, %d filters, precision %d" % (filters, precision), flush=True)
+    maxb = max(max(sizes), 2)
+    net, plain, ref, h_ref = make_pipes(pkg, netgen, orc, 2, filters, 7300, precision, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, filters, 7300, precision, maxb)
+    rounds = 14 if len(sizes) < 4 else 10
+    x = netgen.synthetic_inputs(maxb + rounds, seed=7301)
+    want = {(n, r): plain.forward_batch(x[r:r + n]) for n in sizes for r in range(rounds)}
+    dev = torch.from_numpy(x).cuda()
+    for lanes in (2, pipe.lanes()):
+        for n in sizes:
+            outs = []
+            for r in range(rounds):
+                for k in range(lanes):
+                    p, v = torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")
+                    torch.cuda.synchronize()
+                    d = dev[r:r + n].contiguous()
+                    torch.cuda.synchronize()
+                    pipe.forward_batch_device(n, d.data_ptr(), p.data_ptr(), v.data_ptr(), lane=k)
+                    outs.append((r, d, p, v))
+                if r % 5 == 4:
+                    pipe.sync()
+            pipe.sync()
+            for r, _, p, v in outs:
+                assert np.array_equal(p.cpu().numpy(), want[n, r][0]), (lanes, n, r)
+                assert np.array_equal(v.cpu().numpy(), want[n, r][1]), (lanes, n, r)
+    wrong = []
+
+    def caller(n):
+        for r in range(rounds):
+            pol, val = pipe.forward_batch(x[r:r + n])
+            if not (np.array_equal(pol, want[n, r][0]) and np.array_equal(val, want[n, r][1])):
+                wrong.append((n, r))
+
+    th = [threading.Thread(target=caller, args=(sizes[i % len(sizes)],)) for i in range(3)]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    assert not wrong, wrong
+    pipe.close()
+    plain.close()
