@@ -138,11 +138,9 @@ public:
             throw std::runtime_error(std::string("device is ") + prop.gcnArchName +
                                      ", this library contains gfx950 code only");
         // Small batches leave more of the device idle at every kernel boundary.  Evaluations of
-        // all lanes, a third lane against two: 20x256 fp16, batch 16 to 32 -2..0 %, 40 and 48
-        // +10 %, 52 +7 %, 64 +2 %; 20x384 fp16, batch 16 to 48 +4..7 %; 20x192 fp32, batch 8 +30 %, 32
-        // +4 %, 48 -3 %, 64 -6 %; 20x256 fp32, batch 8 +24 %, 48 and 64 +3 %.  (At batches below 8 one
-        // host thread cannot feed three lanes.)  The line lies where it did for fp16 Winograd
-        // kernels; of today's only 192 filters in fp32 ask for it.
+        // all lanes, a third lane against two: 20x64 fp16, batch 8 +34 %; 20x128 fp16, batch 32 +1 %;
+        // 20x256 fp16, batch 16 +4 %, 32 +1 %, 40 +4 %; 20x192 fp32, batch 8 +1 %, 32 +10 %; 20x256 fp32,
+        // batch 8 -5 %, 48 +8 %.  The line lies where it did for fp16 Winograd kernels.
         m_n_lanes = max_batch <= 48 ? 3 : 2;
         if (const char* e = std::getenv("LZHIP_LANES")) {   // measurement knob: 1..3 lanes
             const int v = std::atoi(e);
