@@ -8,7 +8,9 @@
 // fp32.  2^e brings the operand to the top of half's range, so that lo is a normal number
 // down to 2^-17 of the largest and exact to 2^-39 of it below: for planes from the largest
 // activation of the board (each layer leaves it for the next), for filters from the largest weight of
-// the output channel.  Error against float64 is smaller than the Winograd kernels' (F(4x4,3x3)
+// the output channel.  Channels of different magnitude are brought together beforehand, by powers of two
+// in the filters and in the batch norm that leave every product as it is (balance_channels in
+// hip_pipe.hip); a network that this does not help runs the Winograd kernels.  Error against float64 is smaller than the Winograd kernels' (F(4x4,3x3)
 // amplifies fp32 rounding): figures at conv3x3_f32_serves.
 //
 // The matrix instruction drops bits of its products below the largest term's, downwards (measured: sums
@@ -876,29 +878,36 @@ __device__ __forceinline__ bool filter_3x3(const float* U, int C, int F, int c, 
     return ok;
 }
 
-// peak[k] (bits of a float, zero before): largest magnitude of the output channel's filters
-__global__ __launch_bounds__(256) void filters_f32_peak_k(const float* __restrict__ U, int C, int F,
-                                                          unsigned* __restrict__ peak,
+// Binary exponents of an output channel's largest filter (times 2^-in_exp of its input channel) and of
+// its largest product with an input channel of magnitude 2^mag; both kNoExp before.  (Maxima of
+// integers: the same whatever the order.)
+__global__ __launch_bounds__(256) void filters_f32_peak_k(const float* __restrict__ U,
+                                                          const int* __restrict__ in_exp,
+                                                          const int* __restrict__ mag, int C, int F,
+                                                          int* __restrict__ peak,
+                                                          int* __restrict__ reach,
                                                           int* __restrict__ bad) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= C * F) return;
     const int c = i / F, k = i - c * F;
     double f[3][3];
     if (!filter_3x3(U, C, F, c, k, f)) *bad = 1;
-    float top = 0.0f;
+    double top = 0.0;
 #pragma unroll
-    for (int tap = 0; tap < 9; tap++) top = fmaxf(top, fabsf((float)f[tap / 3][tap % 3]));
-    if (!(top < __builtin_inff())) *bad = 1;
-    atomicMax(peak + k, __builtin_bit_cast(unsigned, top));
-}
-
-// Exponent that the filters of an output channel are scaled by.
-__host__ __device__ static inline int filter_exponent(unsigned peak_bits) {
-    return peak_bits == 0 ? 0 : kFilterTop + 127 - (int)(peak_bits >> 23);
+    for (int tap = 0; tap < 9; tap++) top = fmax(top, fabs(f[tap / 3][tap % 3]));
+    if (!((float)top < __builtin_inff())) {
+        *bad = 1;
+        return;
+    }
+    if (!(top > 0.0)) return;
+    const int e = ilogb(top);
+    atomicMax(peak + k, e - in_exp[c]);
+    if (mag[c] != kNoExp) atomicMax(reach + k, e + mag[c]);
 }
 
 __global__ __launch_bounds__(256) void filters_f32_k(const float* __restrict__ U,
-                                                     const unsigned* __restrict__ peak,
+                                                     const int* __restrict__ in_exp,
+                                                     const int* __restrict__ exp,
                                                      half_t* __restrict__ Wf, int C, int Cp, int F,
                                                      int Kp) {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -906,7 +915,7 @@ __global__ __launch_bounds__(256) void filters_f32_k(const float* __restrict__ U
     const int c = i / F, k = i - c * F;
     double f[3][3];
     filter_3x3(U, C, F, c, k, f);
-    const double scale = ldexp(conv3x3_f32_negated(c, Cp) ? -1.0 : 1.0, filter_exponent(peak[k]));
+    const double scale = ldexp(conv3x3_f32_negated(c, Cp) ? -1.0 : 1.0, exp[k] - in_exp[c]);
 #pragma unroll
     for (int tap = 0; tap < 9; tap++) {
         const double v = f[tap / 3][tap % 3] * scale;
@@ -916,17 +925,38 @@ __global__ __launch_bounds__(256) void filters_f32_k(const float* __restrict__ U
     }
 }
 
-void conv3x3_f32_filters(const float* U, half_t* Wf, unsigned* peak, int C, int Cp, int F, int Kp,
-                         int* bad, hipStream_t s) {
-    const dim3 grid((unsigned)((C * F + 255) / 256));
-    hipLaunchKernelGGL(filters_f32_peak_k, grid, dim3(256), 0, s, U, C, F, peak, bad);
-    hipLaunchKernelGGL(filters_f32_k, grid, dim3(256), 0, s, U, peak, Wf, C, Cp, F, Kp);
+void conv3x3_f32_peaks(const float* U, const int* in_exp, const int* mag, int C, int F, int* peak,
+                       int* reach, int* bad, hipStream_t s) {
+    hipLaunchKernelGGL(filters_f32_peak_k, dim3((unsigned)((C * F + 255) / 256)), dim3(256), 0, s, U,
+                       in_exp, mag, C, F, peak, reach, bad);
 }
 
-float conv3x3_f32_unscale(unsigned peak_bits) { return std::ldexp(1.0f, -filter_exponent(peak_bits)); }
+void conv3x3_f32_filters(const float* U, const int* in_exp, const int* exp, half_t* Wf, int C, int Cp,
+                         int F, int Kp, hipStream_t s) {
+    hipLaunchKernelGGL(filters_f32_k, dim3((unsigned)((C * F + 255) / 256)), dim3(256), 0, s, U, in_exp,
+                       exp, Wf, C, Cp, F, Kp);
+}
 
-void conv3x3_f32_winograd_filters(const half_t* Wf, const unsigned* peak, int C, int Cp, int F, int Kp,
-                                  float* U) {
+// Where the halves lose what fp32 holds.  The lo half of a plane is exact to 2^-40 of the board's largest
+// value, that of a filter to 2^-36 of its output channel's largest.  If the largest product of an
+// output channel is at least 2^-14 of its largest filter times the largest input channel, either
+// error stays below 2^-22 of that product, as it is with operands of the full 22 bits.
+bool conv3x3_f32_holds(int peak, int reach, int top) {
+    return peak == kNoExp || top == kNoExp || reach >= peak + top - 14;
+}
+
+// The exponent of an output channel's filters: their largest comes to kFilterTop.  False if the batch
+// norm's numbers cannot take it in (scale * 2^(out_exp - e), mean * 2^e).
+bool conv3x3_f32_exponent(int peak, float scale, float mean, int out_exp, int& e) {
+    e = peak == kNoExp ? 0 : kFilterTop - peak;
+    auto fits = [](float v, int p) {
+        return !std::isfinite(v) || v == 0.0f || std::isnormal(std::ldexp(v, p));
+    };
+    return fits(scale, out_exp - e) && fits(mean, e);
+}
+
+void conv3x3_f32_winograd_filters(const half_t* Wf, const int* in_exp, const int* exp, int C, int Cp,
+                                  int F, int Kp, float* U) {
     const double s2 = std::sqrt(2.0);
     const double G[6][3] = {{1, 0, 0},
                             {-2.0 / 3, -s2 / 3, -1.0 / 3},
@@ -937,7 +967,7 @@ void conv3x3_f32_winograd_filters(const half_t* Wf, const unsigned* peak, int C,
     for (int k = 0; k < F; k++) {
         for (int c = 0; c < C; c++) {
             const double unscale =
-                std::ldexp(conv3x3_f32_negated(c, Cp) ? -1.0 : 1.0, -filter_exponent(peak[k]));
+                std::ldexp(conv3x3_f32_negated(c, Cp) ? -1.0 : 1.0, in_exp[c] - exp[k]);
             double f[9];
             for (int tap = 0; tap < 9; tap++)
                 f[tap] = unscale * ((double)Wf[conv3x3_f32_index(k, c, tap, 0, Kp)] +

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <condition_variable>
@@ -251,6 +252,8 @@ public:
             (void)hipStreamSynchronize(ln.stream);
             m_layers.clear();
             m_direct = false;
+            m_chan.clear();
+            m_in_scale.release();
             for (auto& l : m_lane) l.peaks.release();
             m_w3.release();
             m_s.clear();
@@ -320,9 +323,10 @@ public:
         }
         std::vector<float> w3((size_t)3 * m_Fp, 0.0f);
         for (int c = 0; c < F; c++) {
-            w3[c] = pol_w[c];
-            w3[m_Fp + c] = pol_w[F + c];
-            w3[2 * m_Fp + c] = val_w[c];
+            const int e = chan(n_layers, c);
+            w3[c] = std::ldexp(pol_w[c], -e);
+            w3[m_Fp + c] = std::ldexp(pol_w[F + c], -e);
+            w3[2 * m_Fp + c] = std::ldexp(val_w[c], -e);
         }
         m_w3.alloc(w3.size());
         HIP_CHECK(hipMemcpy(m_w3.p, w3.data(), w3.size() * sizeof(float), hipMemcpyHostToDevice));
@@ -334,65 +338,184 @@ public:
     }
 
     // Filters of the direct convolution for every layer; false (and nothing kept) if some layer's
-    // U is not the transform of 3x3 filters.
+    // U is not the transform of 3x3 filters, or fp32 operands do not fit into two halves.
     bool build_direct_filters(int n_layers, const float* const* U, const float* const* bn_mean,
                               const float* const* bn_scale) {
-        hipStream_t s = m_lane[0].stream;
-        const int F = m_filters;
         DevBuf<float> stage;
-        DevBuf<uint32_t> peak;
-        DevBuf<int> bad;
-        stage.alloc((size_t)kPos * F * (F > kInPlanes ? F : kInPlanes));
-        bad.alloc(1);
+        stage.alloc((size_t)kPos * m_filters * (m_filters > kInPlanes ? m_filters : kInPlanes));
         bool good = true;
-        for (int l = 0; l < n_layers && good; l++) {
-            Layer& L = m_layers[l];
-            const int C = l == 0 ? kInPlanes : F, Cp = l == 0 ? m_C0p : m_Fp;
-            HIP_CHECK(hipMemcpy(stage.p, U[l], sizeof(float) * (size_t)kPos * C * F,
-                                hipMemcpyHostToDevice));
-            if constexpr (sizeof(P) == 2) {
+        if constexpr (sizeof(P) == 2) {
+            hipStream_t s = m_lane[0].stream;
+            DevBuf<int> bad;
+            bad.alloc(1);
+            for (int l = 0; l < n_layers; l++) {
+                Layer& L = m_layers[l];
+                const int Cp = l == 0 ? m_C0p : m_Fp;
                 L.W3.alloc(conv3x3_filter_count(Cp, m_Fp));
-                conv3x3_filters(stage.p, L.W3.p, C, F, m_Fp, bad.p, s);
-            } else {
-                L.W3.alloc(conv3x3_f32_filter_count(Cp, m_Fp));
-                peak.alloc(F);
-                conv3x3_f32_filters(stage.p, L.W3.p, peak.p, C, Cp, F, m_Fp, bad.p, s);
+                conv3x3_filters(upload_filters(stage, U, l), L.W3.p, channels(l), m_filters, m_Fp, bad.p, s);
+                HIP_CHECK(hipGetLastError());
+                HIP_CHECK(hipStreamSynchronize(s));
             }
-            HIP_CHECK(hipGetLastError());
-            HIP_CHECK(hipStreamSynchronize(s));
-            if constexpr (sizeof(P) == 4) {
-                L.peak.resize(F);
-                HIP_CHECK(hipMemcpy(L.peak.data(), peak.p, sizeof(uint32_t) * F, hipMemcpyDeviceToHost));
-                // the filters' scales have to fit into the batch norm's numbers
-                for (int k = 0; k < F && good; k++) {
-                    const float u = conv3x3_f32_unscale(L.peak[k]);
-                    good = fits(bn_scale[l][k], u) && fits(bn_mean[l][k], 1.0f / u);
-                }
-            }
+            int is_bad = 0;
+            HIP_CHECK(hipMemcpy(&is_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost));
+            good = !is_bad;
+        } else {
+            good = build_split_filters(n_layers, U, bn_mean, bn_scale, stage);
         }
-        int is_bad = 0;
-        HIP_CHECK(hipMemcpy(&is_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost));
-        good = good && !is_bad;
-        if (!good)
+        if (!good) {
             for (auto& L : m_layers) {
                 L.W3.release();
-                L.peak.clear();
+                L.exp.clear();
             }
-        else
+            m_chan.clear();
+            m_in_scale.release();
+        } else {
             // the planes' borders are zero, whatever a push that failed has left there
             for (int i = 0; i < m_n_lanes; i++) {
                 Lane& ln = m_lane[i];
                 HIP_CHECK(hipMemset(ln.act0.p, 0, ln.act0.count * sizeof(P)));
                 for (auto& a : ln.act) HIP_CHECK(hipMemset(a.p, 0, a.count * sizeof(P)));
             }
+        }
         if (good && sizeof(P) == 4)
             for (int i = 0; i < m_n_lanes; i++)
                 m_lane[i].peaks.alloc(2 * conv3x3_f32_slots(m_Fp, m_max_batch) + 2 * (size_t)m_max_batch);
         return good;
     }
-    // Whether v times a power of two is exact: v is no number, zero, or stays a normal one.
-    static bool fits(float v, float power) {
-        return !std::isfinite(v) || v == 0.0f || std::isnormal(v * power);
+    int channels(int l) const { return l == 0 ? kInPlanes : m_filters; }
+    const float* upload_filters(DevBuf<float>& stage, const float* const* U, int l) {
+        HIP_CHECK(hipMemcpy(stage.p, U[l], sizeof(float) * (size_t)kPos * channels(l) * m_filters,
+                            hipMemcpyHostToDevice));
+        return stage.p;
+    }
+
+    // fp32.  A direct tower holds its operands as two halves, relative to the largest of a board and of an
+    // output channel, so channels whose activations lie far below others' would lose bits that fp32
+    // keeps.  What a channel's magnitude is, is estimated from the filters and the batch norm, layer by
+    // layer, as a binary exponent; where estimates of a layer differ by 2^8 or more, planes hold
+    // the smaller channels times a power of two (m_chan), which its producer's batch norm puts in and the
+    // next layer's filters and the heads take out.  Batch norm and ReLU commute with it, so every
+    // product is the one that it would be.  A network whose estimates agree is left as it is.
+    bool build_split_filters(int n_layers, const float* const* U, const float* const* bn_mean,
+                             const float* const* bn_scale, DevBuf<float>& stage) {
+        hipStream_t s = m_lane[0].stream;
+        const int F = m_filters;
+        const size_t wide = F > kInPlanes ? F : kInPlanes;
+        DevBuf<int> in_exp, mag, out;   // out: peak, reach, bad; then the filters' exponents
+        in_exp.alloc(wide);
+        mag.alloc(wide);
+        out.alloc(2 * (size_t)F + 1);
+        auto put = [](DevBuf<int>& d, const std::vector<int>& v) {
+            HIP_CHECK(hipMemcpy(d.p, v.data(), v.size() * sizeof(int), hipMemcpyHostToDevice));
+        };
+        // magnitudes of layer l's input channels: m[0] of the planes, m[l] of layer l - 1's output
+        std::vector<std::vector<int>> m(n_layers + 1, std::vector<int>(F, kNoExp));
+        m[0].assign(kInPlanes, 0);
+        m_chan.assign(n_layers + 1, std::vector<int>(F, 0));
+        m_chan[0] = plane_exponents(U[0]);
+        for (int pass = 0; pass < 2; pass++) {
+            bool holds = true;
+            for (int l = 0; l < n_layers; l++) {
+                Layer& L = m_layers[l];
+                const int C = channels(l), Cp = l == 0 ? m_C0p : m_Fp;
+                upload_filters(stage, U, l);
+                put(in_exp, m_chan[l]);
+                put(mag, m[l]);
+                std::vector<int> ends(2 * (size_t)F + 1, kNoExp);
+                ends[2 * F] = 0;
+                put(out, ends);
+                conv3x3_f32_peaks(stage.p, in_exp.p, mag.p, C, F, out.p, out.p + F, out.p + 2 * F,
+                                  s);
+                HIP_CHECK(hipGetLastError());
+                HIP_CHECK(hipStreamSynchronize(s));
+                HIP_CHECK(hipMemcpy(ends.data(), out.p, ends.size() * sizeof(int), hipMemcpyDeviceToHost));
+                if (ends[2 * F]) return false;
+                int top = kNoExp;
+                for (int c = 0; c < C; c++)
+                    if (m[l][c] != kNoExp) top = std::max(top, m[l][c] + m_chan[l][c]);
+                L.exp.resize(F);
+                for (int k = 0; k < F; k++) {
+                    holds = holds && (l == 0 || conv3x3_f32_holds(ends[k], ends[F + k], top)) &&
+                            conv3x3_f32_exponent(ends[k], bn_scale[l][k], bn_mean[l][k],
+                                                 m_chan[l + 1][k], L.exp[k]);
+                    if (pass == 0) {
+                        const bool second = l >= 2 && l % 2 == 0;
+                        m[l + 1][k] = std::max(second ? m[l - 1][k] : kNoExp,
+                                               magnitude(ends[F + k], bn_scale[l][k], bn_mean[l][k]));
+                    }
+                }
+                put(out, L.exp);
+                if (pass == 0) L.W3.alloc(conv3x3_f32_filter_count(Cp, m_Fp));
+                conv3x3_f32_filters(stage.p, in_exp.p, out.p, L.W3.p, C, Cp, F, m_Fp, s);
+                HIP_CHECK(hipGetLastError());
+                HIP_CHECK(hipStreamSynchronize(s));
+            }
+            if (pass == 1 || !balance_channels(m)) {
+                if (!holds) return false;
+                break;
+            }
+        }
+        std::vector<float> f(kInPlanes);
+        for (int c = 0; c < kInPlanes; c++) f[c] = std::ldexp(1.0f, m_chan[0][c]);
+        if (*std::min_element(f.begin(), f.end()) < 1.0f) {
+            m_in_scale.alloc(kInPlanes);
+            HIP_CHECK(hipMemcpy(m_in_scale.p, f.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
+        }
+        return true;
+    }
+    // Exponents of the input planes, at most 0: the engine's are 0 and 1, but a caller's may be of any
+    // magnitude, which the first layer's filters then make up for.  A plane whose filters are
+    // small in every output channel, beside that channel's largest, is taken down by as much.
+    std::vector<int> plane_exponents(const float* U) const {
+        const int F = m_filters;
+        std::vector<float> most(F, 0.0f), of((size_t)kInPlanes * F, 0.0f);
+        for (int p = 0; p < kPos; p++)
+            for (int c = 0; c < kInPlanes; c++)
+                for (int k = 0; k < F; k++) {
+                    const float v = std::fabs(U[((size_t)p * kInPlanes + c) * F + k]);
+                    most[k] = std::max(most[k], v);
+                    of[(size_t)c * F + k] = std::max(of[(size_t)c * F + k], v);
+                }
+        std::vector<int> e(kInPlanes, 0);
+        for (int c = 0; c < kInPlanes; c++) {
+            int best = kNoExp;
+            for (int k = 0; k < F; k++)
+                if (of[(size_t)c * F + k] > 0.0f)
+                    best = std::max(best, std::ilogb(of[(size_t)c * F + k]) - std::ilogb(most[k]));
+            if (best != kNoExp) e[c] = -std::min(-best / 8 * 8, 96);
+        }
+        return e;
+    }
+    // Exponent of what a channel puts out: its largest product, times what 9 F of them come to (a sum of
+    // F = 64 to 512 random ones is 4 to 12 times the largest), or its batch norm's constant.
+    static int magnitude(int reach, float scale, float mean) {
+        if (!std::isfinite(scale) || scale == 0.0f) return kNoExp;
+        const int s = std::ilogb(scale);
+        const int conv = reach == kNoExp ? kNoExp : s + reach + 3;
+        return std::isfinite(mean) && mean != 0.0f ? std::max(conv, s + std::ilogb(mean)) : conv;
+    }
+    // m_chan from the magnitudes: in whole 2^8, so that ordinary networks keep theirs, and by at most 2^64;
+    // the channels of the residual stream have one exponent throughout, by which none comes above
+    // the largest of its layer anywhere.  False: nothing to move.
+    bool balance_channels(const std::vector<std::vector<int>>& m) {
+        const int n_layers = (int)m.size() - 1, F = m_filters;
+        auto below = [&](int l, int k, int top) { return m[l][k] == kNoExp ? 64 : top - m[l][k]; };
+        std::vector<int> stream(F, 64);
+        bool moved = false;
+        for (int l = 1; l <= n_layers; l++) {
+            const int top = *std::max_element(m[l].begin(), m[l].end());
+            if (top == kNoExp) continue;
+            for (int k = 0; k < F; k++) {
+                if (l % 2) stream[k] = std::min(stream[k], below(l, k, top));
+                else if (m[l][k] != kNoExp) m_chan[l][k] = std::min(below(l, k, top), 64) / 8 * 8;
+            }
+        }
+        for (int l = 1; l <= n_layers; l++)
+            for (int k = 0; k < F; k++) {
+                if (l % 2) m_chan[l][k] = m[n_layers][k] == kNoExp ? 0 : stream[k] / 8 * 8;
+                moved = moved || m_chan[l][k] != 0;
+            }
+        return moved;
     }
 
     void alloc_tiles() {
@@ -729,24 +852,26 @@ public:
         HIP_CHECK(hipMemcpy(d_planes.p, act_in, sizeof(float) * (size_t)n * C * kPts, hipMemcpyHostToDevice));
         P* a_in = (layer == 0) ? ln.act0.p : ln.act[0].p;
         PeakMap peaks{ln.peaks.p, kPts, 1};
+        DevBuf<float> d_own;   // the planes as a forward holds them (m_chan)
         if constexpr (sizeof(P) == 4) {
-            if (m_direct)
-                launch_pack_input_peaks(d_planes.p, a_in, n, C, Cp, peaks.slots, ln.stream, nullptr);
+            if (m_direct) {
+                upload_planes(d_own, act_in, n, C, layer);
+                launch_pack_input_peaks(d_own.p, a_in, n, C, Cp, peaks.slots, nullptr, ln.stream, nullptr);
+            }
         }
         if (sizeof(P) == 2 || !m_direct)
             launch_pack_input<P>(d_planes.p, a_in, m_direct, n, C, Cp, ln.stream, nullptr);
         const P* r = nullptr;
         if (res) {
-            d_res.alloc((size_t)n * F * kPts);
-            HIP_CHECK(hipMemcpy(d_res.p, res, sizeof(float) * (size_t)n * F * kPts, hipMemcpyHostToDevice));
+            upload_planes(d_res, res, n, F, layer + 1);
             launch_pack_input<P>(d_res.p, ln.act[1].p, m_direct, n, F, m_Fp, ln.stream, nullptr);
             r = ln.act[1].p;
         }
         std::vector<float> sc(m_Fp, 0.0f), mn(m_Fp, 0.0f);
         for (int k = 0; k < F; k++) {
-            const float u = L.peak.empty() ? 1.0f : conv3x3_f32_unscale(L.peak[k]);
-            sc[k] = L.scale[k] * u;
-            mn[k] = L.mean[k] / u;
+            const int e = L.exp.empty() ? 0 : L.exp[k];
+            sc[k] = std::ldexp(L.scale[k], chan(layer + 1, k) - e);
+            mn[k] = std::ldexp(L.mean[k], e);
         }
         d_sc.alloc(m_Fp); d_mn.alloc(m_Fp);
         HIP_CHECK(hipMemcpy(d_sc.p, sc.data(), sizeof(float) * m_Fp, hipMemcpyHostToDevice));
@@ -763,7 +888,8 @@ public:
             if constexpr (sizeof(P) == 2)
                 conv3x3_winograd_filters(w3.data(), C, Cp, F, m_Fp, u.data());
             else
-                conv3x3_f32_winograd_filters(w3.data(), L.peak.data(), C, Cp, F, m_Fp, u.data());
+                conv3x3_f32_winograd_filters(w3.data(), m_chan[layer].data(), L.exp.data(), C, Cp, F, m_Fp,
+                                             u.data());
             d_U.alloc(u.size());
             HIP_CHECK(hipMemcpy(d_U.p, u.data(), u.size() * sizeof(P), hipMemcpyHostToDevice));
             d_V.alloc((size_t)kPos * m_Tp * m_Fp);
@@ -813,8 +939,15 @@ public:
                 for (int pt = 0; pt < kPts; pt++)
                     for (int k = 0; k < F; k++)
                         Yout[((size_t)b * F + k) * kPts + pt] =
-                            (float)h[plane_index(m_direct, b, pt) * m_Fp + k];
+                            std::ldexp((float)h[plane_index(m_direct, b, pt) * m_Fp + k], -chan(layer + 1, k));
         }
+    }
+    // Planes [n][C][361], of layer l's input channels, times 2^m_chan, to the device.
+    void upload_planes(DevBuf<float>& d, const float* planes, int n, int C, int l) {
+        std::vector<float> h(planes, planes + (size_t)n * C * kPts);
+        for (size_t i = 0; i < h.size(); i++) h[i] = std::ldexp(h[i], chan(l, (int)(i / kPts % C)));
+        d.alloc(h.size());
+        HIP_CHECK(hipMemcpy(d.p, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
     }
 
     // -------------------------------------------------------------------
@@ -893,7 +1026,7 @@ private:
         DevBuf<P> U;                          // [36][Fp][Cp] (tiled GEMMs)
         DevBuf<P> Uf;                         // fragment order of the streaming GEMM
         DevBuf<half_t> W3;                    // 3x3, fragment order of the direct convolution
-        std::vector<uint32_t> peak;           // (fp32) largest of each output channel's W3
+        std::vector<int> exp;                 // (fp32) exponent of each output channel's W3
         std::vector<float> mean, scale;       // as pushed (unscaled)
         DevBuf<float> d_mean, d_scale;        // with activation scales folded in
         float rfac = 1.0f;
@@ -911,9 +1044,9 @@ private:
         const float s_in = m_s[l], s_out = m_s[l + 1];
         std::vector<float> sc(m_Fp, 0.0f), mn(m_Fp, 0.0f);
         for (int k = 0; k < m_filters; k++) {
-            const float u = L.peak.empty() ? 1.0f : conv3x3_f32_unscale(L.peak[k]);
-            sc[k] = L.scale[k] * (s_in / s_out) * u;
-            mn[k] = L.mean[k] / s_in / u;
+            const int e = L.exp.empty() ? 0 : L.exp[k];
+            sc[k] = std::ldexp(L.scale[k] * (s_in / s_out), chan(l + 1, k) - e);
+            mn[k] = std::ldexp(L.mean[k] / s_in, e);
         }
         const bool second = l >= 2 && (l % 2) == 0;
         L.rfac = second ? m_s[l - 1] / s_out : 1.0f;
@@ -1016,7 +1149,8 @@ private:
         const int Tu = n * kTilesPerBoard;
         LaunchTimer* pack = timer(timed, LZHIP_K_PACK);
         if (!d_in)
-            launch_pack_input_bits<P>(d_bits, w.act0, m_direct, n, kInPlanes, m_C0p, w.peaks, w.stream, pack);
+            launch_pack_input_bits<P>(d_bits, w.act0, m_direct, n, kInPlanes, m_C0p, w.peaks, m_in_scale.p,
+                                      w.stream, pack);
         else if (!pack_with_peaks(w, d_in, n, pack))
             launch_pack_input<P>(d_in, w.act0, m_direct, n, kInPlanes, m_C0p, w.stream, pack);
         if (m_direct) {
@@ -1062,7 +1196,8 @@ private:
     bool pack_with_peaks(const Work& w, const float* d_in, int n, LaunchTimer* t) {
         if constexpr (sizeof(P) == 4) {
             if (w.peaks) {
-                launch_pack_input_peaks(d_in, w.act0, n, kInPlanes, m_C0p, w.peaks, w.stream, t);
+                launch_pack_input_peaks(d_in, w.act0, n, kInPlanes, m_C0p, w.peaks, m_in_scale.p, w.stream,
+                                        t);
                 return true;
             }
         }
@@ -1299,6 +1434,10 @@ private:
         return e != nullptr && std::atoi(e) != 0;
     }();
     bool m_direct = false;               // direct convolutions (set by push_weights)
+    // (direct fp32) planes of layer l's input channel c are held times 2^m_chan[l][c]; the last: the heads'
+    std::vector<std::vector<int>> m_chan;
+    DevBuf<float> m_in_scale;            // 2^m_chan[0], or none where all of it is 0
+    int chan(int l, int c) const { return m_chan.empty() ? 0 : m_chan[l][c]; }
     std::atomic<uint32_t> m_recent{0xffffffu};   // lanes of the last three forwards, a byte each
     bool m_in_place = true;              // tower layers keep V and M in one array (see enqueue_forward)
 };

@@ -54,16 +54,16 @@ struct PeakMap {
     uint32_t* slots = nullptr;
     int mt = 0, tiles_n = 0;
 };
-// (peaks: null, or 2 n slots of input planes, one tile a board)
+// (peaks: null, or 2 n slots of input planes, one tile a board; scale: null, or a factor per plane)
 template <typename P>
 void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, int C, int Cp,
-                            uint32_t* peaks, hipStream_t s, LaunchTimer* t);
+                            uint32_t* peaks, const float* scale, hipStream_t s, LaunchTimer* t);
 template <typename P>
 void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int Cp, hipStream_t s,
                        LaunchTimer* t);
 // The same with the peaks; padded.
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
-                             hipStream_t s, LaunchTimer* t);
+                             const float* scale, hipStream_t s, LaunchTimer* t);
 
 // act [n][361][Cp] -> V [36][Tp][Cp]
 template <typename P>
@@ -131,9 +131,9 @@ void conv3x3_winograd_filters(const _Float16* Wf, int C, int Cp, int F, int Kp, 
 
 // Direct 3x3 convolution of fp32 towers (conv3x3_f32.hip), one launch per layer:
 // X [Cp] -> Y [Kp] = max(0, scale*(conv - mean) + rfac*res) in fp32, padded planes, every operand split in
-// two half-precision numbers.  Wf holds the filters of output channel k times 2^e(k):
-// conv3x3_f32_unscale(peak[k]) = 2^-e(k) belongs into scale, 2^e(k) into mean.  peaks: of X; those of Y
-// go to `slots` (conv3x3_f32_slots words) and are returned.
+// two half-precision numbers.  Wf holds the filters of output channel k and input channel c times
+// 2^(exp[k] - in_exp[c]): X holds channel c times 2^in_exp[c], scale is the caller's times 2^(out_exp[k]
+// - exp[k]), mean times 2^exp[k], and Y comes out times 2^out_exp[k].  peaks: of X; those of Y go to `slots` (conv3x3_f32_slots words) and are returned.
 bool conv3x3_f32_serves(int Kp);
 size_t conv3x3_f32_filter_count(int Cp, int Kp);
 size_t conv3x3_f32_slots(int Kp, int max_batch);
@@ -147,12 +147,19 @@ PeakMap launch_conv3x3_f32_split(const float* X, const _Float16* Wf, const float
                                  const float* bn_scale, const float* bn_mean, float rfac,
                                  const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
                                  hipStream_t s, LaunchTimer* t);
-// Filters of one layer and their peaks (F values, zero before) from U [36][C][F]; *bad as above.
-void conv3x3_f32_filters(const float* U, _Float16* Wf, uint32_t* peak, int C, int Cp, int F, int Kp,
-                         int* bad, hipStream_t s);
-float conv3x3_f32_unscale(uint32_t peak_bits);
-void conv3x3_f32_winograd_filters(const _Float16* Wf, const uint32_t* peak, int C, int Cp, int F, int Kp,
-                                  float* U);
+// Of every output channel of U [36][C][F]: the exponents of its largest filter times 2^-in_exp and of its
+// largest product with inputs of magnitude 2^mag (kNoExp before; kNoExp: none); *bad as above.
+constexpr int kNoExp = -(1 << 28);
+void conv3x3_f32_peaks(const float* U, const int* in_exp, const int* mag, int C, int F, int* peak,
+                       int* reach, int* bad, hipStream_t s);
+// Whether halves hold what fp32 does: exponents as above, of inputs of magnitude up to 2^top.
+bool conv3x3_f32_holds(int peak, int reach, int top);
+bool conv3x3_f32_exponent(int peak, float scale, float mean, int out_exp, int& e);
+// Filters of one layer from U (device), exponents per channel (device).
+void conv3x3_f32_filters(const float* U, const int* in_exp, const int* exp, _Float16* Wf, int C, int Cp,
+                         int F, int Kp, hipStream_t s);
+void conv3x3_f32_winograd_filters(const _Float16* Wf, const int* in_exp, const int* exp, int C, int Cp,
+                                  int F, int Kp, float* U);
 
 // 1x1 head convolutions: act [n][361][Cp] x w[3][Cp] -> pol [n][2][361], val [n][361],
 // both multiplied by out_scale.

@@ -148,45 +148,51 @@ void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int C
 template <typename P>
 __global__ __launch_bounds__(512) void pack_input_bits_k(const uint32_t* __restrict__ bits,
                                                          P* __restrict__ act, bool padded, int C,
-                                                         int Cp, uint32_t* __restrict__ peaks) {
+                                                         int Cp, uint32_t* __restrict__ peaks,
+                                                         const float* __restrict__ scale) {
     __shared__ uint32_t words[kInputWords];
     const int b = blockIdx.x, i = blockIdx.y * 512 + threadIdx.x, pt = i >> 2;
     if (threadIdx.x < kInputWords)
         words[threadIdx.x] = bits[(size_t)b * kInputWords + threadIdx.x];
-    if (peaks && i < 2) peaks[2 * (size_t)b + i] = 0x3f800000u;
+    if (peaks && i < 2) peaks[2 * (size_t)b + i] = 0x3f800000u;   // (no factor is above 1)
     __syncthreads();
     if (pt >= kPts) return;
     pack_point(act + plane_index(padded, b, pt) * Cp, i & 3, C, Cp, [&](int c) {
         const int bit = c * kPts + pt;
-        return (float)((words[bit >> 5] >> (bit & 31)) & 1u);
+        const float v = (float)((words[bit >> 5] >> (bit & 31)) & 1u);
+        return scale ? v * scale[c] : v;
     });
 }
 
 template <typename P>
 void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, int C, int Cp,
-                            uint32_t* peaks, hipStream_t s, LaunchTimer* t) {
+                            uint32_t* peaks, const float* scale, hipStream_t s, LaunchTimer* t) {
     launch(pack_input_bits_k<P>, dim3(n, (kPackThreads + 511) / 512), dim3(512), s, t, bits, act,
-           padded, C, Cp, peaks);
+           padded, C, Cp, peaks, scale);
 }
 
 // Planes and peaks from float planes: the first work-group of a board packs nothing and reads all
 // of it (26 KB); three pack.
 __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restrict__ in,
                                                           float* __restrict__ act, int C, int Cp,
-                                                          uint32_t* __restrict__ peaks) {
+                                                          uint32_t* __restrict__ peaks,
+                                                          const float* __restrict__ scale) {
     const int b = blockIdx.x, tid = threadIdx.x;
     const float* planes = in + (size_t)b * C * kPts;
     if (blockIdx.y > 0) {
         const int i = (blockIdx.y - 1) * 512 + tid, pt = i >> 2;
         if (pt < kPts)
             pack_point(act + plane_index(true, b, pt) * Cp, i & 3, C, Cp,
-                       [&](int c) { return planes[(size_t)c * kPts + pt]; });
+                       [&](int c) {
+                           const float v = planes[(size_t)c * kPts + pt];
+                           return scale ? v * scale[c] : v;
+                       });
         return;
     }
     float top = 0.0f;
 #pragma unroll 13
     for (int i = tid; i < C * kPts; i += 512) {
-        const float v = fabsf(planes[i]);
+        const float v = fabsf(scale ? planes[i] * scale[i / kPts] : planes[i]);
         top = fmaxf(top, v < __builtin_inff() ? v : 0.0f);
     }
     __shared__ float tops[8];
@@ -201,9 +207,9 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
 }
 
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
-                             hipStream_t s, LaunchTimer* t) {
+                             const float* scale, hipStream_t s, LaunchTimer* t) {
     launch(pack_input_peaks_k, dim3(n, 1 + (kPackThreads + 511) / 512), dim3(512), s, t, in, act, C,
-           Cp, peaks);
+           Cp, peaks, scale);
 }
 
 __global__ __launch_bounds__(256) void clear_k(int4v* p, size_t n) {
@@ -2148,7 +2154,8 @@ void launch_heads(const float* pol, const float* val, HeadParams hp, float tempe
     template void launch_pack_input<P>(const float*, P*, bool, int, int, int, hipStream_t,     \
                                        LaunchTimer*);                                          \
     template void launch_pack_input_bits<P>(const uint32_t*, P*, bool, int, int, int,          \
-                                            uint32_t*, hipStream_t, LaunchTimer*);             \
+                                            uint32_t*, const float*, hipStream_t,              \
+                                            LaunchTimer*);                                     \
     template void launch_in_transform<P>(const P*, P*, int, int, int, hipStream_t,             \
                                          LaunchTimer*);                                        \
     template void launch_gemm<P>(const P*, const P*, const P*, P*, int, int, int, int,         \
