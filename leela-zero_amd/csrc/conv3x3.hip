@@ -789,7 +789,7 @@ __global__ __launch_bounds__(256) void filters_3x3_k(const float* __restrict__ U
 #pragma unroll
         for (int x = 0; x < 6; x++) {
             const float v = g[0] * kG[x][0] + g[1] * kG[x][1] + g[2] * kG[x][2];
-            ok = ok && fabsf(v - u[y][x]) <= 1e-4f * peak;
+            ok = ok && fabsf(v - u[y][x]) <= 1e-4f * peak + kFilterFloor;
         }
     }
     if (!ok) *bad = 1;

@@ -18,6 +18,7 @@
 // nothing where they are negative).  Over a tower's layers that adds up, so the filters of the second
 // half of a layer's input channels are stored negated and the sum changes its sign in between: what
 // the one half loses the other gains.
+#include <algorithm>
 #include <cmath>
 #include <stdexcept>
 #include <type_traits>
@@ -815,7 +816,8 @@ bool conv3x3_f32_serves(int Kp) { return Kp % 64 == 0 && Kp <= 512; }
 // f = P U P^T with P = (G^T G)^-1 G^T, the least-squares solution, so that the rounding of U is
 // averaged.  Every filter is checked by transforming it forward again: *bad is set if some u is
 // further from G f G^T than the rounding of a transform in single precision explains (such a U
-// is no transform of a 3x3 filter, and only the Winograd kernels can compute with it).
+// is no transform of a 3x3 filter, and only the Winograd kernels can compute with it); below the smallest
+// normal number, 2^-126, rounding is no longer relative, and may be down to zero.
 __device__ constexpr double kS2 = 1.4142135623730951;
 __device__ constexpr double kGd[6][3] = {{1.0, 0.0, 0.0},
                                          {-2.0 / 3, -kS2 / 3, -1.0 / 3},
@@ -872,7 +874,7 @@ __device__ __forceinline__ bool filter_3x3(const float* U, int C, int F, int c, 
 #pragma unroll
         for (int x = 0; x < 6; x++) {
             const double v = g[0] * kGd[x][0] + g[1] * kGd[x][1] + g[2] * kGd[x][2];
-            ok = ok && fabs(v - U[((size_t)(y * 6 + x) * C + c) * F + k]) <= 4e-6 * peak;
+            ok = ok && fabs(v - U[((size_t)(y * 6 + x) * C + c) * F + k]) <= 4e-6 * peak + kFilterFloor;
         }
     }
     return ok;
@@ -945,14 +947,17 @@ bool conv3x3_f32_holds(int peak, int reach, int top) {
     return peak == kNoExp || top == kNoExp || reach >= peak + top - 14;
 }
 
-// The exponent of an output channel's filters: their largest comes to kFilterTop.  False if the batch
-// norm's numbers cannot take it in (scale * 2^(out_exp - e), mean * 2^e).
+// The exponent of an output channel's filters: their largest comes to kFilterTop, or as far towards it as
+// the batch norm's numbers can take in (scale * 2^(out_exp - e), mean * 2^e).  They are the limit where
+// filters have decayed to nothing: by then the convolution is less than 2^-100 of the mean, or of
+// what channels of the same exponent hold.  False: no exponent does.
 bool conv3x3_f32_exponent(int peak, float scale, float mean, int out_exp, int& e) {
     e = peak == kNoExp ? 0 : kFilterTop - peak;
-    auto fits = [](float v, int p) {
-        return !std::isfinite(v) || v == 0.0f || std::isnormal(std::ldexp(v, p));
-    };
-    return fits(scale, out_exp - e) && fits(mean, e);
+    if (std::isfinite(mean) && mean != 0.0f) e = std::min(e, 126 - std::ilogb(mean));
+    if (!std::isfinite(scale) || scale == 0.0f) return true;
+    const int s = std::ilogb(scale) + out_exp;
+    e = std::min(e, s + 126);
+    return s - e <= 126;
 }
 
 void conv3x3_f32_winograd_filters(const half_t* Wf, const int* in_exp, const int* exp, int C, int Cp,

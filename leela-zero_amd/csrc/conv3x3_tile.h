@@ -137,6 +137,10 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvGrid& g) {
 
 constexpr int kUnits = 256;   // compute units
 
+// What a transformed filter may be off by however small it is: a few sums of numbers that were rounded
+// to zero below 2^-126.
+constexpr float kFilterFloor = 0x1p-123f;
+
 // filters, planes: bytes of a layer's filters and of its input planes
 static inline ConvGrid conv_grid(int tiles_m, int tiles_n, size_t filters, size_t planes) {
     ConvGrid best{};

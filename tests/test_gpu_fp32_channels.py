@@ -173,3 +173,28 @@ def test_layer_with_channels_of_any_magnitude(pkg, netgen, orc, filters, maxb, l
         assert rel_l2(V[i] * back[None, :, None], Vr * back[None, :, None]) <= 1e-5
         assert rel_l2(M[i] * own[0], Mr * own[0]) <= 1e-5
     pipe.close()
+
+
+@pytest.mark.parametrize("precision,filters,maxb", [(0, 64, 4), (0, 128, 40), (1, 128, 40)])
+@pytest.mark.parametrize("size", [1e-40, 1e-42, 3e-36, 1e-30])
+def test_dead_channels_keep_the_direct_kernels(pkg, netgen, precision, filters, maxb, size):
+    """Output channels whose filters have decayed to nearly nothing, below the smallest normal number
+    among them, change neither the results nor the kernels of the others."""
+    print("case: dead channels of %g, precision %d, %d filters" % (size, precision, filters), flush=True)
+    n = 3
+    net = netgen.make_network(2, filters, 8500)
+    rng = np.random.default_rng(8501)
+    for l, k in ((0, 3), (1, 5), (2, 7), (3, 9), (4, 1)):
+        net.conv_w[l][k] = (rng.standard_normal(net.conv_w[l][k].shape) * size).astype(np.float32)
+    net.bn_mean[1][5] = 0.0      # a channel that is dead altogether
+    net.bn_mean[0][3] = 0.0
+    net.bn_var[3][9] = 0.0       # ... and one with the statistics of such a channel
+    x = netgen.synthetic_inputs(n, seed=8502)
+    want = tower_f64(net, x)
+    pipe = make_pipe(pkg, netgen, net, maxb, precision)
+    assert is_direct(pkg, pipe, x)
+    pol, val = pipe.forward_batch(x)
+    tol = 1e-5 if precision == 0 else 2e-2
+    for i in range(n):
+        assert rel_l2(pol[i], want["pol"][i]) <= tol and rel_l2(val[i], want["val"][i]) <= tol, i
+    pipe.close()
