@@ -551,7 +551,9 @@ public:
     // the stream is being captured into a graph no event is recorded or waited for (the
     // captured launches are then ordered by the graph's own dependencies, and replays
     // that overlap with other users of the array race).  The borders of a direct tower's planes are
-    // cleared by each call (another handle's may lie elsewhere); nothing else has to start at
+    // cleared by each call (another handle's may lie elsewhere), by the kernel that packs its input: a
+    // launch of its own for all of the planes cost a call of 1 to 6 blocks 1 to 9 us in fp16 (6x128, 8
+    // positions, with the device to itself: 83, now 71 to 75).  Nothing else has to start at
     // zero: every element a kernel reads for a real tile is written earlier in the same call (rows
     // of V past the last tile feed only rows of M that no kernel reads).
     void forward_device_static(int n, const float* d_in, float* d_pol, float* d_val) override {
@@ -571,7 +573,7 @@ public:
         Work w;
         w.stream = ln.stream;
         w.Tp = kStaticTp;
-        size_t clear = 0;
+        PlaneBorders borders;
         if (m_direct) {
             // a direct tower has no tiles: its planes, padded and one after the other, are all
             // there is, and in fp32 the peaks behind them
@@ -579,14 +581,19 @@ public:
             w.act0 = reinterpret_cast<P*>(base);
             for (int i = 0; i < 3; i++)
                 w.act[i] = reinterpret_cast<P*>(base + cells * (m_C0p + i * m_Fp));
-            clear = cells * (m_C0p + 3 * m_Fp);
-            size_t need = clear;
+            size_t need = cells * (m_C0p + 3 * m_Fp);
             if (sizeof(P) == 4) {
-                w.peaks = reinterpret_cast<uint32_t*>(base + clear);
+                w.peaks = reinterpret_cast<uint32_t*>(base + need);
                 need += peak_words(n) * sizeof(uint32_t);
             }
             if (need > kStaticBytes)
                 throw std::invalid_argument("no room in the static working memory");
+            constexpr int piece = 16 / sizeof(P);
+            borders.planes = reinterpret_cast<decltype(borders.planes)>(base);
+            borders.n = n;
+            borders.w0 = m_C0p / piece;
+            borders.w = m_Fp / piece;
+            w.borders = &borders;
         } else {
             w.V = reinterpret_cast<P*>(base);
             w.M = reinterpret_cast<P*>(base + kStaticTileBytes);
@@ -601,7 +608,6 @@ public:
         std::lock_guard<std::mutex> order(g_scratch_order_mu);
         hipEvent_t ev = g_scratch_event[m_device];
         if (ordered) HIP_CHECK(hipStreamWaitEvent(ln.stream, ev, 0));
-        if (clear) launch_clear(base, clear, ln.stream);
         enqueue_forward(w, n, d_in, nullptr, d_pol, d_val, false);
         HIP_CHECK(hipGetLastError());
         if (ordered) HIP_CHECK(hipEventRecord(ev, ln.stream));
@@ -1001,6 +1007,7 @@ private:
         uint32_t* peaks = nullptr;   // (direct fp32 towers)
         int lanes = 2;               // forwards that may be running side by side (lanes_in_use)
         std::map<int, LayersGraph>* layers = nullptr;   // the lane's (none: plain launches)
+        const PlaneBorders* borders = nullptr;          // to be cleared with the packing
     };
     // Slots of the input planes, then two sets that the layers write in turn.
     size_t peak_words(int n) const { return 2 * (size_t)n + 2 * conv3x3_f32_slots(m_Fp, n); }
@@ -1152,7 +1159,7 @@ private:
             launch_pack_input_bits<P>(d_bits, w.act0, m_direct, n, kInPlanes, m_C0p, w.peaks, m_in_scale.p,
                                       w.stream, pack);
         else if (!pack_with_peaks(w, d_in, n, pack))
-            launch_pack_input<P>(d_in, w.act0, m_direct, n, kInPlanes, m_C0p, w.stream, pack);
+            launch_pack_input<P>(d_in, w.act0, m_direct, n, kInPlanes, m_C0p, w.stream, pack, w.borders);
         if (m_direct) {
             enqueue_direct(w, n, d_pol, d_val, timed);
             return;
@@ -1197,7 +1204,7 @@ private:
         if constexpr (sizeof(P) == 4) {
             if (w.peaks) {
                 launch_pack_input_peaks(d_in, w.act0, n, kInPlanes, m_C0p, w.peaks, m_in_scale.p, w.stream,
-                                        t);
+                                        t, w.borders);
                 return true;
             }
         }

@@ -40,8 +40,12 @@ __host__ __device__ static inline size_t plane_index(bool padded, int b, int pt)
     return padded ? (size_t)(b + 1) * kPadCells + pt + pt / kBoard + 20 : (size_t)b * kPts + pt;
 }
 static inline size_t padded_cells(int n) { return (size_t)(n + 2) * kPadCells; }
-// Clears device memory (a multiple of 16 bytes) by a kernel.
-void launch_clear(void* p, size_t bytes, hipStream_t s);
+// The padded planes of a forward of n boards, one of w0 and then three of w pieces of 16 bytes to a cell
+// one after the other, whose borders the packing kernel is to clear on the way.
+struct PlaneBorders {
+    int __attribute__((ext_vector_type(4)))* planes = nullptr;
+    unsigned n = 0, w0 = 0, w = 0;
+};
 
 // NCHW fp32 planes [n][C][361] -> act [n][361][Cp] (channels >= C zero).
 // 32-bit words of one position's 18 x 361 input planes packed one bit per value.
@@ -60,10 +64,11 @@ void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, in
                             uint32_t* peaks, const float* scale, hipStream_t s, LaunchTimer* t);
 template <typename P>
 void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int Cp, hipStream_t s,
-                       LaunchTimer* t);
+                       LaunchTimer* t, const PlaneBorders* borders = nullptr);
 // The same with the peaks; padded.
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
-                             const float* scale, hipStream_t s, LaunchTimer* t);
+                             const float* scale, hipStream_t s, LaunchTimer* t,
+                             const PlaneBorders* borders = nullptr);
 
 // act [n][361][Cp] -> V [36][Tp][Cp]
 template <typename P>

@@ -121,10 +121,35 @@ __device__ __forceinline__ void pack_point(P* __restrict__ cell, int g, int C, i
     }
 }
 
+// The border of padded planes, as far as a tap of some point reads it: the last cell before the first
+// board, and of every board the row above it and the cell that ends each row, and the row below the
+// last.  Thread i clears a piece of one cell; 39 n + 21 cells of 400 (n + 2).
+__device__ __forceinline__ void clear_border(const PlaneBorders& p, unsigned i) {
+    const unsigned per = p.w0 + 3 * p.w, j = i / per, q = i - j * per;
+    if (j >= 39u * p.n + 21u) return;
+    const unsigned b = (j + 38) / 39, r = j + 38 - b * 39;   // (from the cell before the first board)
+    const unsigned cell = b * kPadCells + (r < 20 ? r : (r - 19) * 20 + 19);
+    const unsigned cells = (p.n + 2) * kPadCells;
+    const unsigned plane = q < p.w0 ? 0u : (q - p.w0) / p.w;
+    const size_t at = q < p.w0 ? (size_t)cell * p.w0 + q
+                               : (size_t)cells * (p.w0 + plane * p.w) + (size_t)cell * p.w +
+                                     (q - p.w0 - plane * p.w);
+    p.planes[at] = int4v{0, 0, 0, 0};
+}
+static unsigned border_pieces(const PlaneBorders* p) {
+    return p ? (39u * p->n + 21u) * (p->w0 + 3 * p->w) : 0u;
+}
+
+// (work-groups from pack_groups on clear borders)
 template <typename P>
 __global__ __launch_bounds__(256) void pack_input_k(const float* __restrict__ in,
                                                     P* __restrict__ act, bool padded, int n, int C,
-                                                    int Cp) {
+                                                    int Cp, unsigned pack_groups,
+                                                    PlaneBorders borders) {
+    if (blockIdx.x >= pack_groups) {
+        clear_border(borders, (blockIdx.x - pack_groups) * 256 + threadIdx.x);
+        return;
+    }
     const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (gid >= (size_t)n * kPackThreads) return;
     const int b = (int)(gid / kPackThreads), i = (int)(gid % kPackThreads), pt = i >> 2;
@@ -135,10 +160,10 @@ __global__ __launch_bounds__(256) void pack_input_k(const float* __restrict__ in
 
 template <typename P>
 void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int Cp, hipStream_t s,
-                       LaunchTimer* t) {
-    const size_t total = (size_t)n * kPackThreads;
-    launch(pack_input_k<P>, dim3((unsigned)((total + 255) / 256)), dim3(256), s, t, in, act,
-           padded, n, C, Cp);
+                       LaunchTimer* t, const PlaneBorders* borders) {
+    const unsigned groups = (unsigned)(((size_t)n * kPackThreads + 255) / 256);
+    launch(pack_input_k<P>, dim3(groups + (border_pieces(borders) + 255) / 256), dim3(256), s, t, in,
+           act, padded, n, C, Cp, groups, borders ? *borders : PlaneBorders());
 }
 
 // The same from bit-packed planes: bit (c*361 + pt) of a board's kInputWords words is
@@ -172,12 +197,18 @@ void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, in
 }
 
 // Planes and peaks from float planes: the first work-group of a board packs nothing and reads all
-// of it (26 KB); three pack.
+// of it (26 KB); three pack; those beyond clear borders.
+constexpr int kPeakGroups = 1 + (kPackThreads + 511) / 512;   // of a board
 __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restrict__ in,
                                                           float* __restrict__ act, int C, int Cp,
                                                           uint32_t* __restrict__ peaks,
-                                                          const float* __restrict__ scale) {
+                                                          const float* __restrict__ scale,
+                                                          PlaneBorders borders) {
     const int b = blockIdx.x, tid = threadIdx.x;
+    if (blockIdx.y >= kPeakGroups) {
+        clear_border(borders, ((blockIdx.y - kPeakGroups) * gridDim.x + b) * 512 + tid);
+        return;
+    }
     const float* planes = in + (size_t)b * C * kPts;
     if (blockIdx.y > 0) {
         const int i = (blockIdx.y - 1) * 512 + tid, pt = i >> 2;
@@ -207,19 +238,10 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
 }
 
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
-                             const float* scale, hipStream_t s, LaunchTimer* t) {
-    launch(pack_input_peaks_k, dim3(n, 1 + (kPackThreads + 511) / 512), dim3(512), s, t, in, act, C,
-           Cp, peaks, scale);
-}
-
-__global__ __launch_bounds__(256) void clear_k(int4v* p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-        p[i] = int4v{0, 0, 0, 0};
-}
-void launch_clear(void* p, size_t bytes, hipStream_t s) {
-    const size_t n = bytes / 16;
-    hipLaunchKernelGGL(clear_k, dim3((unsigned)(n < 256 * 1024 ? (n + 255) / 256 : 1024)), dim3(256), 0, s,
-                       (int4v*)p, n);
+                             const float* scale, hipStream_t s, LaunchTimer* t,
+                             const PlaneBorders* borders) {
+    launch(pack_input_peaks_k, dim3(n, kPeakGroups + (border_pieces(borders) + 512 * n - 1) / (512 * n)),
+           dim3(512), s, t, in, act, C, Cp, peaks, scale, borders ? *borders : PlaneBorders());
 }
 
 // ---------------------------------------------------------------------------
@@ -2152,7 +2174,7 @@ void launch_heads(const float* pol, const float* val, HeadParams hp, float tempe
 // ---------------------------------------------------------------------------
 #define INSTANTIATE(P)                                                                         \
     template void launch_pack_input<P>(const float*, P*, bool, int, int, int, hipStream_t,     \
-                                       LaunchTimer*);                                          \
+                                       LaunchTimer*, const PlaneBorders*);                     \
     template void launch_pack_input_bits<P>(const uint32_t*, P*, bool, int, int, int,          \
                                             uint32_t*, const float*, hipStream_t,              \
                                             LaunchTimer*);                                     \

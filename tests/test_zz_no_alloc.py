@@ -100,3 +100,61 @@ def test_no_alloc_forward_refuses_what_does_not_fit(pkg, netgen):
     with pytest.raises(ValueError, match="256 filters"):
         wide.forward_batch_device_noalloc(2, d_in.data_ptr(), d_pol.data_ptr(), d_val.data_ptr())
     wide.close()
+
+
+@pytest.mark.parametrize("precision_name", ["FP32", "FP16"])
+@pytest.mark.parametrize("filters", [64, 200, 256])
+def test_no_alloc_forward_after_planes_that_are_no_numbers(pkg, netgen, precision_name, filters):
+    """What another handle left in the static array does not reach a result: before each call a network
+    whose filters are no 3x3 ones (its Winograd tiles lie where a direct network has its planes) is given
+    planes of infinities, which leave the array full of NaN.  A call launches the kernels of the
+    plain forward and none beside them."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    precision = getattr(pkg, precision_name)
+    print("case: no-alloc after NaN", precision_name, filters, flush=True)
+    pipe = _pipe(pkg, netgen, 2, filters, 99, precision, 8)
+    net = netgen.make_network(1, 256, seed=100)
+    w, _ = netgen.prepare(net)
+    u = np.array(w.m_conv_weights[1], np.float32).reshape(36, 256, 256)
+    u[14] *= 1.25
+    w.m_conv_weights[1] = u
+    dirty = pkg.HIPScheduler(pkg.FP32, max_batch=8, device=0)
+    dirty.initialize(256)
+    dirty.push_weights(6, 18, 256, w)
+    x = torch.from_numpy(netgen.synthetic_inputs(8, seed=101)).cuda()
+    bad = torch.full((8, 18, 361), float("inf"), device="cuda")
+    pol, val = torch.zeros(8, 722, device="cuda"), torch.zeros(8, 361, device="cuda")
+    torch.cuda.synchronize()
+
+    def kernels(call):
+        with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
+            call()
+            torch.cuda.synchronize()
+        return sum("lzhip" in e.name for e in p.events())
+
+    for n in (8, 1, 5):
+        a, b = torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")
+        torch.cuda.synchronize()
+
+        def plain():
+            pipe.forward_batch_device(n, x.data_ptr(), a.data_ptr(), b.data_ptr())
+            pipe.sync()
+
+        def noalloc():
+            pipe.forward_batch_device_noalloc(n, x.data_ptr(), c.data_ptr(), d.data_ptr())
+            pipe.sync()
+
+        plain()
+        c, d = torch.full_like(a, -7.0), torch.full_like(b, -7.0)
+        dirty.forward_batch_device_noalloc(8, bad.data_ptr(), pol.data_ptr(), val.data_ptr())
+        dirty.sync()
+        torch.cuda.synchronize()
+        noalloc()
+        assert np.isfinite(a.cpu().numpy()).all()
+        assert np.array_equal(c.cpu().numpy(), a.cpu().numpy())
+        assert np.array_equal(d.cpu().numpy(), b.cpu().numpy())
+        count = kernels(plain)
+        assert count >= 5 and kernels(noalloc) == count
+    pipe.close()
+    dirty.close()
