@@ -17,6 +17,7 @@
 #include <stdexcept>
 
 #include "kernels.h"
+#include "layer_graphs.h"
 #include "plane_bits.h"
 
 namespace lzhip {
@@ -980,10 +981,6 @@ public:
 
 private:
     typedef std::tuple<int, const void*, float*, float*> GraphKey;
-    struct LayersGraph {
-        int uses = 0;
-        hipGraphExec_t exec = nullptr;
-    };
     // A lane is a stream with the working buffers of one forward.  Two batches on two
     // lanes run side by side on the device: each kernel's start-up and tail overlap with
     // the other lane's work, which a single chain of dependent kernels cannot do.
@@ -994,7 +991,7 @@ private:
         DevBuf<P> act0, act[3], V, M;
         DevBuf<uint32_t> peaks;   // direct fp32 towers: peak_words
         std::map<GraphKey, hipGraphExec_t> graphs;
-        std::map<int, LayersGraph> layers;   // by 4 n + lanes in use
+        LayerGraphs<hipGraphExec_t> layers;  // by 4 n + lanes in use
     };
     static constexpr int kLanes = 3;   // upper bound; m_n_lanes are in use
 
@@ -1006,7 +1003,7 @@ private:
         int Tp = 0;
         uint32_t* peaks = nullptr;   // (direct fp32 towers)
         int lanes = 2;               // forwards that may be running side by side (lanes_in_use)
-        std::map<int, LayersGraph>* layers = nullptr;   // the lane's (none: plain launches)
+        LayerGraphs<hipGraphExec_t>* layers = nullptr;  // the lane's (none: plain launches)
         const PlaneBorders* borders = nullptr;          // to be cleared with the packing
     };
     // Slots of the input planes, then two sets that the layers write in turn.
@@ -1098,9 +1095,7 @@ private:
     void clear_graphs(Lane& ln) {
         for (auto& kv : ln.graphs) (void)hipGraphExecDestroy(kv.second);
         ln.graphs.clear();
-        for (auto& kv : ln.layers)
-            if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
-        ln.layers.clear();
+        ln.layers.clear([](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); });
     }
     void clear_graphs() {
         for (auto& ln : m_lane) clear_graphs(ln);
@@ -1258,23 +1253,21 @@ private:
     // kernels, and between the lane's own buffers only, so that it is good for any caller's planes
     // and results.  It takes the host thread off the layers' 3.5 us a launch, which is what bounds small
     // networks on several lanes; on one lane, where the kernels are as long as their launches, plain
-    // launches are 3 to 8 % faster.  A graph is made the eighth time that a lane is given a batch size
-    // beside another lane, for eight batch sizes a lane at most.
+    // launches are 3 to 8 % faster.  A lane has graphs of the sixteen most frequent pairs of batch size and
+    // lanes in use at most (LayerGraphs).
     bool launch_layers_graph(const Work& w, int n) {
         if (!w.layers || w.lanes < 2 || !launch_bound(n)) return false;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(w.stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
             return false;
-        const int key = 4 * n + w.lanes;
-        auto it = w.layers->find(key);
-        if (it == w.layers->end()) {
-            if (w.layers->size() >= 8) return false;
-            it = w.layers->emplace(key, LayersGraph()).first;
-        }
-        LayersGraph& g = it->second;
-        if (!g.exec && ++g.uses == 8) g.exec = layers_graph(w, n);
-        if (!g.exec) return false;
-        HIP_CHECK(hipGraphLaunch(g.exec, w.stream));
+        const hipGraphExec_t g = w.layers->use(
+            4 * n + w.lanes, [&] { return layers_graph(w, n); },
+            [&](hipGraphExec_t old) {
+                (void)hipStreamSynchronize(w.stream);   // (its last launch may still be running)
+                (void)hipGraphExecDestroy(old);
+            });
+        if (!g) return false;
+        HIP_CHECK(hipGraphLaunch(g, w.stream));
         return true;
     }
     // Recorded on a stream of its own that no other work is ordered against, so that a call of

@@ -1124,3 +1124,55 @@ def test_layers_replayed_on_several_lanes(pkg, netgen, orc, filters, precision, 
     assert not wrong, wrong
     pipe.close()
     plain.close()
+
+
+def lzhip_events(call):
+    """Names of this library's kernels that call() ran, and how many graphs it launched."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    names = [e.name for e in p.events()]
+    return [n for n in names if "lzhip" in n], sum("GraphLaunch" in n for n in names)
+
+
+def test_frequent_batch_sizes_are_replayed_whatever_came_first(pkg, netgen, orc):
+    """Twenty batch sizes, some of them often enough for a graph each, before the one that is then used
+    throughout: that one is replayed all the same, and gives the bits of the plain launches."""
+    import torch
+    print("case: layer graphs of frequent sizes", flush=True)
+    maxb, lanes = 24, 2
+    net, plain, ref, h_ref = make_pipes(pkg, netgen, orc, 2, 64, 7400, pkg.FP16, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, 64, 7400, pkg.FP16, maxb)
+    x = netgen.synthetic_inputs(maxb, seed=7401)
+    d_in = torch.from_numpy(x).cuda()
+    outs = [(torch.zeros(maxb, 722, device="cuda"), torch.zeros(maxb, 361, device="cuda"))
+            for _ in range(lanes)]
+    torch.cuda.synchronize()
+
+    def forwards(n, reps):
+        for _ in range(reps):
+            for k, (pol, val) in enumerate(outs):
+                pipe.forward_batch_device(n, d_in.data_ptr(), pol.data_ptr(), val.data_ptr(), lane=k)
+        pipe.sync()
+
+    for n in range(1, 21):
+        forwards(n, 3 if n <= 10 else 10)
+    for n, reps in ((22, 12), (24, 40)):
+        forwards(n, reps)
+        want = plain.forward_batch(x[:n])
+        for _ in range(3):
+            kernels, graphs = lzhip_events(lambda: forwards(n, 2))
+            assert graphs == 2 * lanes and len(kernels) == 2 * lanes * 7, (n, graphs, len(kernels))
+            for pol, val in outs:
+                assert np.array_equal(pol.cpu().numpy()[:n], want[0]), n
+                assert np.array_equal(val.cpu().numpy()[:n], want[1]), n
+    for n in range(1, 21):   # as frequent as those: more sizes than a lane has graphs
+        forwards(n, 60)
+        want = plain.forward_batch(x[:n])
+        for pol, val in outs:
+            assert np.array_equal(pol.cpu().numpy()[:n], want[0]), n
+            assert np.array_equal(val.cpu().numpy()[:n], want[1]), n
+    pipe.close()
+    plain.close()

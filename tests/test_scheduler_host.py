@@ -63,3 +63,10 @@ def test_search_under_thread_sanitizer(tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
     assert "WARNING: ThreadSanitizer" not in r.stderr
     assert "search tests passed" in r.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_layer_graphs(tmp_path):
+    r = build_and_run(tmp_path, [], src=[os.path.join(ROOT, "tests", "cpp", "test_layer_graphs.cpp")])
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "layer graph tests passed" in r.stdout
