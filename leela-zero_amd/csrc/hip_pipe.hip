@@ -967,7 +967,7 @@ public:
         if ((int)m_layers.size() * 3 + 2 > kTimerPool)
             throw std::invalid_argument("network too deep for the timer pool");
         m_timer_used = 0;
-        enqueue_forward(ln, n, d_in, nullptr, d_pol, d_val, true);
+        enqueue_forward(ln, n, d_in, nullptr, d_pol, d_val, 1, true);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipStreamSynchronize(ln.stream));
         for (int k = 0; k < LZHIP_K_COUNT; k++) { ms[k] = 0.0f; launches[k] = 0; }
@@ -980,7 +980,7 @@ public:
     }
 
 private:
-    typedef std::tuple<int, const void*, float*, float*> GraphKey;
+    typedef std::tuple<int, int, const void*, float*, float*> GraphKey;   // (n, lanes in use, buffers)
     // A lane is a stream with the working buffers of one forward.  Two batches on two
     // lanes run side by side on the device: each kernel's start-up and tail overlap with
     // the other lane's work, which a single chain of dependent kernels cannot do.
@@ -1085,7 +1085,7 @@ private:
     }
 
     // With LZHIP_GRAPH=1 the launches of a forward (2 + one per layer of a direct tower; 2 + two
-    // per layer with Winograd kernels) are captured once per (batch size, buffers) into a HIP
+    // per layer with Winograd kernels) are captured once per (batch size, lanes in use, buffers) into a HIP
     // graph and replayed, which takes the launch work off the host thread.  Only kernel
     // nodes are captured (no memsets or copies).  On one lane the replay measured no faster
     // than stream launches (40x256 fp16 at batch 16: 0.84 against 0.83 ms; the gaps between
@@ -1112,18 +1112,22 @@ private:
     // d_in: fp32 planes, or, when null, d_bits: the planes one bit per value
     void run_forward(Lane& ln, int n, const float* d_in, const uint32_t* d_bits, float* d_pol,
                      float* d_val) {
+        const int lanes = lanes_in_use(ln);
         if (!m_use_graph) {
-            enqueue_forward(ln, n, d_in, d_bits, d_pol, d_val, false);
+            enqueue_forward(ln, n, d_in, d_bits, d_pol, d_val, lanes, false);
             return;
         }
-        const GraphKey key(n, d_in ? (const void*)d_in : (const void*)d_bits, d_pol, d_val);
+        const GraphKey key(n, lanes, d_in ? (const void*)d_in : (const void*)d_bits, d_pol, d_val);
         auto it = ln.graphs.find(key);
         if (it == ln.graphs.end()) {
-            if (ln.graphs.size() >= 64) clear_graphs(ln);
+            if (ln.graphs.size() >= 64) {
+                HIP_CHECK(hipStreamSynchronize(ln.stream));
+                clear_graphs(ln);
+            }
             hipGraph_t g = nullptr;
             hipGraphExec_t ge = nullptr;
             HIP_CHECK(hipStreamBeginCapture(ln.stream, hipStreamCaptureModeThreadLocal));
-            enqueue_forward(ln, n, d_in, d_bits, d_pol, d_val, false);
+            enqueue_forward(ln, n, d_in, d_bits, d_pol, d_val, lanes, false);
             HIP_CHECK(hipStreamEndCapture(ln.stream, &g));
             const hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
@@ -1139,9 +1143,9 @@ private:
     // later layer adds it back as a skip connection (layer 0 and every block
     // output), and by the last layer for the 1x1 heads.
     void enqueue_forward(Lane& ln, int n, const float* d_in, const uint32_t* d_bits,
-                         float* d_pol, float* d_val, bool timed) {
+                         float* d_pol, float* d_val, int lanes, bool timed) {
         Work w = work_of(ln);
-        w.lanes = timed ? 1 : lanes_in_use(ln);
+        w.lanes = lanes;
         if (!m_use_graph) w.layers = &ln.layers;
         enqueue_forward(w, n, d_in, d_bits, d_pol, d_val, timed);
     }

@@ -1176,3 +1176,42 @@ def test_frequent_batch_sizes_are_replayed_whatever_came_first(pkg, netgen, orc)
             assert np.array_equal(val.cpu().numpy()[:n], want[1]), n
     pipe.close()
     plain.close()
+
+
+@pytest.mark.parametrize("precision,filters,n", [(1, 256, 70), (0, 128, 17), (1, 64, 20)])
+def test_graph_replays_run_the_kernels_of_the_lanes_in_use(pkg, netgen, orc, precision, filters, n):
+    """With LZHIP_GRAPH=1, forwards on one lane and then on several run the kernels that plain
+    launches would: which tiles a layer takes follows the lanes in use, not those at the first call."""
+    import os
+    import torch
+    print("case: graphs and lanes, %d filters precision=%d" % (filters, precision), flush=True)
+    _, plain, _, _ = make_pipes(pkg, netgen, orc, 1, filters, 7500, precision, n)
+    os.environ["LZHIP_GRAPH"] = "1"
+    try:
+        _, pipe, _, _ = make_pipes(pkg, netgen, orc, 1, filters, 7500, precision, n)
+    finally:
+        del os.environ["LZHIP_GRAPH"]
+    x = netgen.synthetic_inputs(n, seed=7501)
+    want = plain.forward_batch(x)
+    d_in = torch.from_numpy(x).cuda()
+    outs = [(torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda"))
+            for _ in range(plain.lanes())]
+    torch.cuda.synchronize()
+
+    def forwards(p, lanes, reps):
+        for _ in range(reps):
+            for k, (pol, val) in enumerate(outs[:lanes]):
+                p.forward_batch_device(n, d_in.data_ptr(), pol.data_ptr(), val.data_ptr(), lane=k)
+        p.sync()
+
+    for lanes in (1, 2, plain.lanes(), 1):
+        ran = []
+        for p in (plain, pipe):
+            forwards(p, lanes, 3)
+            ran.append(sorted(lzhip_events(lambda: forwards(p, lanes, 4))[0]))
+            for pol, val in outs[:lanes]:
+                assert np.array_equal(pol.cpu().numpy(), want[0])
+                assert np.array_equal(val.cpu().numpy(), want[1])
+        assert len(ran[0]) == 4 * lanes * 5 and ran[0] == ran[1], (lanes, ran)
+    pipe.close()
+    plain.close()
