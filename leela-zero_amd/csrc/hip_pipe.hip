@@ -1281,7 +1281,10 @@ private:
         hipGraphExec_t exec = nullptr;
         hipStream_t s = nullptr;
         HIP_CHECK(hipGetLastError());   // (the caller's own, before any of this)
-        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return nullptr;
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
         w.stream = s;
         if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
             std::exception_ptr failed;
