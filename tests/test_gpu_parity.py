@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 def make_pipes(pkg, netgen, orc, blocks, filters, seed, precision, max_batch, winograd=False):
     """winograd: one Winograd position of layer 1 is scaled, which no 3x3 filter can express, so
-    that an fp16 network runs the Winograd kernels whatever its width."""
+    that a network of either precision runs the Winograd kernels whatever its width."""
     net = netgen.make_network(blocks, filters, seed)
     w, h = netgen.prepare(net)
     w_ref, h_ref = netgen.prepare(net, orc.winograd_transform_f, orc.process_bn_var)
@@ -36,18 +36,18 @@ def make_pipes(pkg, netgen, orc, blocks, filters, seed, precision, max_batch, wi
     return net, pipe, ref, h_ref
 
 
-@pytest.mark.parametrize("precision,winograd", [(0, False), (1, False), (1, True)])
+@pytest.mark.parametrize("precision,winograd", [(0, False), (0, True), (1, False), (1, True)])
 @pytest.mark.parametrize("filters,n", [(8, 3), (64, 3), (192, 3), (192, 30), (128, 3), (128, 40),
                                        (256, 3), (256, 16), (256, 20), (256, 40)])
 def test_single_layer_stages(pkg, netgen, orc, precision, winograd, filters, n):
     """V, M and Y of one convolution layer against the oracle's stages, for the input
     layer (18 planes) and a residual-tower layer with a skip connection.  The M stage is
     the check the reference's tuner makes of every GEMM it times, against a plain sgemm
-    (reference src/Tuner.cpp:262-301); in fp32, 128 and 256 filters put the streaming GEMM
-    under it, at 3 boards (one 32-row block per work-group) and at 40 (several
-    blocks per work-group, a last block of 8 rows).  An fp16 layer is a direct convolution: Y is
-    what a forward computes, V and M come from its filters by the tiled kernels.  With filters that
-    are no 3x3 ones (winograd) all three are the stages of such a network's forward."""
+    (reference src/Tuner.cpp:262-301).  A layer is a direct convolution: Y is what a forward
+    computes, V and M come from its filters by the tiled kernels.  With filters that are no 3x3
+    ones (winograd) all three are the stages of such a network's forward; in fp32, 128 and 256
+    filters then put the streaming GEMM under it, at 3 boards (one 32-row block per work-group)
+    and at 40 (several blocks per work-group, a last block of 8 rows)."""
     print("case: single_layer precision=%d filters=%d n=%d" % (precision, filters, n), flush=True)
     net, pipe, ref, _ = make_pipes(pkg, netgen, orc, 1, filters, 40 + filters, precision,
                                    max(4, n), winograd)
@@ -350,16 +350,17 @@ def test_handle_created_from_a_weights_file(pkg, netgen, orc, tmp_path):
         b.close()
 
 
-@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("precision,winograd", [(0, False), (0, True), (1, False)])
 @pytest.mark.parametrize("filters,maxb", [(64, 8), (128, 40), (192, 16), (192, 40), (256, 40)])
-def test_batch_composition_does_not_change_results(pkg, netgen, orc, precision, filters, maxb):
+def test_batch_composition_does_not_change_results(pkg, netgen, orc, precision, winograd, filters, maxb):
     """A position evaluated alone, in a partial batch and in a full batch gives
-    bit-identical planes: rows of the GEMM are independent, and a network's layers run one
-    kernel family at every batch (whatever the tile shapes, blocks per work-group or channel
-    groups the batch selects, a value is summed in the same order).  fp32 at 192 filters takes
-    the streaming GEMM in handles of up to 16 positions and the tiled one in larger ones."""
+    bit-identical planes: points and rows of the GEMM are independent, and a network's layers run
+    one kernel family at every batch (whatever the tile shapes, blocks per work-group or channel
+    groups the batch selects, a value is summed in the same order).  With filters that are no 3x3
+    ones (winograd) fp32 at 192 filters takes the streaming GEMM in handles of up to 16 positions
+    and the tiled one in larger ones."""
     print("case: batch composition %d filters precision=%d" % (filters, precision), flush=True)
-    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, filters, 77, precision, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 2, filters, 77, precision, maxb, winograd)
     x = netgen.synthetic_inputs(maxb, seed=5)
     pol_all, val_all = pipe.forward_batch(x)
     for lo, hi in ((2, 5), (4, 5), (0, min(17, maxb)), (1, min(34, maxb)), (0, 1)):
@@ -544,29 +545,32 @@ def test_graph_replays_match_stream_launches(pkg, netgen, orc):
     plain.close()
 
 
-@pytest.mark.parametrize("precision,filters,maxb,batches", [
-    (1, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
-    (1, 192, 42, (1, 7, 10, 15, 21, 22, 37, 42)),
-    (1, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
-    (0, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
-    (0, 192, 16, (1, 5, 9, 15, 16)),
-    (0, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
+@pytest.mark.parametrize("precision,winograd,filters,maxb,batches", [
+    (1, False, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
+    (1, False, 192, 42, (1, 7, 10, 15, 21, 22, 37, 42)),
+    (1, False, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
+    (0, False, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
+    (0, False, 192, 16, (1, 5, 9, 15, 16)),
+    (0, False, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
+    (0, True, 256, 32, (1, 5, 8, 9, 16, 17, 20, 21, 23, 32)),
+    (0, True, 192, 16, (1, 5, 9, 15, 16)),
+    (0, True, 128, 64, (1, 8, 9, 18, 32, 33, 36, 44, 45, 64)),
 ])
-def test_busy_lanes_and_tile_layouts_give_the_same_bits(pkg, netgen, orc, precision, filters, maxb,
-                                                        batches):
+def test_busy_lanes_and_tile_layouts_give_the_same_bits(pkg, netgen, orc, precision, winograd, filters,
+                                                        maxb, batches):
     """Every batch on one lane alone, and on all lanes at once with many forwards in a row and no
-    synchronisation, gives the same bits; so does an fp32 handle that keeps V and M of the tower's
-    layers in two arrays (LZHIP_INPLACE=0) beside the default that keeps them in one; and the
-    result agrees with the oracle."""
+    synchronisation, gives the same bits; so does, where filters are no 3x3 ones (winograd), an fp32
+    handle that keeps V and M of the tower's layers in two arrays (LZHIP_INPLACE=0) beside the
+    default that keeps them in one; and the result agrees with the oracle."""
     import os
     import torch
     print("case: busy lanes, %d filters precision=%d" % (filters, precision), flush=True)
-    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 4, filters, 3100, precision, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 4, filters, 3100, precision, maxb, winograd)
     pipes = [pipe]
-    if precision == 0:
+    if winograd:
         os.environ["LZHIP_INPLACE"] = "0"
         try:
-            pipes.append(make_pipes(pkg, netgen, orc, 4, filters, 3100, precision, maxb)[1])
+            pipes.append(make_pipes(pkg, netgen, orc, 4, filters, 3100, precision, maxb, winograd)[1])
         finally:
             del os.environ["LZHIP_INPLACE"]
     x = netgen.synthetic_inputs(maxb, seed=3101)
@@ -597,16 +601,17 @@ def test_busy_lanes_and_tile_layouts_give_the_same_bits(pkg, netgen, orc, precis
         p.close()
 
 
-def test_random_batches_on_all_lanes_match_the_plain_forward(pkg, netgen, orc):
-    """A seeded sequence of 400 forwards of random batches (1 to 32 boards, 256 filters) dealt to
+@pytest.mark.parametrize("precision,filters", [(1, 256), (0, 256), (0, 384), (1, 384)])
+def test_random_batches_on_all_lanes_match_the_plain_forward(pkg, netgen, orc, precision, filters):
+    """A seeded sequence of 400 forwards of random batches (1 to 32 boards) dealt to
     random lanes with no synchronisation between them -- so that consecutive forwards of a lane
     change between tiles, and between having the device alone and sharing it -- gives, forward by
     forward, the bits of another handle that runs one batch at a time."""
     import torch
-    print("case: random batches on all lanes", flush=True)
+    print("case: random batches on all lanes, %d filters precision=%d" % (filters, precision), flush=True)
     maxb = 32
-    net, plain, ref, h_ref = make_pipes(pkg, netgen, orc, 3, 256, 3300, pkg.FP16, maxb)
-    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 3, 256, 3300, pkg.FP16, maxb)
+    net, plain, ref, h_ref = make_pipes(pkg, netgen, orc, 3, filters, 3300, precision, maxb)
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 3, filters, 3300, precision, maxb)
     x = netgen.synthetic_inputs(maxb, seed=3301)
     want = {}
     rng = np.random.default_rng(3302)
@@ -689,14 +694,14 @@ def test_error_behaviour_on_device(pkg, netgen):
 @pytest.mark.parametrize("filters,batch", [(128, 1), (128, 9), (128, 30), (128, 52), (128, 72),
                                            (192, 2), (192, 16), (192, 17), (192, 40), (192, 64)])
 def test_streaming_gemm_at_narrower_widths(pkg, netgen, orc, filters, batch, precision):
-    """fp32 nets of 128 filters, and of 192 in handles of up to 16 positions, run the streaming
-    GEMM with 4 and 6 wavefronts per work-group (256 filters: 8); larger handles of 192 filters the
-    tiled one.  fp16 nets whose filters are no 3x3 ones run the tiled GEMM at the same sizes.  The
+    """Nets whose filters are no 3x3 ones.  fp32 nets of 128 filters, and of 192 in handles of up to
+    16 positions, run the streaming GEMM with 4 and 6 wavefronts per work-group (256 filters: 8);
+    larger handles of 192 filters the tiled one, and so do fp16 nets at the same sizes.  The
     batches take different numbers of blocks per work-group, with tile counts that are not
     multiples of the 32-row block."""
     print("case: streaming width %d b%d precision=%d" % (filters, batch, precision), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 5100 + filters, precision,
-                                       batch, winograd=precision == 1)
+                                       batch, winograd=True)
     x = netgen.synthetic_inputs(batch, seed=filters + batch)
     check_outputs(pkg, orc, pipe, ref, h_ref, x, precision,
                   idx=sorted({0, batch // 2, batch - 1}))
@@ -718,15 +723,15 @@ def test_fp16_widths_on_the_tiled_gemm(pkg, netgen, orc, filters, batch):
     pipe.close()
 
 
-@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("precision,winograd", [(0, False), (0, True), (1, False)])
 @pytest.mark.parametrize("filters,batch", [(384, 6), (512, 44), (320, 3)])
-def test_other_widths(pkg, netgen, orc, precision, filters, batch):
-    """Widths other than the benchmark's: 12, 16 and 10 k-slices of the tiled GEMM in fp32, with
-    its large tile at 512 filters; in fp16 direct convolution at 384 and 320 filters and the
-    tiled GEMM's 8 k-slices at 512."""
+def test_other_widths(pkg, netgen, orc, precision, winograd, filters, batch):
+    """Widths other than the benchmark's: direct convolution in fp32, and in fp16 at 384 and 320
+    filters; the tiled GEMM's 8 k-slices in fp16 at 512; and where filters are no 3x3 ones
+    (winograd) its 12, 16 and 10 k-slices in fp32, with its large tile at 512 filters."""
     print("case: width %d b%d precision=%d" % (filters, batch, precision), flush=True)
     net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 4000 + filters, precision,
-                                       batch)
+                                       batch, winograd)
     x = netgen.synthetic_inputs(batch, seed=filters)
     check_outputs(pkg, orc, pipe, ref, h_ref, x, precision, idx=[0, batch - 1])
     pipe.close()
