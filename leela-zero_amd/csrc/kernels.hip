@@ -170,7 +170,7 @@ void launch_pack_input(const float* in, P* act, bool padded, int n, int C, int C
 // plane c at point pt (planes that hold only 0 and 1, which is what the engine feeds).  The
 // words may lie in host memory, across the bus: a work-group fetches its board's once, in one
 // load, and there are three of them to a board.
-template <typename P>
+template <typename P, bool SCALED>
 __global__ __launch_bounds__(512) void pack_input_bits_k(const uint32_t* __restrict__ bits,
                                                          P* __restrict__ act, bool padded, int C,
                                                          int Cp, uint32_t* __restrict__ peaks,
@@ -185,20 +185,23 @@ __global__ __launch_bounds__(512) void pack_input_bits_k(const uint32_t* __restr
     pack_point(act + plane_index(padded, b, pt) * Cp, i & 3, C, Cp, [&](int c) {
         const int bit = c * kPts + pt;
         const float v = (float)((words[bit >> 5] >> (bit & 31)) & 1u);
-        return scale ? v * scale[c] : v;
+        return SCALED ? v * scale[c] : v;
     });
 }
 
+// (A kernel of its own for planes with factors: the test of the pointer at every value cost 37 boards
+// of 128 filters 4 us a call.)
 template <typename P>
 void launch_pack_input_bits(const uint32_t* bits, P* act, bool padded, int n, int C, int Cp,
                             uint32_t* peaks, const float* scale, hipStream_t s, LaunchTimer* t) {
-    launch(pack_input_bits_k<P>, dim3(n, (kPackThreads + 511) / 512), dim3(512), s, t, bits, act,
-           padded, C, Cp, peaks, scale);
+    launch(scale ? pack_input_bits_k<P, true> : pack_input_bits_k<P, false>,
+           dim3(n, (kPackThreads + 511) / 512), dim3(512), s, t, bits, act, padded, C, Cp, peaks, scale);
 }
 
 // Planes and peaks from float planes: the first work-group of a board packs nothing and reads all
 // of it (26 KB); three pack; those beyond clear borders.
 constexpr int kPeakGroups = 1 + (kPackThreads + 511) / 512;   // of a board
+template <bool SCALED>
 __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restrict__ in,
                                                           float* __restrict__ act, int C, int Cp,
                                                           uint32_t* __restrict__ peaks,
@@ -216,14 +219,14 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
             pack_point(act + plane_index(true, b, pt) * Cp, i & 3, C, Cp,
                        [&](int c) {
                            const float v = planes[(size_t)c * kPts + pt];
-                           return scale ? v * scale[c] : v;
+                           return SCALED ? v * scale[c] : v;
                        });
         return;
     }
     float top = 0.0f;
 #pragma unroll 13
     for (int i = tid; i < C * kPts; i += 512) {
-        const float v = fabsf(scale ? planes[i] * scale[i / kPts] : planes[i]);
+        const float v = fabsf(SCALED ? planes[i] * scale[i / kPts] : planes[i]);
         top = fmaxf(top, v < __builtin_inff() ? v : 0.0f);
     }
     __shared__ float tops[8];
@@ -240,7 +243,8 @@ __global__ __launch_bounds__(512) void pack_input_peaks_k(const float* __restric
 void launch_pack_input_peaks(const float* in, float* act, int n, int C, int Cp, uint32_t* peaks,
                              const float* scale, hipStream_t s, LaunchTimer* t,
                              const PlaneBorders* borders) {
-    launch(pack_input_peaks_k, dim3(n, kPeakGroups + (border_pieces(borders) + 512 * n - 1) / (512 * n)),
+    launch(scale ? pack_input_peaks_k<true> : pack_input_peaks_k<false>,
+           dim3(n, kPeakGroups + (border_pieces(borders) + 512 * n - 1) / (512 * n)),
            dim3(512), s, t, in, act, C, Cp, peaks, scale, borders ? *borders : PlaneBorders());
 }
 
