@@ -221,10 +221,11 @@ def gemm_kernel_name(fp16, Fp, B):
 
 def measure_forward(pkg, netgen, torch, blocks, F, precision, B, steps, warmup, lanes_arg,
                     profile_reps, host_buffers=False, blocks_of_k=0, min_block=200, winograd=False):
-    """winograd: one Winograd position of layer 1 is scaled, which no 3x3 filter can express, so
-    that the network runs the Winograd kernels.  One network on the device: evaluations/s of `steps` forwards of B device-resident
+    """One network on the device: evaluations/s of `steps` forwards of B device-resident
     positions (all lanes, and one lane), optionally the same through host buffers, and the
-    per-kernel-class durations with the roofline figures derived from them."""
+    per-kernel-class durations with the roofline figures derived from them.  winograd: one
+    Winograd position of layer 1 is scaled, which no 3x3 filter can express, so that the network
+    runs the Winograd kernels."""
     prec = pkg.FP16 if precision == "fp16" else pkg.FP32
     net = netgen.make_network(blocks, F, seed=2025)
     x = netgen.synthetic_inputs(B, seed=2026)
@@ -486,16 +487,22 @@ def side_config(pkg, netgen, torch, blocks, F, precision, B, args, cpu=False):
     net, x = r.pop("_net"), r.pop("_x")
     r.pop("_pol")
     t = r["roofline_transforms"]["out_in_transform"]
+    notes = {}
+    if precision == "fp32" and r["roofline"]["kernel"].startswith("conv3x3"):
+        notes["gemm_note"] = ("direct convolution: three half-precision products for one of fp32, "
+                              "against the fp16 peak; not to be read beside a share of the fp32 peak")
     if t is None and precision == "fp32":
         # the transforms of a network of the same size whose filters are no 3x3 ones
         t = measure_forward(pkg, netgen, torch, blocks, F, precision, B, 10, 2, 0, 2,
                             winograd=True)["roofline_transforms"]["out_in_transform"]
+        notes["transform_note"] = ("not of this network, which has no transforms: measured on one of the "
+                                   "same size whose filters are no 3x3 ones")
     out = {"value": r["value"], "unit": "evals/s", "lanes": r["lanes"],
            "one_lane": r["one_lane"]["value"], "ms_per_batch_one_lane": r["one_lane"]["ms_per_step"],
            "gemm_frac_of_mfma_peak": r["roofline"]["frac"],
            "gemm_us_per_launch": r["roofline"]["avg_launch_us"],
            "transform_frac_of_hbm_peak": t["frac"] if t else None,
-           "transform_us_per_launch": t["avg_launch_us"] if t else None}
+           "transform_us_per_launch": t["avg_launch_us"] if t else None, **notes}
     if cpu and not args.no_cpu_baseline:
         orc = entry.load_oracle()
         c, _ = cpu_baseline(orc, netgen, net, x, seconds_budget=3.0)

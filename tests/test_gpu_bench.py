@@ -49,12 +49,14 @@ def test_forward_line():
         assert k in cb, k
     assert cb["kind"] == "port" and cb["value"] > 0 and cb["cores"] >= 1
     assert cb["raw_policy_plane_rel_l2_vs_gpu"] < 2e-2      # the spot check against the oracle
-    # an fp16 tower is one direct convolution per layer: no transforms to price; fp32 has them
+    # a tower is one direct convolution per layer: no transforms to price; the fp32 line has those of a
+    # network whose filters are no 3x3 ones, and says so
     assert d["roofline"]["kernel"].startswith("conv3x3")
     assert d["roofline"]["launches_per_forward"] == 5
     for name in ("out_in_transform", "in_transform", "out_transform"):
         assert d["roofline_transforms"][name] is None
     assert 0 < d["fp32"]["transform_frac_of_hbm_peak"] < 1
+    assert "no 3x3" in d["fp32"]["transform_note"] and "half-precision" in d["fp32"]["gemm_note"]
     # the figures beside the headline one: host buffers (PCIe inside the timed region), the
     # repeated blocks, the plain-copy floor, the same net in fp32 and the smaller configurations
     hb = d["host_buffers"]
