@@ -16,8 +16,9 @@ typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 // bounds logic, and the patch of a tile is one run of consecutive cells: every piece that a
 // thread fetches lies a constant distance from its first.  (With dense planes in memory and the border
 // made on the way to LDS an address took some 25 instructions, and up to 13 of them per thread came
-// before the first load: 10x128 fp16 batch 5, 86.8 -> 82.8 us a forward, 15x192 batch 8, 218 -> 209,
-// 20x256 batch 32, 676 -> 664; fp32, with more pieces, 6x128 batch 1, 83 -> 75.)
+// before the first load: 15x192 fp16 batch 8, 217 -> 210 us a forward, 20x256 batch 32, 644 -> 627; 6x128
+// fp32 batch 1, 76 -> 75; nothing where the host's launches are the bound, 10x128 fp16 batch 5, 77 to 87
+// and 83 to 85.)
 constexpr int kCellsPerBoard = kPadCells;
 constexpr int kRowCells = 20;
 // Cells that a tile of mt consecutive rows can reach: its own span (a cell more per board

@@ -138,7 +138,8 @@ void conv3x3_winograd_filters(const _Float16* Wf, int C, int Cp, int F, int Kp, 
 // X [Cp] -> Y [Kp] = max(0, scale*(conv - mean) + rfac*res) in fp32, padded planes, every operand split in
 // two half-precision numbers.  Wf holds the filters of output channel k and input channel c times
 // 2^(exp[k] - in_exp[c]): X holds channel c times 2^in_exp[c], scale is the caller's times 2^(out_exp[k]
-// - exp[k]), mean times 2^exp[k], and Y comes out times 2^out_exp[k].  peaks: of X; those of Y go to `slots` (conv3x3_f32_slots words) and are returned.
+// - exp[k]), mean times 2^exp[k], and Y comes out times 2^out_exp[k].  peaks: of X; those of Y
+// go to `slots` (conv3x3_f32_slots words) and are returned.
 bool conv3x3_f32_serves(int Kp);
 size_t conv3x3_f32_filter_count(int Cp, int Kp);
 size_t conv3x3_f32_slots(int Kp, int max_batch);
