@@ -179,8 +179,20 @@ __global__ __launch_bounds__(512) void pack_input_bits_k(const uint32_t* __restr
     const int b = blockIdx.x, i = blockIdx.y * 512 + threadIdx.x, pt = i >> 2;
     if (threadIdx.x < kInputWords)
         words[threadIdx.x] = bits[(size_t)b * kInputWords + threadIdx.x];
-    if (peaks && i < 2) peaks[2 * (size_t)b + i] = 0x3f800000u;   // (no factor is above 1)
+    if (!SCALED && peaks && i < 2) peaks[2 * (size_t)b + i] = 0x3f800000u;
     __syncthreads();
+    if (SCALED && peaks && blockIdx.y == 0 && threadIdx.x < 64) {
+        // the largest factor of a plane that is not empty, as the float planes' peak would be
+        const int c = threadIdx.x, from = c * kPts, to = from + kPts;
+        float top = 0.0f;
+        for (int w = from >> 5; c < C && w <= (to - 1) >> 5; w++) {
+            const int lo = max(from - w * 32, 0), hi = min(to - w * 32, 32);   // bits [lo, hi) are c's
+            if (words[w] >> lo & (hi - lo == 32 ? ~0u : (1u << (hi - lo)) - 1u)) top = scale[c];
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
+        if (c < 2) peaks[2 * (size_t)b + c] = __builtin_bit_cast(uint32_t, top);
+    }
     if (pt >= kPts) return;
     pack_point(act + plane_index(padded, b, pt) * Cp, i & 3, C, Cp, [&](int c) {
         const int bit = c * kPts + pt;

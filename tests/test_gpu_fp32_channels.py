@@ -198,3 +198,39 @@ def test_dead_channels_keep_the_direct_kernels(pkg, netgen, precision, filters, 
     for i in range(n):
         assert rel_l2(pol[i], want["pol"][i]) <= tol and rel_l2(val[i], want["val"][i]) <= tol, i
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,maxb", [(64, 8), (128, 40)])
+@pytest.mark.parametrize("far", [24, 48])
+def test_planes_in_bits_are_those_in_floats(pkg, netgen, filters, maxb, far):
+    """A plane that is empty in every position, whose filters are 2^far times all others': it sets the
+    factors of the input planes and nothing else.  Positions sent as bits and as floats give the same
+    planes, with the precision of the network whose filters are alike."""
+    print("case: empty plane, %d filters of %d, 2^%d" % (filters, maxb, far), flush=True)
+    import torch
+    n = 3
+    net = netgen.make_network(2, filters, 8600)
+    zero = np.zeros(filters, int)
+    low = spread(net, np.zeros(18, int), zero - far, [zero, zero])
+    low.conv_w[0][:, 17] *= np.float32(2.0 ** far)
+    x = netgen.synthetic_inputs(n, seed=8601)
+    assert not x[:, 17].any()
+    x[1, 16] = 0.0
+    want = tower_f64(net, x)
+    plain, pipe = make_pipe(pkg, netgen, net, maxb), make_pipe(pkg, netgen, low, maxb)
+    base, bits = plain.forward_batch(x), pipe.forward_batch(x)
+    d_in = torch.from_numpy(x).cuda()
+    pol, val = torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")
+    torch.cuda.synchronize()
+    pipe.forward_batch_device(n, d_in.data_ptr(), pol.data_ptr(), val.data_ptr())
+    pipe.sync()
+    assert is_direct(pkg, pipe, x)
+    for i in range(n):
+        one = pipe.forward(x[i])
+        for k, (name, floats) in enumerate((("pol", pol), ("val", val))):
+            assert np.array_equal(floats.cpu().numpy()[i], bits[k][i]), (i, name)
+            assert np.array_equal(one[k], bits[k][i]), (i, name)
+            alike, err = rel_l2(base[k][i], want[name][i]), rel_l2(bits[k][i], want[name][i])
+            assert err <= 2 * alike + 2.0 ** -24, (i, name, err, alike)
+    pipe.close()
+    plain.close()
