@@ -158,3 +158,37 @@ def test_no_alloc_forward_after_planes_that_are_no_numbers(pkg, netgen, precisio
         assert count >= 5 and kernels(noalloc) == count
     pipe.close()
     dirty.close()
+
+
+@pytest.mark.parametrize("precision_name", ["FP32", "FP16"])
+def test_no_alloc_forward_in_a_captured_graph(pkg, netgen, precision_name):
+    """The call recorded into a caller's graph: every replay gives the eager planes, with other handles'
+    calls through the same static array, eager work and synchronisations between the replays."""
+    import torch
+    print("case: no-alloc captured", precision_name, flush=True)
+    pipe = _pipe(pkg, netgen, 2, 128, 102, getattr(pkg, precision_name), 8)
+    other = _pipe(pkg, netgen, 1, 256, 103, pkg.FP32, 8)
+    n = 5
+    x = torch.from_numpy(netgen.synthetic_inputs(8, seed=104)).cuda()
+    planes = x[:n].clone()
+    out = [torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")]
+    rest = [torch.zeros(8, 722, device="cuda"), torch.zeros(8, 361, device="cuda")]
+    torch.cuda.synchronize()
+    stream = torch.cuda.ExternalStream(pipe.stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        pipe.forward_batch_device_noalloc(n, planes.data_ptr(), out[0].data_ptr(), out[1].data_ptr())
+    for rep in range(5):
+        planes.copy_(x[rep % 3:rep % 3 + n])
+        other.forward_batch_device_noalloc(8, x.data_ptr(), rest[0].data_ptr(), rest[1].data_ptr())
+        other.sync()
+        for t in out:
+            t.fill_(-7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = pipe.forward_batch(planes.cpu().numpy())
+        assert np.array_equal(out[0].cpu().numpy(), want[0]), rep
+        assert np.array_equal(out[1].cpu().numpy(), want[1]), rep
+    pipe.close()
+    other.close()
