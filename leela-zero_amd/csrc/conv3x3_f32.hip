@@ -943,8 +943,8 @@ void conv3x3_f32_filters(const float* U, const int* in_exp, const int* exp, half
 // value, that of a filter to 2^-36 of its output channel's largest.  If the largest product of an
 // output channel is at least 2^-14 of its largest filter times the largest input channel, either
 // error stays below 2^-22 of that product, as it is with operands of the full 22 bits.
-bool conv3x3_f32_holds(int peak, int reach, int top) {
-    return peak == kNoExp || top == kNoExp || reach >= peak + top - 14;
+bool conv3x3_f32_holds(int peak, int reach, int top, int most) {
+    return peak == kNoExp || top == kNoExp || reach >= peak + top - most;
 }
 
 // The exponent of an output channel's filters: their largest comes to kFilterTop, or as far towards it as

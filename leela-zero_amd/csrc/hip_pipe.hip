@@ -393,10 +393,12 @@ public:
     // fp32.  A direct tower holds its operands as two halves, relative to the largest of a board and of an
     // output channel, so channels whose activations lie far below others' would lose bits that fp32
     // keeps.  What a channel's magnitude is, is estimated from the filters and the batch norm, layer by
-    // layer, as a binary exponent; where estimates of a layer differ by 2^8 or more, planes hold
-    // the smaller channels times a power of two (m_chan), which its producer's batch norm puts in and the
-    // next layer's filters and the heads take out.  Batch norm and ReLU commute with it, so every
-    // product is the one that it would be.  A network whose estimates agree is left as it is.
+    // layer, as a binary exponent.  Where some output channel's largest product lies 2^8 or more below
+    // its largest filter times the largest input, that layer's input planes hold the smaller channels
+    // times a power of two (m_chan), which the producer's batch norm puts in and the next layer's
+    // filters and the heads take out.  Batch norm and ReLU commute with it, so every product is the
+    // one that it would be.  Any other layer is left as it is: an estimate may be far too high, for a
+    // channel that never fires, and others raised to it would lose bits of their filters.
     bool build_split_filters(int n_layers, const float* const* U, const float* const* bn_mean,
                              const float* const* bn_scale, DevBuf<float>& stage) {
         hipStream_t s = m_lane[0].stream;
@@ -414,6 +416,7 @@ public:
         m[0].assign(kInPlanes, 0);
         m_chan.assign(n_layers + 1, std::vector<int>(F, 0));
         m_chan[0] = plane_exponents(U[0]);
+        std::vector<char> move(n_layers + 1, 0);   // layers whose inputs are to be brought together
         for (int pass = 0; pass < 2; pass++) {
             bool holds = true;
             for (int l = 0; l < n_layers; l++) {
@@ -436,10 +439,11 @@ public:
                     if (m[l][c] != kNoExp) top = std::max(top, m[l][c] + m_chan[l][c]);
                 L.exp.resize(F);
                 for (int k = 0; k < F; k++) {
-                    holds = holds && (l == 0 || conv3x3_f32_holds(ends[k], ends[F + k], top)) &&
+                    holds = holds && (l == 0 || conv3x3_f32_holds(ends[k], ends[F + k], top, 14)) &&
                             conv3x3_f32_exponent(ends[k], bn_scale[l][k], bn_mean[l][k],
                                                  m_chan[l + 1][k], L.exp[k]);
                     if (pass == 0) {
+                        if (l > 0 && !conv3x3_f32_holds(ends[k], ends[F + k], top, 8)) move[l] = 1;
                         const bool second = l >= 2 && l % 2 == 0;
                         m[l + 1][k] = std::max(second ? m[l - 1][k] : kNoExp,
                                                magnitude(ends[F + k], bn_scale[l][k], bn_mean[l][k]));
@@ -451,7 +455,7 @@ public:
                 HIP_CHECK(hipGetLastError());
                 HIP_CHECK(hipStreamSynchronize(s));
             }
-            if (pass == 1 || !balance_channels(m)) {
+            if (pass == 1 || !balance_channels(m, move)) {
                 if (!holds) return false;
                 break;
             }
@@ -488,32 +492,35 @@ public:
         return e;
     }
     // Exponent of what a channel puts out: its largest product, times what 9 F of them come to (a sum of
-    // F = 64 to 512 random ones is 4 to 12 times the largest), or its batch norm's constant.
+    // F = 64 to 512 random ones is 4 to 12 times the largest), or its batch norm's constant where
+    // that adds to it.
     static int magnitude(int reach, float scale, float mean) {
         if (!std::isfinite(scale) || scale == 0.0f) return kNoExp;
         const int s = std::ilogb(scale);
         const int conv = reach == kNoExp ? kNoExp : s + reach + 3;
-        return std::isfinite(mean) && mean != 0.0f ? std::max(conv, s + std::ilogb(mean)) : conv;
+        const bool adds = std::isfinite(mean) && (scale > 0.0f ? mean < 0.0f : mean > 0.0f);
+        return adds ? std::max(conv, s + std::ilogb(mean)) : conv;
     }
-    // m_chan from the magnitudes: in whole 2^8, so that ordinary networks keep theirs, and by at most 2^64;
-    // the channels of the residual stream have one exponent throughout, by which none comes above
-    // the largest of its layer anywhere.  False: nothing to move.
-    bool balance_channels(const std::vector<std::vector<int>>& m) {
+    // m_chan from the magnitudes, for the inputs of the layers that `move` names: in whole 2^8, and by at
+    // most 2^64; the channels of the residual stream have one exponent throughout, by which none comes
+    // above the largest of its layer anywhere.  False: nothing to move.
+    bool balance_channels(const std::vector<std::vector<int>>& m, const std::vector<char>& move) {
         const int n_layers = (int)m.size() - 1, F = m_filters;
         auto below = [&](int l, int k, int top) { return m[l][k] == kNoExp ? 64 : top - m[l][k]; };
         std::vector<int> stream(F, 64);
-        bool moved = false;
+        bool moved = false, move_stream = false;
+        for (int l = 1; l < n_layers; l += 2) move_stream = move_stream || move[l];
         for (int l = 1; l <= n_layers; l++) {
             const int top = *std::max_element(m[l].begin(), m[l].end());
             if (top == kNoExp) continue;
             for (int k = 0; k < F; k++) {
                 if (l % 2) stream[k] = std::min(stream[k], below(l, k, top));
-                else if (m[l][k] != kNoExp) m_chan[l][k] = std::min(below(l, k, top), 64) / 8 * 8;
+                else if (move[l] && m[l][k] != kNoExp) m_chan[l][k] = std::min(below(l, k, top), 64) / 8 * 8;
             }
         }
         for (int l = 1; l <= n_layers; l++)
             for (int k = 0; k < F; k++) {
-                if (l % 2) m_chan[l][k] = m[n_layers][k] == kNoExp ? 0 : stream[k] / 8 * 8;
+                if (l % 2) m_chan[l][k] = !move_stream || m[n_layers][k] == kNoExp ? 0 : stream[k] / 8 * 8;
                 moved = moved || m_chan[l][k] != 0;
             }
         return moved;

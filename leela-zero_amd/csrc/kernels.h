@@ -158,8 +158,9 @@ PeakMap launch_conv3x3_f32_split(const float* X, const _Float16* Wf, const float
 constexpr int kNoExp = -(1 << 28);
 void conv3x3_f32_peaks(const float* U, const int* in_exp, const int* mag, int C, int F, int* peak,
                        int* reach, int* bad, hipStream_t s);
-// Whether halves hold what fp32 does: exponents as above, of inputs of magnitude up to 2^top.
-bool conv3x3_f32_holds(int peak, int reach, int top);
+// Whether an output channel's largest product is at least 2^-most of its largest filter times the largest
+// input (exponents as above, of inputs of magnitude up to 2^top): with most = 14 halves hold what fp32 does.
+bool conv3x3_f32_holds(int peak, int reach, int top, int most);
 bool conv3x3_f32_exponent(int peak, float scale, float mean, int out_exp, int& e);
 // Filters of one layer from U (device), exponents per channel (device).
 void conv3x3_f32_filters(const float* U, const int* in_exp, const int* exp, _Float16* Wf, int C, int Cp,

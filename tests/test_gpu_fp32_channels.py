@@ -234,3 +234,43 @@ def test_planes_in_bits_are_those_in_floats(pkg, netgen, filters, maxb, far):
             assert err <= 2 * alike + 2.0 ** -24, (i, name, err, alike)
     pipe.close()
     plain.close()
+
+
+@pytest.mark.parametrize("filters,maxb", [(64, 8), (128, 40)])
+@pytest.mark.parametrize("scale,mean", [(1.0, 1e8), (2.0 ** 24, 1e3), (2.0 ** 24, -1e-30)])
+def test_channels_that_look_larger_than_they_are(pkg, netgen, filters, maxb, scale, mean):
+    """Channels whose batch norm says that they are 2^20 and more above the others, and that never fire
+    (or, with filters to match, are alike): the others keep their precision."""
+    print("case: scale %g mean %g, %d filters of %d" % (scale, mean, filters, maxb), flush=True)
+    n = 3
+    net = netgen.make_network(2, filters, 8700)
+    where = ((0, 3), (1, 5), (2, 7), (3, 9), (4, 1))
+    for l, k in where:
+        net.bn_mean[l][k] = mean
+        if mean < 0:
+            net.conv_w[l][k] *= np.float32(1.0 / scale)
+    x = netgen.synthetic_inputs(n, seed=8701)
+    w, _ = netgen.prepare(net)
+    for l, k in where:
+        w.m_batchnorm_stddevs[l] = np.array(w.m_batchnorm_stddevs[l], np.float32)
+        w.m_batchnorm_stddevs[l][k] = scale
+    # the same in float64: what never fires is zero whatever its scale; else the scale in the filters
+    same = copy.deepcopy(net)
+    for l, k in where:
+        same.bn_var[l][k] = 1.0 - 1e-5
+        if mean < 0:
+            same.conv_w[l][k] *= np.float32(scale)
+            same.bn_mean[l][k] *= scale
+    want = tower_f64(same, x)
+    pipe = pkg.HIPScheduler(pkg.FP32, maxb)
+    pipe.initialize(filters)
+    pipe.push_weights(6, 18, filters, w)
+    assert is_direct(pkg, pipe, x)
+    plain = make_pipe(pkg, netgen, same, maxb)
+    base, got = plain.forward_batch(x), pipe.forward_batch(x)
+    for i in range(n):
+        for k, name in enumerate(("pol", "val")):
+            alike, err = rel_l2(base[k][i], want[name][i]), rel_l2(got[k][i], want[name][i])
+            assert err <= 2 * alike + 2.0 ** -24, (i, name, err, alike)
+    pipe.close()
+    plain.close()
