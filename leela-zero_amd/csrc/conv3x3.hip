@@ -375,14 +375,13 @@ bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
 //   64 boards   32.0*   29.2*   26.4*   25.1*   28.5*   24.1
 //   80 boards   40.1*   35.6*   32.2*   33.1*   30.2*   37.6*
 //  128 boards   61.0*   54.2*   47.6*   45.6*   44.9*   42.9*
-// Two chains side by side want larger tiles (us per layer and chain): 20 boards 128x64 8.5, 192x64
-// 8.9, 96x64 9.6; 40 boards 192x64 13.3, 128x128 13.4, 128x64 14.3, 192x128 14.8; 64 boards 192x128 19.1,
-// 192x64 20.2; 80 boards 192x128 23.7, 128x128 25.3.  So 128x128 is taken up to one work-group per unit,
-// where it gains either way, and not up to two (72 to 90 boards of 256 filters one chain at a time
-// 37 -> 30, two side by side 4 to 8 % slower).  At other widths the order is the same: 128 filters, 44
-// boards 48x64 7.9, 128x64 6.7 (two chains 5.9 | 4.9), 70 boards 128x128 10.7, 192x128 12.1 (7.2 | 7.9);
-// 384 filters, 13 boards 192x64 16.8, 128x64 13.7 (13.4 | 12.0), 26 boards 128x128 24.0, 192x128 26.2 (19.4 |
-// 19.8).  64 and 192 filters have no tile of 128 channels; there 128x64 is taken up to two work-groups
+// (128x128 with its wavefronts two by two; side by side, as it is now, 40 boards take 16.7.)  Two chains side by
+// side want larger tiles (us per layer and chain): 20 boards 128x64 8.5, 192x64
+// 8.9, 96x64 9.6; 40 boards 192x64 13.3, 128x64 14.3, 192x128 14.8; 64 boards 192x128 19.1,
+// 192x64 20.2; 80 boards 192x128 23.7, 128x128 25.3.  At other widths the order is the same: 128 filters, 44
+// boards 48x64 7.9, 128x64 6.7 (two chains 5.9 | 4.9);
+// 384 filters, 13 boards 192x64 16.8, 128x64 13.7 (13.4 | 12.0).  64 and 192 filters have no tile of 128
+// channels; there 128x64 is taken up to two work-groups
 // per unit (192 filters, 52 boards 128x192 15.9, 128x64 13.6, two chains 12.7 | 12.0; 64 filters, 150 boards
 // 192x64 8.7, 128x64 7.1), and beyond, 128x192 takes the place of 192x128 (192 filters, 70 boards 192x64
 // 17.9, 128x192 16.5).  64 filters, whose one chunk is over soon, keep 48x64 up to three work-groups
@@ -443,37 +442,63 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
         LZ_CONV(3, 2, 1, 2, 6, 3, 0, 2);
         return;
     }
+    // Larger tiles, the lowest that makes one round.  Of 128 channels where the width has them: the four
+    // wavefronts stand side by side, every filter is fetched once and not by two rows of them, and
+    // heights go in steps of 16 points.  Layers of 256 filters, 192x64 and 128x128 (wavefronts two by two) -> this, us:
+    // 24 boards 13.4 -> 12.2 (80x128), 32: 13.6 -> 13.3 (96x128), 40: 18.1 -> 16.7 (128x128), 50: 20.1 -> 18.6
+    // (144x128), 56: 21.5 -> 20.9; of 384, 16 boards 17.0 -> 15.3, 26: 23.6 -> 21.3; of 128, 50 boards 8.6 -> 7.7.
+    // Two or three forwards side by side gain as much from 112x128 on (256 filters, 50 boards, two: 16.4 -> 15.3) and
+    // nothing below (32 boards, two: 10.3 -> 10.6), so there 192x64 stays.
+#define LZ_WIDE(RB)                         \
+    case RB:                                \
+        LZ_CONV(RB, 2, 1, 4, 6, 1, 0, 2);   \
+        return
+    auto wide = [&](int rb) {
+        switch (rb) {
+            LZ_WIDE(5);
+            LZ_WIDE(6);
+            LZ_WIDE(7);
+            LZ_WIDE(8);
+            LZ_WIDE(9);
+            LZ_WIDE(10);
+            default: LZ_CONV(6, 4, 2, 2, 3, 1, 0, 2); return;
+        }
+    };
+#undef LZ_WIDE
+    const bool wide_columns = Kp % 128 == 0;
+    if (wide_columns && lanes == 1) {
+        if (const int rb = one_round_blocks(rows, Kp / 128, 5)) return wide(rb);
+    }
+    // 192 filters, 33 boards 192x64 11.2, 160x64 10.1 us (two side by side 7.6 | 7.1)
+    if (!wide_columns && Kp != 64 && groups(160, 64) <= kUnits) {
+        LZ_CONV(5, 2, 2, 2, 6, 1, 0, 2);
+        return;
+    }
     if (groups(192, 64) <= kUnits) {
         LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);
         return;
     }
-    if (Kp % 128 == 0 && groups(128, 128) <= kUnits) {
-        LZ_CONV(4, 4, 2, 2, 3, 1, 0, 2);
-        return;
+    if (wide_columns) {
+        if (const int rb = one_round_blocks(rows, Kp / 128, 7)) return wide(rb);
     }
     if ((Kp == 64 || Kp == 192) && groups(128, 64) <= 2 * kUnits) {
         LZ_CONV(4, 2, 2, 2, 6, 1, 0, 2);
         return;
     }
     // More than a round of every tile.  What a forward with the device to itself takes is rounds times
-    // tile, whether the last round is full or nearly empty: 10 blocks of 256 filters, 69 to 90 boards
-    // 763 - 791 us on 192x128 and 588 - 649 on 128x128; of 384 filters, 46 to 60 boards 1059 - 1087 and
-    // 821 - 909; of 192 filters, 91 to 120 boards 637 - 659 on 128x192, 527 - 566 on 128x64, 135 boards
+    // tile, whether the last round is full or nearly empty: a layer of 256 filters, 70 boards 36 us on 192x128
+    // and 26 on 112x128, 100 boards 38 and 34 (144x128); 10 blocks of 192 filters, 91 to 120 boards
+    // 637 - 659 us on 128x192, 527 - 566 on 128x64, 135 boards
     // 678 and 590 on 192x64.  Side by side with another forward, which fills the gaps, the tile
     // that reads least is the best one.
+    if (wide_columns) return wide(lanes == 1 ? least_rounds_blocks(rows, Kp / 128) : 12);
     auto rounds = [&](int mt, int cw) { return (groups(mt, cw) + kUnits - 1) / kUnits * mt * cw; };
-    if (lanes == 1 && Kp % 128 == 0 && rounds(128, 128) < rounds(192, 128)) {
-        LZ_CONV(4, 4, 2, 2, 3, 1, 0, 2);
-        return;
-    }
-    if (lanes == 1 && Kp % 128 != 0 && rounds(128, 64) < rounds(192, 64) &&
+    if (lanes == 1 && rounds(128, 64) < rounds(192, 64) &&
         (Kp != 192 || rounds(128, 64) < rounds(128, 192))) {
         LZ_CONV(4, 2, 2, 2, 6, 1, 0, 2);
         return;
     }
-    if (Kp % 128 == 0)
-        LZ_CONV(6, 4, 2, 2, 3, 1, 0, 2);
-    else if (Kp == 192 && (lanes > 1 || rounds(128, 192) <= rounds(192, 64)))
+    if (Kp == 192 && (lanes > 1 || rounds(128, 192) <= rounds(192, 64)))
         LZ_CONV(4, 6, 2, 2, 3, 1, 0, 2);
     else
         LZ_CONV(6, 2, 2, 2, 6, 1, 0, 2);

@@ -493,24 +493,47 @@ PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, f
     if (groups(128, 64) <= kUnits) {
         return LZ_F32(4, 2, 2, 2, 6, 0, 2);
     }
+    // launch_conv3x3's tiles of 128 channels and 160x64.  256 filters, 24 boards 192x64 32.2, 80x128 27.8 us (two side by
+    // side 23.9 | 22.3), 50 boards 192x128 50.4, 144x128 47.9 (42.8 | 41.0); 384 filters, 16 boards 44.6 -> 38.5, 26: 56.4
+    // -> 53.3; 128 filters, 50 boards 19.5 -> 17.4; 192 filters, 33 boards 192x64 26.3, 160x64 23.5 (19.5 | 18.2).
+#define LZ_WIDE(RB) \
+    case RB:        \
+        return LZ_F32(RB, 2, 1, 4, (RB < 9 ? 6 : 3), 0, 2)
+    auto wide = [&](int rb) {
+        switch (rb) {
+            LZ_WIDE(5);
+            LZ_WIDE(6);
+            LZ_WIDE(7);
+            LZ_WIDE(8);
+            LZ_WIDE(9);
+            LZ_WIDE(10);
+            default: return LZ_F32(6, 4, 2, 2, 3, 0, 2);
+        }
+    };
+#undef LZ_WIDE
+    const bool wide_columns = Kp % 128 == 0;
+    if (wide_columns && lanes <= 2) {
+        const int rb = one_round_blocks(rows, Kp / 128, 5);
+        if (rb > 0 && (lanes == 1 || rb != 6)) return wide(rb);
+    }
+    if (!wide_columns && Kp != 64 && groups(160, 64) <= kUnits) {
+        return LZ_F32(5, 2, 2, 2, 6, 0, 2);
+    }
     if (groups(192, 64) <= kUnits) {
         return LZ_F32(6, 2, 2, 2, 6, 0, 2);
     }
-    if (Kp % 128 == 0 && groups(128, 128) <= kUnits) {
-        return LZ_F32(4, 4, 2, 2, 3, 0, 2);
+    if (wide_columns) {
+        if (const int rb = one_round_blocks(rows, Kp / 128, 7)) return wide(rb);
     }
     if ((Kp == 64 || Kp == 192) && groups(128, 64) <= 2 * kUnits) {
         return LZ_F32(4, 2, 2, 2, 6, 0, 2);
     }
-    // (launch_conv3x3's rule: 10 blocks of 256 filters, 70 boards 2002 us on 192x128 and 1518 on 128x128;
-    // of 384 filters, 47 boards 2889 and 2218; of 192 filters, 91 boards 1597 on 128x192 and 1306 on 128x64)
+    // (launch_conv3x3's rule for more than a round)
+    if (wide_columns) return wide(lanes == 1 ? least_rounds_blocks(rows, Kp / 128) : 12);
     auto rounds = [&](int mt, int cw) { return (groups(mt, cw) + kUnits - 1) / kUnits * mt * cw; };
-    if (lanes == 1 && Kp % 128 == 0 && rounds(128, 128) < rounds(192, 128))
-        return LZ_F32(4, 4, 2, 2, 3, 0, 2);
-    if (lanes == 1 && Kp % 128 != 0 && rounds(128, 64) < rounds(192, 64) &&
+    if (lanes == 1 && rounds(128, 64) < rounds(192, 64) &&
         (Kp != 192 || rounds(128, 64) < rounds(128, 192)))
         return LZ_F32(4, 2, 2, 2, 6, 0, 2);
-    if (Kp % 128 == 0) return LZ_F32(6, 4, 2, 2, 3, 0, 2);
     if (Kp == 192 && (lanes > 1 || rounds(128, 192) <= rounds(192, 64)))
         return LZ_F32(4, 6, 2, 2, 3, 0, 2);
     return LZ_F32(6, 2, 2, 2, 6, 0, 2);

@@ -138,6 +138,26 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvGrid& g) {
 
 constexpr int kUnits = 256;   // compute units
 
+// Tiles of 128 channels, 16 rb points high, of a layer of `rows` points and `cols` such columns: the
+// lowest from `lowest` to 10 blocks that makes no more than one work-group per unit (0: none does), and the
+// one that takes the least rounds times tile (12 is the tile of 192x128, which wins where several take the same).
+static inline int one_round_blocks(int rows, int cols, int lowest) {
+    for (int rb = lowest; rb <= 10; rb++)
+        if ((rows + rb * 16 - 1) / (rb * 16) * cols <= kUnits) return rb;
+    return 0;
+}
+static inline int least_rounds_blocks(int rows, int cols) {
+    int best = 12, least = 0;
+    for (int rb = 12; rb >= 5; rb--) {
+        const int work = ((rows + rb * 16 - 1) / (rb * 16) * cols + kUnits - 1) / kUnits * rb;
+        if (rb != 11 && (least == 0 || work < least)) {
+            best = rb;
+            least = work;
+        }
+    }
+    return best;
+}
+
 // What a transformed filter may be off by however small it is: a few sums of numbers that were rounded
 // to zero below 2^-126.
 constexpr float kFilterFloor = 0x1p-123f;

@@ -1007,6 +1007,24 @@ def test_direct_convolution_tiles_of_16_channels(pkg, netgen, orc, filters, batc
     test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches)
 
 
+@pytest.mark.parametrize("precision", [1, 0])
+@pytest.mark.parametrize("filters,batches", [
+    # 80x128 to 160x128 and 192x128 points by channels, the last batch of each and the first of the next
+    (256, (23, 28, 29, 34, 35, 39, 40, 45, 46, 51, 52, 56, 57)),
+    (128, (46, 56, 57, 68, 69, 79, 80, 90, 91, 102, 103, 113, 114)),
+    (384, (15, 18, 19, 22, 23, 26, 27, 30, 31, 33, 34, 37, 38)),
+    (192, (31, 37, 38)), (320, (19, 22, 23)),       # 160x64
+    (256, (70, 81, 100)),                           # more than a round
+])
+def test_direct_convolution_tiles_in_steps_of_16_points(pkg, netgen, orc, precision, filters, batches):
+    """Tiles whose four wavefronts stand side by side, and 160x64, on both sides of every change, with the
+    bounds of the tests above."""
+    if precision == pkg.FP16:
+        test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches)
+    else:
+        test_fp32_direct_convolution(pkg, netgen, orc, filters, max(batches), batches)
+
+
 @pytest.mark.parametrize("filters,maxb", [(128, 40), (192, 16), (192, 40), (256, 9), (384, 28), (512, 44)])
 def test_fp32_filters_of_no_3x3_filter(pkg, netgen, orc, filters, maxb):
     """fp32 networks whose filters are no 3x3 ones run the Winograd kernels: the streaming GEMM, the
