@@ -513,18 +513,25 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // fetched twice or four times, and all wait for the whole patch.  Here every wavefront owns the
 // whole tile and KW-th of the k-steps (HPW halves of a chunk of 64 channels, all nine taps): each
 // operand is fetched once, a wavefront stages its own input channels and waits for nobody, its
-// filters are in flight all at once (D = 9 HPW; two thirds of them where five or more wavefronts
-// share the registers), and the partial sums meet in LDS at the end, in the order of the wavefronts.
+// filters are in flight all at once (D = 9 HPW; less where that would take the registers of another
+// wavefront on the SIMD), and the partial sums meet in LDS at the end, in the order of the wavefronts.
 // Measured per forward of 10 blocks, conv3x3_k -> this with tiles of 32 channels, us: 128 filters, 1 board 99 -> 82, 8 boards
 // 110 -> 92; 192 filters, 1 board 120 -> 98, 5 boards 134 -> 114; 256 filters, 1 board 132 -> 104, 5
 // boards 150 -> 138; of 5 blocks, 1 board: 320 filters 105 -> 60, 384 116 -> 63, 448 131 -> 70, 512
 // 136 -> 76.
-// Tiles of 80x32 and 96x32 points x channels for larger batches take 5 to 13 % off a forward
-// alone (20 blocks of 256 filters, 6 boards 322 -> 285 us) and add 10 to 24 % to two or three side by side,
-// of whose work-groups a unit then holds one; 96x64 and 192x64 gave nothing either way.
+// 96x32 points x channels for larger batches is slower than conv3x3_k (192 filters, 11 boards 244 -> 259 us a
+// forward of 20 blocks, two side by side 162 -> 210), 96x64 and 192x64 gave nothing either way.
 // The order of the sum differs from conv3x3_k's, so a network uses one or the other whatever the
 // batch (conv3x3_splits).
-template <int RB, int NB, int KW, int HPW, int D>
+//
+// PAIRS (192 and 256 filters): the two halves of a chunk are summed apart and then added, which gives the
+// same bits where one wavefront has both halves and where two have one each.  Two take half as long over
+// their steps, their loads and their share of the patch: a forward with the device to itself, 20 blocks of 256
+// filters, 1 board 168 -> 160 us, 2: 193 -> 180, 5: 262 -> 243; of 192, 1 board 147 -> 146, 7: 225 -> 213.  Side by
+// side with other forwards one has both, with the filters of 12 steps ahead instead of all 18, so that a unit
+// holds two work-groups (192 filters, 7 boards, three at once 166 -> 111 us each; 256, 2 boards, two at once
+// 113 -> 107).
+template <int RB, int NB, int KW, int HPW, int D, bool PAIRS>
 __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
     half_t* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
@@ -633,11 +640,14 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     for (int i = 0; i < RB; i++)
         arow[i] = patch_cell(ps, min(i * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
                   (lane >> 4) * 16;
-    float4v acc[RB][NB];
+    constexpr int SUMS = PAIRS ? HPW : 1;
+    float4v acc[SUMS][RB][NB];
 #pragma unroll
-    for (int i = 0; i < RB; i++)
+    for (int h = 0; h < SUMS; h++)
 #pragma unroll
-        for (int j = 0; j < NB; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) acc[h][i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
     int4v a[DA][RB];
     auto aread = [&](int i, int st) {
@@ -660,9 +670,9 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
                     wload((st + D - 1) % D, j, st + D - 1);
 #pragma unroll
             for (int j = 0; j < NB; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                acc[st / 9 % SUMS][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                     __builtin_bit_cast(half8v, w[st % D][j]),
-                    __builtin_bit_cast(half8v, a[st % DA][i]), acc[i][j], 0, 0, 0);
+                    __builtin_bit_cast(half8v, a[st % DA][i]), acc[st / 9 % SUMS][i][j], 0, 0, 0);
             if (st + DA < STEPS) a[st % DA][i] = aread(i, st + DA);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -675,7 +685,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 #pragma unroll
         for (int j = 0; j < NB; j++)
             *reinterpret_cast<float4v*>(lds + ((wave * RB + i) * NB + j) * 1024 + lane * 16) =
-                acc[i][j];
+                SUMS == 2 ? acc[0][i][j] + acc[SUMS - 1][i][j] : acc[0][i][j];
     lds_barrier();
 #pragma unroll
     for (int q = 0; q < QP; q++) {
@@ -692,9 +702,14 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
         HalfE o;
 #pragma unroll
         for (int e = 0; e < E; e++) {
-            float v = part[0][e / 4][e % 4];
+            constexpr int STEP = PAIRS && HPW == 1 ? 2 : 1;
+            auto sum = [&](int k) {
+                const float first = part[k][e / 4][e % 4];
+                return STEP == 2 ? first + part[k + STEP - 1][e / 4][e % 4] : first;
+            };
+            float v = sum(0);
 #pragma unroll
-            for (int k = 1; k < KW; k++) v += part[k][e / 4][e % 4];
+            for (int k = STEP; k < KW; k += STEP) v += sum(k);
             o[e] = (half_t)fminf(
                 fmaxf(0.0f, fmaf((float)rh[e], rfac, fmaf(v, bn[0][cl + e], bn[1][cl + e]))),
                 kActStoreMax);
@@ -713,14 +728,17 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 // has to deliver to a work-group, which is what a layer of one board waits for: against 32 x 32
 // tiles 128 filters 3.8 -> 3.3 us, 192 4.4 -> 3.8, 256 4.9 -> 4.3, 320 5.3 -> 4.7.  48 x 16 is worth
 // 2 to 4 % up to 256 filters (192 filters, 2 boards 4.4 -> 4.3 us) and no longer beyond (384
-// filters, 1 board 5.5 -> 5.7).
+// filters, 1 board 5.5 -> 5.7).  80 x 32 is as fast as conv3x3_k's tiles or faster at 128 to 256 filters (20 blocks, us:
+// 128 filters, 14 boards 204 -> 195, three side by side 98 -> 93; 192, 9 boards 239 -> 239 and 133 -> 131; 256, 7 boards
+// 271 -> 260 and 162 -> 153), and a handle of that size then takes this kernel for its small batches too (1 board
+// of 128, 192, 256 filters 169 -> 133, 185 -> 147, 208 -> 159).
 struct SplitTile {
     int rb, nb;
 };
 static SplitTile split_tile(int n, int Kp) {
-    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}};
+    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}, {5, 2}};
     for (const SplitTile& t : kTiles)
-        if ((t.rb * t.nb != 3 || Kp <= 256) &&
+        if ((t.rb * t.nb != 3 || Kp <= 256) && (t.rb < 5 || (Kp >= 128 && Kp <= 256)) &&
             (n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
     return {0, 0};
 }
@@ -733,8 +751,10 @@ bool conv3x3_splits(int Kp, int max_batch) {
 
 void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                           const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
-                          int Kp, hipStream_t s, LaunchTimer* t) {
-    const SplitTile tile = split_tile(n, Kp);
+                          int Kp, int lanes, hipStream_t s, LaunchTimer* t) {
+    SplitTile tile = split_tile(n, Kp);
+    // (80x32 of 256 filters takes more than half of the LDS: two work-groups on a unit want less)
+    if (lanes > 1 && Kp == 256 && tile.rb == 5) tile = {4, 2};
     if (!conv3x3_splits(Kp, n) || Cp != Kp)
         throw std::invalid_argument("no split convolution for this width or batch");
     const ConvGrid g = conv_grid((n * kPts + tile.rb * 16 - 1) / (tile.rb * 16), Kp / (16 * tile.nb),
@@ -744,23 +764,33 @@ void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, 
                bn_mean, rfac, n, Kp, g);
     };
     // KW wavefronts x HPW halves of a chunk
-#define LZ_SPLIT(KW, HPW, D)                                               \
-    if (tile.nb == 1) {                                                    \
-        if (tile.rb == 2) go(conv3x3_split_k<2, 1, KW, HPW, D>, KW);       \
-        else if constexpr (KW < 5) go(conv3x3_split_k<3, 1, KW, HPW, D>, KW); \
-    } else if (tile.rb == 2) go(conv3x3_split_k<2, 2, KW, HPW, D>, KW);    \
-    else if (tile.rb == 3) go(conv3x3_split_k<3, 2, KW, HPW, D>, KW);      \
-    else if constexpr (KW < 8) go(conv3x3_split_k<4, 2, KW, HPW, D>, KW)
+#define LZ_SPLIT(KW, HPW, D, PAIRS)                                                      \
+    if (tile.nb == 1) {                                                                  \
+        if (tile.rb == 2) go(conv3x3_split_k<2, 1, KW, HPW, D, PAIRS>, KW);              \
+        else if constexpr (KW * HPW <= 8) go(conv3x3_split_k<3, 1, KW, HPW, D, PAIRS>, KW); \
+    } else if (tile.rb == 2) go(conv3x3_split_k<2, 2, KW, HPW, D, PAIRS>, KW);           \
+    else if (tile.rb == 3) go(conv3x3_split_k<3, 2, KW, HPW, D, PAIRS>, KW);             \
+    else if (tile.rb == 4) {                                                             \
+        if constexpr (KW * HPW < 16) go(conv3x3_split_k<4, 2, KW, HPW, D, PAIRS>, KW);   \
+    } else if constexpr (KW * HPW <= 8 && KW >= 3) {                                     \
+        go(conv3x3_split_k<5, 2, KW, HPW, 9, PAIRS>, KW);                                \
+    }
     switch (Kp) {
-        case 64: LZ_SPLIT(2, 1, 9); break;
-        case 128: LZ_SPLIT(4, 1, 9); break;
-        case 192: LZ_SPLIT(3, 2, 18); break;
-        case 256: LZ_SPLIT(4, 2, 18); break;
+        case 64: LZ_SPLIT(2, 1, 9, false); break;
+        case 128: LZ_SPLIT(4, 1, 9, false); break;
+        case 192:
+            if (lanes == 1) { LZ_SPLIT(6, 1, 9, true); }
+            else { LZ_SPLIT(3, 2, 12, true); }
+            break;
+        case 256:
+            if (lanes == 1) { LZ_SPLIT(8, 1, 9, true); }
+            else { LZ_SPLIT(4, 2, 12, true); }
+            break;
         // from here on two wavefronts share a SIMD's registers: two thirds of the filters ahead
-        case 320: LZ_SPLIT(5, 2, 12); break;
-        case 384: LZ_SPLIT(6, 2, 12); break;
-        case 448: LZ_SPLIT(7, 2, 12); break;
-        default: LZ_SPLIT(8, 2, 12); break;   // (the largest is for 3 boards, which no longer fit)
+        case 320: LZ_SPLIT(5, 2, 12, false); break;
+        case 384: LZ_SPLIT(6, 2, 12, false); break;
+        case 448: LZ_SPLIT(7, 2, 12, false); break;
+        default: LZ_SPLIT(8, 2, 12, false); break;   // (the largest is for 3 boards, which no longer fit)
     }
 #undef LZ_SPLIT
 }

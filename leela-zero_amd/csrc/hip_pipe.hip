@@ -1225,7 +1225,7 @@ private:
         if constexpr (sizeof(P) == 2) {
             const bool split = L.Cp == m_Fp && conv3x3_splits(m_Fp, m_max_batch);
             if (split)
-                launch_conv3x3_split(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, s, t);
+                launch_conv3x3_split(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, lanes, s, t);
             else
                 launch_conv3x3(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, lanes, s, t);
         } else {

@@ -1007,6 +1007,17 @@ def test_direct_convolution_tiles_of_16_channels(pkg, netgen, orc, filters, batc
     test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches)
 
 
+@pytest.mark.parametrize("filters,batches", [
+    (128, (1, 11, 12, 14)), (192, (1, 2, 3, 5, 7)), (192, (1, 7, 8, 9)), (256, (1, 2, 3, 5)), (256, (1, 5, 6, 7)),
+    (128, (15,)), (192, (10,)), (256, (8,)),     # the first handles that no longer deal out their sums
+])
+def test_sums_dealt_to_more_wavefronts(pkg, netgen, orc, filters, batches):
+    """Handles whose layers deal their sum to the wavefronts, up to tiles of 80 points: each tile against a
+    float32 convolution, and on several lanes, where a wavefront has two shares of the sum, the bits of one lane."""
+    test_direct_convolution_tiles_of_128_points(pkg, netgen, orc, filters, batches)
+    test_layers_replayed_on_several_lanes(pkg, netgen, orc, filters, pkg.FP16, batches)
+
+
 @pytest.mark.parametrize("precision", [1, 0])
 @pytest.mark.parametrize("filters,batches", [
     # 80x128 to 160x128 and 192x128 points by channels, the last batch of each and the first of the next
