@@ -112,24 +112,32 @@ static PeakIn peak_in(const PeakMap& p) {
             (unsigned)((((uint64_t)1 << 32) + p.mt - 1) / p.mt),
             (unsigned)((((uint64_t)1 << 31) + p.tiles_n - 1) / p.tiles_n)};
 }
-// Requests a board's slots (LOADS per lane) and takes their maximum.
+// The most slots a board may have: it meets 360 / mt + 2 rows of tiles at most.
+static constexpr int peak_slots(int mt, int tiles_n) { return (360 / mt + 2) * tiles_n; }
+static void peaks_fit(const PeakMap& p, int loads) {
+    if (peak_slots(p.mt, p.tiles_n) > 64 * loads) throw std::logic_error("a board of more peaks than are read");
+}
+// Requests up to MAX x 64 slots of a board, the first ALL x 64 without a look at how many there are, and takes
+// their maximum.  Behind a branch that is taken a request is waited for at the branch's end, with everything
+// requested before it: small batches, whose tiles are small, had two to five of those before their planes.
+// Without them a forward of 15 layers of 192 filters takes 198 us instead of 215 for 1 board, 20 of 256 283
+// instead of 307 (2 boards 344, 359), 20 of 128 216 instead of 227, 10 of 512 255 instead of 272.
+template <int ALL, int MAX>
 struct BoardPeak {
-    static constexpr int kLoads = 8;
-    unsigned v[kLoads];
-    int count = 0;
+    unsigned v[MAX];
     __device__ __forceinline__ void load(const PeakIn& p, unsigned board, unsigned lane) {
         const unsigned first = board * kPts, t0 = __umulhi(first, p.inv_m);
-        const unsigned tiles = __umulhi(first + kPts - 1, p.inv_m) - t0 + 1;
-        count = (int)(tiles * p.tiles_n);
+        const unsigned tiles = __umulhi(first + kPts - 1, p.inv_m) - t0 + 1, count = tiles * p.tiles_n;
         const unsigned late = t0 * p.mt < first ? 1u : 0u;   // the first tile's second board
         const __amdgpu_buffer_rsrc_t r =
             make_rsrc(p.slots + (size_t)t0 * 2 * p.tiles_n, (size_t)tiles * 2 * p.tiles_n * 4);
 #pragma unroll
-        for (int k = 0; k < kLoads; k++) {
-            v[k] = 0;
-            if (k * 64 < count) {
+        for (int k = 0; k < MAX; k++) {
+            if (k >= ALL) v[k] = 0;
+            if (k < ALL || k * 64 < (int)count) {
                 const unsigned i = lane + k * 64, t = __umulhi(i * 2u, p.inv_n);
                 const unsigned at = (t * 2 + (t == 0 ? late : 0u)) * p.tiles_n + i - t * p.tiles_n;
+                // (beyond the last row of tiles this lies outside the buffer: 0)
                 v[k] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(r, at * 4u, 0, 0);
             }
         }
@@ -137,11 +145,10 @@ struct BoardPeak {
     __device__ __forceinline__ unsigned get() const {
         unsigned top = v[0];
 #pragma unroll
-        for (int k = 1; k < kLoads; k++) top = max(top, v[k]);
+        for (int k = 1; k < MAX; k++) top = max(top, v[k]);
         return wave_max(top);
     }
 };
-
 // Scales of a tile's first board and of the next one, and their reciprocals.
 struct TileScales {
     float s0, s1, u0, u1;
@@ -150,8 +157,9 @@ struct TileScales {
 __device__ __forceinline__ unsigned second_board(const PatchStart& s) {
     return (s.mb + 2) * kCellsPerBoard - s.q0;
 }
+template <int ALL, int MAX>
 struct TilePeaks {
-    BoardPeak a, b;
+    BoardPeak<ALL, MAX> a, b;
     bool two;   // the tile reaches a second board
     __device__ __forceinline__ void load(const PeakIn& p, const PatchStart& s, int m0, int mt, int rows,
                                          unsigned lane) {
@@ -244,7 +252,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     __builtin_amdgcn_sched_barrier(0);
 
     const PatchStart ps = patch_start(m0);
-    TilePeaks tp;
+    TilePeaks<0, 2> tp;
     tp.load(peaks, ps, m0, MT, rows, lane);
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 4);
     const unsigned xrow = (unsigned)Cp * 4u;     // bytes of a cell in memory
@@ -446,6 +454,7 @@ static PeakMap launch_f32_as(const float* X, const half_t* Wf, const float* res,
     constexpr int MT = WR * RB * 16, CW = WN * NB * 16;
     const ConvGrid g = conv_grid((n * kPts + MT - 1) / MT, Kp / CW, (size_t)36 * Cp * Kp,
                                  (size_t)n * kPts * Cp * 4);
+    peaks_fit(peaks, 2);
     launch(conv3x3_f32_k<RB, NB, WR, WN, D, CC, OCC>, dim3(8 * g.share), dim3(64 * WR * WN), s, t, X,
            Wf, res, Y, bn_scale, bn_mean, rfac, peak_in(peaks), slots, n, Cp, Kp, g);
     return {slots, MT, Kp / CW};
@@ -550,6 +559,12 @@ PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, f
 // A tile is 16 channels wide where that makes no more than one work-group per unit: with hi
 // and lo parts the filters are twice as many bytes as in fp16, and what the L1 delivers to a unit
 // (filters of NB * 16 channels, planes of conv_cells(RB * 16) cells) is what a tile waits for.
+//
+// The peaks come from a layer of the same tiles, or from conv3x3_f32_k's 32x64 of the first layer.
+static constexpr int split_peak_loads(int rb, int nb, int filters) {
+    const int own = peak_slots(rb * 16, filters / (nb * 16)), first = peak_slots(32, filters / 64);
+    return ((own > first ? own : first) + 63) / 64;
+}
 template <int RB, int NB, int KW, int HPW, int D>
 __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     const float* __restrict__ X, const half_t* __restrict__ Wf, const float* __restrict__ res,
@@ -599,7 +614,8 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     };
     filters(0, F0);
     const PatchStart ps = patch_start(m0);
-    TilePeaks tp;
+    constexpr int PEAKS = split_peak_loads(RB, NB, Cp);
+    TilePeaks<PEAKS, PEAKS> tp;
     tp.load(peaks, ps, m0, MT, rows, lane);
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 4);
     constexpr unsigned xrow = Cp * 4;   // bytes of a cell in memory
@@ -783,6 +799,7 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
         throw std::invalid_argument("no split convolution for this width or batch");
     const ConvGrid g = conv_grid((n * kPts + tile.rb * 16 - 1) / (tile.rb * 16), Kp / (16 * tile.nb),
                                  (size_t)36 * Cp * Kp, (size_t)n * kPts * Cp * 4);
+    peaks_fit(peaks, split_peak_loads(tile.rb, tile.nb, Kp));
     auto go = [&](auto kernel, int waves) {
         launch(kernel, dim3(8 * g.share), dim3(64 * waves), s, t, X, Wf, res, Y, bn_scale, bn_mean,
                rfac, peak_in(peaks), slots, n, Kp, g);

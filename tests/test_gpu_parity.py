@@ -1072,6 +1072,34 @@ def test_fp32_range_and_values_that_are_no_numbers(pkg, netgen, orc):
     pipe.close()
 
 
+@pytest.mark.parametrize("filters,maxb,batches", [
+    (64, 8, (1, 8)), (192, 8, (1, 2, 3, 8)), (256, 5, (1, 2, 3, 5)), (320, 4, (1, 2, 4)), (384, 3, (1, 2, 3)),
+    (448, 3, (1, 3)), (512, 4, (1, 2, 3, 4)), (512, 9, (1, 4, 9)),
+])
+def test_fp32_largest_planes_in_the_last_tile(pkg, netgen, orc, filters, maxb, batches):
+    """fp32 layers whose results are 1e6 times larger in their last channel: read with the scale of the other
+    tiles' peaks they would leave fp16's range.  The bound is that of planes of any magnitude above."""
+    net = netgen.make_network(1, filters, 6970 + filters)
+    for layer in (0, 1):
+        net.conv_w[layer][-1] *= 1e6
+    w, h = netgen.prepare(net)
+    w_ref, h_ref = netgen.prepare(net, orc.winograd_transform_f, orc.process_bn_var)
+    ref = orc.OraclePipe()
+    ref.initialize(filters)
+    ref.push_weights(6, 18, filters, w_ref)
+    pipe = pkg.HIPScheduler(pkg.FP32, maxb)
+    pipe.initialize(filters)
+    pipe.push_weights(6, 18, filters, w)
+    x = netgen.synthetic_inputs(maxb, seed=6971)
+    for n in batches:
+        print("case: fp32 peaks, %d filters, %d boards of %d" % (filters, n, maxb), flush=True)
+        pol, val = pipe.forward_batch(x[:n])
+        for i in {0, n - 1}:
+            rp, rv = ref.forward(x[i])
+            assert rel_l2(pol[i], rp) <= 1e-5 and rel_l2(val[i], rv) <= 1e-5, (n, i)
+    pipe.close()
+
+
 @pytest.mark.parametrize("n", [1, 31, 32, 33, 100])
 def test_heads_at_the_edges_of_their_tiles(pkg, netgen, orc, n):
     """The fully connected heads work on tiles of 32 positions by 32 outputs, and sixteen
