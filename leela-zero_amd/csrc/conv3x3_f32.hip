@@ -560,24 +560,35 @@ PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, f
 // and lo parts the filters are twice as many bytes as in fp16, and what the L1 delivers to a unit
 // (filters of NB * 16 channels, planes of conv_cells(RB * 16) cells) is what a tile waits for.
 //
+// A unit has four SIMDs: two wavefronts leave two of them idle, five and six leave two or three with half the
+// work of the others.  There WR x WN wavefronts share the channels, and each has its rows or columns of
+// blocks; they stage the planes together.  Measured per forward of 10 blocks, us, WR * WN = 1 -> here (one at a
+// time | two side by side): 64 filters, 1 board 96 -> 93 | 52 -> 50, 6: 111 -> 104 | 66 -> 64, 11: 115 -> 104 |
+// 71 -> 71, 22: 152 -> 118 | 88 -> 73, 34: 179 -> 137 | 102 -> 88; 192 filters, 8 boards 227 -> 217 | 164 ->
+// 158, 15: 302 -> 288 | 255 -> 241; 320, 6: 375 -> 356 | 325 -> 313; 384, 5: 386 -> 372 | 341 -> 332.  Tiles of 32
+// channels and less of 192 filters and more stay: halves of their blocks fetch more from LDS per instruction
+// (192 filters, 5 boards 187 -> 212), and so does 64 filters' 64x64 in quarters (45 boards 162 -> 174).  Four
+// and eight wavefronts fill the SIMDs as they are (128 filters, 8 boards 155 -> 168, 256, 8: 277 -> 295).
+//
 // The peaks come from a layer of the same tiles, or from conv3x3_f32_k's 32x64 of the first layer.
 static constexpr int split_peak_loads(int rb, int nb, int filters) {
     const int own = peak_slots(rb * 16, filters / (nb * 16)), first = peak_slots(32, filters / 64);
     return ((own > first ? own : first) + 63) / 64;
 }
-template <int RB, int NB, int KW, int HPW, int D>
-__global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
+template <int RB, int NB, int KW, int HPW, int D, int WR, int WN>
+__global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
     const float* __restrict__ X, const half_t* __restrict__ Wf, const float* __restrict__ res,
     float* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
     float rfac, PeakIn peaks, unsigned* __restrict__ slots, int n, int Kp, ConvGrid g) {
-    constexpr int Cp = kF32Chunk * HPW * KW, NT = 64 * KW;
+    constexpr int Cp = kF32Chunk * HPW * KW, WS = WR * WN, NT = 64 * KW * WS;
+    constexpr int RBW = RB / WR, NBW = NB / WN;   // a wavefront's blocks
     constexpr int MT = RB * 16, CW = NB * 16, CELLS = conv_cells(MT);
     constexpr int STR = 144, SLICE = (CELLS + 1) * STR;
-    constexpr int PPC = 8, NP = (CELLS * PPC + 63) / 64;
+    constexpr int PPC = 8, NP = (CELLS * PPC + 64 * WS - 1) / (64 * WS);
     constexpr int STEPS = kF32Steps * HPW;
-    constexpr int BLOCKS = RB * NB, QB = (BLOCKS + KW - 1) / KW;   // a wavefront finishes QB blocks
+    constexpr int BLOCKS = RB * NB, QB = (BLOCKS + KW * WS - 1) / (KW * WS);   // a wavefront finishes QB blocks
     constexpr int BYTES = KW * (SLICE > BLOCKS * 1024 ? SLICE : BLOCKS * 1024);
-    static_assert(D <= STEPS && D <= kF32Lookahead && CW <= NT && MT <= kPts, "tile");
+    static_assert(D <= STEPS && D <= kF32Lookahead && CW <= NT && MT <= kPts && RB % WR == 0 && NB % WN == 0, "tile");
     __shared__ __attribute__((aligned(16))) unsigned char lds[BYTES];
     __shared__ __attribute__((aligned(16))) float bn[2][CW];
     __shared__ unsigned red[NT / 64][2];
@@ -588,6 +599,8 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     const int rows = n * kPts, m0 = tm * MT;
     const unsigned tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const int kw = WS == 1 ? wave : wave % KW, ww = WS == 1 ? 0 : wave / KW;   // its channels; its part of the tile
+    const int wr = ww / WN, wn = ww % WN;
 
     const unsigned bnoff = tid < (unsigned)CW ? (tn * CW + tid) * 4u : 0xfffffff0u;
     const float scale = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
@@ -595,10 +608,10 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     const float mean = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                                                      make_rsrc(bn_mean, Kp * 4), bnoff, 0, 0));
     const unsigned wstep = (unsigned)Kp * 64u;
-    const unsigned ws = (unsigned)(wave * STEPS) * wstep + (unsigned)(tn * NB) * 1024u;
+    const unsigned ws = (unsigned)(kw * STEPS) * wstep + (unsigned)(tn * NB + wn * NBW) * 1024u;
     const __amdgpu_buffer_rsrc_t rW =
         make_rsrc(Wf, ((size_t)18 * Cp / 32 + kF32Lookahead) * Kp * 64);
-    int4v w[D][NB];
+    int4v w[D][NBW];
     auto wload = [&](int slot, int j, unsigned st) {
         w[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(rW, lane * 16u + j * 1024, ws + st * wstep, 0);
     };
@@ -608,7 +621,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
 #pragma unroll
         for (int d = 0; d < D - 1; d++)
 #pragma unroll
-            for (int j = 0; j < NB; j++)
+            for (int j = 0; j < NBW; j++)
                 if (d >= from && d < to) wload(d, j, d);
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -619,10 +632,10 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     tp.load(peaks, ps, m0, MT, rows, lane);
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(X, (size_t)(n + 2) * kCellsPerBoard * Cp * 4);
     constexpr unsigned xrow = Cp * 4;   // bytes of a cell in memory
-    const unsigned xoff = (ps.q0 + lane / PPC) * xrow + (lane % PPC) * 16u;
+    const unsigned xoff = (ps.q0 + ww * (64 / PPC) + lane / PPC) * xrow + (lane % PPC) * 16u;
     auto xload = [&](int i, int h) {   // piece i of the wavefront's chunk h
         return __builtin_amdgcn_raw_buffer_load_b128(
-            rX, xoff, i * (64 / PPC) * xrow + (wave * HPW + h) * 128, 0);
+            rX, xoff, i * WS * (64 / PPC) * xrow + (kw * HPW + h) * 128, 0);
     };
     int4v stg[NP];
 #pragma unroll
@@ -640,7 +653,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     const int cl = 4 * (int)(lane >> 4);   // first of this lane's 4 channels of a block
 #pragma unroll
     for (int q = 0; q < QB; q++) {
-        const int id = q * KW + wave, local = id / NB * 16 + (int)(lane & 15);
+        const int id = q * KW * WS + wave, local = id / NB * 16 + (int)(lane & 15);
         ro[q] = id < BLOCKS && m0 + local < rows
                     ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + tn * CW + id % NB * 16 + cl) * 4u
                     : 0xfffffff0u;
@@ -651,11 +664,11 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
         for (int q = 0; q < QB; q++)
             rr[q] = __builtin_amdgcn_raw_buffer_load_b128(rR, ro[q], 0, 0);
     }
-    unsigned char* const own = lds + wave * SLICE;
+    unsigned char* const own = lds + kw * SLICE;
     auto stage = [&]() {
 #pragma unroll
         for (int i = 0; i < NP; i++) {
-            const unsigned cell = lane / PPC + i * (64 / PPC);
+            const unsigned cell = lane / PPC + (i * WS + ww) * (64 / PPC);
             store_split(own + (i < NP - 1 ? cell : min(cell, (unsigned)CELLS)) * STR + lane % PPC * 8u,
                         stg[i], cell < second_board(ps) ? ts.s0 : ts.s1);
         }
@@ -670,19 +683,19 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
         bn[0][tid] = scale;
         bn[1][tid] = -scale * mean;
     }
-    unsigned arow[RB];
+    unsigned arow[RBW];
 #pragma unroll
-    for (int i = 0; i < RB; i++)
-        arow[i] = patch_cell(ps, min(i * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
+    for (int i = 0; i < RBW; i++)
+        arow[i] = patch_cell(ps, min((wr * RBW + i) * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
                   (lane >> 4) * 16;
-    float4v acc[RB][NB];
+    float4v acc[RBW][NBW];
 #pragma unroll
-    for (int i = 0; i < RB; i++)
+    for (int i = 0; i < RBW; i++)
 #pragma unroll
-        for (int j = 0; j < NB; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < NBW; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
-    constexpr int AT = RB * NB >= 6 ? 1 : 2;   // taps read ahead
-    int4v a[AT][2][RB];   // [tap][hi, lo]
+    constexpr int AT = RBW * NBW >= 6 ? 1 : 2;   // taps read ahead
+    int4v a[AT][2][RBW];   // [tap][hi, lo]
     auto aread = [&](int i, int part, int tap) {
         return *reinterpret_cast<const int4v*>(own + arow[i] + ((tap / 3) * 20 + tap % 3) * STR +
                                                part * 64);
@@ -690,33 +703,37 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     static_assert(HPW <= 2, "chunks of a wavefront");
 #pragma unroll
     for (int h = 0; h < HPW; h++) {
-        if (h > 0) stage();
-        if (h > 0 && (wave * HPW + h) * 2 == KW * HPW) {   // KW is odd: the middle one
+        if (h > 0) {
+            if constexpr (WS > 1) lds_barrier();
+            stage();
+        }
+        if constexpr (WS > 1) lds_barrier();
+        if (h > 0 && (kw * HPW + h) * 2 == KW * HPW) {   // KW is odd: the middle one
 #pragma unroll
-            for (int i = 0; i < RB; i++)
+            for (int i = 0; i < RBW; i++)
 #pragma unroll
-                for (int j = 0; j < NB; j++) acc[i][j] = -acc[i][j];
+                for (int j = 0; j < NBW; j++) acc[i][j] = -acc[i][j];
         }
 #pragma unroll
         for (int p = 0; p < 2 * AT; p++)
 #pragma unroll
-            for (int i = 0; i < RB; i++) a[p / 2][p & 1][i] = aread(i, p & 1, p / 2);
+            for (int i = 0; i < RBW; i++) a[p / 2][p & 1][i] = aread(i, p & 1, p / 2);
 #pragma unroll
         for (int sc = 0; sc < kF32Steps; sc++) {
             const int st = h * kF32Steps + sc, part = sc & 1, tap = sc / 2;
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < RB; i++) {
+            for (int i = 0; i < RBW; i++) {
 #pragma unroll
-                for (int j = 0; j < NB; j++)
-                    if (i == (RB >= NB ? j : 0) && st + D - 1 < STEPS)
+                for (int j = 0; j < NBW; j++)
+                    if (i == (RBW >= NBW ? j : 0) && st + D - 1 < STEPS)
                         wload((st + D - 1) % D, j, st + D - 1);
 #pragma unroll
-                for (int j = 0; j < NB; j++)
+                for (int j = 0; j < NBW; j++)
                     acc[i][j] = mfma(w[st % D][j], a[tap % AT][0][i], acc[i][j]);
                 if (part == 0) {
 #pragma unroll
-                    for (int j = 0; j < NB; j++)
+                    for (int j = 0; j < NBW; j++)
                         acc[i][j] = mfma(w[st % D][j], a[tap % AT][1][i], acc[i][j]);
                 }
                 if (tap + AT < 9) a[tap % AT][1 - part][i] = aread(i, 1 - part, tap + AT);
@@ -728,17 +745,17 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
     // partial sums through LDS: [wavefront][block][64 lanes][4]
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < RB; i++)
+    for (int i = 0; i < RBW; i++)
 #pragma unroll
-        for (int j = 0; j < NB; j++)
-            *reinterpret_cast<float4v*>(lds + (wave * BLOCKS + i * NB + j) * 1024 + lane * 16) =
+        for (int j = 0; j < NBW; j++)
+            *reinterpret_cast<float4v*>(lds + (kw * BLOCKS + (wr * RBW + i) * NB + wn * NBW + j) * 1024 + lane * 16) =
                 acc[i][j];
     lds_barrier();
     float top0 = 0.0f, top1 = 0.0f;
     const int m1 = ((int)ps.mb + 1) * kPts;   // first row of the tile's second board
 #pragma unroll
     for (int q = 0; q < QB; q++) {
-        const int id = q * KW + wave;
+        const int id = q * KW * WS + wave;
         if (id >= BLOCKS) continue;
         float4v part[KW];
 #pragma unroll
@@ -762,7 +779,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
         top0 = fmaxf(top0, m < m1 ? top : 0.0f);
         top1 = fmaxf(top1, m >= m1 && m < rows ? top : 0.0f);
     }
-    leave_peaks<KW>(red, slots, tm, tn, Kp / CW, wave, top0, top1);
+    leave_peaks<KW * WS>(red, slots, tm, tn, Kp / CW, wave, top0, top1);
 }
 
 // The tile, in blocks of 16 points and of 16 channels: the smallest that makes at most one work-group per
@@ -772,17 +789,19 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_f32_split_k(
 // side): 128 filters, 12 boards 116 -> 86 | 134 -> 105, 22: 116 -> 93 | 148 -> 126; 192 filters, 8: 140 -> 103 |
 // 169 -> 147, 15: 143 -> 128 | 194 -> 199; 256 filters, 6: 175 -> 114 | 210 -> 160, 11: 176 -> 132 | 235 -> 227;
 // 320 filters, 6: 201 -> 152 | 254 -> 252; 384 filters, 4: 231 -> 150 | 293 -> 222; 512 filters, 4: 293 -> 179 |
-// 385 -> 320.  Left out: 64x64 for 64 filters, whose two wavefronts leave half a unit idle (40 boards 87 ->
-// 96), and above 256, where the registers do not hold it (320 filters, 8 boards 199 -> 245); 96x64 (256
-// filters, 16 boards 191 -> 193 | 299 -> 324).
+// 385 -> 320.  Left out: 64x64 above 256 filters, where the registers do not hold it (320 filters, 8
+// boards 199 -> 245); 96x64 (256 filters, 16 boards 191 -> 193 | 299 -> 324).  64 filters take 32x64 for 48x32
+// and 64x32: two thirds of the bytes per instruction (per forward of 10 blocks with the wavefronts below, 16
+// boards 121 -> 112, 22 boards 129 -> 118).
 struct SplitTile {
     int rb, nb;
 };
 static SplitTile f32_split_tile(int n, int Kp) {
-    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}, {3, 4}, {4, 4}};
-    for (const SplitTile& t : kTiles)
-        if ((t.rb * t.nb < 16 || (Kp >= 128 && Kp <= 256)) &&
-            (n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
+    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {2, 4}, {3, 2}, {4, 2}, {3, 4}, {4, 4}};
+    for (const SplitTile& t : kTiles) {
+        if (t.rb == 2 && t.nb == 4 ? Kp != 64 : t.rb * t.nb == 16 && Kp > 256) continue;
+        if ((n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
+    }
     return {0, 0};
 }
 
@@ -804,19 +823,29 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
         launch(kernel, dim3(8 * g.share), dim3(64 * waves), s, t, X, Wf, res, Y, bn_scale, bn_mean,
                rfac, peak_in(peaks), slots, n, Kp, g);
     };
-    // KW wavefronts x HPW chunks
+    // KW x WR x WN wavefronts, HPW chunks each
+#define LZ_TILE(RB, NB, KW, HPW, D, WR, WN) go(conv3x3_f32_split_k<RB, NB, KW, HPW, D, WR, WN>, KW * WR * WN)
 #define LZ_SPLIT(KW, HPW, D)                                                                  \
     if (tile.nb == 4) {                                                                       \
-        if (tile.rb == 3) go(conv3x3_f32_split_k<3, 4, KW, HPW, (HPW == 2 ? 3 : 5)>, KW);     \
-        else if constexpr (HPW == 1) go(conv3x3_f32_split_k<4, 4, KW, HPW, 4>, KW);           \
+        constexpr int WN = KW == 5 || KW == 6 ? 2 : 1;                                        \
+        if (tile.rb == 3) LZ_TILE(3, 4, KW, HPW, (HPW == 2 ? 3 : 5), 1, WN);                  \
+        else if constexpr (HPW == 1) LZ_TILE(4, 4, KW, HPW, 4, 1, WN);                        \
     } else if (tile.nb == 1) {                                                                \
-        if (tile.rb == 2) go(conv3x3_f32_split_k<2, 1, KW, HPW, D>, KW);                      \
-        else go(conv3x3_f32_split_k<3, 1, KW, HPW, D>, KW);                                   \
-    } else if (tile.rb == 2) go(conv3x3_f32_split_k<2, 2, KW, HPW, D>, KW);                   \
-    else if (tile.rb == 3) go(conv3x3_f32_split_k<3, 2, KW, HPW, D>, KW);                     \
-    else go(conv3x3_f32_split_k<4, 2, KW, HPW, (D < 18 ? 9 : D)>, KW)
+        if (tile.rb == 2) LZ_TILE(2, 1, KW, HPW, D, 1, 1);                                    \
+        else LZ_TILE(3, 1, KW, HPW, D, 1, 1);                                                 \
+    } else if (tile.rb == 2) LZ_TILE(2, 2, KW, HPW, D, 1, 1);                                 \
+    else if (tile.rb == 3) LZ_TILE(3, 2, KW, HPW, D, 1, 1);                                   \
+    else LZ_TILE(4, 2, KW, HPW, (D < 18 ? 9 : D), 1, 1)
     switch (Kp) {
-        case 64: LZ_SPLIT(2, 1, 18); break;
+        case 64:
+            if (tile.nb == 4) {
+                if (tile.rb == 2) LZ_TILE(2, 4, 2, 1, 9, 1, 2);
+                else if (tile.rb == 3) LZ_TILE(3, 4, 2, 1, 5, 1, 2);
+                else LZ_TILE(4, 4, 2, 1, 4, 2, 1);
+            } else if (tile.nb == 2) LZ_TILE(2, 2, 2, 1, 18, 2, 1);
+            else if (tile.rb == 2) LZ_TILE(2, 1, 2, 1, 18, 2, 1);
+            else LZ_TILE(3, 1, 2, 1, 18, 3, 1);
+            break;
         case 128: LZ_SPLIT(4, 1, 18); break;
         case 192: LZ_SPLIT(6, 1, 18); break;
         case 256: LZ_SPLIT(8, 1, 18); break;
@@ -826,6 +855,7 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
         default: LZ_SPLIT(8, 2, 12); break;
     }
 #undef LZ_SPLIT
+#undef LZ_TILE
     return {slots, tile.rb * 16, Kp / (16 * tile.nb)};
 }
 

@@ -1036,6 +1036,17 @@ def test_direct_convolution_tiles_in_steps_of_16_points(pkg, netgen, orc, precis
         test_fp32_direct_convolution(pkg, netgen, orc, filters, max(batches), batches)
 
 
+@pytest.mark.parametrize("filters,maxb,batches", [
+    (64, 46, (45, 46)), (64, 45, (1, 5, 6, 8, 9, 11, 12, 22, 23, 34, 35, 45)),
+    (192, 15, (1, 7, 8, 11, 12, 15)), (320, 6, (1, 4, 5, 6)), (384, 5, (1, 3, 4, 5)),
+])
+def test_fp32_tiles_dealt_to_wavefronts(pkg, netgen, orc, filters, maxb, batches):
+    """fp32 tiles whose blocks are dealt to two or three wavefronts, the smallest and the largest batch of each,
+    with the bounds of the test above; position 0 has the same bits in all of them, also on several lanes."""
+    test_fp32_direct_convolution(pkg, netgen, orc, filters, maxb, batches)
+    test_layers_replayed_on_several_lanes(pkg, netgen, orc, filters, pkg.FP32, batches)
+
+
 @pytest.mark.parametrize("filters,maxb", [(128, 40), (192, 16), (192, 40), (256, 9), (384, 28), (512, 44)])
 def test_fp32_filters_of_no_3x3_filter(pkg, netgen, orc, filters, maxb):
     """fp32 networks whose filters are no 3x3 ones run the Winograd kernels: the streaming GEMM, the
