@@ -13,7 +13,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(CSRC, "liblzhip.so")
 
-SOURCES = ["kernels.hip", "conv3x3.hip", "conv3x3_f32.hip", "hip_pipe.hip", "hip_scheduler.cpp", "goboard.cpp", "search.cpp",
+SOURCES = ["kernels.hip", "conv3x3.hip", "conv3x3_f32.hip", "conv3x3_first.hip", "hip_pipe.hip", "hip_scheduler.cpp", "goboard.cpp", "search.cpp",
            "weights_file.cpp",
            "c_api.cpp"]
 

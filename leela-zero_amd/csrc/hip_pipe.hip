@@ -1160,6 +1160,17 @@ private:
                          float* d_pol, float* d_val, bool timed) {
         const int nl = (int)m_layers.size();
         const int Tu = n * kTilesPerBoard;
+        if constexpr (sizeof(P) == 2) {
+            // (Forwards side by side replay their layers as one launch, from the lane's own planes; those in
+            // the static array do not.  A timed pass tells packing and convolutions apart.)
+            if (m_direct && d_in && !timed && (w.lanes == 1 || w.borders) && conv3x3_first_serves(m_Fp, n)) {
+                const Layer& L = m_layers[0];
+                launch_conv3x3_first(d_in, L.W3.p, w.act[0], L.d_scale.p, L.d_mean.p, n, m_C0p, m_Fp, w.stream,
+                                     w.borders);
+                enqueue_direct(w, n, d_pol, d_val, timed, 1);
+                return;
+            }
+        }
         LaunchTimer* pack = timer(timed, LZHIP_K_PACK);
         if (!d_in)
             launch_pack_input_bits<P>(d_bits, w.act0, m_direct, n, kInPlanes, m_C0p, w.peaks, m_in_scale.p,
@@ -1167,7 +1178,7 @@ private:
         else if (!pack_with_peaks(w, d_in, n, pack))
             launch_pack_input<P>(d_in, w.act0, m_direct, n, kInPlanes, m_C0p, w.stream, pack, w.borders);
         if (m_direct) {
-            enqueue_direct(w, n, d_pol, d_val, timed);
+            enqueue_direct(w, n, d_pol, d_val, timed, 0);
             return;
         }
         launch_in_transform<P>(w.act0, w.V, n, m_C0p, w.Tp, w.stream, timer(timed, LZHIP_K_IN));
@@ -1238,13 +1249,14 @@ private:
     }
 
     // The layer loop of a direct tower: one launch per layer.
-    // All layers of a direct tower, from the packed planes to the last activation, which is returned.
-    const P* enqueue_layers(const Work& w, int n, bool timed) {
+    // The layers of a direct tower from `first` on, 0 (from the packed planes) or 1, to the last activation, which
+    // is returned.
+    const P* enqueue_layers(const Work& w, int n, bool timed, int first) {
         const int nl = (int)m_layers.size();
         const P* last = w.act[0];
         PeakMap peaks{w.peaks, kPts, 1};
         int cur = 0, nxt = 2;   // block input (skip) / block output; 1 lies between
-        for (int l = 0; l < nl; l++) {
+        for (int l = first; l < nl; l++) {
             Layer& L = m_layers[l];
             const bool second = l >= 2 && (l % 2) == 0;
             const P* in = l == 0 ? w.act0 : second ? w.act[1] : w.act[cur];
@@ -1296,7 +1308,7 @@ private:
         if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
             std::exception_ptr failed;
             try {
-                enqueue_layers(w, n, false);
+                enqueue_layers(w, n, false, 0);
             } catch (...) {
                 failed = std::current_exception();
             }
@@ -1323,10 +1335,10 @@ private:
     bool launch_bound(int n) const {
         return (size_t)n * m_Fp * m_Fp <= (sizeof(P) == 2 ? 5u * 256 * 256 : 8u * 64 * 64);
     }
-    void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed) {
+    void enqueue_direct(const Work& w, int n, float* d_pol, float* d_val, bool timed, int first) {
         const int nl = (int)m_layers.size();
         const P* last = last_activation(w);
-        if (timed || !launch_layers_graph(w, n)) last = enqueue_layers(w, n, timed);
+        if (first > 0 || timed || !launch_layers_graph(w, n)) last = enqueue_layers(w, n, timed, first);
         launch_head_conv<P>(last, true, m_w3.p, m_s[nl], d_pol, d_val, n, m_Fp, w.stream,
                             timer(timed, LZHIP_K_HEAD));
     }

@@ -41,7 +41,7 @@ __host__ __device__ static inline size_t plane_index(bool padded, int b, int pt)
 }
 static inline size_t padded_cells(int n) { return (size_t)(n + 2) * kPadCells; }
 // The padded planes of a forward of n boards, one of w0 and then three of w pieces of 16 bytes to a cell
-// one after the other, whose borders the packing kernel is to clear on the way.
+// one after the other, whose borders the kernel that reads the input is to clear on the way.
 struct PlaneBorders {
     int __attribute__((ext_vector_type(4)))* planes = nullptr;
     unsigned n = 0, w0 = 0, w = 0;
@@ -133,6 +133,12 @@ void conv3x3_filters(const float* U, _Float16* Wf, int C, int F, int Kp, int* ba
 // The way back, on the host: Winograd filters [36][Kp][Cp] of the filters as stored (padding of
 // U is left as it is).
 void conv3x3_winograd_filters(const _Float16* Wf, int C, int Cp, int F, int Kp, _Float16* U);
+
+// The first layer of a direct fp16 tower from planes as floats [n][18][361] (conv3x3_first.hip): the results of
+// launch_pack_input and launch_conv3x3, for batches that it serves (measured; see there).  Cp = 64.
+bool conv3x3_first_serves(int Kp, int n);
+void launch_conv3x3_first(const float* planes, const _Float16* Wf, _Float16* Y, const float* bn_scale,
+                          const float* bn_mean, int n, int Cp, int Kp, hipStream_t s, const PlaneBorders* borders);
 
 // Direct 3x3 convolution of fp32 towers (conv3x3_f32.hip), one launch per layer:
 // X [Cp] -> Y [Kp] = max(0, scale*(conv - mean) + rfac*res) in fp32, padded planes, every operand split in

@@ -1036,6 +1036,23 @@ def test_direct_convolution_tiles_in_steps_of_16_points(pkg, netgen, orc, precis
         test_fp32_direct_convolution(pkg, netgen, orc, filters, max(batches), batches)
 
 
+@pytest.mark.parametrize("filters,last", [(24, 16), (64, 16), (128, 16), (192, 16), (256, 16), (512, 16)])
+def test_first_layer_from_the_callers_planes(pkg, netgen, orc, filters, last):
+    """fp16 batches whose first layer reads the planes as floats, up to the last that does and the next one, which
+    packs them: the same bits, with values that are not 0 and 1 and some beyond the stored range."""
+    net, pipe, ref, h_ref = make_pipes(pkg, netgen, orc, 1, filters, 7150 + filters, pkg.FP16, last + 1)
+    x = netgen.synthetic_inputs(last + 1, seed=7151)
+    rng = np.random.default_rng(7152)
+    x.reshape(last + 1, -1)[:] += rng.standard_normal(x.shape).reshape(last + 1, -1).astype(np.float32) * 0.1
+    x.reshape(last + 1, -1)[:, ::997] = 7e4
+    print("case: first layer, %d filters, %d boards" % (filters, last), flush=True)
+    pol, val = pipe.forward_batch(x)
+    for n in (1, 2, 9, last):
+        p, v = pipe.forward_batch(x[:n])
+        assert np.array_equal(p, pol[:n]) and np.array_equal(v, val[:n]), n
+    pipe.close()
+
+
 @pytest.mark.parametrize("filters,maxb,batches", [
     (64, 46, (45, 46)), (64, 45, (1, 5, 6, 8, 9, 11, 12, 22, 23, 34, 35, 45)),
     (192, 15, (1, 7, 8, 11, 12, 15)), (320, 6, (1, 4, 5, 6)), (384, 5, (1, 3, 4, 5)),
