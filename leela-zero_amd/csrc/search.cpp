@@ -151,13 +151,17 @@ HeadWeights::HeadWeights(const lzhip_head_weights& w) {
     bn_val_mean = w.bn_val_mean[0];
     bn_val_scale = w.bn_val_scale[0];
     const int pin = 2 * kPoints, pout = kPoints + 1;
-    ip_pol_wt.resize((size_t)pin * pout);
+    ip_pol_wt.resize((size_t)pin * (kPolRow / 16));   // (padding 0)
+    float* pol_wt = reinterpret_cast<float*>(ip_pol_wt.data());
     for (int o = 0; o < pout; o++)
-        for (int i = 0; i < pin; i++) ip_pol_wt[(size_t)i * pout + o] = w.ip_pol_w[(size_t)o * pin + i];
+        for (int i = 0; i < pin; i++)
+            pol_wt[(size_t)i * kPolRow + o] = w.ip_pol_w[(size_t)o * pin + i];
     ip_pol_b.assign(w.ip_pol_b, w.ip_pol_b + pout);
-    ip1_val_wt.resize((size_t)kPoints * 256);
+    ip1_val_wt.resize((size_t)kPoints * (256 / 16));
+    float* val_wt = reinterpret_cast<float*>(ip1_val_wt.data());
     for (int o = 0; o < 256; o++)
-        for (int i = 0; i < kPoints; i++) ip1_val_wt[(size_t)i * 256 + o] = w.ip1_val_w[(size_t)o * kPoints + i];
+        for (int i = 0; i < kPoints; i++)
+            val_wt[(size_t)i * 256 + o] = w.ip1_val_w[(size_t)o * kPoints + i];
     ip1_val_b.assign(w.ip1_val_b, w.ip1_val_b + 256);
     ip2_val_w.assign(w.ip2_val_w, w.ip2_val_w + 256);
     ip2_val_b = w.ip2_val_b[0];
@@ -228,10 +232,11 @@ template <int N> struct Fc {
 
 void heads_on_host(const HeadWeights& w, int n, const float* pol, const float* val,
                    float softmax_temp, float* policy, float* winrate) {
-    constexpr int pout = kPoints + 1, pin = 2 * kPoints, kBlock = 8, vout = 256;
-    static FcRows* const fc_pol = Fc<pout>::best();
+    constexpr int pout = kPoints + 1, prow = HeadWeights::kPolRow, pin = 2 * kPoints, kBlock = 8, vout = 256;
+    static FcRows* const fc_pol = Fc<prow>::best();
     static FcRows* const fc_val = Fc<vout>::best();
-    float x[kBlock * pin], y[kBlock * pout];
+    float x[kBlock * pin];
+    alignas(64) float y[kBlock * prow];
     for (int p0 = 0; p0 < n; p0 += kBlock) {
         const int m = std::min(kBlock, n - p0);
         for (int p = 0; p < m; p++) {
@@ -240,11 +245,12 @@ void heads_on_host(const HeadWeights& w, int n, const float* pol, const float* v
                 for (int i = 0; i < kPoints; i++)
                     x[p * pin + c * kPoints + i] =
                         w.bn_pol_scale[c] * (src[c * kPoints + i] - w.bn_pol_mean[c]);
-            for (int o = 0; o < pout; o++) y[p * pout + o] = w.ip_pol_b[o];
+            for (int o = 0; o < pout; o++) y[p * prow + o] = w.ip_pol_b[o];
+            for (int o = pout; o < prow; o++) y[p * prow + o] = 0.0f;
         }
-        fc_pol(w.ip_pol_wt.data(), x, pin, pin, y, m);
+        fc_pol(reinterpret_cast<const float*>(w.ip_pol_wt.data()), x, pin, pin, y, m);
         for (int p = 0; p < m; p++) {
-            const float* logits = y + p * pout;
+            const float* logits = y + p * prow;
             float* out = policy + (size_t)(p0 + p) * pout;
             float alpha = logits[0];
             for (int o = 1; o < pout; o++) alpha = std::max(alpha, logits[o]);
@@ -261,7 +267,7 @@ void heads_on_host(const HeadWeights& w, int n, const float* pol, const float* v
                 x[p * pin + i] = w.bn_val_scale * (src[i] - w.bn_val_mean);
             for (int o = 0; o < vout; o++) y[p * vout + o] = w.ip1_val_b[o];
         }
-        fc_val(w.ip1_val_wt.data(), x, kPoints, pin, y, m);
+        fc_val(reinterpret_cast<const float*>(w.ip1_val_wt.data()), x, kPoints, pin, y, m);
         for (int p = 0; p < m; p++) {
             const float* hid = y + p * vout;
             float out = w.ip2_val_b;

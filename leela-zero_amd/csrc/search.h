@@ -58,11 +58,17 @@ struct Netresult {
 
 // Head parameters, laid out for the host loops (FC weights input-major).
 struct HeadWeights {
+    // Rows of the FC weights are whole cache lines: a row of 362 floats starts anywhere in one, and every
+    // vector of it is then two loads (8 positions 50 -> 37 us, one 7.2 -> 5.3).
+    static constexpr int kPolRow = 368;
+    struct alignas(64) Line {
+        float v[16];
+    };
     explicit HeadWeights(const lzhip_head_weights& w);
     float bn_pol_mean[2], bn_pol_scale[2], bn_val_mean, bn_val_scale;
-    std::vector<float> ip_pol_wt;   // [722][362]
+    std::vector<Line> ip_pol_wt;    // [722][kPolRow / 16], padding 0
     std::vector<float> ip_pol_b;    // [362]
-    std::vector<float> ip1_val_wt;  // [361][256]
+    std::vector<Line> ip1_val_wt;   // [361][256 / 16]
     std::vector<float> ip1_val_b;   // [256]
     std::vector<float> ip2_val_w;   // [256]
     float ip2_val_b;
