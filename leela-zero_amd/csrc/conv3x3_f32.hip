@@ -245,11 +245,19 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     auto wload = [&](int slot, int j, unsigned st) {
         w[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(rW, wv + j * 1024, ws + st * wstep, 0);
     };
+    // The filters of two k-steps go before the planes, the others behind them (CC == 0): 6 blocks of 256 filters, 12
+    // boards 248 -> 243 us, of 128, 32 boards 165 -> 162, of 192, 30 boards 276 -> 269, of 384, 8 boards 331 ->
+    // 326; 20 boards of 256 filters and more within 1 %.
+    constexpr int F0 = DB && D - 1 > 2 ? 2 : D - 1;
+    auto filters = [&](int from, int to) {
 #pragma unroll
-    for (int d = 0; d < D - 1; d++)
+        for (int d = 0; d < D - 1; d++)
 #pragma unroll
-        for (int j = 0; j < NB; j++) wload(d, j, d);
-    __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < NB; j++)
+                if (d >= from && d < to) wload(d, j, d);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    filters(0, F0);
 
     const PatchStart ps = patch_start(m0);
     TilePeaks<0, 2> tp;
@@ -304,6 +312,8 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
         int4v stg[NP];
 #pragma unroll
         for (int i = 0; i < NP; i++) stg[i] = xload(i, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        filters(F0, D - 1);
         if constexpr (EARLY) first_res();
         ts = tp.scales();
 #pragma unroll
