@@ -81,6 +81,19 @@ __device__ __forceinline__ float4v mfma(int4v w, int4v x, float4v acc) {
                                                   __builtin_bit_cast(half8v, x), acc, 0, 0, 0);
 }
 
+// Of conv3x3_k's order in LDS (CellPitch) these kernels take what costs no address: a lane's point is conv_point's,
+// and quarters 2 i and 2 i + 1 of a cell's 32 channels stand an even number of 16 bytes apart, so that of the 16
+// lanes served together eight meet odd and eight even slots, but in blocks that a board row ends in.  (Its longer
+// rows cost more than they gave.)  With quarters and points in their natural order nearly every read took two
+// turns, 17 % of a launch of 15x192, 8 boards.  A forward, us: 15x192, 1 board 198 -> 191, 2 boards 238 -> 223, 8: 319
+// -> 316; 20x256, 1 board 286 -> 272; 10x512, 1 board 256 -> 235; conv3x3_f32_k, 6 blocks: 256 filters, 1 board 151 ->
+// 141, 8: 198 -> 191, 64: 740 -> 737; 128, 1 board 100 -> 93; 192, 8 boards 160 -> 153; 384, 24 boards 657 -> 650.
+//
+// Place of quarter q of a cell's 32 channels, in 16 bytes.
+__device__ __forceinline__ unsigned f32_slot(unsigned q) { return 2 * (q & 1) + (q >> 1); }
+// Byte of piece x of a cell: channels 4 x to 4 x + 3.
+__device__ __forceinline__ unsigned f32_piece(unsigned x) { return f32_slot(x >> 1) * 16 + (x & 1) * 8; }
+
 // Largest value of a wavefront, in every lane.
 __device__ __forceinline__ unsigned wave_max(unsigned v) {
     auto step = [&](auto ctrl, auto rows) {
@@ -270,14 +283,14 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
         return __builtin_amdgcn_raw_buffer_load_b128(rX, xoff, i * (NT / PPC) * xrow + at, 0);
     };
     // LDS address of piece i: a constant distance from piece 0 (the last may lie past the end)
-    const unsigned lst = (tid / PPC) * STR + (tid % PPC) * 8u;
+    const unsigned lst = (tid / PPC) * STR + f32_piece(tid % PPC);
     TileScales ts;
     unsigned tv = tid;   // (opaque in every chunk: the scales of the pieces are not held)
     auto put = [&](int i, unsigned buffer, int4v bits) {
         const unsigned cell = tv / PPC + i * (NT / PPC);
         const unsigned at = i < NP - 1 || (CELLS * PPC) % NT == 0
                                 ? lst + i * (NT / PPC) * STR
-                                : min(cell, (unsigned)CELLS) * STR + (tid % PPC) * 8u;
+                                : min(cell, (unsigned)CELLS) * STR + f32_piece(tid % PPC);
         store_split(lds + buffer + at, bits, cell < second_board(ps) ? ts.s0 : ts.s1);
     };
 
@@ -288,9 +301,9 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     int4v rr[RQ][NB];
 #pragma unroll
     for (int i = 0; i < RB; i++) {
-        const int local = (wr * RB + i) * 16 + (int)(lane & 15);
+        const int local = (wr * RB + i) * 16 + conv_point(lane);
         const unsigned cell = patch_cell(ps, min(local, rows - 1 - m0));
-        arow[i] = cell * STR + (lane >> 4) * 16;
+        arow[i] = cell * STR + f32_slot(lane >> 4) * 16;
         ro[i] = m0 + local < rows ? ((ps.q0 + kPointCell + cell) * Kp + ch0) * 4u : 0xfffff000u;
     }
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 4;
@@ -432,7 +445,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     const int m1 = ((int)ps.mb + 1) * kPts;   // first row of the tile's second board
 #pragma unroll
     for (int i = 0; i < RB; i++) {
-        const int m = m0 + (wr * RB + i) * 16 + (int)(lane & 15);
+        const int m = m0 + (wr * RB + i) * 16 + conv_point(lane);
         const float unscale = m < m1 ? -ts.u0 : -ts.u1;   // (the sum ends negated)
         float top = 0.0f;
 #pragma unroll
@@ -663,7 +676,7 @@ __global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
     const int cl = 4 * (int)(lane >> 4);   // first of this lane's 4 channels of a block
 #pragma unroll
     for (int q = 0; q < QB; q++) {
-        const int id = q * KW * WS + wave, local = id / NB * 16 + (int)(lane & 15);
+        const int id = q * KW * WS + wave, local = id / NB * 16 + conv_point(lane);
         ro[q] = id < BLOCKS && m0 + local < rows
                     ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + tn * CW + id % NB * 16 + cl) * 4u
                     : 0xfffffff0u;
@@ -679,7 +692,7 @@ __global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
 #pragma unroll
         for (int i = 0; i < NP; i++) {
             const unsigned cell = lane / PPC + (i * WS + ww) * (64 / PPC);
-            store_split(own + (i < NP - 1 ? cell : min(cell, (unsigned)CELLS)) * STR + lane % PPC * 8u,
+            store_split(own + (i < NP - 1 ? cell : min(cell, (unsigned)CELLS)) * STR + f32_piece(lane % PPC),
                         stg[i], cell < second_board(ps) ? ts.s0 : ts.s1);
         }
     };
@@ -696,8 +709,8 @@ __global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
     unsigned arow[RBW];
 #pragma unroll
     for (int i = 0; i < RBW; i++)
-        arow[i] = patch_cell(ps, min((wr * RBW + i) * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
-                  (lane >> 4) * 16;
+        arow[i] = patch_cell(ps, min((wr * RBW + i) * 16 + conv_point(lane), rows - 1 - m0)) * STR +
+                  f32_slot(lane >> 4) * 16;
     float4v acc[RBW][NBW];
 #pragma unroll
     for (int i = 0; i < RBW; i++)
@@ -772,7 +785,7 @@ __global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
         for (int k = 0; k < KW; k++)
             part[k] = *reinterpret_cast<const float4v*>(lds + (k * BLOCKS + id) * 1024 + lane * 16);
         const float4v r = __builtin_bit_cast(float4v, rr[q]);
-        const int m = m0 + id / NB * 16 + (int)(lane & 15), c = id % NB * 16 + cl;
+        const int m = m0 + id / NB * 16 + conv_point(lane), c = id % NB * 16 + cl;
         const float unscale = m < m1 ? ts.u0 : ts.u1;
         float top = 0.0f;
         float4v o;

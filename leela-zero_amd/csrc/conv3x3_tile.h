@@ -65,8 +65,8 @@ __device__ __forceinline__ unsigned patch_cell(const PatchStart& s, unsigned loc
 // Counted in a loop of reads: 4 cycles each; 8 with the pieces and points in their natural order, 12
 // where 16 points end a board row.  It shows where 192x64 tiles load the LDS most: 20x256 batch 32 640 ->
 // 614 us a forward, two side by side 979 -> 924; 16 boards 830 -> 820 of 40 blocks, the others within 1 %.
-// conv3x3_split_k and the fp32 kernels keep the natural order: they wait for other things, and the
-// addresses cost them more (10x128 fp16 batch 5 84 -> 93, 10x256 fp32 batch 64 1280 -> 1292).
+// The fp32 kernels have the order of points and quarters without the longer rows (f32_slot), conv3x3_split_k
+// keeps the natural one: longer rows cost addresses (10x128 fp16 batch 5 84 -> 93, 10x256 fp32 batch 64 1280 -> 1292).
 template <int STR>
 struct CellPitch {
     static_assert(STR % 32 == 16, "an odd number of slots");
