@@ -609,10 +609,17 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
     const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
     const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
+    // The order of points and quarters in LDS (CellPitch) where more than four wavefronts' worth of channels is read:
+    // 15x192, 8 boards 177 -> 174.5 us a forward, two side by side 110 -> 106.5; 20x256, two of 1 board 93.6 -> 90.1, of 5
+    // boards 144 -> 141; 10x320, 1 board 94.7 -> 89.9. 64 filters, 1 board, lost by it (110.4 -> 111.5), 128 gained
+    // nothing for one.
+    constexpr bool SPREAD = KW * HPW > 4;
+    const int point = SPREAD ? conv_point(lane) : (int)(lane & 15);   // this lane's, of a block of 16
+    auto slot = [](unsigned q) { return SPREAD ? quarter_slot(q) : q; };
     const int cl = E * (int)(lane >> 4);   // first of this lane's channels
 #pragma unroll
     for (int q = 0; q < QP; q++) {
-        const int i = q * KW + wave, local = i * 16 + (int)(lane & 15);
+        const int i = q * KW + wave, local = i * 16 + point;
         ro[q] = i < RB && m0 + local < rows
                     ? ((ps.q0 + kPointCell + patch_cell(ps, local)) * Kp + channel(cl)) * 2u
                     : 0xfffffff0u;
@@ -629,7 +636,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     for (int i = 0; i < NP; i++) {
         const unsigned piece = lane + i * 64, cell = piece / PPC;
         *reinterpret_cast<int4v*>(own + (cell < (unsigned)CELLS ? cell : (unsigned)CELLS) * STR +
-                                  piece % PPC * 16u) = stg[i];
+                                  (piece % PPC / 4 * 4 + slot(piece % 4)) * 16u) = stg[i];
     }
     if (tid < (unsigned)CW) {
         bn[0][tid] = scale;
@@ -638,8 +645,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     unsigned arow[RB];
 #pragma unroll
     for (int i = 0; i < RB; i++)
-        arow[i] = patch_cell(ps, min(i * 16 + (int)(lane & 15), rows - 1 - m0)) * STR +
-                  (lane >> 4) * 16;
+        arow[i] = patch_cell(ps, min(i * 16 + point, rows - 1 - m0)) * STR + slot(lane >> 4) * 16;
     constexpr int SUMS = PAIRS ? HPW : 1;
     float4v acc[SUMS][RB][NB];
 #pragma unroll

@@ -88,11 +88,8 @@ __device__ __forceinline__ float4v mfma(int4v w, int4v x, float4v acc) {
 // turns, 17 % of a launch of 15x192, 8 boards.  A forward, us: 15x192, 1 board 198 -> 191, 2 boards 238 -> 223, 8: 319
 // -> 316; 20x256, 1 board 286 -> 272; 10x512, 1 board 256 -> 235; conv3x3_f32_k, 6 blocks: 256 filters, 1 board 151 ->
 // 141, 8: 198 -> 191, 64: 740 -> 737; 128, 1 board 100 -> 93; 192, 8 boards 160 -> 153; 384, 24 boards 657 -> 650.
-//
-// Place of quarter q of a cell's 32 channels, in 16 bytes.
-__device__ __forceinline__ unsigned f32_slot(unsigned q) { return 2 * (q & 1) + (q >> 1); }
 // Byte of piece x of a cell: channels 4 x to 4 x + 3.
-__device__ __forceinline__ unsigned f32_piece(unsigned x) { return f32_slot(x >> 1) * 16 + (x & 1) * 8; }
+__device__ __forceinline__ unsigned f32_piece(unsigned x) { return quarter_slot(x >> 1) * 16 + (x & 1) * 8; }
 
 // Largest value of a wavefront, in every lane.
 __device__ __forceinline__ unsigned wave_max(unsigned v) {
@@ -303,7 +300,7 @@ __global__ __launch_bounds__(64 * WR * WN, OCC) void conv3x3_f32_k(
     for (int i = 0; i < RB; i++) {
         const int local = (wr * RB + i) * 16 + conv_point(lane);
         const unsigned cell = patch_cell(ps, min(local, rows - 1 - m0));
-        arow[i] = cell * STR + f32_slot(lane >> 4) * 16;
+        arow[i] = cell * STR + quarter_slot(lane >> 4) * 16;
         ro[i] = m0 + local < rows ? ((ps.q0 + kPointCell + cell) * Kp + ch0) * 4u : 0xfffff000u;
     }
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 4;
@@ -710,7 +707,7 @@ __global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
 #pragma unroll
     for (int i = 0; i < RBW; i++)
         arow[i] = patch_cell(ps, min((wr * RBW + i) * 16 + conv_point(lane), rows - 1 - m0)) * STR +
-                  f32_slot(lane >> 4) * 16;
+                  quarter_slot(lane >> 4) * 16;
     float4v acc[RBW][NBW];
 #pragma unroll
     for (int i = 0; i < RBW; i++)
