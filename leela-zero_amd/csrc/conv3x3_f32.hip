@@ -83,11 +83,12 @@ __device__ __forceinline__ float4v mfma(int4v w, int4v x, float4v acc) {
 
 // Of conv3x3_k's order in LDS (CellPitch) these kernels take what costs no address: a lane's point is conv_point's,
 // and quarters 2 i and 2 i + 1 of a cell's 32 channels stand an even number of 16 bytes apart, so that of the 16
-// lanes served together eight meet odd and eight even slots, but in blocks that a board row ends in.  (Its longer
-// rows cost more than they gave.)  With quarters and points in their natural order nearly every read took two
-// turns, 17 % of a launch of 15x192, 8 boards.  A forward, us: 15x192, 1 board 198 -> 191, 2 boards 238 -> 223, 8: 319
-// -> 316; 20x256, 1 board 286 -> 272; 10x512, 1 board 256 -> 235; conv3x3_f32_k, 6 blocks: 256 filters, 1 board 151 ->
-// 141, 8: 198 -> 191, 64: 740 -> 737; 128, 1 board 100 -> 93; 192, 8 boards 160 -> 153; 384, 24 boards 657 -> 650.
+// lanes served together eight meet odd and eight even slots, but in blocks that a board row ends in. (Its longer rows
+// cost more than they gave.) With quarters and points in their natural order nearly every read took two turns, 17 %
+// of a launch of 15x192, 8 boards, now 9; 40x256, 64 boards: 20, now 10. A forward, us: 15x192, 1 board 198 -> 191, 2
+// boards 238 -> 223, 8: 319 -> 316; 20x256, 1 board 286 -> 272; 10x512, 1 board 256 -> 235; conv3x3_f32_k, 6 blocks:
+// 256 filters, 1 board 151 -> 141, 8: 198 -> 191, 64: 740 -> 737; 128, 1 board 100 -> 93; 192, 8 boards 160 -> 153;
+// 384, 24 boards 657 -> 650.
 // Byte of piece x of a cell: channels 4 x to 4 x + 3.
 __device__ __forceinline__ unsigned f32_piece(unsigned x) { return quarter_slot(x >> 1) * 16 + (x & 1) * 8; }
 
