@@ -564,6 +564,8 @@ public:
     // positions, with the device to itself: 83, now 71 to 75).  Nothing else has to start at
     // zero: every element a kernel reads for a real tile is written earlier in the same call (rows
     // of V past the last tile feed only rows of M that no kernel reads).
+    // Calls wait for one another, so each takes the tiles of a forward alone (8 blocks of 256 fp16 filters, a handle
+    // of 7 positions: 6 positions 134 us with the tiles of two lanes, 111 so; 7: 135, 111).
     void forward_device_static(int n, const float* d_in, float* d_pol, float* d_val) override {
         Lane& ln = m_lane[0];
         std::lock_guard<std::mutex> lk(ln.mu);
@@ -1009,7 +1011,7 @@ private:
         P *act0 = nullptr, *act[3] = {nullptr, nullptr, nullptr}, *V = nullptr, *M = nullptr;
         int Tp = 0;
         uint32_t* peaks = nullptr;   // (direct fp32 towers)
-        int lanes = 2;               // forwards that may be running side by side (lanes_in_use)
+        int lanes = 1;               // forwards that may be running side by side (lanes_in_use)
         LayerGraphs<hipGraphExec_t>* layers = nullptr;  // the lane's (none: plain launches)
         const PlaneBorders* borders = nullptr;          // to be cleared with the packing
     };
@@ -1161,9 +1163,9 @@ private:
         const int nl = (int)m_layers.size();
         const int Tu = n * kTilesPerBoard;
         if constexpr (sizeof(P) == 2) {
-            // (Forwards side by side replay their layers as one launch, from the lane's own planes; those in
-            // the static array do not.  A timed pass tells packing and convolutions apart.)
-            if (m_direct && d_in && !timed && (w.lanes == 1 || w.borders) && conv3x3_first_serves(m_Fp, n)) {
+            // (Forwards side by side replay their layers as one launch, from the lane's own planes.  A timed
+            // pass tells packing and convolutions apart.)
+            if (m_direct && d_in && !timed && w.lanes == 1 && conv3x3_first_serves(m_Fp, n)) {
                 const Layer& L = m_layers[0];
                 launch_conv3x3_first(d_in, L.W3.p, w.act[0], L.d_scale.p, L.d_mean.p, n, m_C0p, m_Fp, w.stream,
                                      w.borders);

@@ -161,6 +161,33 @@ def test_no_alloc_forward_after_planes_that_are_no_numbers(pkg, netgen, precisio
 
 
 @pytest.mark.parametrize("precision_name", ["FP32", "FP16"])
+@pytest.mark.parametrize("filters,max_batch,sizes", [(64, 8, (8,)), (192, 9, (1, 8)), (256, 7, (1, 6, 7))])
+def test_no_alloc_forward_runs_the_kernels_of_a_forward_alone(pkg, netgen, precision_name, filters, max_batch,
+                                                              sizes):
+    """Each call waits for the one before it, whatever its handle, and has the device to itself: it launches the
+    kernels, tiles included, that the plain forward launches on one lane, with the same bits."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    print("case: no-alloc kernels", precision_name, filters, max_batch, flush=True)
+    pipe = _pipe(pkg, netgen, 1, filters, 105, getattr(pkg, precision_name), max_batch)
+    x = torch.from_numpy(netgen.synthetic_inputs(max_batch, seed=106)).cuda()
+    for n in sizes:
+        ran, got = [], []
+        for forward in (pipe.forward_batch_device, pipe.forward_batch_device_noalloc):
+            pol, val = torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")
+            torch.cuda.synchronize()
+            with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
+                forward(n, x.data_ptr(), pol.data_ptr(), val.data_ptr())
+                pipe.sync()
+                torch.cuda.synchronize()
+            ran.append(sorted(e.name for e in p.events() if "lzhip" in e.name))
+            got.append((pol.cpu().numpy(), val.cpu().numpy()))
+        assert len(ran[0]) >= 4 and ran[0] == ran[1], (n, ran)
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), n
+    pipe.close()
+
+
+@pytest.mark.parametrize("precision_name", ["FP32", "FP16"])
 def test_no_alloc_forward_in_a_captured_graph(pkg, netgen, precision_name):
     """The call recorded into a caller's graph: every replay gives the eager planes, with other handles'
     calls through the same static array, eager work and synchronisations between the replays."""
