@@ -833,8 +833,12 @@ bool conv3x3_f32_splits(int Kp, int max_batch) {
 PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* res, float* Y,
                                  const float* bn_scale, const float* bn_mean, float rfac,
                                  const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
-                                 hipStream_t s, LaunchTimer* t) {
-    const SplitTile tile = f32_split_tile(n, Kp);
+                                 int lanes, hipStream_t s, LaunchTimer* t) {
+    SplitTile tile = f32_split_tile(n, Kp);
+    // Three forwards of 64 filters side by side have wavefronts enough: 64x64 gives way to 48x64, which a unit holds
+    // four of (per forward of 8 blocks, 36 boards 67.7 -> 65.7 us, 42: 75.4 -> 72.4, 45: 79.1 -> 77.1; conv3x3_f32_k's
+    // 96x64 took 66.7, 70.4 and 74.1 there), and 48x16 is not dealt (6: 38.8 -> 37.6, 8: 41.3 -> 36.4).
+    if (lanes > 2 && Kp == 64 && tile.rb == 4 && tile.nb == 4) tile = {3, 4};
     if (!conv3x3_f32_splits(Kp, n) || Cp != Kp)
         throw std::invalid_argument("no split convolution for this width or batch");
     const ConvGrid g = conv_grid((n * kPts + tile.rb * 16 - 1) / (tile.rb * 16), Kp / (16 * tile.nb),
@@ -865,7 +869,8 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
                 else LZ_TILE(4, 4, 2, 1, 4, 2, 1);
             } else if (tile.nb == 2) LZ_TILE(2, 2, 2, 1, 18, 2, 1);
             else if (tile.rb == 2) LZ_TILE(2, 1, 2, 1, 18, 2, 1);
-            else LZ_TILE(3, 1, 2, 1, 18, 3, 1);
+            else if (lanes <= 2) LZ_TILE(3, 1, 2, 1, 18, 3, 1);
+            else LZ_TILE(3, 1, 2, 1, 18, 1, 1);
             break;
         case 128: LZ_SPLIT(4, 1, 18); break;
         case 192: LZ_SPLIT(6, 1, 18); break;

@@ -1244,7 +1244,7 @@ private:
         } else {
             const bool split = L.Cp == m_Fp && conv3x3_f32_splits(m_Fp, m_max_batch);
             peaks = split ? launch_conv3x3_f32_split(in, L.W3.p, res, out, scale, mean, rfac, peaks,
-                                                     slots, n, L.Cp, m_Fp, s, t)
+                                                     slots, n, L.Cp, m_Fp, lanes, s, t)
                           : launch_conv3x3_f32(in, L.W3.p, res, out, scale, mean, rfac, peaks, slots,
                                                n, L.Cp, m_Fp, lanes, s, t);
         }

@@ -158,7 +158,7 @@ bool conv3x3_f32_splits(int Kp, int max_batch);
 PeakMap launch_conv3x3_f32_split(const float* X, const _Float16* Wf, const float* res, float* Y,
                                  const float* bn_scale, const float* bn_mean, float rfac,
                                  const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
-                                 hipStream_t s, LaunchTimer* t);
+                                 int lanes, hipStream_t s, LaunchTimer* t);
 // Of every output channel of U [36][C][F]: the exponents of its largest filter times 2^-in_exp and of its
 // largest product with inputs of magnitude 2^mag (kNoExp before; kNoExp: none); *bad as above.
 constexpr int kNoExp = -(1 << 28);

@@ -1305,3 +1305,38 @@ def test_graph_replays_run_the_kernels_of_the_lanes_in_use(pkg, netgen, orc, pre
         assert len(ran[0]) == 4 * lanes * 5 and ran[0] == ran[1], (lanes, ran)
     pipe.close()
     plain.close()
+
+
+@pytest.mark.parametrize("maxb,n", [(11, 6), (11, 8), (45, 8), (45, 36), (45, 45)])
+def test_fp32_tiles_of_64_filters_on_three_lanes(pkg, netgen, orc, maxb, n):
+    """Three fp32 forwards of 64 filters side by side take tiles of 48 points on fewer wavefronts, or in place of 64
+    points, than a forward alone: other kernels and the same bits."""
+    import torch
+    print("case: three lanes, 64 filters, %d boards of %d" % (n, maxb), flush=True)
+    _, plain, _, _ = make_pipes(pkg, netgen, orc, 1, 64, 7600, pkg.FP32, maxb)
+    _, pipe, _, _ = make_pipes(pkg, netgen, orc, 1, 64, 7600, pkg.FP32, maxb)
+    assert pipe.lanes() == 3
+    x = netgen.synthetic_inputs(n, seed=7601)
+    want = plain.forward_batch(x)
+    d_in = torch.from_numpy(x).cuda()
+    outs = [(torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")) for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def forwards(lanes):
+        for k, (pol, val) in enumerate(outs[:lanes]):
+            pipe.forward_batch_device(n, d_in.data_ptr(), pol.data_ptr(), val.data_ptr(), lane=k)
+        pipe.sync()
+
+    ran = {}
+    for lanes in (1, 3):
+        for _ in range(3):
+            forwards(lanes)
+        for pol, val in outs[:lanes]:
+            pol.zero_(), val.zero_()
+        torch.cuda.synchronize()
+        ran[lanes] = set(lzhip_events(lambda: forwards(lanes))[0])
+        for pol, val in outs[:lanes]:
+            assert np.array_equal(pol.cpu().numpy(), want[0]) and np.array_equal(val.cpu().numpy(), want[1]), lanes
+    assert ran[1] and ran[3] - ran[1], ran
+    pipe.close()
+    plain.close()
