@@ -469,8 +469,9 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
     if (wide_columns && lanes == 1) {
         if (const int rb = one_round_blocks(rows, Kp / 128, 5)) return wide(rb);
     }
-    // 192 filters, 33 boards 192x64 11.2, 160x64 10.1 us (two side by side 7.6 | 7.1)
-    if (!wide_columns && Kp != 64 && groups(160, 64) <= kUnits) {
+    // 192 filters, 33 boards 192x64 11.2, 160x64 10.1 us (two side by side 7.6 | 7.1).  Three side by side have nothing
+    // from it and lose some (8 blocks of 320 filters, 20 boards 517 -> 527 us a forward of each, of 192, 33 boards 343 -> 346).
+    if (!wide_columns && Kp != 64 && lanes <= 2 && groups(160, 64) <= kUnits) {
         LZ_CONV(5, 2, 2, 2, 6, 1, 0, 2);
         return;
     }

@@ -1340,3 +1340,49 @@ def test_fp32_tiles_of_64_filters_on_three_lanes(pkg, netgen, orc, maxb, n):
     assert ran[1] and ran[3] - ran[1], ran
     pipe.close()
     plain.close()
+
+
+@pytest.mark.parametrize("precision,filters,n,tiles", [
+    (1, 320, 20, "aab"), (1, 192, 33, "aab"),       # 160x64 points by channels, or 192x64
+    (1, 128, 46, "abb"), (1, 256, 24, "abb"), (1, 384, 17, "abb"),      # 80x128, or 192x64
+    (0, 256, 24, "aab"), (0, 256, 30, "abb"), (0, 384, 17, "aab"), (0, 192, 33, "aaa"),
+    (1, 256, 70, "ab"), (1, 192, 91, "ab"), (0, 256, 70, "ab"),         # more than a round
+])
+def test_large_tiles_on_one_lane_and_beside_others(pkg, netgen, orc, precision, filters, n, tiles):
+    """Forwards on one, two and three lanes give the same bits.  `tiles` has a letter for each number of lanes: equal
+    letters run the same kernels, others do not."""
+    import torch
+    print("case: large tiles beside others, %d filters, %d boards, precision %d" % (filters, n, precision), flush=True)
+    _, pipe, _, _ = make_pipes(pkg, netgen, orc, 1, filters, 7700, precision, n)
+    assert pipe.lanes() == len(tiles)
+    x = [netgen.synthetic_inputs(n, seed=7701 + k) for k in range(len(tiles))]
+    d_in = [torch.from_numpy(v).cuda() for v in x]
+    outs = [(torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")) for _ in tiles]
+    torch.cuda.synchronize()
+
+    def forward(planes, lane):
+        pol, val = outs[lane]
+        pipe.forward_batch_device(n, d_in[planes].data_ptr(), pol.data_ptr(), val.data_ptr(), lane=lane)
+
+    want = []
+    for k in range(len(tiles)):
+        for _ in range(3):
+            forward(k, 0)
+        pipe.sync()
+        want.append([o.cpu().numpy() for o in outs[0]])
+    ran = []
+    for lanes in range(1, len(tiles) + 1):
+        for _ in range(3):
+            for k in range(lanes):
+                forward(k, k)
+        pipe.sync()
+        for pol, val in outs:
+            pol.zero_(), val.zero_()
+        torch.cuda.synchronize()
+        ran.append(set(lzhip_events(lambda: [forward(k, k) for k in range(lanes)] + [pipe.sync()])[0]))
+        for k in range(lanes):
+            assert all(np.array_equal(o.cpu().numpy(), w) for o, w in zip(outs[k], want[k])), (lanes, k)
+    for i in range(len(tiles)):
+        for j in range(i):
+            assert ran[i] and (ran[i] == ran[j]) == (tiles[i] == tiles[j]), (i + 1, j + 1, ran)
+    pipe.close()
