@@ -1386,3 +1386,48 @@ def test_large_tiles_on_one_lane_and_beside_others(pkg, netgen, orc, precision, 
         for j in range(i):
             assert ran[i] and (ran[i] == ran[j]) == (tiles[i] == tiles[j]), (i + 1, j + 1, ran)
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,maxb,sizes", [
+    (128, 17, (1, 16)), (384, 17, (1, 9, 16)), (448, 9, (1, 9)), (512, 8, (1, 8)), (1024, 4, (1, 4)),
+])
+def test_first_layer_kernel_against_packed_planes(pkg, netgen, orc, filters, maxb, sizes):
+    """Direct fp16 networks of all widths: a forward alone convolves the caller's planes in one launch, forwards side by side
+    pack them first, and planes of 0 and 1 from host memory travel as bits.  Same bits from all three, with other values
+    and some beyond the stored range from the first two."""
+    import torch
+    _, pipe, _, _ = make_pipes(pkg, netgen, orc, 1, filters, 7800 + filters, pkg.FP16, maxb)
+    rng = np.random.default_rng(7801)
+    for n in sizes:
+        print("case: first layer, %d filters, %d boards of %d" % (filters, n, maxb), flush=True)
+        stones = netgen.synthetic_inputs(n, seed=7802)
+        other = stones + rng.standard_normal(stones.shape).astype(np.float32) * 0.1
+        other.reshape(n, -1)[:, ::997] = 7e4
+        for x, bits in ((stones, True), (other, False)):
+            d_in = torch.from_numpy(x).cuda()
+            outs = [(torch.zeros(n, 722, device="cuda"), torch.zeros(n, 361, device="cuda")) for _ in range(2)]
+            torch.cuda.synchronize()
+
+            def forwards(lanes):
+                for k, (pol, val) in enumerate(outs[:lanes]):
+                    pipe.forward_batch_device(n, d_in.data_ptr(), pol.data_ptr(), val.data_ptr(), lane=k)
+                pipe.sync()
+
+            got = []
+            for lanes in (1, 2):
+                for _ in range(3):
+                    forwards(lanes)
+                for pol, val in outs:
+                    pol.zero_(), val.zero_()
+                torch.cuda.synchronize()
+                ran = lzhip_events(lambda: forwards(lanes))[0]
+                first = sum("conv3x3_first_k" in e for e in ran)
+                packs = sum("pack_input_k" in e for e in ran)
+                assert (first, packs) == ((1, 0) if lanes == 1 else (0, 2)), (n, lanes, ran)
+                got += [[o.cpu().numpy() for o in outs[k]] for k in range(lanes)]
+            if bits:
+                got.append(pipe.forward_batch(x))
+            for other_way in got[1:]:
+                assert all(np.array_equal(a, b) for a, b in zip(got[0], other_way)), n
+            assert np.isfinite(got[0][0]).all() and np.abs(got[0][0]).max() > 0
+    pipe.close()
