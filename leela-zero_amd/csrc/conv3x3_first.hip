@@ -116,10 +116,13 @@ __global__ __launch_bounds__(kThreads) void conv3x3_first_k(
 
 // Measured per forward of 10 blocks, us, two launches -> this one: 64 filters, 1 board 79 -> 76, 16: 80.3 -> 77.6; 128
 // filters, 1: 73 -> 70, 5: 78.4 -> 75.9, 8: 96.4 -> 94.0, 16: 108.2 -> 105.8; 192 filters, 1: 100.5 -> 97.6, 8: 124.8 ->
-// 122.4, 16: 158.5 -> 156.4; 256 filters, 4: 127.6 -> 123.0, 8: 144.5 -> 141.6, 16: 198.0 -> 195.7; 512, 16: 407 -> 406.
-// Larger batches keep the two launches that their profiles and replays are counted in: what is saved is the
-// same 2 us or less of a longer forward (192 filters, 22 boards 164.6 -> 163.6, 256, 32: 282 -> 280, 64: 480 -> 479),
-// and at 256 filters two forwards of 32 side by side lost by it (229 -> 233).
+// 122.4, 16: 158.5 -> 156.4; 256 filters, 4: 127.6 -> 123.0, 8: 144.5 -> 141.6, 16: 198.0 -> 195.7 (two versions one after
+// the other; timed in turn, 128 filters at 5 boards is 82.0 -> 81.3, within the spread).
+// What is saved is a launch, and what it costs grows with the batch: a tile of 32 points fetches the planes and the filters
+// that launch_conv3x3's share among up to 192 points.  So 256 filters lose from 64 boards on (8 blocks, 367.7 -> 371.3;
+// 128: 672.9 -> 680.4).  The line lies where every width was still measured to gain; between it and that loss a
+// forward alone would gain 2 to 4 us more (64 filters, 64 boards 89.6 -> 86.6; 128, 64: 143.6 -> 141.3; 192, 64: 276.0 ->
+// 273.0; 256, 32: 213.9 -> 211.4) or nothing (384, 17: 248.9 -> 248.3, 44: 516.0 -> 517.8).
 bool conv3x3_first_serves(int Kp, int n) { return Kp % kCols == 0 && n <= 16; }
 
 void launch_conv3x3_first(const float* planes, const half_t* Wf, half_t* Y, const float* bn_scale,
