@@ -125,6 +125,10 @@ static PeakIn peak_in(const PeakMap& p) {
 }
 // The most slots a board may have: it meets 360 / mt + 2 rows of tiles at most.
 static constexpr int peak_slots(int mt, int tiles_n) { return (360 / mt + 2) * tiles_n; }
+// Whether a layer's peaks, two a tile, lie within what conv3x3_f32_slots keeps for them.
+static void slots_fit(int tiles_m, int tiles_n, int Kp, int n) {
+    if (2 * (size_t)tiles_m * tiles_n > conv3x3_f32_slots(Kp, n)) throw std::logic_error("more peaks than slots");
+}
 static void peaks_fit(const PeakMap& p, int loads) {
     if (peak_slots(p.mt, p.tiles_n) > 64 * loads) throw std::logic_error("a board of more peaks than are read");
 }
@@ -476,6 +480,7 @@ static PeakMap launch_f32_as(const float* X, const half_t* Wf, const float* res,
     const ConvGrid g = conv_grid((n * kPts + MT - 1) / MT, Kp / CW, (size_t)36 * Cp * Kp,
                                  (size_t)n * kPts * Cp * 4);
     peaks_fit(peaks, 2);
+    slots_fit(g.tiles_m, Kp / CW, Kp, n);
     launch(conv3x3_f32_k<RB, NB, WR, WN, D, CC, OCC>, dim3(8 * g.share), dim3(64 * WR * WN), s, t, X,
            Wf, res, Y, bn_scale, bn_mean, rfac, peak_in(peaks), slots, n, Cp, Kp, g);
     return {slots, MT, Kp / CW};
@@ -844,6 +849,7 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
     const ConvGrid g = conv_grid((n * kPts + tile.rb * 16 - 1) / (tile.rb * 16), Kp / (16 * tile.nb),
                                  (size_t)36 * Cp * Kp, (size_t)n * kPts * Cp * 4);
     peaks_fit(peaks, split_peak_loads(tile.rb, tile.nb, Kp));
+    slots_fit(g.tiles_m, Kp / (16 * tile.nb), Kp, n);
     auto go = [&](auto kernel, int waves) {
         launch(kernel, dim3(8 * g.share), dim3(64 * waves), s, t, X, Wf, res, Y, bn_scale, bn_mean,
                rfac, peak_in(peaks), slots, n, Kp, g);
@@ -885,8 +891,9 @@ PeakMap launch_conv3x3_f32_split(const float* X, const half_t* Wf, const float* 
     return {slots, tile.rb * 16, Kp / (16 * tile.nb)};
 }
 
-// Tiles of up to 64 points come in grids of at most three work-groups per unit, larger ones have
-// at least 96 points and 64 channels.
+// Two peaks a tile.  Tiles of less than 96x64 points by channels come in grids of at most three work-groups per unit; larger
+// ones are fewer than those of 96x64 would be, by their area (the smallest are 128x64 and 80x128).  Every launch
+// looks that its own fit (slots_fit).
 size_t conv3x3_f32_slots(int Kp, int max_batch) {
     const size_t large = (size_t)(max_batch * kPts / 96 + 1) * (Kp / 64);
     return 2 * (large > 3 * kUnits ? large : 3 * kUnits);
