@@ -1431,3 +1431,33 @@ def test_first_layer_kernel_against_packed_planes(pkg, netgen, orc, filters, max
                 assert all(np.array_equal(a, b) for a, b in zip(got[0], other_way)), n
             assert np.isfinite(got[0][0]).all() and np.abs(got[0][0]).max() > 0
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,maxb,batches", [
+    # sums dealt to the wavefronts: every tile of a handle
+    (64, 45, (5, 6, 8, 9, 11, 12, 22, 23, 34, 35, 45)), (128, 23, (4, 5, 8, 11, 12, 22, 23)),
+    (192, 15, (3, 7, 8, 11, 12, 15)), (256, 11, (2, 5, 6, 8, 11)), (320, 6, (2, 4, 5, 6)), (384, 5, (2, 3, 4, 5)),
+    (512, 4, (2, 3, 4)),
+    # and not: small tiles, steps of 16 points by 128 channels, 160x64, more than a round
+    (64, 182, (22, 35, 68, 91, 137, 182)), (128, 114, (17, 34, 46, 57, 68, 80, 91, 103, 114)),
+    (192, 91, (11, 16, 22, 31, 38, 61, 91)), (256, 70, (8, 12, 17, 23, 29, 35, 40, 46, 52, 57, 70)),
+    (320, 28, (9, 13, 19, 23, 28)), (384, 38, (5, 8, 15, 19, 23, 27, 31, 34, 38)),
+])
+def test_fp32_tiles_give_a_position_the_same_bits(pkg, netgen, orc, filters, maxb, batches):
+    """One layer of an fp32 handle with a skip connection: the first position of every batch, and the last one, whose tile
+    is the ragged one, have the bits that they have alone, whatever tile the batch takes and however large
+    the boards beside them are."""
+    _, pipe, _, _ = make_pipes(pkg, netgen, orc, 1, filters, 7900 + filters, pkg.FP32, maxb)
+    rng = np.random.default_rng(filters + maxb)
+    a = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float32)
+    r = np.abs(rng.standard_normal((maxb, filters, 361))).astype(np.float32)
+    size = 10.0 ** rng.integers(-12, 13, maxb).astype(np.float32)
+    a *= size[:, None, None]
+    r *= size[:, None, None]
+    first = pipe.debug_layer(2, a[:1], r[:1])[2]
+    for n in batches:
+        print("case: fp32 bits, %d filters, %d boards of %d" % (filters, n, maxb), flush=True)
+        got = pipe.debug_layer(2, a[:n], r[:n])[2]
+        last = pipe.debug_layer(2, a[n - 1:n], r[n - 1:n])[2]
+        assert np.array_equal(got[0], first[0]) and np.array_equal(got[n - 1], last[0]), n
+    pipe.close()
