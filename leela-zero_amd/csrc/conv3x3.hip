@@ -525,14 +525,15 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // The order of the sum differs from conv3x3_k's, so a network uses one or the other whatever the
 // batch (conv3x3_splits).
 //
-// PAIRS (192 and 256 filters): the two halves of a chunk are summed apart and then added, which gives the
-// same bits where one wavefront has both halves and where two have one each.  Two take half as long over
-// their steps, their loads and their share of the patch: a forward with the device to itself, 20 blocks of 256
-// filters, 1 board 168 -> 160 us, 2: 193 -> 180, 5: 262 -> 243; of 192, 1 board 147 -> 146, 7: 225 -> 213.  Side by
-// side with other forwards one has both, with the filters of 12 steps ahead instead of all 18, so that a unit
-// holds two work-groups (192 filters, 7 boards, three at once 166 -> 111 us each; 256, 2 boards, two at once
-// 113 -> 107).
-template <int RB, int NB, int KW, int HPW, int D, bool PAIRS>
+// Left out, because they sum in another order than networks of these widths had before, and give other bits: a
+// wavefront for each half of a chunk at 192 and 256 filters, the halves summed apart (8 blocks, us, one forward at a
+// time | two side by side: 192 filters, 7 boards 93.6 -> 90.5 | 111.5 -> 115.2; 256, 1 board 71.1 -> 71.4 | 80.1 -> 81.6, 5:
+// 101.6 -> 103.0 | 120.5 -> 123.1; at 320 and 384 slower: 1 board 75.8 -> 79.0 and 93.3 -> 98.7), and tiles of 80x32 for the handles
+// of 12 to 14 boards of 128 filters, 8 and 9 of 192, 6 and 7 of 256, which are conv3x3_k's (0 to 7 % faster).
+// Side by side with other forwards 192 and 256 filters have the filters of 12 steps ahead instead of all 18, so that
+// a unit holds two work-groups (192 filters, 7 boards, three at once 166 -> 111 us each; 256, 2 boards, two at
+// once 113 -> 107).
+template <int RB, int NB, int KW, int HPW, int D>
 __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
     half_t* __restrict__ Y, const float* __restrict__ bn_scale, const float* __restrict__ bn_mean,
@@ -610,10 +611,10 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const size_t ybytes = (size_t)(n + 2) * kCellsPerBoard * Kp * 2;
     const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
     const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
-    // The order of points and quarters in LDS (CellPitch) where more than four wavefronts' worth of channels is read:
-    // 15x192, 8 boards 177 -> 174.5 us a forward, two side by side 110 -> 106.5; 20x256, two of 1 board 93.6 -> 90.1, of 5
-    // boards 144 -> 141; 10x320, 1 board 94.7 -> 89.9. 64 filters, 1 board, lost by it (110.4 -> 111.5), 128 gained
-    // nothing for one.
+    // The order of points and quarters in LDS (CellPitch) where more than four wavefronts' worth of channels is read (8
+    // blocks, us, one forward at a time | two side by side: 192 filters, 7 boards 95.5 -> 93.6 | 115.4 -> 111.5; 256, 1: 73.5 ->
+    // 71.1 | 81.9 -> 80.1, 5: 105.9 -> 101.6 | 124.2 -> 120.5; 320, 1: 78.5 -> 73.9 | 100.8 -> 97.1). 64 filters, 1 board, lost by
+    // it (110.4 -> 111.5 of 20 blocks), 128 gained nothing for one.
     constexpr bool SPREAD = KW * HPW > 4;
     const int point = SPREAD ? conv_point(lane) : (int)(lane & 15);   // this lane's, of a block of 16
     auto slot = [](unsigned q) { return SPREAD ? quarter_slot(q) : q; };
@@ -647,14 +648,11 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 #pragma unroll
     for (int i = 0; i < RB; i++)
         arow[i] = patch_cell(ps, min(i * 16 + point, rows - 1 - m0)) * STR + slot(lane >> 4) * 16;
-    constexpr int SUMS = PAIRS ? HPW : 1;
-    float4v acc[SUMS][RB][NB];
+    float4v acc[RB][NB];
 #pragma unroll
-    for (int h = 0; h < SUMS; h++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-        for (int i = 0; i < RB; i++)
-#pragma unroll
-            for (int j = 0; j < NB; j++) acc[h][i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < NB; j++) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
     int4v a[DA][RB];
     auto aread = [&](int i, int st) {
@@ -677,9 +675,9 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
                     wload((st + D - 1) % D, j, st + D - 1);
 #pragma unroll
             for (int j = 0; j < NB; j++)
-                acc[st / 9 % SUMS][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                     __builtin_bit_cast(half8v, w[st % D][j]),
-                    __builtin_bit_cast(half8v, a[st % DA][i]), acc[st / 9 % SUMS][i][j], 0, 0, 0);
+                    __builtin_bit_cast(half8v, a[st % DA][i]), acc[i][j], 0, 0, 0);
             if (st + DA < STEPS) a[st % DA][i] = aread(i, st + DA);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -692,7 +690,7 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 #pragma unroll
         for (int j = 0; j < NB; j++)
             *reinterpret_cast<float4v*>(lds + ((wave * RB + i) * NB + j) * 1024 + lane * 16) =
-                SUMS == 2 ? acc[0][i][j] + acc[SUMS - 1][i][j] : acc[0][i][j];
+                acc[i][j];
     lds_barrier();
 #pragma unroll
     for (int q = 0; q < QP; q++) {
@@ -709,14 +707,9 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
         HalfE o;
 #pragma unroll
         for (int e = 0; e < E; e++) {
-            constexpr int STEP = PAIRS && HPW == 1 ? 2 : 1;
-            auto sum = [&](int k) {
-                const float first = part[k][e / 4][e % 4];
-                return STEP == 2 ? first + part[k + STEP - 1][e / 4][e % 4] : first;
-            };
-            float v = sum(0);
+            float v = part[0][e / 4][e % 4];
 #pragma unroll
-            for (int k = STEP; k < KW; k += STEP) v += sum(k);
+            for (int k = 1; k < KW; k++) v += part[k][e / 4][e % 4];
             o[e] = (half_t)fminf(
                 fmaxf(0.0f, fmaf((float)rh[e], rfac, fmaf(v, bn[0][cl + e], bn[1][cl + e]))),
                 kActStoreMax);
@@ -735,17 +728,14 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
 // has to deliver to a work-group, which is what a layer of one board waits for: against 32 x 32
 // tiles 128 filters 3.8 -> 3.3 us, 192 4.4 -> 3.8, 256 4.9 -> 4.3, 320 5.3 -> 4.7.  48 x 16 is worth
 // 2 to 4 % up to 256 filters (192 filters, 2 boards 4.4 -> 4.3 us) and no longer beyond (384
-// filters, 1 board 5.5 -> 5.7).  80 x 32 is as fast as conv3x3_k's tiles or faster at 128 to 256 filters (20 blocks, us:
-// 128 filters, 14 boards 204 -> 195, three side by side 98 -> 93; 192, 9 boards 239 -> 239 and 133 -> 131; 256, 7 boards
-// 271 -> 260 and 162 -> 153), and a handle of that size then takes this kernel for its small batches too (1 board
-// of 128, 192, 256 filters 169 -> 133, 185 -> 147, 208 -> 159).
+// filters, 1 board 5.5 -> 5.7).
 struct SplitTile {
     int rb, nb;
 };
 static SplitTile split_tile(int n, int Kp) {
-    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}, {5, 2}};
+    constexpr SplitTile kTiles[] = {{2, 1}, {3, 1}, {2, 2}, {3, 2}, {4, 2}};
     for (const SplitTile& t : kTiles)
-        if ((t.rb * t.nb != 3 || Kp <= 256) && (t.rb < 5 || (Kp >= 128 && Kp <= 256)) &&
+        if ((t.rb * t.nb != 3 || Kp <= 256) &&
             (n * kPts + t.rb * 16 - 1) / (t.rb * 16) * (Kp / (16 * t.nb)) <= kUnits) return t;
     return {0, 0};
 }
@@ -759,9 +749,7 @@ bool conv3x3_splits(int Kp, int max_batch) {
 void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                           const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
                           int Kp, int lanes, hipStream_t s, LaunchTimer* t) {
-    SplitTile tile = split_tile(n, Kp);
-    // (80x32 of 256 filters takes more than half of the LDS: two work-groups on a unit want less)
-    if (lanes > 1 && Kp == 256 && tile.rb == 5) tile = {4, 2};
+    const SplitTile tile = split_tile(n, Kp);
     if (!conv3x3_splits(Kp, n) || Cp != Kp)
         throw std::invalid_argument("no split convolution for this width or batch");
     const ConvGrid g = conv_grid((n * kPts + tile.rb * 16 - 1) / (tile.rb * 16), Kp / (16 * tile.nb),
@@ -771,33 +759,29 @@ void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, 
                bn_mean, rfac, n, Kp, g);
     };
     // KW wavefronts x HPW halves of a chunk
-#define LZ_SPLIT(KW, HPW, D, PAIRS)                                                      \
-    if (tile.nb == 1) {                                                                  \
-        if (tile.rb == 2) go(conv3x3_split_k<2, 1, KW, HPW, D, PAIRS>, KW);              \
-        else if constexpr (KW * HPW <= 8) go(conv3x3_split_k<3, 1, KW, HPW, D, PAIRS>, KW); \
-    } else if (tile.rb == 2) go(conv3x3_split_k<2, 2, KW, HPW, D, PAIRS>, KW);           \
-    else if (tile.rb == 3) go(conv3x3_split_k<3, 2, KW, HPW, D, PAIRS>, KW);             \
-    else if (tile.rb == 4) {                                                             \
-        if constexpr (KW * HPW < 16) go(conv3x3_split_k<4, 2, KW, HPW, D, PAIRS>, KW);   \
-    } else if constexpr (KW * HPW <= 8 && KW >= 3) {                                     \
-        go(conv3x3_split_k<5, 2, KW, HPW, 9, PAIRS>, KW);                                \
-    }
+#define LZ_SPLIT(KW, HPW, D)                                               \
+    if (tile.nb == 1) {                                                    \
+        if (tile.rb == 2) go(conv3x3_split_k<2, 1, KW, HPW, D>, KW);       \
+        else if constexpr (KW < 5) go(conv3x3_split_k<3, 1, KW, HPW, D>, KW); \
+    } else if (tile.rb == 2) go(conv3x3_split_k<2, 2, KW, HPW, D>, KW);    \
+    else if (tile.rb == 3) go(conv3x3_split_k<3, 2, KW, HPW, D>, KW);      \
+    else if constexpr (KW < 8) go(conv3x3_split_k<4, 2, KW, HPW, D>, KW)
     switch (Kp) {
-        case 64: LZ_SPLIT(2, 1, 9, false); break;
-        case 128: LZ_SPLIT(4, 1, 9, false); break;
+        case 64: LZ_SPLIT(2, 1, 9); break;
+        case 128: LZ_SPLIT(4, 1, 9); break;
         case 192:
-            if (lanes == 1) { LZ_SPLIT(6, 1, 9, true); }
-            else { LZ_SPLIT(3, 2, 12, true); }
+            if (lanes == 1) { LZ_SPLIT(3, 2, 18); }
+            else { LZ_SPLIT(3, 2, 12); }
             break;
         case 256:
-            if (lanes == 1) { LZ_SPLIT(8, 1, 9, true); }
-            else { LZ_SPLIT(4, 2, 12, true); }
+            if (lanes == 1) { LZ_SPLIT(4, 2, 18); }
+            else { LZ_SPLIT(4, 2, 12); }
             break;
-        // from here on two wavefronts share a SIMD's registers: two thirds of the filters ahead
-        case 320: LZ_SPLIT(5, 2, 12, false); break;
-        case 384: LZ_SPLIT(6, 2, 12, false); break;
-        case 448: LZ_SPLIT(7, 2, 12, false); break;
-        default: LZ_SPLIT(8, 2, 12, false); break;   // (the largest is for 3 boards, which no longer fit)
+        // five wavefronts and more share the SIMDs' registers: two thirds of the filters ahead
+        case 320: LZ_SPLIT(5, 2, 12); break;
+        case 384: LZ_SPLIT(6, 2, 12); break;
+        case 448: LZ_SPLIT(7, 2, 12); break;
+        default: LZ_SPLIT(8, 2, 12); break;   // (the largest is for 3 boards, which no longer fit)
     }
 #undef LZ_SPLIT
 }

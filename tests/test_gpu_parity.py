@@ -1461,3 +1461,43 @@ def test_fp32_tiles_give_a_position_the_same_bits(pkg, netgen, orc, filters, max
         last = pipe.debug_layer(2, a[n - 1:n], r[n - 1:n])[2]
         assert np.array_equal(got[0], first[0]) and np.array_equal(got[n - 1], last[0]), n
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,batches", [(192, (1, 3, 7)), (256, (1, 2, 5))])
+def test_sum_of_64_channels_is_one_chain(pkg, netgen, orc, filters, batches):
+    """fp16 layers of 192 and 256 filters, handles that deal their sums: 64 input channels are summed one k-step after
+    the other, by whichever wavefronts, so that a network's outputs stay what they are.  Channels 0 to 31 bring 1.5 * 2^24,
+    where fp32 has steps of 2; channels 32 to 63 then bring 0.5 in each of nine steps, which is lost nine times (summed
+    apart they would be 4); the next 64 channels take the first sum away."""
+    net = netgen.make_network(1, filters, 8000 + filters)
+    w2 = np.zeros_like(net.conv_w[2])
+    w2[:, 0, 1, 1], w2[:, 64, 1, 1] = 4096.0, -4096.0
+    w2[:, 32] = 0.5
+    net.conv_w[2] = w2
+    net.bn_mean[2][:], net.bn_var[2][:] = -1.0, 1.0
+    w, _ = netgen.prepare(net)
+    pipe = pkg.HIPScheduler(pkg.FP16, max(batches))
+    pipe.initialize(filters)
+    pipe.push_weights(6, 18, filters, w)
+    for n in batches:
+        print("case: one chain, %d filters, %d boards" % (filters, n), flush=True)
+        a = np.zeros((n, filters, 361), np.float32)
+        a[:, 0], a[:, 64], a[:, 32] = 6144.0, 6144.0, 1.0
+        got = pipe.debug_layer(2, a, np.zeros_like(a))[2].reshape(n, filters, 19, 19)[:, :, 1:18, 1:18]
+        assert np.abs(got - 1.0).max() <= 2.0 ** -10, (n, got.min(), got.max())
+    pipe.close()
+
+
+@pytest.mark.parametrize("filters,handles", [(128, (12, 14)), (192, (8, 9)), (256, (6, 7))])
+def test_handles_past_the_dealt_sums_have_the_bits_of_large_ones(pkg, netgen, orc, filters, handles):
+    """fp16 handles whose largest batch is just past 64 points x 32 channels on every unit give the bits of a handle of 32."""
+    print("case: handles of %s, %d filters" % (handles, filters), flush=True)
+    x = netgen.synthetic_inputs(max(handles), seed=8101)
+    _, large, _, _ = make_pipes(pkg, netgen, orc, 2, filters, 8100, pkg.FP16, 32)
+    for maxb in handles:
+        _, pipe, _, _ = make_pipes(pkg, netgen, orc, 2, filters, 8100, pkg.FP16, maxb)
+        for n in (1, maxb):
+            want, got = large.forward_batch(x[:n]), pipe.forward_batch(x[:n])
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), (maxb, n)
+        pipe.close()
+    large.close()
