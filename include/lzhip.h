@@ -251,7 +251,10 @@ int lzhip_get_act_scales(lzhip_handle* h, float* out, int n);
 
 /* One forward of n device-resident positions with every kernel launch timed
  * individually by the device's own begin/end timestamps.  ms[LZHIP_K_COUNT]
- * receives the summed duration per class, launches[...] the launch counts. */
+ * receives the summed duration per class, launches[...] the launch counts.
+ * Packing and the first layer are always launches of their own here, as in forwards
+ * beside others; a direct fp16 forward of up to 16 positions that has the device to
+ * itself does both in one launch, which is of neither class (the same results). */
 int lzhip_profile_forward(lzhip_handle* h, int n, const void* d_in, void* d_pol, void* d_val,
                           float* ms, int* launches);
 

@@ -452,7 +452,8 @@ class HIPScheduler:
         return lib().lzhip_stream(self._h)
 
     def profile_forward(self, n, d_in, d_pol, d_val):
-        """Per-kernel-class device time (ms) and launch counts of one forward."""
+        """Per-kernel-class device time (ms) and launch counts of one forward, packing and the first layer
+        as launches of their own (a forward of up to 16 positions alone has one for both in fp16)."""
         self._need()
         ms = np.zeros(K_COUNT, dtype=np.float32)
         cnt = (ctypes.c_int * K_COUNT)()

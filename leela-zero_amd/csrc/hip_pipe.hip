@@ -1163,8 +1163,8 @@ private:
         const int nl = (int)m_layers.size();
         const int Tu = n * kTilesPerBoard;
         if constexpr (sizeof(P) == 2) {
-            // (Forwards side by side replay their layers as one launch, from the lane's own planes.  A timed
-            // pass tells packing and convolutions apart.)
+            // (Forwards side by side replay their layers as one launch, from the lane's own planes.  A timed pass
+            // reports packing and every convolution as launches of their own, whatever the batch.)
             if (m_direct && d_in && !timed && w.lanes == 1 && conv3x3_first_serves(m_Fp, n)) {
                 const Layer& L = m_layers[0];
                 launch_conv3x3_first(d_in, L.W3.p, w.act[0], L.d_scale.p, L.d_mean.p, n, m_C0p, m_Fp, w.stream,
