@@ -375,10 +375,10 @@ bool conv3x3_serves(int Kp, int max_batch, int elem_bytes) {
 //   64 boards   32.0*   29.2*   26.4*   25.1*   28.5*   24.1
 //   80 boards   40.1*   35.6*   32.2*   33.1*   30.2*   37.6*
 //  128 boards   61.0*   54.2*   47.6*   45.6*   44.9*   42.9*
-// (128x128 with its wavefronts two by two; side by side, as it is now, 40 boards take 16.7.)  Two chains side by
-// side want larger tiles (us per layer and chain): 20 boards 128x64 8.5, 192x64
-// 8.9, 96x64 9.6; 40 boards 192x64 13.3, 128x64 14.3, 192x128 14.8; 64 boards 192x128 19.1,
-// 192x64 20.2; 80 boards 192x128 23.7, 128x128 25.3.  At other widths the order is the same: 128 filters, 44
+// (128x128 with its wavefronts two by two, a kernel that is gone; side by side, as they are now, 40 boards take
+// 16.7.)  Two chains side by side want larger tiles (us per layer and chain): 20 boards 128x64 8.5, 192x64 8.9, 96x64
+// 9.6; 40 boards 192x64 13.3, 128x64 14.3, 192x128 14.8; 64 boards 192x128 19.1, 192x64 20.2; 80 boards 192x128
+// 23.7.  At other widths the order is the same: 128 filters, 44
 // boards 48x64 7.9, 128x64 6.7 (two chains 5.9 | 4.9);
 // 384 filters, 13 boards 192x64 16.8, 128x64 13.7 (13.4 | 12.0).  64 and 192 filters have no tile of 128
 // channels; there 128x64 is taken up to two work-groups

@@ -487,10 +487,9 @@ static PeakMap launch_f32_as(const float* X, const half_t* Wf, const float* res,
 }
 
 // The tiles and their order are conv3x3_k's (launch_conv3x3).  Measured, us per layer of a chain (two chains
-// side by side, per chain): 256 filters, 20 boards 192x64 31.8, 128x64 24.5 (21.9 | 20.2), 40 boards 192x128
-// 50.5, 128x128 42.2 (37.8 | 36.6); 192 filters, 28 boards 192x64 25.1, 128x64 19.7 (30 boards 19.5 | 17.3), 46 boards
-// 128x192 40.0, 128x64 32.4 (28.1 | 25.3); 384 filters, 13 boards 192x64 44.7, 128x64 33.5 (32.1 | 29.1), 26 boards
-// 192x128 72.0, 128x128 58.7.
+// side by side, per chain): 256 filters, 20 boards 192x64 31.8, 128x64 24.5 (21.9 | 20.2); 192 filters, 28 boards
+// 192x64 25.1, 128x64 19.7 (30 boards 19.5 | 17.3), 46 boards 128x192 40.0, 128x64 32.4 (28.1 | 25.3); 384 filters, 13
+// boards 192x64 44.7, 128x64 33.5 (32.1 | 29.1).
 PeakMap launch_conv3x3_f32(const float* X, const half_t* Wf, const float* res, float* Y,
                            const float* bn_scale, const float* bn_mean, float rfac,
                            const PeakMap& peaks, uint32_t* slots, int n, int Cp, int Kp,
@@ -801,6 +800,9 @@ __global__ __launch_bounds__(64 * KW * WR * WN, 1) void conv3x3_f32_split_k(
             o[e] = fmaxf(0.0f, fmaf(r[e], rfac, fmaf(v * unscale, bn[0][c + e], bn[1][c + e])));
             top = fmaxf(top, finite(o[e]));
         }
+        // (Through the cache, unlike the other convolutions: tiles of 16 channels, half a cache line each, are slower
+        // written through, 8 blocks of 128 filters, 1 board 92.2 -> 95.0 us, of 256 115.7 -> 117.4; those of 64 channels
+        // would be 1 to 2 % faster, 22 boards of 128 filters 165.3 -> 162.2, 11 of 256 243.6 -> 240.8.)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, o), rY, ro[q], 0, 0);
         top0 = fmaxf(top0, m < m1 ? top : 0.0f);
         top1 = fmaxf(top1, m >= m1 && m < rows ? top : 0.0f);

@@ -65,8 +65,8 @@ __device__ __forceinline__ unsigned patch_cell(const PatchStart& s, unsigned loc
 // Counted in a loop of reads: 4 cycles each; 8 with the pieces and points in their natural order, 12
 // where 16 points end a board row.  It shows where 192x64 tiles load the LDS most: 20x256 batch 32 640 ->
 // 614 us a forward, two side by side 979 -> 924; 16 boards 830 -> 820 of 40 blocks, the others within 1 %.
-// The fp32 kernels and conv3x3_split_k have the order of points and quarters (quarter_slot) without the longer
-// rows, which cost them addresses (10x128 fp16 batch 5 84 -> 93, 10x256 fp32 batch 64 1280 -> 1292).
+// The fp32 kernels, and conv3x3_split_k from 192 filters on, have the order of points and quarters (quarter_slot)
+// without the longer rows, which cost them addresses (10x128 fp16 batch 5 84 -> 93, 10x256 fp32 batch 64 1280 -> 1292).
 template <int STR>
 struct CellPitch {
     static_assert(STR % 32 == 16, "an odd number of slots");
