@@ -525,14 +525,14 @@ void launch_conv3x3(const half_t* X, const half_t* Wf, const half_t* res, half_t
 // The order of the sum differs from conv3x3_k's, so a network uses one or the other whatever the
 // batch (conv3x3_splits).
 //
-// Left out, because they sum in another order than networks of these widths had before, and give other bits: a
-// wavefront for each half of a chunk at 192 and 256 filters, the halves summed apart (8 blocks, us, one forward at a
-// time | two side by side: 192 filters, 7 boards 93.6 -> 90.5 | 111.5 -> 115.2; 256, 1 board 71.1 -> 71.4 | 80.1 -> 81.6, 5:
-// 101.6 -> 103.0 | 120.5 -> 123.1; at 320 and 384 slower: 1 board 75.8 -> 79.0 and 93.3 -> 98.7), and tiles of 80x32 for the handles
-// of 12 to 14 boards of 128 filters, 8 and 9 of 192, 6 and 7 of 256, which are conv3x3_k's (0 to 7 % faster).
-// Side by side with other forwards 192 and 256 filters have the filters of 12 steps ahead instead of all 18, so that
-// a unit holds two work-groups (192 filters, 7 boards, three at once 166 -> 111 us each; 256, 2 boards, two at
-// once 113 -> 107).
+// From 192 filters on a wavefront has the filters of 12 of its 18 steps ahead: with all of them a unit holds one
+// work-group of 192 or 256 filters, and a forward alone waits longer for its first ones too (8 blocks, us, one at a time |
+// two side by side, 18 -> 12: 192 filters, 1 board 58.8 -> 57.3, 7: 91.9 -> 87.3 | 138 -> 112; 256, 1: 66.0 -> 63.2, 5:
+// 101.4 -> 96.7; three side by side, 192 filters, 7 boards 203 -> 140).
+// Left out: a wavefront for each half of a chunk at 192 and 256 filters, the halves summed apart, which gives other bits
+// and is slower (192 filters, 7 boards 87.9 | 115.1; 256, 1: 64.9 | 81.5, 5: 102.5 | 125.0; at 320 and 384 too, 1 board
+// 75.8 -> 79.0 and 93.3 -> 98.7); and tiles of 80x32 for the handles of 12 to 14 boards of 128 filters, 8 and 9 of 192, 6
+// and 7 of 256, which are conv3x3_k's and would get other bits (0 to 7 % faster).
 template <int RB, int NB, int KW, int HPW, int D>
 __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const half_t* __restrict__ X, const half_t* __restrict__ Wf, const half_t* __restrict__ res,
@@ -612,9 +612,9 @@ __global__ __launch_bounds__(64 * KW, 1) void conv3x3_split_k(
     const __amdgpu_buffer_rsrc_t rY = make_rsrc(Y, ybytes);
     const __amdgpu_buffer_rsrc_t rR = make_rsrc(res != nullptr ? res : Y, ybytes);
     // The order of points and quarters in LDS (CellPitch) where more than four wavefronts' worth of channels is read (8
-    // blocks, us, one forward at a time | two side by side: 192 filters, 7 boards 95.5 -> 93.6 | 115.4 -> 111.5; 256, 1: 73.5 ->
-    // 71.1 | 81.9 -> 80.1, 5: 105.9 -> 101.6 | 124.2 -> 120.5; 320, 1: 78.5 -> 73.9 | 100.8 -> 97.1). 64 filters, 1 board, lost by
-    // it (110.4 -> 111.5 of 20 blocks), 128 gained nothing for one.
+    // blocks, us: 320 filters, 1 board 78.5 -> 73.9, 384, 3: 119.5 -> 116.2; two side by side: 192 filters, 7 boards 115.4 ->
+    // 111.5; 256, 1: 81.9 -> 80.1, 5: 124.2 -> 120.5). 64 filters, 1 board, lost by it (20 blocks 110.4 -> 111.5), 128 gained
+    // nothing for one.
     constexpr bool SPREAD = KW * HPW > 4;
     const int point = SPREAD ? conv_point(lane) : (int)(lane & 15);   // this lane's, of a block of 16
     auto slot = [](unsigned q) { return SPREAD ? quarter_slot(q) : q; };
@@ -748,7 +748,7 @@ bool conv3x3_splits(int Kp, int max_batch) {
 
 void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, half_t* Y,
                           const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
-                          int Kp, int lanes, hipStream_t s, LaunchTimer* t) {
+                          int Kp, hipStream_t s, LaunchTimer* t) {
     const SplitTile tile = split_tile(n, Kp);
     if (!conv3x3_splits(Kp, n) || Cp != Kp)
         throw std::invalid_argument("no split convolution for this width or batch");
@@ -769,15 +769,9 @@ void launch_conv3x3_split(const half_t* X, const half_t* Wf, const half_t* res, 
     switch (Kp) {
         case 64: LZ_SPLIT(2, 1, 9); break;
         case 128: LZ_SPLIT(4, 1, 9); break;
-        case 192:
-            if (lanes == 1) { LZ_SPLIT(3, 2, 18); }
-            else { LZ_SPLIT(3, 2, 12); }
-            break;
-        case 256:
-            if (lanes == 1) { LZ_SPLIT(4, 2, 18); }
-            else { LZ_SPLIT(4, 2, 12); }
-            break;
-        // five wavefronts and more share the SIMDs' registers: two thirds of the filters ahead
+        // (from here on two thirds of the filters ahead)
+        case 192: LZ_SPLIT(3, 2, 12); break;
+        case 256: LZ_SPLIT(4, 2, 12); break;
         case 320: LZ_SPLIT(5, 2, 12); break;
         case 384: LZ_SPLIT(6, 2, 12); break;
         case 448: LZ_SPLIT(7, 2, 12); break;

@@ -564,8 +564,7 @@ public:
     // positions, with the device to itself: 83, now 71 to 75).  Nothing else has to start at
     // zero: every element a kernel reads for a real tile is written earlier in the same call (rows
     // of V past the last tile feed only rows of M that no kernel reads).
-    // Calls wait for one another, so each takes the tiles of a forward alone (8 blocks of 256 fp16 filters, a handle
-    // of 7 positions: 6 positions 134 us with the tiles of two lanes, 111 so; 7: 135, 111).
+    // Calls wait for one another, so each takes the kernels of a forward alone.
     void forward_device_static(int n, const float* d_in, float* d_pol, float* d_val) override {
         Lane& ln = m_lane[0];
         std::lock_guard<std::mutex> lk(ln.mu);
@@ -1238,7 +1237,7 @@ private:
         if constexpr (sizeof(P) == 2) {
             const bool split = L.Cp == m_Fp && conv3x3_splits(m_Fp, m_max_batch);
             if (split)
-                launch_conv3x3_split(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, lanes, s, t);
+                launch_conv3x3_split(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, s, t);
             else
                 launch_conv3x3(in, L.W3.p, res, out, scale, mean, rfac, n, L.Cp, m_Fp, lanes, s, t);
         } else {

@@ -126,7 +126,7 @@ void launch_conv3x3(const _Float16* X, const _Float16* Wf, const _Float16* res, 
 bool conv3x3_splits(int Kp, int max_batch);
 void launch_conv3x3_split(const _Float16* X, const _Float16* Wf, const _Float16* res, _Float16* Y,
                           const float* bn_scale, const float* bn_mean, float rfac, int n, int Cp,
-                          int Kp, int lanes, hipStream_t s, LaunchTimer* t);
+                          int Kp, hipStream_t s, LaunchTimer* t);
 // Filters of one layer from U [36][C][F] fp32 on the device; *bad (device) is set if U is not
 // the Winograd transform of 3x3 filters.
 void conv3x3_filters(const float* U, _Float16* Wf, int C, int F, int Kp, int* bad, hipStream_t s);
