@@ -143,6 +143,9 @@ constexpr int kUnits = 256;   // compute units
 // Tiles of 128 channels, 16 rb points high, of a layer of `rows` points and `cols` such columns: the
 // lowest from `lowest` to 10 blocks that makes no more than one work-group per unit (0: none does), and the
 // one that takes the least rounds times tile (12 is the tile of 192x128, which wins where several take the same).
+// 80x128, of which that can be three rounds or more, reads most and is in it for 128 filters only, where a layer has
+// two chunks (4 blocks, us, 80x128 and the next: 128 filters, 162 boards 153.2, 155.8; 256, 81 boards 252.7, 245.6, 137:
+// 413.3, 395.4; 384, 53 boards 340.0, 332.3, fp32 953, 909).
 static inline int one_round_blocks(int rows, int cols, int lowest) {
     for (int rb = lowest; rb <= 10; rb++)
         if ((rows + rb * 16 - 1) / (rb * 16) * cols <= kUnits) return rb;
@@ -150,7 +153,7 @@ static inline int one_round_blocks(int rows, int cols, int lowest) {
 }
 static inline int least_rounds_blocks(int rows, int cols) {
     int best = 12, least = 0;
-    for (int rb = 12; rb >= 5; rb--) {
+    for (int rb = 12; rb >= (cols == 1 ? 5 : 6); rb--) {
         const int work = ((rows + rb * 16 - 1) / (rb * 16) * cols + kUnits - 1) / kUnits * rb;
         if (rb != 11 && (least == 0 || work < least)) {
             best = rb;

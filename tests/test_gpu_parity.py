@@ -1501,3 +1501,27 @@ def test_handles_past_the_dealt_sums_have_the_bits_of_large_ones(pkg, netgen, or
             assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), (maxb, n)
         pipe.close()
     large.close()
+
+
+@pytest.mark.parametrize("precision,filters,n,like", [(1, 384, 53, 59), (0, 384, 53, 59), (1, 256, 81, 89)])
+def test_no_third_round_of_the_smallest_tiles(pkg, netgen, orc, precision, filters, n, like):
+    """Three rounds of 80x128 points by channels are slower than two of 128x128, which a forward of a few boards more takes."""
+    import torch
+    print("case: rounds, %d filters, %d and %d boards, precision %d" % (filters, n, like, precision), flush=True)
+    _, pipe, _, _ = make_pipes(pkg, netgen, orc, 1, filters, 8200, precision, like)
+    d_in = torch.from_numpy(netgen.synthetic_inputs(like, seed=8201)).cuda()
+    outs = {b: (torch.zeros(b, 722, device="cuda"), torch.zeros(b, 361, device="cuda")) for b in (n, like)}
+    torch.cuda.synchronize()
+
+    def forward(b):
+        pipe.forward_batch_device(b, d_in.data_ptr(), outs[b][0].data_ptr(), outs[b][1].data_ptr())
+        pipe.sync()
+
+    ran = {}
+    for b in outs:
+        forward(b)
+        ran[b] = set(lzhip_events(lambda: forward(b))[0])
+    assert ran[n] and ran[n] == ran[like], ran
+    for a, b in zip(outs[n], outs[like]):
+        assert np.array_equal(a.cpu().numpy(), b.cpu().numpy()[:n])
+    pipe.close()
