@@ -143,9 +143,10 @@ constexpr int kUnits = 256;   // compute units
 // Tiles of 128 channels, 16 rb points high, of a layer of `rows` points and `cols` such columns: the
 // lowest from `lowest` to 10 blocks that makes no more than one work-group per unit (0: none does), and the
 // one that takes the least rounds times tile (12 is the tile of 192x128, which wins where several take the same).
-// 80x128, of which that can be three rounds or more, reads most and is in it for 128 filters only, where a layer has
-// two chunks (4 blocks, us, 80x128 and the next: 128 filters, 162 boards 153.2, 155.8; 256, 81 boards 252.7, 245.6, 137:
-// 413.3, 395.4; 384, 53 boards 340.0, 332.3, fp32 953, 909).
+// A tile costs as much as two blocks of points more than it has: by its blocks alone three rounds of 80x128 would
+// beat two of 128x128, and five of 112x128 three of 192x128, and do not (4 blocks, us: 256 filters, 81 boards 252.7 on 80x128,
+// 245.6 on 128x128, 137: 413.3, 395.4 on 144x128; 384, 53: 340.0, 332.3 on 128x128, fp32 953, 909; 122: 768 on 112x128, 735 on
+// 192x128).  Over 80 batches of 128 to 384 filters, the tile so chosen is 0.3 % from the best one, by the blocks alone 0.6.
 static inline int one_round_blocks(int rows, int cols, int lowest) {
     for (int rb = lowest; rb <= 10; rb++)
         if ((rows + rb * 16 - 1) / (rb * 16) * cols <= kUnits) return rb;
@@ -153,8 +154,8 @@ static inline int one_round_blocks(int rows, int cols, int lowest) {
 }
 static inline int least_rounds_blocks(int rows, int cols) {
     int best = 12, least = 0;
-    for (int rb = 12; rb >= (cols == 1 ? 5 : 6); rb--) {
-        const int work = ((rows + rb * 16 - 1) / (rb * 16) * cols + kUnits - 1) / kUnits * rb;
+    for (int rb = 12; rb >= 5; rb--) {
+        const int rounds = ((rows + rb * 16 - 1) / (rb * 16) * cols + kUnits - 1) / kUnits, work = rounds * (rb + 2);
         if (rb != 11 && (least == 0 || work < least)) {
             best = rb;
             least = work;

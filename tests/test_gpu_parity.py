@@ -1525,3 +1525,9 @@ def test_no_third_round_of_the_smallest_tiles(pkg, netgen, orc, precision, filte
     for a, b in zip(outs[n], outs[like]):
         assert np.array_equal(a.cpu().numpy(), b.cpu().numpy()[:n])
     pipe.close()
+
+
+@pytest.mark.parametrize("filters,n,like", [(384, 38, 122), (256, 57, 187)])
+def test_no_more_rounds_of_smaller_tiles(pkg, netgen, orc, filters, n, like):
+    """Five rounds of 112x128 or seven of 80x128 are slower than three of 192x128, the tile of a full round."""
+    test_no_third_round_of_the_smallest_tiles(pkg, netgen, orc, pkg.FP16, filters, n, like)
